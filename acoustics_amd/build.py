@@ -22,6 +22,8 @@ ARCH = os.environ.get("FDTD_OFFLOAD_ARCH", "gfx950")
 # (source, compiled as HIP device code?)
 SOURCES = [
     ("kernels.hip", True),
+    ("resident.hip", True),
+    ("resident_plan.cpp", True),
     ("device_scene.cpp", True),
     ("solver.cpp", True),
     ("batch.cpp", True),

@@ -32,7 +32,7 @@ fdtd_status BatchRunner::rebuild(hipStream_t st)
         const int id = (int)devs.size();
         devs.push_back(scenes[i]->dev);
         const size_t before = tiles.size();
-        scenes[i]->append_tiles(id, tile_plan(plan), tiles, terms);
+        if (!res[i]) scenes[i]->append_tiles(id, tile_plan(plan), tiles, terms);
         slot_tiles[i] = tiles.size() - before;
         if (scenes[i]->needs_motion_kernel()) motion.push_back({id});
         members.push_back((int)i);
@@ -40,6 +40,10 @@ fdtd_status BatchRunner::rebuild(hipStream_t st)
     prog_tiles = tiles.size();
     dead_tiles = 0;
     if (devs.empty()) { prog.release(); return FDTD_OK; }
+    if (!res_listed) {
+        const fdtd_status s = list_resident(st);
+        if (s != FDTD_OK) return s;
+    }
     const bool fused = tile_plan(plan).fused;
     size_t npre = motion.size();
     for (const SceneDev &d : devs) npre += d.n_spk ? 1 : 0;
@@ -66,6 +70,64 @@ fdtd_status BatchRunner::rebuild(hipStream_t st)
     if (s != FDTD_OK) return s;
     FDTD_HIP_TRY(hipEventRecord(pdone[b], st));
     return FDTD_OK;
+}
+
+bool BatchRunner::all_resident() const
+{
+    for (size_t i = 0; i < scenes.size(); ++i)
+        if (scenes[i] && !res[i]) return false;
+    return true;
+}
+
+// A finished scene's workgroups return at once on its device clock, so the
+// launches keep their lists until a scene leaves the resident set.
+fdtd_status BatchRunner::list_resident(hipStream_t st)
+{
+    for (int shape = 0; shape < RES_SHAPES; ++shape) {
+        std::vector<const ResidentScene *> list;
+        for (size_t i = 0; i < scenes.size(); ++i)
+            if (scenes[i] && res[i] && res[i]->plan.shape == shape) list.push_back(res[i].get());
+        const fdtd_status s = res_prog[shape].upload(list, st);
+        if (s != FDTD_OK) return s;
+    }
+    res_listed = true;
+    return FDTD_OK;
+}
+
+fdtd_status BatchRunner::settle(hipStream_t st)
+{
+    FDTD_HIP_TRY(hipStreamSynchronize(st));
+    bool gave_up = false;
+    for (const ResidentProgram &p : res_prog) {
+        if (p.trouble && *p.trouble > 1) { set_last_error("a resident launch lost its neighbours"); return FDTD_ERR_DEVICE; }
+        gave_up = gave_up || p.gave_up();
+    }
+    if (!gave_up) return FDTD_OK;
+    for (size_t i = 0; i < scenes.size(); ++i) {
+        if (!scenes[i] || !res[i]) continue;
+        DeviceScene &D = *scenes[i];
+        long long at = 0;
+        fdtd_status s = resident_reopen(D.dev, &at);
+        if (s != FDTD_OK) return s;
+        const long long due = std::min<long long>(taken, D.target);
+        if (at >= due) continue;
+        // the steps it lacks, and from now on all of its steps, by the step kernels
+        std::vector<TileDesc> tiles;
+        std::vector<TermRef> terms;
+        D.append_tiles(0, tile_plan(default_tile_plan(D.S)), tiles, terms);
+        StepProgram own;
+        s = own.upload({D.dev}, tiles, terms, st, tile_plan(default_tile_plan(D.S)).fused);
+        if (s == FDTD_OK) s = own.enqueue(st, at, (int)(due - at));
+        FDTD_HIP_TRY(hipStreamSynchronize(st));
+        own.release();
+        if (s != FDTD_OK) return s;
+        res[i]->release();
+        res[i].reset();
+    }
+    for (ResidentProgram &p : res_prog)
+        if (p.trouble) *p.trouble = 0;
+    res_listed = false;
+    return rebuild(st);
 }
 
 void BatchRunner::drop_graph()
@@ -173,7 +235,23 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
             if (s != FDTD_OK) return s;
         }
         const int want = (int)std::min<long long>(left, remaining);
-        if (graph_steps > 0 && want >= graph_steps) {
+        if (any_resident()) {
+            // the step kernels of the other scenes, then the block of the
+            // resident ones, then every scene's clock
+            const int blk = std::min(want, (int)AMP_ROWS);
+            for (int k = 0; k < blk && prog_tiles > 0; ++k) {
+                const fdtd_status s = prog.enqueue_step(st, taken + k, k);
+                if (s != FDTD_OK) return s;
+            }
+            for (ResidentProgram &p : res_prog) {
+                const fdtd_status s = p.enqueue(st, blk);
+                if (s != FDTD_OK) return s;
+            }
+            FDTD_HIP_TRY(launch_advance(prog.d_scenes, prog.nscenes, blk, st));
+            taken += blk;
+            left -= blk;
+            ++blocks;
+        } else if (graph_steps > 0 && want >= graph_steps) {
             if (!exec) {
                 fdtd_status s = build_graph(st);
                 if (s != FDTD_OK) return s;
@@ -257,7 +335,8 @@ fdtd_status run_time_chunks(const fdtd_scene &scene, int64_t num_steps, const fd
         if (!any) break;
         st = R.advance(b->stream, block);
         if (st != FDTD_OK) break;
-        if (hipStreamSynchronize(b->stream) != hipSuccess) { set_last_error("stream synchronize failed"); st = FDTD_ERR_DEVICE; break; }
+        st = R.settle(b->stream);
+        if (st != FDTD_OK) break;
         for (int c = 0; c < K && st == FDTD_OK; ++c) {
             Monitor &m = mon[c];
             if (!m.live) continue;
@@ -332,11 +411,16 @@ static fdtd_status batch_fill(fdtd_batch *b, const fdtd_scene *scenes, const int
         }
         st = ds->allocate_and_upload(b->stream, std::max(1, num_steps[i]), num_steps[i]);
         if (st != FDTD_OK) { ds->release(); return st; }
+        // a tile plan that the caller asked for is what runs
+        auto rs = std::make_unique<ResidentScene>();
+        const bool resident = !(opt.tile_config >= 0 && opt.tile_config < kNumTilePlans) && rs->build(*ds, b->stream);
+        R.res.push_back(resident ? std::move(rs) : nullptr);
         R.scenes.push_back(std::move(ds));
         R.targets.push_back(num_steps[i]);
         R.done.push_back(num_steps[i] == 0);
     }
     if (opt.tile_config >= 0 && opt.tile_config < kNumTilePlans) { R.plan = opt.tile_config; return R.rebuild(b->stream); }
+    if (R.all_resident()) return R.rebuild(b->stream);   // no step kernel to tune
     return R.autotune(b->stream);
 }
 
@@ -378,7 +462,8 @@ fdtd_status fdtd_batch_run(fdtd_batch *b)
     for (long long t : b->R.targets) mx = std::max(mx, t);
     fdtd_status st = fdtd_batch_step(b, (int)std::max<long long>(0, mx - b->R.taken));
     if (st != FDTD_OK) return st;
-    FDTD_HIP_TRY(hipStreamSynchronize(b->stream));
+    const fdtd_status s = b->R.settle(b->stream);
+    if (s != FDTD_OK) return s;
     b->R.reap();
     return FDTD_OK;
 }
@@ -393,7 +478,8 @@ fdtd_status fdtd_batch_steps_done(fdtd_batch *b, int scene, int64_t *steps)
 fdtd_status fdtd_batch_read_listener_series(fdtd_batch *b, int scene, double *out)
 {
     if (!b || scene < 0 || scene >= (int)b->R.scenes.size()) return FDTD_ERR_INVALID;
-    FDTD_HIP_TRY(hipStreamSynchronize(b->stream));
+    const fdtd_status s = b->R.settle(b->stream);
+    if (s != FDTD_OK) return s;
     b->R.reap();
     const DeviceScene &D = *b->R.scenes[scene];
     const long long rows = std::min<long long>(b->R.taken, b->R.targets[scene]);
@@ -457,6 +543,7 @@ fdtd_status fdtd_batch_destroy(fdtd_batch *b)
     b->R.reap();
     b->R.prog.release();
     b->R.free_buffers();
+    if (b->stream) resident_forget_stream(b->stream);
     b->R.release_scenes();
     if (b->own_stream && b->stream) (void)hipStreamDestroy(b->stream);
     delete b;

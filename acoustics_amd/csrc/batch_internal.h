@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "device_scene.h"
+#include "resident.h"
 
 namespace fdtd {
 
@@ -29,6 +30,11 @@ struct BatchRunner {
     size_t pbytes = 0;
     int pnext = 0;
     std::vector<hipGraphExec_t> retired;
+    // scenes that run resident (slot i: null when scene i does not), and their
+    // launches by tile shape
+    std::vector<std::unique_ptr<ResidentScene>> res;
+    ResidentProgram res_prog[RES_SHAPES];
+    bool res_listed = false;
     int plan = 0;
     int graph_steps = 32;
     hipGraphExec_t exec = nullptr;
@@ -43,11 +49,20 @@ struct BatchRunner {
     void free_buffers();                              // with the stream idle
     fdtd_status autotune(hipStream_t st);
     fdtd_status advance(hipStream_t st, int nsteps);
+    bool any_resident() const { return res_prog[RES_FINE].n > 0 || res_prog[RES_COARSE].n > 0; }
+    bool all_resident() const;
+    fdtd_status list_resident(hipStream_t st);        // (re)builds the resident launches
+    // Waits for the stream and completes blocks that a resident launch gave up.
+    fdtd_status settle(hipStream_t st);
     void release_scenes()
     {
         for (auto &s : scenes)
             if (s) s->release();
         scenes.clear();
+        for (auto &r : res)
+            if (r) r->release();
+        res.clear();
+        for (ResidentProgram &p : res_prog) p.release();
     }
     ~BatchRunner();
 };

@@ -54,8 +54,13 @@ __host__ __device__ inline int slot_next(long long s) { return (int)(s & 1); }
 
 // clock words of a scene; CLK_TIME holds the bits of the simulation time of
 // step clock[CLK_STEP], accumulated from the start time by adding dt once per
-// step, as the reference's clock runs (_simulationTime += dt)
-enum : int { CLK_STEP = 0, CLK_TARGET = 1, CLK_DONE = 2, CLK_TIME = 3, CLK_WORDS = 4 };
+// step, as the reference's clock runs (_simulationTime += dt).  CLK_ARRIVED
+// and CLK_GATE belong to a resident launch (resident.h): its workgroups that
+// have arrived, and whether they run (GATE_RUN) or give the block up
+// (GATE_GIVEN_UP, for good); the advance kernel shuts the gate again and leaves
+// the counter of a scene that gave up where it is.
+enum : int { CLK_STEP = 0, CLK_TARGET = 1, CLK_DONE = 2, CLK_TIME = 3, CLK_ARRIVED = 4, CLK_GATE = 5, CLK_WORDS = 8 };
+enum : unsigned long long { GATE_SHUT = 0, GATE_RUN = 1, GATE_GIVEN_UP = 2 };
 
 // the clock words of step s of a scene starting at t_start (host side)
 inline void clock_words(unsigned long long *clk, long long s, unsigned long long target, double t_start, double dt)
@@ -69,6 +74,7 @@ inline void clock_words(unsigned long long *clk, long long s, unsigned long long
     clk[CLK_TARGET] = target;
     clk[CLK_DONE] = 0ULL;
     clk[CLK_TIME] = tb;
+    for (int q = CLK_ARRIVED; q < CLK_WORDS; ++q) clk[q] = 0ULL;
 }
 
 // Steps are launched in blocks: the kernels of the k-th step of a block run

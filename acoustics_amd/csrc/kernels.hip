@@ -22,29 +22,9 @@
 #include <climits>
 
 #include "linalg.h"
+#include "stencil.h"
 
 namespace fdtd {
-
-// Pointers read out of a SceneDev are generic to the compiler, which then
-// emits flat memory instructions; those count against both the vector-memory
-// and the LDS counters, so every wait becomes a full wait.  Every scene array
-// lives in device global memory: casting to the global address space gives
-// global_load/global_store with vmcnt-only waits, and read-only tables cast to
-// the constant address space are fetched with scalar loads when the index is
-// uniform across the wavefront.
-#if defined(__HIP_DEVICE_COMPILE__)
-#define AS_GLOBAL __attribute__((address_space(1)))
-#define AS_CONST __attribute__((address_space(4)))
-#else  // the host pass only parses device code
-#define AS_GLOBAL
-#define AS_CONST
-#endif
-template <class T>
-__device__ __forceinline__ AS_GLOBAL T *gmem(T *p) { return (AS_GLOBAL T *)p; }
-template <class T>
-__device__ __forceinline__ const AS_GLOBAL T *gmem(const T *p) { return (const AS_GLOBAL T *)p; }
-template <class T>
-__device__ __forceinline__ const AS_CONST T *cmem(const T *p) { return (const AS_CONST T *)p; }
 
 // a_s(obj, t): the sources whose acceleration vector is a_n times the normal
 // (Gaussian impulse; HarmonicVibrationalSource::Evaluate,
@@ -141,18 +121,6 @@ __device__ __forceinline__ float speaker_at(const SceneDev &S, int i, int j, int
 // x_g = sum_q M_gq p_q + sum_o m_go a_n(o), FP64, in row order.  Computed where
 // it is used (the object-adjacent cell next to the ghost, and listener terms),
 // four independent index loads and gathers at a time.
-// -f h grad_p . cell_n of a rasterised ghost (f = 1 with centre sampling,
-// 0.75 with seven samples), grad_p = -rho (a_s n_b + a_v) (MAC_Grid.cpp:
-// 1256-1281): k_raster a_s, plus k_vec a_v along the ghost's axis in a
-// scene with acceleration noise
-__device__ __forceinline__ double raster_accel_term(const SceneDev &S, const GhostDev &gd, long long step)
-{
-    const AS_GLOBAL double *acc = gmem(S.acc_tab) + amp_row(step) * S.n_ch + gd.obj * S.n_cpo;
-    double v = gd.k_raster * acc[0];
-    if (S.n_cpo > 1) v = fma(gd.k_vec, acc[1 + gd.vaxis], v);
-    return v;
-}
-
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double coupled_ghost(const SceneDev &S, int g, const AS_GLOBAL float *__restrict__ pcur,
                                                 long long step)
@@ -213,21 +181,6 @@ __device__ __forceinline__ void emit_ghost_terms(const SceneDev &S, const TileDe
 // ---------------------------------------------------------------------------
 // interior leapfrog
 // ---------------------------------------------------------------------------
-// The leapfrog update in increment form, p^{n+1} = p^n + ((p^n - p^{n-1}) +
-// lam2 sum_q (p_q - p^n)).  A smooth field changes little between steps and
-// between neighbours, so every difference here is exact in FP32 (Sterbenz:
-// operands within a factor of two) and the only rounding at the scale of p
-// itself is the last addition.  Forming 2 p^n - p^{n-1} and the six-neighbour
-// sum instead rounds three times at that scale per step, and the rounding
-// errors, fed back as velocity, add up along every propagation path: 1.3e-4
-// relative L2 at the listeners after 4000 steps at 256^3, against 1e-4 allowed.
-__device__ __forceinline__ float leapfrog1(float c, float prev, float xm, float xp, float ym, float yp, float zm, float zp,
-                                           float lam2)
-{
-    const float lap = ((xm - c) + (xp - c)) + ((ym - c) + (yp - c)) + ((zm - c) + (zp - c));
-    return c + fmaf(lam2, lap, c - prev);
-}
-
 __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step, bool skip_check)
 {
     const int tk = t.tk_log2;
@@ -257,7 +210,7 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
                 for (int s = 0; s < S.n_psrc; ++s) {
                     const PSrcDev ps = cmem(S.psrc)[s];
                     const AS_CONST float *g = cmem(S.gtab);
-                    pn += gmem(S.src_tab)[amp_row(step) * S.n_psrc + s] * g[ps.goff[0] + i] * g[ps.goff[1] + j] * g[ps.goff[2] + k];
+                    pn = add_source(pn, gmem(S.src_tab)[amp_row(step) * S.n_psrc + s], g[ps.goff[0] + i], g[ps.goff[1] + j], g[ps.goff[2] + k]);
                 }
             if (t.src && S.n_spk) pn += speaker_at(S, i, j, k);
             if (!skip_check || !gmem(S.skip)[idx]) {
@@ -304,7 +257,7 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
             for (int s = 0; s < S.n_psrc; ++s) {
                 const PSrcDev ps = cmem(S.psrc)[s];
                 const AS_CONST float *g = cmem(S.gtab);
-                pn += gmem(S.src_tab)[amp_row(step) * S.n_psrc + s] * g[ps.goff[0] + i] * g[ps.goff[1] + j] * g[ps.goff[2] + k];
+                pn = add_source(pn, gmem(S.src_tab)[amp_row(step) * S.n_psrc + s], g[ps.goff[0] + i], g[ps.goff[1] + j], g[ps.goff[2] + k]);
             }
         if (t.src && S.n_spk) pn += speaker_at(S, i, j, k);
         if (!skip_check || !gmem(S.skip)[idx]) {
@@ -436,28 +389,6 @@ __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileD
 // branch of PML_pressureUpdateCollocated, 496-508), with the merged
 // transverse state of PmlSlab for cells damped along the slab axis only.
 // ---------------------------------------------------------------------------
-// Face velocity update on one axis for a face whose old value is v, between
-// pressures pl (left) and pr (right); inactive faces stay at zero.  The fma
-// is explicit: a face is computed by the two cells that share it and both
-// must round it the same way.
-__device__ __forceinline__ float face_update(bool active, float4 c, float v, float pl, float pr)
-{
-    return active ? fmaf(c.y, pr - pl, c.x * v) : 0.f;
-}
-
-// Split pressure update pDir <- f3 pDir + f5/h (v_R - v_L).
-__device__ __forceinline__ float split_update(float4 c, float q, float dv)
-{
-    return fmaf(c.w, dv, c.z * q);
-}
-
-// One transverse axis of the merged update: f5h (f2_R (p_R - p) - f2_L (p - p_L)),
-// cL the cell's table entry (its low face and itself), cR the high face's.
-__device__ __forceinline__ float transverse_term(float4 cL, float4 cR, float pl, float pc, float pr)
-{
-    return cL.w * fmaf(cR.y, pr - pc, -(cL.y * (pc - pl)));
-}
-
 // Loads and stores at a 32-bit byte offset from a wavefront-uniform base, so
 // the compiler can use the scalar-base form of global memory instructions
 // (one VGPR per address instead of a 64-bit pair).  Offsets stay below 4 GiB:
@@ -613,9 +544,9 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
         float pn;
         if (m) {
             float lap = 0.f;
-            if constexpr (A != 0) lap += transverse_term(cxC, cxR, pm, pc, pp);
-            if constexpr (A != 1) lap += transverse_term(cyL, cyR, ym, pc, yp);
-            if constexpr (A != 2) lap += transverse_term(czL, czR, zm, pc, zp);
+            if constexpr (A != 0) lap = transverse_add(lap, cxC.w, cxC.y, cxR.y, pm, pc, pp);
+            if constexpr (A != 1) lap = transverse_add(lap, cyL.w, cyL.y, cyR.y, ym, pc, yp);
+            if constexpr (A != 2) lap = transverse_add(lap, czL.w, czL.y, czR.y, zm, pc, zp);
             // p^{n+1} = p^n + (pDir_A^{n+1} - pDir_A^n) + d^{n+1}: only
             // increments are rounded before the last addition
             const float dn = qd + lap;
@@ -841,22 +772,6 @@ __device__ __forceinline__ void mac_vec_tile(const SceneDev &S, const TileDesc &
 // ---------------------------------------------------------------------------
 // bulk cells next to rigid objects (FP64)
 // ---------------------------------------------------------------------------
-// One axis of the ghost-aware Laplacian (MAC_Grid::
-// pressureFieldLaplacianGhostCell, MAC_Grid.cpp:187-299) at a cell with
-// pressure c, neighbours nm / np and ghost values gm / gp where the
-// neighbour is solid: the plain 3-point stencil with ghost values (centre
-// sampling, 247-266), or the non-uniform one for ghosts 3h/4 away (seven
-// samples, 268-286).
-__device__ __forceinline__ double ghost_lap_axis(int seven, bool ghm, bool ghp, double gm, double gp, double nm, double np,
-                                                 double c)
-{
-    const double m = ghm ? gm : nm, p = ghp ? gp : np;
-    if (!seven || (!ghm && !ghp)) return p + m - 2.0 * c;
-    if (ghm && ghp) return (gp + gm - 2.0 * c) / (9.0 / 16.0);
-    if (ghp) return (gp + 0.75 * nm - (7.0 / 4.0) * c) / (21.0 / 32.0);
-    return (0.75 * np + gm - (7.0 / 4.0) * c) / (21.0 / 32.0);
-}
-
 __device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
 {
     const int r = t.i0 + (int)threadIdx.x;
@@ -897,7 +812,7 @@ __device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &
             pn = 2.0 * c - (double)pprev[idx] - S.kcalp * (double)gmem(S.lapv)[idx] + (S.c2k2 + S.kcalp) * lc;
             gmem(S.lapv)[idx] = (float)lc;
         } else {
-            pn = 2.0 * c - (double)pprev[idx] + lap * S.lam2;
+            pn = special_update(c, (double)pprev[idx], lap, S.lam2);
         }
     }
     if (S.n_psrc > 0) {
@@ -1314,7 +1229,7 @@ __global__ __launch_bounds__(256) void advance_kernel(const SceneDev *__restrict
     AS_GLOBAL unsigned long long *clk = gmem(S.clock);
     const long long step = (long long)clk[CLK_STEP], target = (long long)clk[CLK_TARGET];
     if (step >= target) return;
-    const long long base = min(step + (long long)n, target);
+    const long long base = clk[CLK_GATE] == GATE_GIVEN_UP ? step : min(step + (long long)n, target);
     // the times of steps base .. base + AMP_ROWS - 1, accumulated from the
     // clock's time by one addition of dt per step (the reference's clock)
     __shared__ double tt[AMP_ROWS];
@@ -1356,6 +1271,8 @@ __global__ __launch_bounds__(256) void advance_kernel(const SceneDev *__restrict
     if (threadIdx.x == 0) {
         clk[CLK_STEP] = (unsigned long long)base;
         clk[CLK_TIME] = (unsigned long long)__double_as_longlong(tt[0]);
+        clk[CLK_ARRIVED] = 0ULL;
+        if (clk[CLK_GATE] == GATE_RUN) clk[CLK_GATE] = GATE_SHUT;
     }
 }
 

@@ -1,0 +1,800 @@
+// resident.hip -- a block of steps of whole scenes held on the chip.
+//
+// Bound: the exchange between workgroups.  A step needs the neighbours' face
+// pressures of the step before, and one hop through the memory side (a store
+// of one workgroup to a load of another) takes 1.3-1.6 us with up to 256
+// workgroups in flight, 1.9 us with 512, 3.0 us with 1024; the arithmetic of
+// a step is 0.3-1.6 us of the SIMDs and nothing is read from or written to
+// HBM.  Each face pressure travels in one 8-byte word with the step's tag
+// above it, so the data is its own flag: no store has to be acknowledged
+// before a flag is raised, and no load follows a flag (with flags the same
+// exchange took 1.8-3.3 us).  The words of a face are contiguous over lanes:
+// stored column by column instead, the exchange took 14-24 us.
+#include <climits>
+
+#include "resident.h"
+#include "stencil.h"
+
+namespace fdtd {
+
+namespace {
+
+template <int SHAPE>
+struct Shape;
+// small grids: as many workgroups as possible
+template <>
+struct Shape<RES_FINE> {
+    static constexpr int plain = 8, one = 8, more = 8, cs = 12, words = 5, recs = 2, waves = 3;
+};
+// larger grids: as many cells per workgroup as registers and LDS hold
+template <>
+struct Shape<RES_COARSE> {
+    static constexpr int plain = 16, one = 12, more = 8, cs = 20, words = 6, recs = 3, waves = 3;
+};
+
+typedef unsigned long long u64;
+
+__device__ __forceinline__ void send_word(u64 *p, u64 v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 take_word(const u64 *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The value, computed anew: offsets of the last stores would otherwise be
+// carried in registers through all steps.
+__device__ __forceinline__ int anew(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// face word w of a tile: the face, and the cell of that face (LDS place of
+// the cell itself and of its neighbour across the face, global cell across it)
+struct FaceCell {
+    int own, halo;      // LDS words
+    int i, j, k;        // the neighbour's cell
+};
+
+template <int CS>
+__device__ __forceinline__ FaceCell face_cell(const ResTile &t, int w)
+{
+    const int nyz = t.by * t.bz, nxz = t.bx * t.bz, nxy = t.bx * t.by, P = t.bz + 2;
+    FaceCell f;
+    if (w < 2 * nyz) {
+        const int hi = w >= nyz, c = w - hi * nyz, y = c / t.bz, z = c - y * t.bz;
+        const int col = ((y + 1) * P + z + 1) * CS;
+        f.own = col + (hi ? t.bx - 1 : 0);
+        f.halo = col + (hi ? t.bx : CS - 1);
+        f.i = hi ? t.i0 + t.bx : t.i0 - 1;
+        f.j = t.j0 + y;
+        f.k = t.k0 + z;
+        return f;
+    }
+    w -= 2 * nyz;
+    if (w < 2 * nxz) {
+        const int hi = w >= nxz, c = w - hi * nxz, x = c / t.bz, z = c - x * t.bz;
+        f.own = ((hi ? t.by : 1) * P + z + 1) * CS + x;
+        f.halo = ((hi ? t.by + 1 : 0) * P + z + 1) * CS + x;
+        f.i = t.i0 + x;
+        f.j = hi ? t.j0 + t.by : t.j0 - 1;
+        f.k = t.k0 + z;
+        return f;
+    }
+    w -= 2 * nxz;
+    const int hi = w >= nxy, c = w - hi * nxy, x = c / t.by, y = c - x * t.by;
+    f.own = ((y + 1) * P + (hi ? t.bz : 1)) * CS + x;
+    f.halo = ((y + 1) * P + (hi ? t.bz + 1 : 0)) * CS + x;
+    f.i = t.i0 + x;
+    f.j = t.j0 + y;
+    f.k = hi ? t.k0 + t.bz : t.k0 - 1;
+    return f;
+}
+
+// Fills a scene's route table, one workgroup per tile: the tile on the other
+// side of each face word and the word there that stands for the own cell.
+template <int CS>
+__global__ __launch_bounds__(RES_THREADS) void route_kernel(const ResScene *__restrict__ scene)
+{
+    const ResScene R = *cmem(scene);
+    const SceneDev S = *cmem(R.S);
+    const ResTile t = cmem(R.tiles)[blockIdx.x];
+    for (int w = (int)threadIdx.x; w < t.words; w += RES_THREADS) {
+        const FaceCell f = face_cell<CS>(t, w);
+        ResRoute r;
+        r.lds = (uint32_t)f.own | ((uint32_t)f.halo << 16);
+        r.to = RES_NOWHERE;
+        if (f.i >= 0 && f.j >= 0 && f.k >= 0 && f.i < S.n[0] && f.j < S.n[1] && f.k < S.n[2]) {
+            const int x[3] = {f.i, f.j, f.k};
+            for (int b = 0; b < R.nboxes; ++b) {
+                const ResBox B = cmem(R.boxes)[b];
+                int at[3];
+                bool in = true;
+                for (int d = 0; d < 3; ++d) {
+                    at[d] = x[d] - B.lo[d];
+                    in = in && at[d] >= 0 && at[d] < B.len[d];
+                }
+                if (!in) continue;
+                const int q = B.first + ((at[0] / B.size[0]) * B.count[1] + at[1] / B.size[1]) * B.count[2] + at[2] / B.size[2];
+                const ResTile o = gmem(R.tiles)[q];
+                const int nyz = o.by * o.bz, nxz = o.bx * o.bz, nxy = o.bx * o.by;
+                const int li = x[0] - o.i0, lj = x[1] - o.j0, lk = x[2] - o.k0;
+                // the own cell is across the neighbour's opposite face
+                int word;
+                if (f.i < t.i0) word = nyz + lj * o.bz + lk;
+                else if (f.i >= t.i0 + t.bx) word = lj * o.bz + lk;
+                else if (f.j < t.j0) word = 2 * nyz + nxz + li * o.bz + lk;
+                else if (f.j >= t.j0 + t.by) word = 2 * nyz + li * o.bz + lk;
+                else if (f.k < t.k0) word = 2 * (nyz + nxz) + nxy + li * o.by + lj;
+                else word = 2 * (nyz + nxz) + li * o.by + lj;
+                r.to = o.word0 + (uint32_t)word;
+                break;
+            }
+        }
+        gmem(R.route)[t.word0 + (uint32_t)w] = r;
+    }
+}
+
+// the x table entry of face / cell i: a wall face gets zero factors
+__device__ __forceinline__ float4 x_entry(const SceneDev &S, int i)
+{
+    float4 c = gmem(S.coef[0])[min(i, S.n[0])];
+    if (i <= 0 || i >= S.n[0]) { c.x = 0.f; c.y = 0.f; }
+    return c;
+}
+
+// What a workgroup carries through its steps besides the class's registers.
+template <int SHAPE>
+struct Frame {
+    using C = Shape<SHAPE>;
+    const SceneDev &S;
+    const ResScene &R;
+    const ResTile &t;
+    float *A, *B;               // this step's pressures and the next's, in LDS
+    float4 *X;                  // x table of the tile's cells and faces, in LDS
+    long long step0;
+    int steps;
+    uint32_t tag;
+    int *trouble;
+    // own column
+    bool act;
+    int ly, lz, col;            // col: LDS word of the column's first cell
+    int P;                      // LDS words from a column to the next along y
+    // face words
+    ResRoute route[C::words];
+    // the tile's listener terms: this thread's first one
+    bool has_term;
+    TermRef term;
+    int term_at;
+    int ring0;                  // ring row of step0
+    bool stuck;
+
+    __device__ Frame(const SceneDev &S_, const ResScene &R_, const ResTile &t_) : S(S_), R(R_), t(t_) {}
+
+    __device__ __forceinline__ int place(int cell) const
+    {
+        const int i = cell / S.sx, r = cell - i * S.sx, j = r / S.sy, k = r - j * S.sy;
+        return ((j - t.j0 + 1) * (t.bz + 2) + (k - t.k0 + 1)) * C::cs + (i - t.i0);
+    }
+
+    // p^{step} of the tile and its halo, both buffers cleared before
+    __device__ __forceinline__ void load()
+    {
+        const int tid = (int)threadIdx.x, n = 2 * RES_LDS_COLUMNS * C::cs;
+        for (int q = tid; q < n; q += RES_THREADS) A[q] = 0.f;
+        P = (t.bz + 2) * C::cs;
+        act = tid < t.by * t.bz;
+        ly = act ? tid / t.bz : 0;
+        lz = act ? tid - ly * t.bz : 0;
+        col = ((ly + 1) * (t.bz + 2) + lz + 1) * C::cs;
+        if (tid <= C::plain) X[tid] = x_entry(S, t.i0 + tid);
+        __syncthreads();
+        const AS_GLOBAL float *pc = gmem(S.field + (size_t)slot_cur(step0) * S.npad);
+        if (act) {
+            const int idx = t.i0 * S.sx + (t.j0 + ly) * S.sy + t.k0 + lz;
+#pragma unroll
+            for (int i = 0; i < C::plain; ++i)
+                if (i < t.bx) A[col + i] = pc[idx + i * S.sx];
+        }
+#pragma unroll
+        for (int m = 0; m < C::words; ++m) {
+            const int w = tid + m * RES_THREADS;
+            route[m].to = RES_NOWHERE;
+            route[m].lds = 0;
+            if (w < t.words) {
+                route[m] = gmem(R.route)[t.word0 + (uint32_t)w];
+                if (route[m].to != RES_NOWHERE) {
+                    const FaceCell f = face_cell<C::cs>(t, w);
+                    A[f.halo] = pc[f.i * S.sx + f.j * S.sy + f.k];
+                }
+            }
+        }
+        has_term = t.tb + tid < t.te;
+        term_at = 0;
+        ring0 = (int)(step0 % S.cap);
+        if (has_term) {
+            term = gmem(R.terms)[t.tb + tid];
+            term_at = place(term.kind == 0 ? term.cell : gmem(S.ghosts)[term.cell].nbr);
+        }
+        stuck = false;
+    }
+
+    // fresh, now: ring rows of the step that made the pressures now held and
+    // of the step about to run (-1: none in this block)
+    __device__ __forceinline__ void emit(const TermRef &r, int at, int fresh, int now, long long step) const
+    {
+        // a cell's term belongs to the step that made the pressure now held,
+        // a ghost's to the step about to run
+        double v = (double)A[at];
+        int row = fresh;
+        if (r.kind != 0) {
+            if (now < 0) return;
+            v += raster_accel_term(S, gmem(S.ghosts)[r.cell], step);
+            row = now;
+        } else if (fresh < 0) {
+            return;
+        }
+        gmem(S.terms)[(size_t)(row < S.cap ? row : row - S.cap) * S.T + r.slot] = r.beta * v;
+    }
+    // before step s of the block (s == steps: after the last)
+    __device__ __forceinline__ void terms(int s) const
+    {
+        if (t.te == t.tb) return;
+        const int fresh = s > 0 ? ring0 + s - 1 : -1, now = s < steps ? ring0 + s : -1;
+        if (has_term) emit(term, term_at, fresh, now, step0 + s);
+        for (int q = t.tb + (int)threadIdx.x + RES_THREADS; q < t.te; q += RES_THREADS) {
+            const TermRef r = gmem(R.terms)[q];
+            emit(r, place(r.kind == 0 ? r.cell : gmem(S.ghosts)[r.cell].nbr), fresh, now, step0 + s);
+        }
+    }
+
+    // sends the tile's faces of the step just made and waits for the
+    // neighbours' (all of B's own cells are written and visible)
+    __device__ __forceinline__ void exchange(int s)
+    {
+        const uint32_t mark = tag + (uint32_t)s;
+        u64 *buf = R.words + (size_t)(mark & 1u) * R.nwords;
+#pragma unroll
+        for (int m = 0; m < C::words; ++m)
+            if (route[m].to != RES_NOWHERE)
+                send_word(buf + route[m].to, ((u64)mark << 32) | __float_as_uint(B[route[m].lds & 0xffffu]));
+        const u64 *in = buf + t.word0 + threadIdx.x;
+        u64 v[C::words];
+        for (int spins = 0; !stuck; ++spins) {
+#pragma unroll
+            for (int m = 0; m < C::words; ++m)
+                if (route[m].to != RES_NOWHERE) v[m] = take_word(in + m * RES_THREADS);
+            bool ok = true;
+#pragma unroll
+            for (int m = 0; m < C::words; ++m)
+                if (route[m].to != RES_NOWHERE) ok = ok && (uint32_t)(v[m] >> 32) == mark;
+            if (ok) break;
+            if (spins > (1 << 22)) {
+                // the neighbours are on the device, so this does not happen;
+                // it keeps every wave's exit certain
+                stuck = true;
+                __hip_atomic_store(trouble, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+        // (nothing lies beyond a wall: that halo stays zero)
+#pragma unroll
+        for (int m = 0; m < C::words; ++m)
+            if (route[m].lds) B[route[m].lds >> 16] = route[m].to != RES_NOWHERE ? __uint_as_float((uint32_t)v[m]) : 0.f;
+    }
+    __device__ __forceinline__ void turn()
+    {
+        float *q = A;
+        A = B;
+        B = q;
+    }
+
+    // the last two levels of the own cells, into the slots of step step0 + steps
+    __device__ __forceinline__ void store_pressure() const
+    {
+        if (!act) return;
+        const long long s = step0 + steps;
+        AS_GLOBAL float *pc = gmem(S.field + (size_t)slot_cur(s) * S.npad), *pp = gmem(S.field + (size_t)slot_next(s) * S.npad);
+        const int idx = t.i0 * S.sx + (t.j0 + anew(ly)) * S.sy + t.k0 + lz;
+#pragma unroll
+        for (int i = 0; i < C::plain; ++i)
+            if (i < t.bx) {
+                pc[idx + i * S.sx] = A[col + i];
+                pp[idx + i * S.sx] = B[col + i];
+            }
+    }
+};
+
+// four cells of a column and their neighbours: cells 4 q .. 4 q + 3
+struct Quad {
+    float c[4], xm, xp, yl[4], yr[4], zl[4], zr[4];
+};
+template <int CS>
+__device__ __forceinline__ Quad quad(const float *A, int col, int P, int q)
+{
+    Quad u;
+    const float *a = A + col + 4 * q;
+    const float4 c = *(const float4 *)a, yl = *(const float4 *)(a - P), yr = *(const float4 *)(a + P);
+    const float4 zl = *(const float4 *)(a - CS), zr = *(const float4 *)(a + CS);
+    u.xp = a[4];
+    u.xm = q == 0 ? A[col + CS - 1] : a[-1];
+    u.c[0] = c.x; u.c[1] = c.y; u.c[2] = c.z; u.c[3] = c.w;
+    u.yl[0] = yl.x; u.yl[1] = yl.y; u.yl[2] = yl.z; u.yl[3] = yl.w;
+    u.yr[0] = yr.x; u.yr[1] = yr.y; u.yr[2] = yr.z; u.yr[3] = yr.w;
+    u.zl[0] = zl.x; u.zl[1] = zl.y; u.zl[2] = zl.z; u.zl[3] = zl.w;
+    u.zr[0] = zr.x; u.zr[1] = zr.y; u.zr[2] = zr.z; u.zr[3] = zr.w;
+    return u;
+}
+// Writes cells 4 q .. 4 q + 3 of the column.  Cells past the tile's last are
+// written too: the first of them is the place of the x-high halo, which the
+// exchange then fills in, and no cell of the tile reads the others.
+__device__ __forceinline__ void put_quad(float *B, int col, int q, const float *o)
+{
+    *(float4 *)(B + col + 4 * q) = make_float4(o[0], o[1], o[2], o[3]);
+}
+
+// Undamped cells: leapfrog, pressure sources, and the object-adjacent cells
+// of the tile in FP64 by one thread per record.
+template <int SHAPE>
+__device__ __forceinline__ void run_plain(Frame<SHAPE> &F)
+{
+    using C = Shape<SHAPE>;
+    constexpr int NB = C::plain, NR = C::recs;
+    const SceneDev &S = F.S;
+    const ResTile &t = F.t;
+    const int tid = (int)threadIdx.x;
+    float prev[NB];
+    uint32_t skip = 0;
+    const float lam2 = S.lam2f;
+    const int j = t.j0 + F.ly, k = t.k0 + F.lz;   // (threads without a column: the first one's)
+    {
+        const AS_GLOBAL float *pp = gmem(S.field + (size_t)slot_next(F.step0) * S.npad);
+        const int idx = t.i0 * S.sx + j * S.sy + k;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) prev[i] = pp[idx + min(i, t.bx - 1) * S.sx];
+        if (t.skip)
+            for (int i = 0; i < t.bx; ++i) skip |= (gmem(S.skip)[idx + i * S.sx] ? 1u : 0u) << i;
+    }
+    // records: place, last level, the ghost term's factor per side
+    int rat[NR], rmask[NR], robj[NR];
+    float rprev[NR];
+    double rk[NR][6];
+    if (t.re > t.rb) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            rat[r] = -1;
+            const int q = t.rb + tid + r * RES_THREADS;
+            if (q >= t.re) continue;
+            const SpecialRec rec = gmem(S.recs)[gmem(F.R.recs)[q]];
+            rat[r] = F.place(rec.cell);
+            rprev[r] = gmem(S.field + (size_t)slot_next(F.step0) * S.npad)[rec.cell];
+            rmask[r] = (rec.flags & 1) << 6;
+            robj[r] = 0;
+            for (int e = 0; e < 6; ++e) {
+                rk[r][e] = 0.0;
+                if (rec.gid[e] < 0) continue;
+                const GhostDev gd = gmem(S.ghosts)[rec.gid[e]];
+                rmask[r] |= 1 << e;
+                robj[r] = gd.obj;
+                rk[r][e] = gd.k_raster;
+            }
+        }
+    }
+    for (int s = 0; s < F.steps; ++s) {
+        const long long step = F.step0 + s;
+        F.terms(s);
+        double racc[NR];
+        if (t.re > t.rb) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) racc[r] = rat[r] >= 0 ? gmem(S.acc_tab)[amp_row(step) * S.n_ch + robj[r] * S.n_cpo] : 0.0;
+        }
+        if (F.act) {
+#pragma unroll
+            for (int q = 0; q < NB / 4; ++q) {
+                if (4 * q >= t.bx) continue;
+                const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[e] = leapfrog1(u.c[e], prev[4 * q + e], e ? u.c[e - 1] : u.xm, e < 3 ? u.c[e + 1] : u.xp, u.yl[e], u.yr[e],
+                                     u.zl[e], u.zr[e], lam2);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) prev[4 * q + e] = u.c[e];
+                if (!t.skip) put_quad(F.B, F.col, q, o);
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (4 * q + e < t.bx && !(skip >> (4 * q + e) & 1)) F.B[F.col + 4 * q + e] = o[e];
+                }
+            }
+            if (t.src)
+                for (int p = 0; p < S.n_psrc; ++p) {
+                    // an amplitude of zero (the pulse is over) adds nothing
+                    const float a = gmem(S.src_tab)[amp_row(step) * S.n_psrc + p];
+                    if (a == 0.f) continue;
+                    const PSrcDev ps = cmem(S.psrc)[p];
+                    const float gy = gmem(S.gtab)[ps.goff[1] + j], gz = gmem(S.gtab)[ps.goff[2] + k];
+                    for (int i = 0; i < t.bx; ++i)
+                        if (!(skip >> i & 1)) F.B[F.col + i] = add_source(F.B[F.col + i], a, cmem(S.gtab)[ps.goff[0] + t.i0 + i], gy, gz);
+                }
+        }
+        if (t.re > t.rb) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                if (rat[r] < 0) continue;
+                const float *a = F.A + rat[r];
+                const int x = rat[r] % C::cs;
+                const float cf = a[0];
+                const double c = cf;
+                const double nb[6] = {x == 0 ? a[C::cs - 1] : a[-1], a[1], a[-F.P], a[F.P], a[-C::cs], a[C::cs]};
+                double g[6];
+#pragma unroll
+                for (int e = 0; e < 6; ++e) g[e] = (rmask[r] >> e & 1) ? c + rk[r][e] * racc[r] : 0.0;
+                double lap = 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    lap += ghost_lap_axis(S.seven, rmask[r] >> (2 * d) & 1, rmask[r] >> (2 * d + 1) & 1, g[2 * d], g[2 * d + 1],
+                                          nb[2 * d], nb[2 * d + 1], c);
+                double pn = (rmask[r] >> 6 & 1) ? c : special_update(c, (double)rprev[r], lap, S.lam2);
+                if (S.n_psrc > 0) {
+                    const int cx = rat[r] / C::cs, y = cx / (t.bz + 2) - 1, z = cx % (t.bz + 2) - 1;
+                    for (int p = 0; p < S.n_psrc; ++p) {
+                        const PSrcDev ps = cmem(S.psrc)[p];
+                        const AS_GLOBAL float *g3 = gmem(S.gtab);
+                        pn += (double)(gmem(S.src_tab)[amp_row(step) * S.n_psrc + p] * g3[ps.goff[0] + t.i0 + x] *
+                                       g3[ps.goff[1] + t.j0 + y] * g3[ps.goff[2] + t.k0 + z]);
+                    }
+                }
+                rprev[r] = cf;
+                F.B[rat[r]] = (float)pn;
+            }
+        }
+        __syncthreads();
+        F.exchange(s);
+        F.turn();
+        __syncthreads();
+    }
+    F.terms(F.steps);
+    F.store_pressure();
+}
+
+// Face and cell coefficients of the own column along y or z.
+struct AxisCoef {
+    float l1, l2, r1, r2, c3, c5;   // faces low and high {f1, f2}, cell {f3, f5/h}; a wall face stays at zero
+};
+__device__ __forceinline__ AxisCoef axis_coef(const SceneDev &S, int d, int i)
+{
+    const float4 lo = gmem(S.coef[d])[i], hi = gmem(S.coef[d])[i + 1];
+    AxisCoef a;
+    a.l1 = i > 0 ? lo.x : 0.f;
+    a.l2 = i > 0 ? lo.y : 0.f;
+    a.r1 = i + 1 < S.n[d] ? hi.x : 0.f;
+    a.r2 = i + 1 < S.n[d] ? hi.y : 0.f;
+    a.c3 = lo.z;
+    a.c5 = lo.w;
+    return a;
+}
+__device__ __forceinline__ float face_step(float f1, float f2, float v, float pl, float pr)
+{
+    return fmaf(f2, pr - pl, f1 * v);
+}
+__device__ __forceinline__ float split_step(float f3, float f5, float q, float dv)
+{
+    return fmaf(f5, dv, f3 * q);
+}
+// compact offsets of the own column's cells and faces in its slab
+struct SlabAt {
+    const PmlSlab &sl;
+    int e1, e2, li, lj, lk;
+    __device__ SlabAt(const PmlSlab &s, const ResTile &t, int ly, int lz)
+        : sl(s), e1(s.e[1]), e2(s.e[2]), li(t.i0 - s.lo[0]), lj(t.j0 + ly - s.lo[1]), lk(t.k0 + lz - s.lo[2]) {}
+    __device__ __forceinline__ int cell(int i) const { return ((li + i) * e1 + lj) * e2 + lk; }   // and the x face
+    __device__ __forceinline__ int fy(int i, int h) const { return ((li + i) * (e1 + 1) + lj + h) * e2 + lk; }
+    __device__ __forceinline__ int fz(int i, int h) const { return ((li + i) * e1 + lj) * (e2 + 1) + lk + h; }
+};
+
+// Cells damped along axis D only (the merged PML state): pDir along D, both
+// faces along D, and the increment of the transverse sum.
+template <int SHAPE, int D>
+__device__ __forceinline__ void run_one(Frame<SHAPE> &F)
+{
+    using C = Shape<SHAPE>;
+    constexpr int NB = C::one;
+    const SceneDev &S = F.S;
+    const ResTile &t = F.t;
+    const PmlSlab sl = cmem(S.slabs)[t.slab];
+    const SlabAt at(sl, t, F.ly, F.lz);
+    AS_GLOBAL float *pq = gmem(S.pd[D] + sl.cell_base), *pi = gmem(S.pd[D == 0 ? 1 : 0] + sl.cell_base);
+    float q0[NB], dd[NB], vl[D == 0 ? NB + 1 : NB], vr[D == 0 ? 1 : NB];
+    const AxisCoef cy = axis_coef(S, 1, t.j0 + F.ly), cz = axis_coef(S, 2, t.k0 + F.lz);
+    {
+        const AS_GLOBAL float *v = gmem((F.step0 & 1 ? S.vel[1][D] : S.vel[0][D]) + sl.v_base[D]);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int e = min(i, t.bx - 1);
+            q0[i] = pq[at.cell(e)];
+            dd[i] = pi[at.cell(e)];
+            if (D == 0) vl[i] = v[at.cell(e)];
+            if (D == 1) { vl[i] = v[at.fy(e, 0)]; vr[i] = v[at.fy(e, 1)]; }
+            if (D == 2) { vl[i] = v[at.fz(e, 0)]; vr[i] = v[at.fz(e, 1)]; }
+        }
+        if (D == 0) {
+            // the high face of the last cell (compile-time places only)
+            const float last = v[at.cell(t.bx)];
+#pragma unroll
+            for (int i = 1; i <= NB; ++i)
+                if (i == t.bx) vl[i] = last;
+        }
+    }
+    const float4 xp0 = cmem(S.coef[0])[t.i0];   // D != 0: x is plain over the tile, one entry for all
+    for (int s = 0; s < F.steps; ++s) {
+        F.terms(s);
+        if (F.act) {
+            float before = 0.f;                 // D == 0: the updated low face of the next cell
+#pragma unroll
+            for (int q = 0; q < NB / 4; ++q) {
+                if (4 * q >= t.bx) continue;
+                const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 4 * q + e;
+                    const float c = u.c[e], xm = e ? u.c[e - 1] : u.xm, xp = e < 3 ? u.c[e + 1] : u.xp;
+                    float n, lap = 0.f;
+                    const float qo = q0[i];
+                    if (D == 0) {
+                        const float4 xl = F.X[i], xr = F.X[i + 1];
+                        if (i == 0) before = face_step(xl.x, xl.y, vl[0], xm, c);
+                        const float after = face_step(xr.x, xr.y, vl[i + 1], c, xp);
+                        n = split_step(xl.z, xl.w, qo, after - before);
+                        vl[i] = before;
+                        before = after;
+                        if (e == 3) vl[i + 1] = after;
+                    } else if (D == 1) {
+                        vl[i] = face_step(cy.l1, cy.l2, vl[i], u.yl[e], c);
+                        vr[i] = face_step(cy.r1, cy.r2, vr[i], c, u.yr[e]);
+                        n = split_step(cy.c3, cy.c5, qo, vr[i] - vl[i]);
+                    } else {
+                        vl[i] = face_step(cz.l1, cz.l2, vl[i], u.zl[e], c);
+                        vr[i] = face_step(cz.r1, cz.r2, vr[i], c, u.zr[e]);
+                        n = split_step(cz.c3, cz.c5, qo, vr[i] - vl[i]);
+                    }
+                    if (D != 0) lap = transverse_add(lap, xp0.w, xp0.y, xp0.y, xm, c, xp);
+                    if (D != 1) lap = transverse_add(lap, cy.c5, cy.l2, cy.r2, u.yl[e], c, u.yr[e]);
+                    if (D != 2) lap = transverse_add(lap, cz.c5, cz.l2, cz.r2, u.zl[e], c, u.zr[e]);
+                    const float dn = dd[i] + lap, dA = n - qo;
+                    dd[i] = dn;
+                    q0[i] = n;
+                    o[e] = c + (dA + dn);
+                }
+                put_quad(F.B, F.col, q, o);
+            }
+        }
+        __syncthreads();
+        F.exchange(s);
+        F.turn();
+        __syncthreads();
+    }
+    F.terms(F.steps);
+    F.store_pressure();
+    if (!F.act) return;
+    const SlabAt to(sl, t, anew(F.ly), anew(F.lz));
+    AS_GLOBAL float *v = gmem(((F.step0 + F.steps) & 1 ? S.vel[1][D] : S.vel[0][D]) + sl.v_base[D]);
+#pragma unroll
+    for (int i = 0; i <= NB; ++i) {
+        if (i < NB && i < t.bx) {
+            pq[to.cell(i)] = q0[i];
+            pi[to.cell(i)] = dd[i];
+            if (D == 1) { v[to.fy(i, 0)] = vl[i]; if (F.ly == t.by - 1) v[to.fy(i, 1)] = vr[i]; }
+            if (D == 2) { v[to.fz(i, 0)] = vl[i]; if (F.lz == t.bz - 1) v[to.fz(i, 1)] = vr[i]; }
+        }
+        if (D == 0 && i <= t.bx) v[to.cell(i)] = vl[i];
+    }
+}
+
+// Cells damped along two or three axes: three split pressures, the faces of
+// all three axes (a face of two tiles is kept by both, computed alike).
+template <int SHAPE>
+__device__ __forceinline__ void run_more(Frame<SHAPE> &F)
+{
+    using C = Shape<SHAPE>;
+    constexpr int NB = C::more;
+    const SceneDev &S = F.S;
+    const ResTile &t = F.t;
+    const PmlSlab sl = cmem(S.slabs)[t.slab];
+    const SlabAt at(sl, t, F.ly, F.lz);
+    float q0[NB], q1[NB], q2[NB], vx[NB + 1], yl[NB], yr[NB], zl[NB], zr[NB];
+    const AxisCoef cy = axis_coef(S, 1, t.j0 + F.ly), cz = axis_coef(S, 2, t.k0 + F.lz);
+    {
+        const int b = (int)(F.step0 & 1);
+        const AS_GLOBAL float *v0 = gmem((b ? S.vel[1][0] : S.vel[0][0]) + sl.v_base[0]), *v1 = gmem((b ? S.vel[1][1] : S.vel[0][1]) + sl.v_base[1]);
+        const AS_GLOBAL float *v2 = gmem((b ? S.vel[1][2] : S.vel[0][2]) + sl.v_base[2]);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int e = min(i, t.bx - 1), c = at.cell(e);
+            vx[i] = v0[c];
+            q0[i] = gmem(S.pd[0] + sl.cell_base)[c];
+            q1[i] = gmem(S.pd[1] + sl.cell_base)[c];
+            q2[i] = gmem(S.pd[2] + sl.cell_base)[c];
+            yl[i] = v1[at.fy(e, 0)];
+            yr[i] = v1[at.fy(e, 1)];
+            zl[i] = v2[at.fz(e, 0)];
+            zr[i] = v2[at.fz(e, 1)];
+        }
+        const float last = v0[at.cell(t.bx)];
+#pragma unroll
+        for (int i = 1; i <= NB; ++i)
+            if (i == t.bx) vx[i] = last;
+    }
+    for (int s = 0; s < F.steps; ++s) {
+        F.terms(s);
+        if (F.act) {
+            float before = 0.f;
+#pragma unroll
+            for (int q = 0; q < NB / 4; ++q) {
+                if (4 * q >= t.bx) continue;
+                const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 4 * q + e;
+                    const float c = u.c[e], xm = e ? u.c[e - 1] : u.xm, xp = e < 3 ? u.c[e + 1] : u.xp;
+                    const float4 xl = F.X[i], xr = F.X[i + 1];
+                    if (i == 0) before = face_step(xl.x, xl.y, vx[0], xm, c);
+                    const float after = face_step(xr.x, xr.y, vx[i + 1], c, xp);
+                    q0[i] = split_step(xl.z, xl.w, q0[i], after - before);
+                    vx[i] = before;
+                    before = after;
+                    if (e == 3) vx[i + 1] = after;
+                    yl[i] = face_step(cy.l1, cy.l2, yl[i], u.yl[e], c);
+                    yr[i] = face_step(cy.r1, cy.r2, yr[i], c, u.yr[e]);
+                    q1[i] = split_step(cy.c3, cy.c5, q1[i], yr[i] - yl[i]);
+                    zl[i] = face_step(cz.l1, cz.l2, zl[i], u.zl[e], c);
+                    zr[i] = face_step(cz.r1, cz.r2, zr[i], c, u.zr[e]);
+                    q2[i] = split_step(cz.c3, cz.c5, q2[i], zr[i] - zl[i]);
+                    o[e] = q0[i] + q1[i] + q2[i];
+                }
+                put_quad(F.B, F.col, q, o);
+            }
+        }
+        __syncthreads();
+        F.exchange(s);
+        F.turn();
+        __syncthreads();
+    }
+    F.terms(F.steps);
+    F.store_pressure();
+    if (!F.act) return;
+    const SlabAt to(sl, t, anew(F.ly), anew(F.lz));
+    const int b = (int)((F.step0 + F.steps) & 1);
+    AS_GLOBAL float *v0 = gmem((b ? S.vel[1][0] : S.vel[0][0]) + sl.v_base[0]), *v1 = gmem((b ? S.vel[1][1] : S.vel[0][1]) + sl.v_base[1]);
+    AS_GLOBAL float *v2 = gmem((b ? S.vel[1][2] : S.vel[0][2]) + sl.v_base[2]);
+#pragma unroll
+    for (int i = 0; i <= NB; ++i) {
+        if (i <= t.bx) v0[to.cell(i)] = vx[i];
+        if (i < NB && i < t.bx) {
+            const int c = to.cell(i);
+            gmem(S.pd[0] + sl.cell_base)[c] = q0[i];
+            gmem(S.pd[1] + sl.cell_base)[c] = q1[i];
+            gmem(S.pd[2] + sl.cell_base)[c] = q2[i];
+            v1[to.fy(i, 0)] = yl[i];
+            if (F.ly == t.by - 1) v1[to.fy(i, 1)] = yr[i];
+            v2[to.fz(i, 0)] = zl[i];
+            if (F.lz == t.bz - 1) v2[to.fz(i, 1)] = zr[i];
+        }
+    }
+}
+
+// One workgroup per tile.  No workgroup changes anything before all of its
+// scene have arrived, so a scene whose workgroups cannot all be on the device
+// at once (another resident launch holds it) gives the block up whole: the
+// last to arrive and the first to lose patience settle it by one
+// compare-and-swap on the gate.  Past the gate every neighbour is running, so
+// every later wait ends.
+template <int SHAPE>
+__global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_kernel(const ResItem *__restrict__ items, int nsteps,
+                                                                                   uint32_t tag, int wait_limit, int *trouble)
+{
+    extern __shared__ __align__(16) float lds[];
+    __shared__ int gate;
+    __shared__ float4 xtab[Shape<SHAPE>::plain + 1];
+    const ResItem it = items[blockIdx.x];
+    if (!it.scene) return;
+    // uniform data by way of the constant address space: scalar loads, scalar registers
+    const ResScene R = *cmem(it.scene);
+    const SceneDev S = *cmem(R.S);
+    const ResTile t = cmem(R.tiles)[it.tile];
+    u64 *clk = S.clock;
+    Frame<SHAPE> F(S, R, t);
+    F.step0 = (long long)clk[CLK_STEP];
+    const long long left = (long long)clk[CLK_TARGET] - F.step0;
+    if (left <= 0) return;
+    F.steps = (int)min((long long)nsteps, left);
+    F.tag = tag;
+    F.trouble = trouble;
+    F.X = xtab;
+    F.A = lds;
+    F.B = lds + RES_LDS_COLUMNS * Shape<SHAPE>::cs;
+    if (threadIdx.x == 0) {
+        u64 expect = GATE_SHUT;
+        const u64 n = __hip_atomic_fetch_add(&clk[CLK_ARRIVED], 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1ULL;
+        if (n == (u64)R.ntiles)
+            __hip_atomic_compare_exchange_strong(&clk[CLK_GATE], &expect, (u64)GATE_RUN, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+    }
+    F.load();
+    if (threadIdx.x == 0) {
+        u64 g;
+        for (int spins = 0; (g = take_word(&clk[CLK_GATE])) == GATE_SHUT; ++spins) {
+            if (spins >= wait_limit) {
+                u64 expect = GATE_SHUT;
+                if (__hip_atomic_compare_exchange_strong(&clk[CLK_GATE], &expect, (u64)GATE_GIVEN_UP, __ATOMIC_RELAXED,
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                    __hip_atomic_store(trouble, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            } else {
+                __builtin_amdgcn_s_sleep(4);
+            }
+        }
+        gate = g == GATE_RUN;
+    }
+    __syncthreads();
+    if (!gate) return;
+    switch (t.damped) {
+    case 0: run_plain<SHAPE>(F); break;
+    case 1: run_one<SHAPE, 0>(F); break;
+    case 2: run_one<SHAPE, 1>(F); break;
+    case 4: run_one<SHAPE, 2>(F); break;
+    default: run_more<SHAPE>(F); break;
+    }
+}
+
+}  // namespace
+
+ResShape resident_shape(int shape)
+{
+    auto of = [](auto c) {
+        using C = decltype(c);
+        return ResShape{C::plain, C::one, C::more, C::cs, C::words * RES_THREADS, C::recs * RES_THREADS};
+    };
+    return shape == RES_FINE ? of(Shape<RES_FINE>{}) : of(Shape<RES_COARSE>{});
+}
+
+static size_t lds_bytes(int shape) { return sizeof(float) * 2 * (size_t)RES_LDS_COLUMNS * resident_shape(shape).column_words; }
+
+int resident_capacity(int shape)
+{
+    int dev = 0, cus = 0, per = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    const size_t bytes = lds_bytes(shape);
+    const hipError_t e = shape == RES_FINE
+                             ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, resident_kernel<RES_FINE>, RES_THREADS, bytes)
+                             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, resident_kernel<RES_COARSE>, RES_THREADS, bytes);
+    if (e != hipSuccess) return 0;
+    return per * cus;
+}
+
+hipError_t launch_resident_routes(const ResScene *scene, int ntiles, int shape, hipStream_t s)
+{
+    if (ntiles <= 0) return hipSuccess;
+    if (shape == RES_FINE)
+        hipLaunchKernelGGL(route_kernel<Shape<RES_FINE>::cs>, dim3(ntiles), dim3(RES_THREADS), 0, s, scene);
+    else
+        hipLaunchKernelGGL(route_kernel<Shape<RES_COARSE>::cs>, dim3(ntiles), dim3(RES_THREADS), 0, s, scene);
+    return hipGetLastError();
+}
+
+hipError_t launch_resident(int shape, const ResItem *items, int n, int nsteps, uint32_t tag, int wait_limit,
+                           int *trouble, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    const size_t bytes = lds_bytes(shape);
+    if (shape == RES_FINE)
+        hipLaunchKernelGGL(resident_kernel<RES_FINE>, dim3(n), dim3(RES_THREADS), bytes, s, items, nsteps, tag, wait_limit, trouble);
+    else
+        hipLaunchKernelGGL(resident_kernel<RES_COARSE>, dim3(n), dim3(RES_THREADS), bytes, s, items, nsteps, tag, wait_limit, trouble);
+    return hipGetLastError();
+}
+
+}  // namespace fdtd

@@ -1,0 +1,406 @@
+// resident_plan.cpp -- which scenes run resident, how they are cut into tiles, and
+// the launch lists of resident scenes.
+#include "resident.h"
+
+#include <algorithm>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
+
+#include "device_scene.h"
+
+namespace fdtd {
+
+const char *resident_refusal(const SceneSetup &S)
+{
+    if (S.scheme != FDTD_SCHEME_COLLOCATED) return "staggered scheme";
+    if (S.abc) return "Engquist boundary";
+    if (S.moving) return "moving objects";
+    if (S.visc) return "air viscosity";
+    if (!S.cons.empty()) return "plane constraints";
+    if (!S.spk.empty()) return "speaker sources";
+    if (S.boundary != FDTD_BOUNDARY_RASTERIZE) return "coupled ghost cells";
+    if (S.n_cpo != 1) return "acceleration noise";
+    if (S.slabs.empty()) return "no PML";
+    for (const PmlSlab &sl : S.slabs)
+        if (!sl.merge) return "split PML state";
+    // a cell is damped along an axis exactly where that axis's segment says
+    // so, and every face of a damped cell but the walls is a PML face
+    for (int d = 0; d < 3; ++d) {
+        for (int i = 0; i < S.n[d]; ++i)
+            if ((S.cpml[d][i] != 0) == axis_plain(S, d, i)) return "PML cells without damping";
+        for (int i = 1; i < S.n[d]; ++i)
+            if ((S.fpml[d][i] != 0) != (S.cpml[d][i - 1] || S.cpml[d][i])) return "PML faces off the PML cells";
+        for (int i = S.inner_lo[d]; i < S.inner_hi[d]; ++i)
+            if (S.f2[d][i] != S.f2[d][S.inner_lo[d]] || S.f2[d][i + 1] != S.f2[d][S.inner_lo[d]] ||
+                S.f5h[d][i] != S.f5h[d][S.inner_lo[d]])
+                return "uneven coefficients outside the PML";
+    }
+    // a record takes one object's acceleration
+    for (const SpecialRec &r : S.special) {
+        int obj = -1;
+        for (int q = 0; q < 6; ++q) {
+            if (r.gid[q] < 0) continue;
+            if (obj >= 0 && S.ghosts[r.gid[q]].obj != obj) return "a cell between two objects";
+            obj = S.ghosts[r.gid[q]].obj;
+        }
+    }
+    return nullptr;
+}
+
+int ResPlan::tile_of(int i, int j, int k) const
+{
+    const int x[3] = {i, j, k};
+    for (const ResBox &b : boxes) {
+        int q[3];
+        bool in = true;
+        for (int d = 0; d < 3; ++d) {
+            const int at = x[d] - b.lo[d];
+            in = in && at >= 0 && at < b.len[d];
+            q[d] = at / b.size[d];
+        }
+        if (in) return b.first + (q[0] * b.count[1] + q[1]) * b.count[2] + q[2];
+    }
+    return -1;
+}
+
+static int pieces(int len, int most) { return (len + most - 1) / most; }
+
+bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
+{
+    const SceneSetup &S = D.S;
+    const ResShape sh = resident_shape(shape);
+    P = ResPlan();
+    P.shape = shape;
+    uint64_t words = 0;
+    for (int c = 0; c < 27; ++c) {
+        const int seg[3] = {c / 9, c / 3 % 3, c % 3};
+        ResBox b{};
+        bool some = true;
+        for (int d = 0; d < 3; ++d) {
+            const int cut[4] = {0, S.inner_lo[d], S.inner_hi[d], S.n[d]};
+            b.lo[d] = cut[seg[d]];
+            b.len[d] = cut[seg[d] + 1] - cut[seg[d]];
+            if (seg[d] != 1) b.damped |= 1 << d;
+            some = some && b.len[d] > 0;
+        }
+        if (!some) continue;
+        const int axes = (b.damped & 1) + (b.damped >> 1 & 1) + (b.damped >> 2 & 1);
+        const int most = axes == 0 ? sh.plain : axes == 1 ? sh.one : sh.more;
+        b.size[0] = pieces(b.len[0], pieces(b.len[0], most));
+        // y and z edges: the fewest tiles, then the least face per tile
+        int best = 1 << 30, face = 1 << 30;
+        for (int m = 1; m <= b.len[1]; ++m) {
+            const int y = pieces(b.len[1], m);
+            int z = std::min(b.len[2], RES_COLUMNS / y);
+            while (z > 1 && 2 * (y * z + b.size[0] * (y + z)) > sh.max_words) --z;
+            if (z < 1 || 2 * (y * z + b.size[0] * (y + z)) > sh.max_words) continue;
+            const int mz = pieces(b.len[2], z);
+            z = pieces(b.len[2], mz);
+            if ((y + 2) * (z + 2) > RES_LDS_COLUMNS) continue;
+            const int n = pieces(b.len[1], y) * mz;
+            if (n < best || (n == best && y + z < face)) {
+                best = n;
+                face = y + z;
+                b.size[1] = y;
+                b.size[2] = z;
+            }
+        }
+        if (best == 1 << 30) return false;
+        for (int d = 0; d < 3; ++d) b.count[d] = pieces(b.len[d], b.size[d]);
+        b.first = (int)P.tiles.size();
+        b.slab = -1;
+        for (int q = 0; q < (int)S.slabs.size() && b.damped; ++q) {
+            bool in = true;
+            for (int d = 0; d < 3; ++d)
+                in = in && b.lo[d] >= S.slabs[q].lo[d] && b.lo[d] + b.len[d] <= S.slabs[q].lo[d] + S.slabs[q].e[d];
+            if (in) b.slab = q;
+        }
+        if (b.damped && b.slab < 0) return false;
+        // one damped axis is the slab's own
+        if (axes == 1 && S.slabs[b.slab].axis != (b.damped == 1 ? 0 : b.damped == 2 ? 1 : 2)) return false;
+        for (int x = 0; x < b.count[0]; ++x)
+            for (int y = 0; y < b.count[1]; ++y)
+                for (int z = 0; z < b.count[2]; ++z) {
+                    ResTile t{};
+                    t.i0 = b.lo[0] + x * b.size[0];
+                    t.j0 = b.lo[1] + y * b.size[1];
+                    t.k0 = b.lo[2] + z * b.size[2];
+                    t.bx = std::min(b.size[0], b.lo[0] + b.len[0] - t.i0);
+                    t.by = std::min(b.size[1], b.lo[1] + b.len[1] - t.j0);
+                    t.bz = std::min(b.size[2], b.lo[2] + b.len[2] - t.k0);
+                    t.damped = b.damped;
+                    t.slab = b.slab;
+                    t.words = 2 * (t.by * t.bz + t.bx * t.bz + t.bx * t.by);
+                    t.word0 = (uint32_t)words;
+                    words += (uint64_t)((t.words + 7) & ~7);
+                    const int lo[3] = {t.i0, t.j0, t.k0}, hi[3] = {t.i0 + t.bx, t.j0 + t.by, t.k0 + t.bz};
+                    for (const PSrcHost &p : S.psrc) {
+                        bool hit = b.damped == 0;
+                        for (int d = 0; d < 3; ++d) hit = hit && lo[d] < p.hi[d] && hi[d] > p.lo[d];
+                        t.src |= hit;
+                    }
+                    for (const SpecialBox &bx : S.boxes) {
+                        bool hit = b.damped == 0;
+                        for (int d = 0; d < 3; ++d) hit = hit && lo[d] < bx.hi[d] && hi[d] > bx.lo[d];
+                        t.skip |= hit;
+                    }
+                    P.tiles.push_back(t);
+                }
+        P.boxes.push_back(b);
+    }
+    if (words >= RES_NOWHERE) return false;
+    P.nwords = (uint32_t)words;
+    // records and listener terms by tile
+    const int sy = S.n[2], sx = S.n[1] * S.n[2];
+    auto tile_of = [&](int cell) { return P.tile_of(cell / sx, cell % sx / sy, cell % sy); };
+    std::vector<std::pair<int, int>> by;
+    for (int r = 0; r < (int)S.special.size(); ++r) by.push_back({tile_of(S.special[r].cell), r});
+    std::sort(by.begin(), by.end());
+    for (const auto &e : by) {
+        if (e.first < 0) return false;
+        ResTile &t = P.tiles[e.first];
+        if (t.damped || !t.skip) return false;
+        if (t.re == t.rb) t.rb = (int)P.recs.size();
+        P.recs.push_back(e.second);
+        t.re = (int)P.recs.size();
+        if (t.re - t.rb > sh.max_recs) return false;
+    }
+    by.clear();
+    for (int q = 0; q < (int)S.lst_terms.size(); ++q) {
+        const ListenerTerm &lt = S.lst_terms[q];
+        by.push_back({tile_of(lt.kind == 0 ? lt.index : S.ghosts[lt.index].nbr), q});
+    }
+    std::sort(by.begin(), by.end());
+    for (const auto &e : by) {
+        if (e.first < 0) return false;
+        ResTile &t = P.tiles[e.first];
+        const ListenerTerm &lt = S.lst_terms[e.second];
+        if (t.te == t.tb) t.tb = (int)P.terms.size();
+        P.terms.push_back({0, e.second, lt.kind, lt.kind == 0 ? (int)D.to_dev(lt.index) : lt.index, lt.beta});
+        t.te = (int)P.terms.size();
+    }
+    return true;
+}
+
+std::string resident_check(const DeviceScene &D, int shape)
+{
+    const SceneSetup &S = D.S;
+    if (resident_refusal(S)) return std::string();
+    ResPlan P;
+    if (!resident_plan(D, shape, P)) return std::string();
+    const ResShape sh = resident_shape(shape);
+    std::vector<uint8_t> hit((size_t)S.N, 0);
+    std::vector<int> recs(S.special.size(), 0), terms(S.lst_terms.size(), 0);
+    uint64_t word = 0;
+    for (size_t q = 0; q < P.tiles.size(); ++q) {
+        const ResTile &t = P.tiles[q];
+        const int axes = (t.damped & 1) + (t.damped >> 1 & 1) + (t.damped >> 2 & 1);
+        const int most = axes == 0 ? sh.plain : axes == 1 ? sh.one : sh.more;
+        if (t.bx < 1 || t.by < 1 || t.bz < 1 || t.bx > most || t.by * t.bz > RES_COLUMNS) return "resident tile too large";
+        if ((t.by + 2) * (t.bz + 2) > RES_LDS_COLUMNS || t.words > sh.max_words) return "resident tile's halo too large";
+        if (t.words != 2 * (t.by * t.bz + t.bx * t.bz + t.bx * t.by)) return "resident tile's face words";
+        if (t.word0 < word || (uint64_t)t.word0 + (uint64_t)t.words > P.nwords) return "resident tiles share exchange words";
+        word = (uint64_t)t.word0 + (uint64_t)t.words;
+        for (int i = t.i0; i < t.i0 + t.bx; ++i)
+            for (int j = t.j0; j < t.j0 + t.by; ++j)
+                for (int k = t.k0; k < t.k0 + t.bz; ++k) {
+                    if (i < 0 || j < 0 || k < 0 || i >= S.n[0] || j >= S.n[1] || k >= S.n[2]) return "resident tile outside the grid";
+                    if (hit[((size_t)i * S.n[1] + j) * S.n[2] + k]++) return "a cell lies in two resident tiles";
+                    const int damped = (S.cpml[0][i] ? 1 : 0) | (S.cpml[1][j] ? 2 : 0) | (S.cpml[2][k] ? 4 : 0);
+                    if (damped != t.damped) return "a resident tile's class does not fit its cells";
+                    if (P.tile_of(i, j, k) != (int)q) return "resident tile lookup";
+                }
+        for (int r = t.rb; r < t.re; ++r) ++recs[P.recs[r]];
+        if (t.re - t.rb > sh.max_recs || (t.re > t.rb && (t.damped || !t.skip))) return "resident records";
+        for (int r = t.tb; r < t.te; ++r) ++terms[P.terms[r].slot];
+    }
+    for (uint8_t h : hit)
+        if (h != 1) return "a cell lies in no resident tile";
+    for (int c : recs)
+        if (c != 1) return "an object-adjacent record is not in exactly one resident tile";
+    for (int c : terms)
+        if (c != 1) return "a listener term is not in exactly one resident tile";
+    return std::string();
+}
+
+bool ResidentScene::build(const DeviceScene &D, hipStream_t st, size_t max_bytes)
+{
+    release();
+    if (resident_refusal(D.S)) return false;
+    bool ok = false;
+    for (int shape = RES_FINE; shape < RES_SHAPES && !ok; ++shape)
+        ok = resident_plan(D, shape, plan) && ((int)plan.tiles.size() + 7) / 8 * 8 <= resident_capacity(shape);
+    if (!ok) return false;
+    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t b[7] = {al(sizeof(ResScene)), al(sizeof(ResTile) * plan.tiles.size()), al(sizeof(ResBox) * plan.boxes.size()),
+                         al(sizeof(int32_t) * plan.recs.size()), al(sizeof(TermRef) * plan.terms.size()),
+                         al(sizeof(ResRoute) * (size_t)plan.nwords), al(sizeof(unsigned long long) * 2 * (size_t)plan.nwords)};
+    bytes = 0;
+    for (size_t x : b) bytes += x;
+    if (bytes > max_bytes) { bytes = 0; return false; }
+    if (hipMalloc(&mem, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        mem = nullptr;
+        bytes = 0;
+        return false;
+    }
+    char *at[7];
+    char *p = mem;
+    for (int q = 0; q < 7; ++q) { at[q] = p; p += b[q]; }
+    dev = reinterpret_cast<ResScene *>(at[0]);
+    ResScene R{};
+    R.S = D.self;
+    R.tiles = reinterpret_cast<ResTile *>(at[1]);
+    R.boxes = reinterpret_cast<ResBox *>(at[2]);
+    R.recs = reinterpret_cast<int32_t *>(at[3]);
+    R.terms = reinterpret_cast<TermRef *>(at[4]);
+    R.route = reinterpret_cast<ResRoute *>(at[5]);
+    R.words = reinterpret_cast<unsigned long long *>(at[6]);
+    R.nwords = plan.nwords;
+    R.ntiles = (int)plan.tiles.size();
+    R.nboxes = (int)plan.boxes.size();
+    // the tables in one copy
+    std::vector<char> stage((size_t)(at[5] - mem), 0);
+    auto put = [&](int q, const void *src, size_t n) { if (n) std::memcpy(stage.data() + (at[q] - mem), src, n); };
+    put(0, &R, sizeof R);
+    put(1, plan.tiles.data(), sizeof(ResTile) * plan.tiles.size());
+    put(2, plan.boxes.data(), sizeof(ResBox) * plan.boxes.size());
+    put(3, plan.recs.data(), sizeof(int32_t) * plan.recs.size());
+    put(4, plan.terms.data(), sizeof(TermRef) * plan.terms.size());
+    ok = hipMemcpyAsync(mem, stage.data(), stage.size(), hipMemcpyHostToDevice, st) == hipSuccess &&
+         hipMemsetAsync(at[6], 0, b[6], st) == hipSuccess &&
+         launch_resident_routes(dev, R.ntiles, plan.shape, st) == hipSuccess && hipStreamSynchronize(st) == hipSuccess;
+    if (!ok) release();
+    return ok;
+}
+
+void ResidentScene::release()
+{
+    if (mem) (void)hipFree(mem);
+    mem = nullptr;
+    dev = nullptr;
+    bytes = 0;
+}
+
+fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &scenes, hipStream_t st)
+{
+    if (items) (void)hipFree(items);
+    items = nullptr;
+    n = 0;
+    if (scenes.empty()) return FDTD_OK;
+    std::vector<ResItem> list;
+    shape = scenes[0]->plan.shape;
+    // Workgroups are dispatched in list order, and a scene starts when all of
+    // its own are on the device: scenes that fill the device together stand
+    // next to each other (largest first, each into the first group with room).
+    const int room = resident_capacity(shape);
+    std::vector<const ResidentScene *> order(scenes);
+    std::stable_sort(order.begin(), order.end(), [](const ResidentScene *a, const ResidentScene *b) {
+        return a->plan.tiles.size() > b->plan.tiles.size();
+    });
+    std::vector<std::vector<const ResidentScene *>> groups;
+    std::vector<int> used;
+    for (const ResidentScene *s : order) {
+        const int m = ((int)s->plan.tiles.size() + 7) / 8 * 8;
+        size_t g = 0;
+        while (g < groups.size() && used[g] + m > room) ++g;
+        if (g == groups.size()) { groups.emplace_back(); used.push_back(0); }
+        groups[g].push_back(s);
+        used[g] += m;
+    }
+    order.clear();
+    for (const auto &g : groups) order.insert(order.end(), g.begin(), g.end());
+    for (const ResidentScene *s : order) {
+        const int m = (int)s->plan.tiles.size(), per = (m + 7) / 8;
+        // workgroup w runs on XCD w % 8: a run of consecutive tiles per XCD,
+        // so that most neighbours share one (1024 workgroups: 3.0 us per
+        // exchange against 3.9 with tiles dealt out in turn)
+        for (int w = 0; w < 8 * per; ++w) {
+            const int t = (w % 8) * per + w / 8;
+            list.push_back(t < m ? ResItem{s->dev, t, 0} : ResItem{nullptr, 0, 0});
+        }
+    }
+    n = (int)list.size();
+    if (!trouble) {
+        FDTD_HIP_TRY(hipHostMalloc(&trouble, sizeof(int)));
+        *trouble = 0;
+    }
+    if (!wait_limit) {
+        // about a second; another launch that holds the device for longer
+        // sends this one's scenes to the step kernels
+        const char *w = std::getenv("FDTD_RESIDENT_WAIT");
+        wait_limit = w ? std::atoi(w) : 1 << 20;
+    }
+    FDTD_HIP_TRY(hipMalloc(&items, sizeof(ResItem) * list.size()));
+    FDTD_HIP_TRY(hipMemcpyAsync(items, list.data(), sizeof(ResItem) * list.size(), hipMemcpyHostToDevice, st));
+    FDTD_HIP_TRY(hipStreamSynchronize(st));
+    return FDTD_OK;
+}
+
+// Two resident launches on different streams could each hold a part of the
+// device and wait for the rest of it until both give up.  So launches of one
+// process follow each other on a device: a launch on another stream than the
+// one before waits for that stream's work so far.
+namespace {
+constexpr int kMaxDevices = 64;
+std::mutex g_order;
+hipStream_t g_last[kMaxDevices] = {};
+bool g_used[kMaxDevices] = {};
+}  // namespace
+
+static fdtd_status follow_last(hipStream_t st)
+{
+    int dev = 0;
+    FDTD_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices) return FDTD_ERR_DEVICE;
+    if (g_used[dev] && g_last[dev] != st) {
+        hipEvent_t e;
+        FDTD_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        hipError_t r = hipEventRecord(e, g_last[dev]);
+        if (r == hipSuccess) r = hipStreamWaitEvent(st, e, 0);
+        (void)hipEventDestroy(e);
+        FDTD_HIP_TRY(r);
+    }
+    g_used[dev] = true;
+    g_last[dev] = st;
+    return FDTD_OK;
+}
+
+void resident_forget_stream(hipStream_t st)
+{
+    std::lock_guard<std::mutex> lk(g_order);
+    for (int d = 0; d < kMaxDevices; ++d)
+        if (g_used[d] && g_last[d] == st) g_used[d] = false;
+}
+
+fdtd_status resident_reopen(const SceneDev &dev, long long *step)
+{
+    unsigned long long clk[CLK_WORDS];
+    FDTD_HIP_TRY(hipMemcpy(clk, dev.clock, sizeof clk, hipMemcpyDeviceToHost));
+    *step = (long long)clk[CLK_STEP];
+    clk[CLK_GATE] = GATE_SHUT;
+    FDTD_HIP_TRY(hipMemcpy(dev.clock + CLK_GATE, &clk[CLK_GATE], sizeof clk[0], hipMemcpyHostToDevice));
+    return FDTD_OK;
+}
+
+fdtd_status ResidentProgram::enqueue(hipStream_t st, int nsteps)
+{
+    std::lock_guard<std::mutex> lk(g_order);
+    const fdtd_status s = follow_last(st);
+    if (s != FDTD_OK) return s;
+    FDTD_HIP_TRY(launch_resident(shape, items, n, nsteps, tag, wait_limit, trouble, st));
+    tag += (uint32_t)nsteps + 1;
+    return FDTD_OK;
+}
+
+void ResidentProgram::release()
+{
+    if (items) (void)hipFree(items);
+    items = nullptr;
+    n = 0;
+    if (trouble) (void)hipHostFree(trouble);
+    trouble = nullptr;
+}
+
+}  // namespace fdtd

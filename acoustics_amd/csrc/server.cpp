@@ -27,6 +27,7 @@
 #include <thread>
 
 #include "device_scene.h"
+#include "resident.h"
 
 using namespace fdtd;
 
@@ -53,6 +54,7 @@ struct Request {
     // scene id 0 and term indices from 0; a rebuild only renumbers them
     std::vector<TileDesc> tiles;
     std::vector<TermRef> terms;
+    ResidentScene res;            // blocks run resident while res.mem is held
 };
 
 }  // namespace
@@ -77,11 +79,14 @@ struct fdtd_server {
     // host enqueues a block far faster than the device runs it, and a
     // rebuild needs no graph capture)
     StepProgram prog;
+    ResidentProgram res_prog[RES_SHAPES];
     bool dirty = true;
     int block = 64;
 
     void run();
     fdtd_status rebuild();
+    fdtd_status run_block();
+    fdtd_status settle();
     void finish(Request *r, fdtd_status st);
 };
 
@@ -89,6 +94,7 @@ void fdtd_server::finish(Request *r, fdtd_status st)
 {
     r->status = st;
     r->finished = Clock::now();
+    r->res.release();
     if (r->dev) { r->dev->release(); r->dev.reset(); }
     resident -= (int64_t)r->bytes;
     if (st == FDTD_OK) ++stats.completed;
@@ -104,15 +110,73 @@ fdtd_status fdtd_server::rebuild()
     std::vector<TileDesc> tiles;
     std::vector<TermRef> terms;
     std::vector<MotionDesc> motion;
+    std::vector<const ResidentScene *> resident_list[RES_SHAPES];
     for (Request *r : active) {
+        if (r->res.mem) resident_list[r->res.plan.shape].push_back(&r->res);
         const int id = (int)devs.size();
         devs.push_back(r->dev->dev);
         const int tb = (int)terms.size();
+        if (!r->res.mem && r->tiles.empty()) r->dev->append_tiles(0, tile_plan(0), r->tiles, r->terms);
+        if (r->res.mem) continue;
         for (TermRef q : r->terms) { q.scene = id; terms.push_back(q); }
         for (TileDesc t : r->tiles) { t.scene = id; t.tb += tb; t.te += tb; tiles.push_back(t); }
         if (r->dev->needs_motion_kernel()) motion.push_back({id});
     }
+    for (int shape = 0; shape < RES_SHAPES; ++shape) {
+        const fdtd_status s = res_prog[shape].upload(resident_list[shape], stream);
+        if (s != FDTD_OK) return s;
+    }
     return prog.upload(devs, tiles, terms, stream, tile_plan(0).fused, motion);
+}
+
+// One block of every active request: the step kernels of those that are not
+// resident, the resident launches, and the clocks, AMP_ROWS steps at a time.
+fdtd_status fdtd_server::run_block()
+{
+    if (res_prog[RES_FINE].n == 0 && res_prog[RES_COARSE].n == 0) return prog.enqueue(stream, 0, block);
+    bool kernels = false;
+    for (int k = 0; k < NUM_KINDS; ++k) kernels = kernels || prog.ntiles[k] > 0;
+    for (int done = 0; done < block;) {
+        const int blk = std::min(block - done, (int)AMP_ROWS);
+        for (int k = 0; k < blk && kernels; ++k) {
+            const fdtd_status s = prog.enqueue_step(stream, done + k, k);
+            if (s != FDTD_OK) return s;
+        }
+        for (ResidentProgram &p : res_prog) {
+            const fdtd_status s = p.enqueue(stream, blk);
+            if (s != FDTD_OK) return s;
+        }
+        FDTD_HIP_TRY(launch_advance(prog.d_scenes, prog.nscenes, blk, stream));
+        done += blk;
+    }
+    return FDTD_OK;
+}
+
+// After a block (the stream is idle): requests whose resident launch gave up
+// are where their clocks say and go on with the step kernels.
+fdtd_status fdtd_server::settle()
+{
+    bool gave_up = false;
+    for (const ResidentProgram &p : res_prog) {
+        if (p.trouble && *p.trouble > 1) return FDTD_ERR_DEVICE;
+        gave_up = gave_up || p.gave_up();
+    }
+    if (!gave_up) return FDTD_OK;
+    for (Request *r : active) {
+        if (!r->res.mem) continue;
+        long long at = 0;
+        const fdtd_status s = resident_reopen(r->dev->dev, &at);
+        if (s != FDTD_OK) return s;
+        if (at >= std::min<long long>(r->launched + block, r->steps)) continue;
+        r->launched = at - block;   // (the caller adds the block)
+        resident -= (int64_t)r->res.bytes;
+        r->bytes -= r->res.bytes;
+        r->res.release();
+        dirty = true;
+    }
+    for (ResidentProgram &p : res_prog)
+        if (p.trouble) *p.trouble = 0;
+    return FDTD_OK;
 }
 
 void fdtd_server::run()
@@ -151,8 +215,8 @@ void fdtd_server::run()
         // the block of the current resident set starts first; the admitted
         // requests upload on their own stream while it runs, and join the
         // work list at the next rebuild
-        const bool run_block = !active.empty() && !dirty;
-        if (run_block && prog.enqueue(stream, 0, block) != FDTD_OK) {
+        const bool stepping = !active.empty() && !dirty;
+        if (stepping && run_block() != FDTD_OK) {
             (void)hipStreamSynchronize(stream);
             std::lock_guard<std::mutex> lk(mu);
             set_last_error("step block failed on the device");
@@ -167,12 +231,20 @@ void fdtd_server::run()
             r->dev = std::make_unique<DeviceScene>();
             r->dev->S = std::move(r->setup);
             fdtd_status s = r->dev->allocate_and_upload(upload, std::max(1, r->steps), r->steps);
-            if (s == FDTD_OK) r->dev->append_tiles(0, tile_plan(0), r->tiles, r->terms);
+            // resident where it fits the device and the budget
+            if (s == FDTD_OK && r->res.build(*r->dev, upload, (size_t)std::max<int64_t>(0, opt.hbm_budget_bytes - resident))) {
+                std::lock_guard<std::mutex> lk(mu);
+                r->bytes += r->res.bytes;
+                resident += (int64_t)r->res.bytes;
+                stats.peak_resident_bytes = std::max(stats.peak_resident_bytes, resident);
+            } else if (s == FDTD_OK) {
+                r->dev->append_tiles(0, tile_plan(0), r->tiles, r->terms);
+            }
             std::lock_guard<std::mutex> lk(mu);
             if (s != FDTD_OK) { finish(r, s); done_cv.notify_all(); continue; }
             fresh.push_back(r);
         }
-        if (run_block && hipStreamSynchronize(stream) != hipSuccess) {
+        if (stepping && (hipStreamSynchronize(stream) != hipSuccess || settle() != FDTD_OK)) {
             std::lock_guard<std::mutex> lk(mu);
             set_last_error("step block failed on the device");
             for (Request *r : active) finish(r, FDTD_ERR_DEVICE);
@@ -186,7 +258,7 @@ void fdtd_server::run()
             // a client that sees a request finished may take (and free) it at
             // once, so no worker list may still hold it when the lock drops
             std::lock_guard<std::mutex> lk(mu);
-            if (run_block) {
+            if (stepping) {
                 ++stats.blocks_run;
                 // every kEvictCheckBlocks blocks, a request whose latest
                 // listener row is no longer finite (a blown-up scene: NaN
@@ -240,6 +312,9 @@ void fdtd_server::run()
         }
     }
     prog.release();
+    (void)hipStreamSynchronize(stream);
+    resident_forget_stream(stream);
+    for (ResidentProgram &p : res_prog) p.release();
     std::lock_guard<std::mutex> lk(mu);
     for (Request *r : active) finish(r, FDTD_ERR_CANCELLED);
     active.clear();
@@ -382,6 +457,10 @@ fdtd_status fdtd_plan_check(const fdtd_scene *scene, int tile_config, int64_t *n
     }
     for (int h : rec_hits)
         if (h != 1) return fail("an object-adjacent record is covered " + std::to_string(h) + " times");
+    for (int shape = 0; shape < RES_SHAPES; ++shape) {
+        const std::string e2 = resident_check(D, shape);
+        if (!e2.empty()) return fail(e2);
+    }
     if (n_tiles) {
         int64_t n = 0;
         for (int k = 0; k < NUM_KINDS; ++k) n += (int64_t)lists[k].size();

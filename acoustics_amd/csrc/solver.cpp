@@ -10,6 +10,7 @@
 #include <new>
 
 #include "device_scene.h"
+#include "resident.h"
 
 using namespace fdtd;
 
@@ -20,6 +21,10 @@ const std::string &get_last_error();
 struct fdtd_handle {
     DeviceScene D;
     StepProgram prog;
+    // blocks of steps with the scene held on the chip, where it fits (the
+    // step kernels run single steps, and the whole scene elsewhere)
+    ResidentScene res;
+    ResidentProgram res_prog;
     hipStream_t stream = nullptr;
     bool own_stream = false;
     int tile = 0;
@@ -129,7 +134,12 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
         if (h->D.needs_motion_kernel()) motion.push_back({0});
         st = h->prog.upload({h->D.dev}, tiles, terms, h->stream, tile_plan(h->tile).fused, motion);
     }
+    // a tile plan or graph blocks that the caller asked for are what runs
+    if (st == FDTD_OK && opt.tile_config < 0 && h->graph_steps == 0 && h->res.build(h->D, h->stream))
+        st = h->res_prog.upload({&h->res}, h->stream);
     if (st != FDTD_OK) {
+        h->res_prog.release();
+        h->res.release();
         h->prog.release();
         h->D.release();
         if (h->own_stream) (void)hipStreamDestroy(h->stream);
@@ -153,10 +163,38 @@ fdtd_status fdtd_destroy(fdtd_handle *h)
     for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
     if (h->call_begin) (void)hipEventDestroy(h->call_begin);
     if (h->call_end) (void)hipEventDestroy(h->call_end);
+    resident_forget_stream(h->stream);
+    h->res_prog.release();
+    h->res.release();
     h->prog.release();
     h->D.release();
     if (h->own_stream) (void)hipStreamDestroy(h->stream);
     delete h;
+    return FDTD_OK;
+}
+
+// Waits for the stream and completes steps that a resident launch gave up
+// (its workgroups could not all be on the device at once): the step kernels
+// run them, and the scene from then on.
+static fdtd_status settle(fdtd_handle *h)
+{
+    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    if (!h->res_prog.trouble || *h->res_prog.trouble == 0) return FDTD_OK;
+    if (*h->res_prog.trouble > 1) { set_last_error("a resident launch lost its neighbours"); return FDTD_ERR_DEVICE; }
+    *h->res_prog.trouble = 0;
+    h->res_prog.n = 0;
+    long long at = 0;
+    {
+        const fdtd_status st = resident_reopen(h->D.dev, &at);
+        if (st != FDTD_OK) return st;
+    }
+    for (long long s = at; s < h->step;) {
+        const int n = (int)std::min({h->step - s, (long long)AMP_ROWS, (long long)h->D.series_cap});
+        const fdtd_status st = h->prog.enqueue(h->stream, s, n);
+        if (st != FDTD_OK) return st;
+        s += n;
+    }
+    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
     return FDTD_OK;
 }
 
@@ -165,7 +203,10 @@ static fdtd_status flush_series(fdtd_handle *h)
 {
     const int L = h->D.S.L;
     if (h->flushed == h->step) return FDTD_OK;
-    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    {
+        const fdtd_status st = settle(h);
+        if (st != FDTD_OK) return st;
+    }
     if (L == 0) { h->flushed = h->step; return FDTD_OK; }
     const long long rows = h->step - h->flushed;
     const int cap = h->D.series_cap;
@@ -196,6 +237,16 @@ static fdtd_status build_graph(fdtd_handle *h)
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) { set_last_error(std::string("graph instantiate: ") + hipGetErrorString(e)); return FDTD_ERR_DEVICE; }
     return FDTD_OK;
+}
+
+// Fewer steps than this run as step kernels: a resident launch loads and
+// stores the whole state.
+constexpr int kResidentSteps = 4;
+
+static bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
 }
 
 fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
@@ -244,6 +295,10 @@ fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
                 if (st != FDTD_OK) return st;
             }
             FDTD_HIP_TRY(hipGraphLaunch(h->graph_exec, h->stream));
+        } else if (h->res_prog.n > 0 && !per_step && block >= kResidentSteps && !capturing(h->stream)) {
+            fdtd_status st = h->res_prog.enqueue(h->stream, block);
+            if (st != FDTD_OK) return st;
+            FDTD_HIP_TRY(launch_advance(h->D.self, 1, block, h->stream));
         } else {
             fdtd_status st = h->prog.enqueue(h->stream, h->step, block, per_step ? &h->ev[2 * done] : nullptr);
             if (st != FDTD_OK) return st;
@@ -259,8 +314,7 @@ fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
 fdtd_status fdtd_synchronize(fdtd_handle *h)
 {
     if (!h) return FDTD_ERR_INVALID;
-    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
-    return FDTD_OK;
+    return settle(h);
 }
 
 fdtd_status fdtd_set_timing(fdtd_handle *h, int enable)
@@ -319,7 +373,8 @@ fdtd_status fdtd_read_listener_series(fdtd_handle *h, int64_t first, int64_t n, 
 fdtd_status fdtd_read_pressure(fdtd_handle *h, double *out)
 {
     if (!h || !out) return FDTD_ERR_INVALID;
-    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    const fdtd_status st = settle(h);
+    if (st != FDTD_OK) return st;
     const int slot = slot_cur(h->step);  // p^{step}: the newest field
     std::vector<float> tmp((size_t)h->D.S.N);
     FDTD_HIP_TRY(h->D.download_grid(h->D.slot(slot), tmp.data()));
@@ -442,7 +497,10 @@ fdtd_status fdtd_save_snapshot(fdtd_handle *h, const char *pattern, const char *
         return FDTD_ERR_UNSUPPORTED;
     }
     FDTD_HIP_TRY(hipSetDevice(h->D.device));
-    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    {
+        const fdtd_status st = settle(h);
+        if (st != FDTD_OK) return st;
+    }
     const SceneSetup &S = h->D.S;
     const long long N = S.N, s = h->step;
     const bool mac = S.scheme == FDTD_SCHEME_STAGGERED;
@@ -583,7 +641,10 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
         return FDTD_ERR_UNSUPPORTED;
     }
     FDTD_HIP_TRY(hipSetDevice(h->D.device));
-    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    {
+        const fdtd_status st = settle(h);
+        if (st != FDTD_OK) return st;
+    }
     const SceneSetup &S = h->D.S;
     const long long N = S.N;
     const bool mac = S.scheme == FDTD_SCHEME_STAGGERED;
