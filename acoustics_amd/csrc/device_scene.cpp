@@ -62,6 +62,8 @@ struct Layout {
     SceneDev *self;
 };
 
+static int amp_rows(const SceneSetup &S) { return S.amp_rows ? S.amp_rows : (int)AMP_ROWS; }
+
 // cells of a moving scene's reclassified box
 static size_t moving_cells(const SceneSetup &S)
 {
@@ -128,16 +130,16 @@ void carve(const SceneSetup &S, int cap, Carver &cs, Carver &c, Layout &L)
     L.oc_w = c.take<double>(S.oc_w.size());
     L.terms = c.take<double>((size_t)cap * std::max<size_t>(1, S.lst_terms.size()));
     L.clock = c.take<unsigned long long>(CLK_WORDS);
-    L.t_tab = c.take<double>(AMP_ROWS);
-    L.acc_tab = c.take<double>((size_t)AMP_ROWS * S.objs.size() * S.n_cpo);
-    L.src_tab = c.take<float>((size_t)AMP_ROWS * S.psrc.size());
+    L.t_tab = c.take<double>(amp_rows(S));
+    L.acc_tab = c.take<double>((size_t)amp_rows(S) * S.objs.size() * S.n_cpo);
+    L.src_tab = c.take<float>((size_t)amp_rows(S) * S.psrc.size());
     L.spk = c.take<double>(8 * S.spk.size());
     L.spk_samples = c.take<double>(S.spk_samples.size());
     L.spk_field = c.take<float>(S.spk.empty() ? 0 : (size_t)(S.spk_hi[0] - S.spk_lo[0]) * (S.spk_hi[1] - S.spk_lo[1]) * (S.spk_hi[2] - S.spk_lo[2]));
     L.ucls = c.take<uint8_t>(2 * moving_cells(S));
     L.mobj = c.take<MoveDev>(S.moving ? S.objs.size() : 0);
     L.kin = c.take<double>(S.kin.size());
-    L.pose = c.take<Geom>(S.moving ? (size_t)AMP_ROWS * S.objs.size() : 0);
+    L.pose = c.take<Geom>(S.moving ? (size_t)amp_rows(S) * S.objs.size() : 0);
     L.ughost = c.take<double>(6 * moving_cells(S));
     L.self = c.take<SceneDev>(1);
 }
@@ -226,7 +228,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
     FDTD_HIP_TRY(hipMemsetAsync(L.terms, 0, sizeof(double) * (size_t)cap * std::max<size_t>(1, S.lst_terms.size()), st));
     // the acceleration ring reads as zero where no object refills it (a
     // constraint's ghost entries weight it by zero)
-    FDTD_HIP_TRY(hipMemsetAsync(L.acc_tab, 0, sizeof(double) * std::max<size_t>(1, (size_t)AMP_ROWS * S.objs.size() * S.n_cpo), st));
+    FDTD_HIP_TRY(hipMemsetAsync(L.acc_tab, 0, sizeof(double) * std::max<size_t>(1, (size_t)amp_rows(S) * S.objs.size() * S.n_cpo), st));
     std::vector<char> staging;  // pageable copies are synchronised before return
     auto up = [&](void *dst, const void *src, size_t bytes) -> hipError_t {
         if (!bytes) return hipSuccess;
@@ -371,6 +373,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
     D.seven = S.sampling == FDTD_SAMPLE_SEVEN ? 1 : 0;
     D.n_cpo = S.n_cpo;
     D.n_ch = D.n_obj * S.n_cpo;
+    D.amp_rows = amp_rows(S);
     D.t_tab = L.t_tab;
     D.acc_tab = L.acc_tab;
     D.src_tab = L.src_tab;

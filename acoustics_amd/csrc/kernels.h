@@ -79,11 +79,13 @@ inline void clock_words(unsigned long long *clk, long long s, unsigned long long
 
 // Steps are launched in blocks: the kernels of the k-th step of a block run
 // step clock[CLK_STEP] + k, and one advance kernel after the block moves the
-// counter on.  The per-step amplitudes live in a ring of AMP_ROWS rows (step
-// s in row s & (AMP_ROWS - 1)) that the advance kernel refills for the next
-// AMP_ROWS steps, so a block is at most AMP_ROWS steps long.
-enum : int { AMP_ROWS = 64 };
-__host__ __device__ inline int amp_row(long long s) { return (int)(s & (AMP_ROWS - 1)); }
+// counter on.  The per-step amplitudes live in a ring of SceneDev::amp_rows rows
+// (a power of two; step s in row s & (amp_rows - 1)) that the advance kernel
+// keeps filled for the next amp_rows steps, so a block is at most that long.
+// AMP_ROWS is what scenes have unless their memory is bounded: a resident
+// block costs about 15 us beside its steps, 10% of a 64^3 step with blocks of
+// 64 and 3% with 256.
+enum : int { AMP_ROWS = 256, AMP_ROWS_BOUNDED = 64 };
 
 // a moving object: its pose at t = 0 and its constant velocity and angular velocity
 // Motion of one object: constant velocity v and angular velocity w from
@@ -147,9 +149,10 @@ struct SceneDev {
     int seven;
     int n_cpo, n_ch;            // amplitude channels per object (1, or 4 with acceleration noise), n_obj n_cpo
     // time-dependent amplitudes, one ring row per step (amp_row):
-    double *t_tab;              // [AMP_ROWS] the accumulated time of the step (CLK_TIME)
-    double *acc_tab;            // [AMP_ROWS][n_ch] channel o n_cpo: a_s(o, t_s); o n_cpo + 1 + d: a_v(o, t_s)[d]
-    float *src_tab;             // [AMP_ROWS][n_psrc] S(t_s + dt/2) dt without the spatial factor
+    int amp_rows;
+    double *t_tab;              // [amp_rows] the accumulated time of the step (CLK_TIME)
+    double *acc_tab;            // [amp_rows][n_ch] channel o n_cpo: a_s(o, t_s); o n_cpo + 1 + d: a_v(o, t_s)[d]
+    float *src_tab;             // [amp_rows][n_psrc] S(t_s + dt/2) dt without the spatial factor
     long long src_steps;        // time-parallel chunk: sources act in steps < src_steps (-1: always)
     // speaker sources: per source {px, py, pz, w, t0, period, off, n} and the samples
     int n_spk;
@@ -167,10 +170,13 @@ struct SceneDev {
     uint8_t *ucls;              // [2][u_n0 u_n1 u_n2], z fastest: 1 bulk, 0 solid
     const MoveDev *mobj;        // [n_obj]
     const double *kin;          // keyframes, 8 doubles each
-    Geom *pose;                 // [AMP_ROWS][n_obj]
+    Geom *pose;                 // [amp_rows][n_obj]
     double *ughost;             // [6][u cells]: ghost term of each solid neighbour of a fluid cell (-x, +x, ..., +z)
     double h, rho, bmin[3];
 };
+
+// ring row of step s's amplitudes, times and poses
+__host__ __device__ inline int amp_row(const SceneDev &S, long long s) { return (int)(s & (long long)(S.amp_rows - 1)); }
 
 // A listener term handled by the tile that produces its sample: kind 0 is
 // the new pressure of flat cell `cell`; kind 1 the value of ghost entry
@@ -220,8 +226,8 @@ enum : int { KIND_INTERIOR = 0, KIND_PML = 1, KIND_SPECIAL = 2, NUM_KINDS = 3, K
 hipError_t launch_step(int kind, const SceneDev *scenes, const TileDesc *tiles, int ntiles, int nhead, const TermRef *terms,
                        const unsigned long long *order_clock, int k, hipStream_t s);
 // Moves every scene of the launch n steps on (clamped to its target) and
-// refills its amplitude and pose rings for the AMP_ROWS steps from there;
-// n = 0 only fills the rings.
+// keeps its amplitude and pose rings filled for the steps from there; n = 0
+// fills the rings anew.
 hipError_t launch_advance(const SceneDev *scenes, int nscenes, int n, hipStream_t s);
 // Moving objects, before the step kernels of step clock + k, in one launch:
 // per-step reclassification of each scene's box, zeroed new solid cells,

@@ -74,7 +74,8 @@ extern "C" fdtd_status fdtd_solve_noalloc(const fdtd_scene *scene, int num_steps
         set_last_error("moving objects are planned up to stop_time (" + std::to_string(D.S.mv_steps) + " steps)");
         return FDTD_ERR_INVALID;
     }
-    const int cap = AMP_ROWS;   // one step block of listener rows, read out after each block
+    D.S.amp_rows = AMP_ROWS_BOUNDED;   // the scratch is bounded
+    const int cap = AMP_ROWS_BOUNDED;   // one step block of listener rows, read out after each block
     size_t state_b = 0, table_b = 0;
     DeviceScene::region_bytes(D.S, cap, &state_b, &table_b);
     if (fields_bytes_needed) *fields_bytes_needed = (int64_t)state_b;

@@ -21,9 +21,7 @@ namespace fdtd {
 // Cells of one class form up to 27 boxes (the products of the three segments
 // of each axis: damped, plain, damped); each is cut into tiles of at most
 // RES_COLUMNS columns along x.
-// RES_LDS_COLUMNS bounds a tile's columns with the halo columns around them,
-// one number for every scene, so that scenes share launches.
-enum : int { RES_THREADS = 256, RES_COLUMNS = 256, RES_LDS_COLUMNS = 18 * 18 };
+enum : int { RES_THREADS = 256, RES_COLUMNS = 256 };
 
 struct ResBox {
     int32_t lo[3], len[3];      // cells
@@ -36,9 +34,10 @@ struct ResBox {
 
 struct ResTile {
     int32_t i0, j0, k0, bx, by, bz;
+    int32_t pitch;              // LDS words from one row of columns (along z) to the next
     int32_t damped, slab;
     uint32_t word0;             // its first word in the exchange buffer and in the route table
-    int32_t words;              // faces' cells: x low, x high, y low, y high, z low, z high
+    int32_t words;              // faces' cells: x low, x high, y low, y high, z low, z high (one more word follows)
     int32_t tb, te;             // listener terms
     int32_t rb, re;             // object-adjacent records
     int32_t src, skip;          // meets a pressure source's box; holds object cells
@@ -47,10 +46,9 @@ struct ResTile {
 // where the own cell next to a face word is sent, and the LDS places of that
 // cell (low half) and of the halo cell received for the word (high half)
 struct ResRoute {
-    uint32_t to;                // word of the neighbour's buffer (RES_NOWHERE: a wall)
+    uint32_t to;                // word of the neighbour's buffer
     uint32_t lds;
 };
-enum : uint32_t { RES_NOWHERE = 0xffffffffu };
 
 // device block of one resident scene
 struct ResScene {
@@ -75,7 +73,7 @@ struct ResItem {
 // of a column (its cells, the x-high halo after them, the x-low halo last).
 struct ResShape {
     int plain, one, more;
-    int column_words;
+    int column_words, lds_words;  // of one of the two buffers
     int max_words, max_recs;    // face words and records a tile may hold
 };
 enum : int { RES_FINE = 0, RES_COARSE = 1, RES_SHAPES = 2 };
@@ -90,6 +88,7 @@ struct ResPlan {
     std::vector<ResBox> boxes;
     std::vector<ResTile> tiles;
     std::vector<int32_t> recs;
+    std::vector<int32_t> order; // tiles in the order of their dispatch
     std::vector<TermRef> terms;
     uint32_t nwords = 0;
     int tile_of(int i, int j, int k) const;

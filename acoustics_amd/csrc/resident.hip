@@ -3,13 +3,25 @@
 // Bound: the exchange between workgroups.  A step needs the neighbours' face
 // pressures of the step before, and one hop through the memory side (a store
 // of one workgroup to a load of another) takes 1.3-1.6 us with up to 256
-// workgroups in flight, 1.9 us with 512, 3.0 us with 1024; the arithmetic of
-// a step is 0.3-1.6 us of the SIMDs and nothing is read from or written to
-// HBM.  Each face pressure travels in one 8-byte word with the step's tag
-// above it, so the data is its own flag: no store has to be acknowledged
-// before a flag is raised, and no load follows a flag (with flags the same
-// exchange took 1.8-3.3 us).  The words of a face are contiguous over lanes:
-// stored column by column instead, the exchange took 14-24 us.
+// workgroups in flight, 1.9 us with 512, 3.0 us with 1024 (a bare exchange of
+// 1024 words each); nothing else is read from or written to memory.  Measured
+// per step: 64^3 with a 10-cell PML (206 workgroups) 2.1 us, of which the
+// arithmetic alone 0.9 and the exchange alone 1.5 (the step kernels: 6.6);
+// 128^3 with a 12-cell PML (733) 5.4 us, 2.9 and 5.0 (17.9).
+//
+// * Each face pressure travels in one 8-byte word with the step's tag above
+//   it, so the data is its own flag: no store is waited for before a flag is
+//   raised, and no load follows a flag (with flags and 4-byte data the bare
+//   exchange took 1.8-2.4 us with 256 workgroups, 3.1-4.0 with 1024).
+// * The words of a face are contiguous over lanes and start on a 128-byte
+//   line (128^3: 6.4 -> 5.9 us per step; word by column instead of by lane, a
+//   bare exchange took 14-24 us).
+// * No lane branches on whether it has a word, and what only some steps or
+//   tiles need (scene pointers for sources, records, rarer listener terms) is
+//   loaded where it is used: 64^3 2.95 -> 2.39 us per step.
+// * Cells' PML and leapfrog history is in registers, pressures in two LDS
+//   buffers with x fastest, so a thread's column and its four neighbours'
+//   columns are 16-byte reads.
 #include <climits>
 
 #include "resident.h"
@@ -24,21 +36,21 @@ struct Shape;
 // small grids: as many workgroups as possible
 template <>
 struct Shape<RES_FINE> {
-    static constexpr int plain = 8, one = 8, more = 8, cs = 12, words = 5, recs = 2, waves = 3;
+    static constexpr int plain = 8, one = 8, more = 8, cs = 12, words = 4, recs = 2, waves = 3, lds = 4608;
 };
 // larger grids: as many cells per workgroup as registers and LDS hold
 template <>
 struct Shape<RES_COARSE> {
-    static constexpr int plain = 16, one = 12, more = 8, cs = 20, words = 6, recs = 3, waves = 3;
+    static constexpr int plain = 16, one = 12, more = 8, cs = 20, words = 6, recs = 3, waves = 3, lds = 6500;
 };
 
 typedef unsigned long long u64;
 
-__device__ __forceinline__ void send_word(u64 *p, u64 v)
+__device__ __forceinline__ void send_word(AS_GLOBAL u64 *p, u64 v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ u64 take_word(const u64 *p)
+__device__ __forceinline__ u64 take_word(const AS_GLOBAL u64 *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -56,56 +68,76 @@ __device__ __forceinline__ int anew(int v)
 struct FaceCell {
     int own, halo;      // LDS words
     int i, j, k;        // the neighbour's cell
+    bool real;          // (the last words of a face stand for no cell)
 };
+
+// Words of a face, rounded up to whole 128-byte lines: a line then has one
+// sender per neighbour.
+__device__ __forceinline__ int face_words(int n) { return (n + 15) & ~15; }
 
 template <int CS>
 __device__ __forceinline__ FaceCell face_cell(const ResTile &t, int w)
 {
-    const int nyz = t.by * t.bz, nxz = t.bx * t.bz, nxy = t.bx * t.by, P = t.bz + 2;
+    const int nyz = face_words(t.by * t.bz), nxz = face_words(t.bx * t.bz), nxy = face_words(t.bx * t.by);
+    const int P = t.pitch;
     FaceCell f;
     if (w < 2 * nyz) {
         const int hi = w >= nyz, c = w - hi * nyz, y = c / t.bz, z = c - y * t.bz;
-        const int col = ((y + 1) * P + z + 1) * CS;
+        const int col = (y + 1) * P + (z + 1) * CS;
         f.own = col + (hi ? t.bx - 1 : 0);
         f.halo = col + (hi ? t.bx : CS - 1);
         f.i = hi ? t.i0 + t.bx : t.i0 - 1;
         f.j = t.j0 + y;
         f.k = t.k0 + z;
+        f.real = y < t.by;
         return f;
     }
     w -= 2 * nyz;
     if (w < 2 * nxz) {
         const int hi = w >= nxz, c = w - hi * nxz, x = c / t.bz, z = c - x * t.bz;
-        f.own = ((hi ? t.by : 1) * P + z + 1) * CS + x;
-        f.halo = ((hi ? t.by + 1 : 0) * P + z + 1) * CS + x;
+        f.own = (hi ? t.by : 1) * P + (z + 1) * CS + x;
+        f.halo = (hi ? t.by + 1 : 0) * P + (z + 1) * CS + x;
         f.i = t.i0 + x;
         f.j = hi ? t.j0 + t.by : t.j0 - 1;
         f.k = t.k0 + z;
+        f.real = x < t.bx;
         return f;
     }
     w -= 2 * nxz;
     const int hi = w >= nxy, c = w - hi * nxy, x = c / t.by, y = c - x * t.by;
-    f.own = ((y + 1) * P + (hi ? t.bz : 1)) * CS + x;
-    f.halo = ((y + 1) * P + (hi ? t.bz + 1 : 0)) * CS + x;
+    f.own = (y + 1) * P + (hi ? t.bz : 1) * CS + x;
+    f.halo = (y + 1) * P + (hi ? t.bz + 1 : 0) * CS + x;
     f.i = t.i0 + x;
     f.j = t.j0 + y;
     f.k = hi ? t.k0 + t.bz : t.k0 - 1;
+    f.real = x < t.bx;
     return f;
 }
 
 // Fills a scene's route table, one workgroup per tile: the tile on the other
-// side of each face word and the word there that stands for the own cell.
+// side of each face word and the word there that stands for the own cell.  A
+// wall's words go to the tile itself (the halo beyond a wall equals the cell
+// before it; the wall face's zero factors keep its velocity at zero), and lanes
+// without a word share one more that goes nowhere else: every lane of the
+// exchange then does the same.
 template <int CS>
 __global__ __launch_bounds__(RES_THREADS) void route_kernel(const ResScene *__restrict__ scene)
 {
     const ResScene R = *cmem(scene);
     const SceneDev S = *cmem(R.S);
     const ResTile t = cmem(R.tiles)[blockIdx.x];
-    for (int w = (int)threadIdx.x; w < t.words; w += RES_THREADS) {
-        const FaceCell f = face_cell<CS>(t, w);
+    for (int w = (int)threadIdx.x; w <= t.words; w += RES_THREADS) {
         ResRoute r;
+        r.to = t.word0 + (uint32_t)w;
+        r.lds = 0;              // (an unused corner of the halo)
+        FaceCell f;
+        f.real = false;
+        if (w < t.words) f = face_cell<CS>(t, w);
+        if (!f.real) {
+            gmem(R.route)[t.word0 + (uint32_t)w] = r;
+            continue;
+        }
         r.lds = (uint32_t)f.own | ((uint32_t)f.halo << 16);
-        r.to = RES_NOWHERE;
         if (f.i >= 0 && f.j >= 0 && f.k >= 0 && f.i < S.n[0] && f.j < S.n[1] && f.k < S.n[2]) {
             const int x[3] = {f.i, f.j, f.k};
             for (int b = 0; b < R.nboxes; ++b) {
@@ -119,7 +151,7 @@ __global__ __launch_bounds__(RES_THREADS) void route_kernel(const ResScene *__re
                 if (!in) continue;
                 const int q = B.first + ((at[0] / B.size[0]) * B.count[1] + at[1] / B.size[1]) * B.count[2] + at[2] / B.size[2];
                 const ResTile o = gmem(R.tiles)[q];
-                const int nyz = o.by * o.bz, nxz = o.bx * o.bz, nxy = o.bx * o.by;
+                const int nyz = face_words(o.by * o.bz), nxz = face_words(o.bx * o.bz), nxy = face_words(o.bx * o.by);
                 const int li = x[0] - o.i0, lj = x[1] - o.j0, lk = x[2] - o.k0;
                 // the own cell is across the neighbour's opposite face
                 int word;
@@ -145,50 +177,74 @@ __device__ __forceinline__ float4 x_entry(const SceneDev &S, int i)
     return c;
 }
 
+// The pointer, read anew: what is loaded through it is loaded there, and not
+// carried in scalar registers through all steps.
+template <class T>
+__device__ __forceinline__ const T *anew(const T *p)
+{
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+template <class T>
+__device__ __forceinline__ AS_GLOBAL T *at_byte(T *base, uint32_t off)
+{
+    return (AS_GLOBAL T *)((AS_GLOBAL char *)base + off);
+}
+
 // What a workgroup carries through its steps besides the class's registers.
 template <int SHAPE>
 struct Frame {
     using C = Shape<SHAPE>;
-    const SceneDev &S;
-    const ResScene &R;
-    const ResTile &t;
+    const SceneDev *scene;
+    const ResScene *res;
+    const ResTile *tile;
     float *A, *B;               // this step's pressures and the next's, in LDS
     float4 *X;                  // x table of the tile's cells and faces, in LDS
     long long step0;
     int steps;
     uint32_t tag;
     int *trouble;
+    int bx;
     // own column
     bool act;
     int ly, lz, col;            // col: LDS word of the column's first cell
     int P;                      // LDS words from a column to the next along y
-    // face words
-    ResRoute route[C::words];
+    // face words: where they go (bytes), LDS places of the own cell and of the halo (bytes, 16 bits each)
+    u64 *words;
+    uint32_t half;              // bytes of one parity's words
+    uint32_t to[C::words], lds[C::words];
+    uint32_t word0;             // byte of this tile's first word
+    int nwords;
     // the tile's listener terms: this thread's first one
-    bool has_term;
-    TermRef term;
+    bool terms_here, has_term, more_terms;
+    double *term_to;            // its place in ring row 0
+    double term_beta;
     int term_at;
-    int ring0;                  // ring row of step0
+    int ring0, cap;             // ring row of step0, rows
+    uint32_t row_bytes;
     bool stuck;
 
-    __device__ Frame(const SceneDev &S_, const ResScene &R_, const ResTile &t_) : S(S_), R(R_), t(t_) {}
+    // the scene, for code off the step loop's usual path
+    __device__ __forceinline__ SceneDev scene_now() const { return *cmem(anew(scene)); }
 
-    __device__ __forceinline__ int place(int cell) const
+    __device__ __forceinline__ static int place(const SceneDev &S, const ResTile &t, int cell)
     {
         const int i = cell / S.sx, r = cell - i * S.sx, j = r / S.sy, k = r - j * S.sy;
-        return ((j - t.j0 + 1) * (t.bz + 2) + (k - t.k0 + 1)) * C::cs + (i - t.i0);
+        return (j - t.j0 + 1) * t.pitch + (k - t.k0 + 1) * C::cs + (i - t.i0);
     }
 
     // p^{step} of the tile and its halo, both buffers cleared before
-    __device__ __forceinline__ void load()
+    __device__ __forceinline__ void load(const SceneDev &S, const ResScene &R, const ResTile &t)
     {
-        const int tid = (int)threadIdx.x, n = 2 * RES_LDS_COLUMNS * C::cs;
+        const int tid = (int)threadIdx.x, n = 2 * C::lds;
         for (int q = tid; q < n; q += RES_THREADS) A[q] = 0.f;
-        P = (t.bz + 2) * C::cs;
+        bx = t.bx;
+        P = t.pitch;
         act = tid < t.by * t.bz;
         ly = act ? tid / t.bz : 0;
         lz = act ? tid - ly * t.bz : 0;
-        col = ((ly + 1) * (t.bz + 2) + lz + 1) * C::cs;
+        col = (ly + 1) * P + (lz + 1) * C::cs;
         if (tid <= C::plain) X[tid] = x_entry(S, t.i0 + tid);
         __syncthreads();
         const AS_GLOBAL float *pc = gmem(S.field + (size_t)slot_cur(step0) * S.npad);
@@ -198,90 +254,101 @@ struct Frame {
             for (int i = 0; i < C::plain; ++i)
                 if (i < t.bx) A[col + i] = pc[idx + i * S.sx];
         }
+        words = R.words;
+        half = R.nwords * 8u;
+        word0 = t.word0 * 8u;
+        nwords = t.words;
 #pragma unroll
         for (int m = 0; m < C::words; ++m) {
-            const int w = tid + m * RES_THREADS;
-            route[m].to = RES_NOWHERE;
-            route[m].lds = 0;
+            const int w = min(tid + m * RES_THREADS, t.words);
+            const ResRoute r = gmem(R.route)[t.word0 + (uint32_t)w];
+            to[m] = r.to * 8u;
+            lds[m] = r.lds * 4u;
             if (w < t.words) {
-                route[m] = gmem(R.route)[t.word0 + (uint32_t)w];
-                if (route[m].to != RES_NOWHERE) {
-                    const FaceCell f = face_cell<C::cs>(t, w);
+                const FaceCell f = face_cell<C::cs>(t, w);
+                if (f.real && f.i >= 0 && f.j >= 0 && f.k >= 0 && f.i < S.n[0] && f.j < S.n[1] && f.k < S.n[2])
                     A[f.halo] = pc[f.i * S.sx + f.j * S.sy + f.k];
-                }
             }
         }
+        // one term per thread of the usual kind (a cell's new pressure) is
+        // kept ready; others are looked up each step
+        terms_here = t.te > t.tb;
         has_term = t.tb + tid < t.te;
         term_at = 0;
+        cap = S.cap;
         ring0 = (int)(step0 % S.cap);
+        row_bytes = 8u * (uint32_t)S.T;
+        more_terms = t.te - t.tb > RES_THREADS;
         if (has_term) {
-            term = gmem(R.terms)[t.tb + tid];
-            term_at = place(term.kind == 0 ? term.cell : gmem(S.ghosts)[term.cell].nbr);
+            const TermRef r = gmem(R.terms)[t.tb + tid];
+            term_to = S.terms + r.slot;
+            term_beta = r.beta;
+            if (r.kind == 0) term_at = place(S, t, r.cell);
+            else { has_term = false; more_terms = true; }
         }
+        more_terms = __any(more_terms);
         stuck = false;
     }
 
-    // fresh, now: ring rows of the step that made the pressures now held and
-    // of the step about to run (-1: none in this block)
-    __device__ __forceinline__ void emit(const TermRef &r, int at, int fresh, int now, long long step) const
-    {
-        // a cell's term belongs to the step that made the pressure now held,
-        // a ghost's to the step about to run
-        double v = (double)A[at];
-        int row = fresh;
-        if (r.kind != 0) {
-            if (now < 0) return;
-            v += raster_accel_term(S, gmem(S.ghosts)[r.cell], step);
-            row = now;
-        } else if (fresh < 0) {
-            return;
-        }
-        gmem(S.terms)[(size_t)(row < S.cap ? row : row - S.cap) * S.T + r.slot] = r.beta * v;
-    }
-    // before step s of the block (s == steps: after the last)
+    // Step s has been made: a cell's term takes its new pressure (in B), a
+    // ghost's its value in that step (from A).
     __device__ __forceinline__ void terms(int s) const
     {
-        if (t.te == t.tb) return;
-        const int fresh = s > 0 ? ring0 + s - 1 : -1, now = s < steps ? ring0 + s : -1;
-        if (has_term) emit(term, term_at, fresh, now, step0 + s);
-        for (int q = t.tb + (int)threadIdx.x + RES_THREADS; q < t.te; q += RES_THREADS) {
+        if (!terms_here) return;
+        const int row = ring0 + s < cap ? ring0 + s : ring0 + s - cap;
+        if (has_term) *(AS_GLOBAL double *)((AS_GLOBAL char *)term_to + (size_t)row * row_bytes) = term_beta * (double)B[term_at];
+        if (!more_terms) return;
+        const SceneDev S = scene_now();
+        const ResScene R = *cmem(anew(res));
+        const ResTile t = *cmem(anew(tile));
+        for (int q = t.tb + (int)threadIdx.x; q < t.te; q += RES_THREADS) {
             const TermRef r = gmem(R.terms)[q];
-            emit(r, place(r.kind == 0 ? r.cell : gmem(S.ghosts)[r.cell].nbr), fresh, now, step0 + s);
+            if (r.kind == 0 && q < t.tb + RES_THREADS) continue;
+            double v;
+            if (r.kind == 0) v = (double)B[place(S, t, r.cell)];
+            else {
+                const GhostDev g = gmem(S.ghosts)[r.cell];
+                v = (double)A[place(S, t, g.nbr)] + raster_accel_term(S, g, step0 + s);
+            }
+            gmem(S.terms)[(size_t)row * S.T + r.slot] = r.beta * v;
         }
     }
 
-    // sends the tile's faces of the step just made and waits for the
-    // neighbours' (all of B's own cells are written and visible)
-    __device__ __forceinline__ void exchange(int s)
+    // sends the tile's faces of step s, just made (all of B's own cells are
+    // written and visible)
+    __device__ __forceinline__ void send(int s) const
     {
         const uint32_t mark = tag + (uint32_t)s;
-        u64 *buf = R.words + (size_t)(mark & 1u) * R.nwords;
+        u64 *buf = words + ((mark & 1u) ? half / 8u : 0u);
+        float v[C::words];
 #pragma unroll
-        for (int m = 0; m < C::words; ++m)
-            if (route[m].to != RES_NOWHERE)
-                send_word(buf + route[m].to, ((u64)mark << 32) | __float_as_uint(B[route[m].lds & 0xffffu]));
-        const u64 *in = buf + t.word0 + threadIdx.x;
+        for (int m = 0; m < C::words; ++m) v[m] = *(const float *)((const char *)B + (lds[m] & 0xffffu));
+#pragma unroll
+        for (int m = 0; m < C::words; ++m) send_word(at_byte(buf, to[m]), ((u64)mark << 32) | __float_as_uint(v[m]));
+    }
+    // waits for the neighbours' faces of step s
+    __device__ __forceinline__ void receive(int s)
+    {
+        const uint32_t mark = tag + (uint32_t)s;
+        u64 *buf = words + ((mark & 1u) ? half / 8u : 0u);
         u64 v[C::words];
-        for (int spins = 0; !stuck; ++spins) {
+        for (int spins = 0;; ++spins) {
+            uint32_t miss = 0;
 #pragma unroll
             for (int m = 0; m < C::words; ++m)
-                if (route[m].to != RES_NOWHERE) v[m] = take_word(in + m * RES_THREADS);
-            bool ok = true;
+                v[m] = take_word(at_byte(buf, word0 + 8u * (uint32_t)min((int)threadIdx.x + m * RES_THREADS, nwords)));
 #pragma unroll
-            for (int m = 0; m < C::words; ++m)
-                if (route[m].to != RES_NOWHERE) ok = ok && (uint32_t)(v[m] >> 32) == mark;
-            if (ok) break;
+            for (int m = 0; m < C::words; ++m) miss |= (uint32_t)(v[m] >> 32) ^ mark;
+            if (miss == 0 || stuck) break;
             if (spins > (1 << 22)) {
                 // the neighbours are on the device, so this does not happen;
                 // it keeps every wave's exit certain
                 stuck = true;
-                __hip_atomic_store(trouble, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(const_cast<int *>(anew((const int *)trouble)), 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
         }
-        // (nothing lies beyond a wall: that halo stays zero)
 #pragma unroll
-        for (int m = 0; m < C::words; ++m)
-            if (route[m].lds) B[route[m].lds >> 16] = route[m].to != RES_NOWHERE ? __uint_as_float((uint32_t)v[m]) : 0.f;
+        for (int m = 0; m < C::words; ++m) *(float *)((char *)B + (lds[m] >> 16)) = __uint_as_float((uint32_t)v[m]);
     }
     __device__ __forceinline__ void turn()
     {
@@ -291,7 +358,7 @@ struct Frame {
     }
 
     // the last two levels of the own cells, into the slots of step step0 + steps
-    __device__ __forceinline__ void store_pressure() const
+    __device__ __forceinline__ void store_pressure(const SceneDev &S, const ResTile &t) const
     {
         if (!act) return;
         const long long s = step0 + steps;
@@ -306,20 +373,32 @@ struct Frame {
     }
 };
 
-// four cells of a column and their neighbours: cells 4 q .. 4 q + 3
+// The own column, the x halos beside it, and four cells of the columns around
+// it: cells 4 q .. 4 q + 3.
+template <int CS, int NB>
+struct Column {
+    float c[NB + 1], before;    // cells 0 .. NB (cell bx is the x-high halo); the x-low halo
+    __device__ __forceinline__ Column(const float *A, int col)
+    {
+#pragma unroll
+        for (int q = 0; q < NB / 4; ++q) {
+            const float4 v = *(const float4 *)(A + col + 4 * q);
+            c[4 * q] = v.x; c[4 * q + 1] = v.y; c[4 * q + 2] = v.z; c[4 * q + 3] = v.w;
+        }
+        c[NB] = A[col + NB];
+        before = A[col + CS - 1];
+    }
+};
 struct Quad {
-    float c[4], xm, xp, yl[4], yr[4], zl[4], zr[4];
+    float yl[4], yr[4], zl[4], zr[4];
 };
 template <int CS>
 __device__ __forceinline__ Quad quad(const float *A, int col, int P, int q)
 {
     Quad u;
     const float *a = A + col + 4 * q;
-    const float4 c = *(const float4 *)a, yl = *(const float4 *)(a - P), yr = *(const float4 *)(a + P);
+    const float4 yl = *(const float4 *)(a - P), yr = *(const float4 *)(a + P);
     const float4 zl = *(const float4 *)(a - CS), zr = *(const float4 *)(a + CS);
-    u.xp = a[4];
-    u.xm = q == 0 ? A[col + CS - 1] : a[-1];
-    u.c[0] = c.x; u.c[1] = c.y; u.c[2] = c.z; u.c[3] = c.w;
     u.yl[0] = yl.x; u.yl[1] = yl.y; u.yl[2] = yl.z; u.yl[3] = yl.w;
     u.yr[0] = yr.x; u.yr[1] = yr.y; u.yr[2] = yr.z; u.yr[3] = yr.w;
     u.zl[0] = zl.x; u.zl[1] = zl.y; u.zl[2] = zl.z; u.zl[3] = zl.w;
@@ -337,16 +416,16 @@ __device__ __forceinline__ void put_quad(float *B, int col, int q, const float *
 // Undamped cells: leapfrog, pressure sources, and the object-adjacent cells
 // of the tile in FP64 by one thread per record.
 template <int SHAPE>
-__device__ __forceinline__ void run_plain(Frame<SHAPE> &F)
+__device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, const ResTile &t)
 {
     using C = Shape<SHAPE>;
     constexpr int NB = C::plain, NR = C::recs;
-    const SceneDev &S = F.S;
-    const ResTile &t = F.t;
     const int tid = (int)threadIdx.x;
     float prev[NB];
     uint32_t skip = 0;
     const float lam2 = S.lam2f;
+    const int i0 = t.i0, src = t.src ? S.n_psrc : 0;
+    const bool skips = t.skip, records = t.re > t.rb;
     const int j = t.j0 + F.ly, k = t.k0 + F.lz;   // (threads without a column: the first one's)
     {
         const AS_GLOBAL float *pp = gmem(S.field + (size_t)slot_next(F.step0) * S.npad);
@@ -366,10 +445,10 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F)
             rat[r] = -1;
             const int q = t.rb + tid + r * RES_THREADS;
             if (q >= t.re) continue;
-            const SpecialRec rec = gmem(S.recs)[gmem(F.R.recs)[q]];
-            rat[r] = F.place(rec.cell);
+            const SpecialRec rec = gmem(S.recs)[gmem(cmem(F.res)->recs)[q]];
+            rat[r] = F.place(S, t, rec.cell);
             rprev[r] = gmem(S.field + (size_t)slot_next(F.step0) * S.npad)[rec.cell];
-            rmask[r] = (rec.flags & 1) << 6;
+            rmask[r] = (rec.flags & 1) << 6 | rat[r] % F.P % C::cs << 8;   // (its x place above the bits)
             robj[r] = 0;
             for (int e = 0; e < 6; ++e) {
                 rk[r][e] = 0.0;
@@ -381,50 +460,63 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F)
             }
         }
     }
+    // amplitudes of a step, fetched while the exchange of the one before runs
+    double racc[NR];
+    float amp = 0.f;
+    const AS_GLOBAL float *src_tab = gmem(S.src_tab);
+    const int amp_last = S.amp_rows - 1;
+    auto amplitudes = [&](long long step) {
+        if (records) {
+            const SceneDev Z = F.scene_now();
+#pragma unroll
+            for (int r = 0; r < NR; ++r) racc[r] = rat[r] >= 0 ? gmem(Z.acc_tab)[amp_row(Z, step) * Z.n_ch + robj[r]] : 0.0;
+        }
+        if (src) amp = src_tab[(int)(step & amp_last) * src];
+    };
+    amplitudes(F.step0);
     for (int s = 0; s < F.steps; ++s) {
         const long long step = F.step0 + s;
-        F.terms(s);
-        double racc[NR];
-        if (t.re > t.rb) {
-#pragma unroll
-            for (int r = 0; r < NR; ++r) racc[r] = rat[r] >= 0 ? gmem(S.acc_tab)[amp_row(step) * S.n_ch + robj[r] * S.n_cpo] : 0.0;
-        }
         if (F.act) {
+            const Column<C::cs, NB> w(F.A, F.col);
 #pragma unroll
             for (int q = 0; q < NB / 4; ++q) {
-                if (4 * q >= t.bx) continue;
+                if (4 * q >= F.bx) continue;
                 const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
                 float o[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    o[e] = leapfrog1(u.c[e], prev[4 * q + e], e ? u.c[e - 1] : u.xm, e < 3 ? u.c[e + 1] : u.xp, u.yl[e], u.yr[e],
-                                     u.zl[e], u.zr[e], lam2);
+                    o[e] = leapfrog1(w.c[4 * q + e], prev[4 * q + e], 4 * q + e ? w.c[4 * q + e - 1] : w.before, w.c[4 * q + e + 1],
+                                     u.yl[e], u.yr[e], u.zl[e], u.zr[e], lam2);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) prev[4 * q + e] = u.c[e];
-                if (!t.skip) put_quad(F.B, F.col, q, o);
+                for (int e = 0; e < 4; ++e) prev[4 * q + e] = w.c[4 * q + e];
+                if (!skips) put_quad(F.B, F.col, q, o);
                 else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (4 * q + e < t.bx && !(skip >> (4 * q + e) & 1)) F.B[F.col + 4 * q + e] = o[e];
+                        if (4 * q + e < F.bx && !(skip >> (4 * q + e) & 1)) F.B[F.col + 4 * q + e] = o[e];
                 }
             }
-            if (t.src)
-                for (int p = 0; p < S.n_psrc; ++p) {
-                    // an amplitude of zero (the pulse is over) adds nothing
-                    const float a = gmem(S.src_tab)[amp_row(step) * S.n_psrc + p];
+            // an amplitude of zero (the pulse is over) adds nothing
+            if (src && (amp != 0.f || src > 1)) {
+                const SceneDev Z = F.scene_now();
+                for (int p = 0; p < Z.n_psrc; ++p) {
+                    const float a = p == 0 ? amp : gmem(Z.src_tab)[amp_row(Z, step) * Z.n_psrc + p];
                     if (a == 0.f) continue;
-                    const PSrcDev ps = cmem(S.psrc)[p];
-                    const float gy = gmem(S.gtab)[ps.goff[1] + j], gz = gmem(S.gtab)[ps.goff[2] + k];
-                    for (int i = 0; i < t.bx; ++i)
-                        if (!(skip >> i & 1)) F.B[F.col + i] = add_source(F.B[F.col + i], a, cmem(S.gtab)[ps.goff[0] + t.i0 + i], gy, gz);
+                    const PSrcDev ps = cmem(Z.psrc)[p];
+                    const float gy = gmem(Z.gtab)[ps.goff[1] + j], gz = gmem(Z.gtab)[ps.goff[2] + k];
+                    for (int i = 0; i < F.bx; ++i)
+                        if (!(skip >> i & 1)) F.B[F.col + i] = add_source(F.B[F.col + i], a, cmem(Z.gtab)[ps.goff[0] + i0 + i], gy, gz);
                 }
+            }
         }
-        if (t.re > t.rb) {
+        if (records) {
+            const SceneDev Z = F.scene_now();
+            const ResTile u = *cmem(anew(F.tile));
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 if (rat[r] < 0) continue;
                 const float *a = F.A + rat[r];
-                const int x = rat[r] % C::cs;
+                const int x = rmask[r] >> 8;
                 const float cf = a[0];
                 const double c = cf;
                 const double nb[6] = {x == 0 ? a[C::cs - 1] : a[-1], a[1], a[-F.P], a[F.P], a[-C::cs], a[C::cs]};
@@ -434,16 +526,16 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F)
                 double lap = 0.0;
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
-                    lap += ghost_lap_axis(S.seven, rmask[r] >> (2 * d) & 1, rmask[r] >> (2 * d + 1) & 1, g[2 * d], g[2 * d + 1],
+                    lap += ghost_lap_axis(Z.seven, rmask[r] >> (2 * d) & 1, rmask[r] >> (2 * d + 1) & 1, g[2 * d], g[2 * d + 1],
                                           nb[2 * d], nb[2 * d + 1], c);
-                double pn = (rmask[r] >> 6 & 1) ? c : special_update(c, (double)rprev[r], lap, S.lam2);
-                if (S.n_psrc > 0) {
-                    const int cx = rat[r] / C::cs, y = cx / (t.bz + 2) - 1, z = cx % (t.bz + 2) - 1;
-                    for (int p = 0; p < S.n_psrc; ++p) {
-                        const PSrcDev ps = cmem(S.psrc)[p];
-                        const AS_GLOBAL float *g3 = gmem(S.gtab);
-                        pn += (double)(gmem(S.src_tab)[amp_row(step) * S.n_psrc + p] * g3[ps.goff[0] + t.i0 + x] *
-                                       g3[ps.goff[1] + t.j0 + y] * g3[ps.goff[2] + t.k0 + z]);
+                double pn = (rmask[r] >> 6 & 1) ? c : special_update(c, (double)rprev[r], lap, Z.lam2);
+                if (Z.n_psrc > 0) {
+                    const int y = rat[r] / F.P - 1, z = rat[r] % F.P / C::cs - 1;
+                    for (int p = 0; p < Z.n_psrc; ++p) {
+                        const PSrcDev ps = cmem(Z.psrc)[p];
+                        const AS_GLOBAL float *g3 = gmem(Z.gtab);
+                        pn += (double)(gmem(Z.src_tab)[amp_row(Z, step) * Z.n_psrc + p] * g3[ps.goff[0] + u.i0 + x] *
+                                       g3[ps.goff[1] + u.j0 + y] * g3[ps.goff[2] + u.k0 + z]);
                     }
                 }
                 rprev[r] = cf;
@@ -451,12 +543,14 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F)
             }
         }
         __syncthreads();
-        F.exchange(s);
+        F.send(s);
+        F.terms(s);
+        amplitudes(step + 1);
+        F.receive(s);
         F.turn();
         __syncthreads();
     }
-    F.terms(F.steps);
-    F.store_pressure();
+    F.store_pressure(F.scene_now(), *cmem(anew(F.tile)));
 }
 
 // Face and cell coefficients of the own column along y or z.
@@ -497,12 +591,10 @@ struct SlabAt {
 // Cells damped along axis D only (the merged PML state): pDir along D, both
 // faces along D, and the increment of the transverse sum.
 template <int SHAPE, int D>
-__device__ __forceinline__ void run_one(Frame<SHAPE> &F)
+__device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, const ResTile &t)
 {
     using C = Shape<SHAPE>;
     constexpr int NB = C::one;
-    const SceneDev &S = F.S;
-    const ResTile &t = F.t;
     const PmlSlab sl = cmem(S.slabs)[t.slab];
     const SlabAt at(sl, t, F.ly, F.lz);
     AS_GLOBAL float *pq = gmem(S.pd[D] + sl.cell_base), *pi = gmem(S.pd[D == 0 ? 1 : 0] + sl.cell_base);
@@ -529,18 +621,18 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F)
     }
     const float4 xp0 = cmem(S.coef[0])[t.i0];   // D != 0: x is plain over the tile, one entry for all
     for (int s = 0; s < F.steps; ++s) {
-        F.terms(s);
         if (F.act) {
+            const Column<C::cs, NB> w(F.A, F.col);
             float before = 0.f;                 // D == 0: the updated low face of the next cell
 #pragma unroll
             for (int q = 0; q < NB / 4; ++q) {
-                if (4 * q >= t.bx) continue;
+                if (4 * q >= F.bx) continue;
                 const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
                 float o[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = 4 * q + e;
-                    const float c = u.c[e], xm = e ? u.c[e - 1] : u.xm, xp = e < 3 ? u.c[e + 1] : u.xp;
+                    const float c = w.c[i], xm = i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
                     float n, lap = 0.f;
                     const float qo = q0[i];
                     if (D == 0) {
@@ -572,36 +664,39 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F)
             }
         }
         __syncthreads();
-        F.exchange(s);
+        F.send(s);
+        F.terms(s);
+        F.receive(s);
         F.turn();
         __syncthreads();
     }
-    F.terms(F.steps);
-    F.store_pressure();
+    const SceneDev Z = F.scene_now();
+    const ResTile u = *cmem(anew(F.tile));
+    F.store_pressure(Z, u);
     if (!F.act) return;
-    const SlabAt to(sl, t, anew(F.ly), anew(F.lz));
-    AS_GLOBAL float *v = gmem(((F.step0 + F.steps) & 1 ? S.vel[1][D] : S.vel[0][D]) + sl.v_base[D]);
+    const PmlSlab zl_ = cmem(Z.slabs)[u.slab];
+    const SlabAt to(zl_, u, anew(F.ly), anew(F.lz));
+    AS_GLOBAL float *zq = gmem(Z.pd[D] + zl_.cell_base), *zi = gmem(Z.pd[D == 0 ? 1 : 0] + zl_.cell_base);
+    AS_GLOBAL float *v = gmem(((F.step0 + F.steps) & 1 ? Z.vel[1][D] : Z.vel[0][D]) + zl_.v_base[D]);
 #pragma unroll
     for (int i = 0; i <= NB; ++i) {
-        if (i < NB && i < t.bx) {
-            pq[to.cell(i)] = q0[i];
-            pi[to.cell(i)] = dd[i];
-            if (D == 1) { v[to.fy(i, 0)] = vl[i]; if (F.ly == t.by - 1) v[to.fy(i, 1)] = vr[i]; }
-            if (D == 2) { v[to.fz(i, 0)] = vl[i]; if (F.lz == t.bz - 1) v[to.fz(i, 1)] = vr[i]; }
+        if (i < NB && i < u.bx) {
+            zq[to.cell(i)] = q0[i];
+            zi[to.cell(i)] = dd[i];
+            if (D == 1) { v[to.fy(i, 0)] = vl[i]; if (F.ly == u.by - 1) v[to.fy(i, 1)] = vr[i]; }
+            if (D == 2) { v[to.fz(i, 0)] = vl[i]; if (F.lz == u.bz - 1) v[to.fz(i, 1)] = vr[i]; }
         }
-        if (D == 0 && i <= t.bx) v[to.cell(i)] = vl[i];
+        if (D == 0 && i <= u.bx) v[to.cell(i)] = vl[i];
     }
 }
 
 // Cells damped along two or three axes: three split pressures, the faces of
 // all three axes (a face of two tiles is kept by both, computed alike).
 template <int SHAPE>
-__device__ __forceinline__ void run_more(Frame<SHAPE> &F)
+__device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, const ResTile &t)
 {
     using C = Shape<SHAPE>;
     constexpr int NB = C::more;
-    const SceneDev &S = F.S;
-    const ResTile &t = F.t;
     const PmlSlab sl = cmem(S.slabs)[t.slab];
     const SlabAt at(sl, t, F.ly, F.lz);
     float q0[NB], q1[NB], q2[NB], vx[NB + 1], yl[NB], yr[NB], zl[NB], zr[NB];
@@ -628,18 +723,18 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F)
             if (i == t.bx) vx[i] = last;
     }
     for (int s = 0; s < F.steps; ++s) {
-        F.terms(s);
         if (F.act) {
+            const Column<C::cs, NB> w(F.A, F.col);
             float before = 0.f;
 #pragma unroll
             for (int q = 0; q < NB / 4; ++q) {
-                if (4 * q >= t.bx) continue;
+                if (4 * q >= F.bx) continue;
                 const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
                 float o[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = 4 * q + e;
-                    const float c = u.c[e], xm = e ? u.c[e - 1] : u.xm, xp = e < 3 ? u.c[e + 1] : u.xp;
+                    const float c = w.c[i], xm = i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
                     const float4 xl = F.X[i], xr = F.X[i + 1];
                     if (i == 0) before = face_step(xl.x, xl.y, vx[0], xm, c);
                     const float after = face_step(xr.x, xr.y, vx[i + 1], c, xp);
@@ -659,29 +754,33 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F)
             }
         }
         __syncthreads();
-        F.exchange(s);
+        F.send(s);
+        F.terms(s);
+        F.receive(s);
         F.turn();
         __syncthreads();
     }
-    F.terms(F.steps);
-    F.store_pressure();
+    const SceneDev Z = F.scene_now();
+    const ResTile u = *cmem(anew(F.tile));
+    F.store_pressure(Z, u);
     if (!F.act) return;
-    const SlabAt to(sl, t, anew(F.ly), anew(F.lz));
+    const PmlSlab zl_ = cmem(Z.slabs)[u.slab];
+    const SlabAt to(zl_, u, anew(F.ly), anew(F.lz));
     const int b = (int)((F.step0 + F.steps) & 1);
-    AS_GLOBAL float *v0 = gmem((b ? S.vel[1][0] : S.vel[0][0]) + sl.v_base[0]), *v1 = gmem((b ? S.vel[1][1] : S.vel[0][1]) + sl.v_base[1]);
-    AS_GLOBAL float *v2 = gmem((b ? S.vel[1][2] : S.vel[0][2]) + sl.v_base[2]);
+    AS_GLOBAL float *v0 = gmem((b ? Z.vel[1][0] : Z.vel[0][0]) + zl_.v_base[0]), *v1 = gmem((b ? Z.vel[1][1] : Z.vel[0][1]) + zl_.v_base[1]);
+    AS_GLOBAL float *v2 = gmem((b ? Z.vel[1][2] : Z.vel[0][2]) + zl_.v_base[2]);
 #pragma unroll
     for (int i = 0; i <= NB; ++i) {
-        if (i <= t.bx) v0[to.cell(i)] = vx[i];
-        if (i < NB && i < t.bx) {
+        if (i <= u.bx) v0[to.cell(i)] = vx[i];
+        if (i < NB && i < u.bx) {
             const int c = to.cell(i);
-            gmem(S.pd[0] + sl.cell_base)[c] = q0[i];
-            gmem(S.pd[1] + sl.cell_base)[c] = q1[i];
-            gmem(S.pd[2] + sl.cell_base)[c] = q2[i];
+            gmem(Z.pd[0] + zl_.cell_base)[c] = q0[i];
+            gmem(Z.pd[1] + zl_.cell_base)[c] = q1[i];
+            gmem(Z.pd[2] + zl_.cell_base)[c] = q2[i];
             v1[to.fy(i, 0)] = yl[i];
-            if (F.ly == t.by - 1) v1[to.fy(i, 1)] = yr[i];
+            if (F.ly == u.by - 1) v1[to.fy(i, 1)] = yr[i];
             v2[to.fz(i, 0)] = zl[i];
-            if (F.lz == t.bz - 1) v2[to.fz(i, 1)] = zr[i];
+            if (F.lz == u.bz - 1) v2[to.fz(i, 1)] = zr[i];
         }
     }
 }
@@ -706,7 +805,10 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
     const SceneDev S = *cmem(R.S);
     const ResTile t = cmem(R.tiles)[it.tile];
     u64 *clk = S.clock;
-    Frame<SHAPE> F(S, R, t);
+    Frame<SHAPE> F;
+    F.scene = R.S;
+    F.res = it.scene;
+    F.tile = R.tiles + it.tile;
     F.step0 = (long long)clk[CLK_STEP];
     const long long left = (long long)clk[CLK_TARGET] - F.step0;
     if (left <= 0) return;
@@ -715,7 +817,7 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
     F.trouble = trouble;
     F.X = xtab;
     F.A = lds;
-    F.B = lds + RES_LDS_COLUMNS * Shape<SHAPE>::cs;
+    F.B = lds + Shape<SHAPE>::lds;
     if (threadIdx.x == 0) {
         u64 expect = GATE_SHUT;
         const u64 n = __hip_atomic_fetch_add(&clk[CLK_ARRIVED], 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1ULL;
@@ -723,10 +825,10 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
             __hip_atomic_compare_exchange_strong(&clk[CLK_GATE], &expect, (u64)GATE_RUN, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
     }
-    F.load();
+    F.load(S, R, t);
     if (threadIdx.x == 0) {
         u64 g;
-        for (int spins = 0; (g = take_word(&clk[CLK_GATE])) == GATE_SHUT; ++spins) {
+        for (int spins = 0; (g = take_word(gmem(&clk[CLK_GATE]))) == GATE_SHUT; ++spins) {
             if (spins >= wait_limit) {
                 u64 expect = GATE_SHUT;
                 if (__hip_atomic_compare_exchange_strong(&clk[CLK_GATE], &expect, (u64)GATE_GIVEN_UP, __ATOMIC_RELAXED,
@@ -741,11 +843,11 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
     __syncthreads();
     if (!gate) return;
     switch (t.damped) {
-    case 0: run_plain<SHAPE>(F); break;
-    case 1: run_one<SHAPE, 0>(F); break;
-    case 2: run_one<SHAPE, 1>(F); break;
-    case 4: run_one<SHAPE, 2>(F); break;
-    default: run_more<SHAPE>(F); break;
+    case 0: run_plain<SHAPE>(F, S, t); break;
+    case 1: run_one<SHAPE, 0>(F, S, t); break;
+    case 2: run_one<SHAPE, 1>(F, S, t); break;
+    case 4: run_one<SHAPE, 2>(F, S, t); break;
+    default: run_more<SHAPE>(F, S, t); break;
     }
 }
 
@@ -755,12 +857,12 @@ ResShape resident_shape(int shape)
 {
     auto of = [](auto c) {
         using C = decltype(c);
-        return ResShape{C::plain, C::one, C::more, C::cs, C::words * RES_THREADS, C::recs * RES_THREADS};
+        return ResShape{C::plain, C::one, C::more, C::cs, C::lds, C::words * RES_THREADS, C::recs * RES_THREADS};
     };
     return shape == RES_FINE ? of(Shape<RES_FINE>{}) : of(Shape<RES_COARSE>{});
 }
 
-static size_t lds_bytes(int shape) { return sizeof(float) * 2 * (size_t)RES_LDS_COLUMNS * resident_shape(shape).column_words; }
+static size_t lds_bytes(int shape) { return sizeof(float) * 2 * (size_t)resident_shape(shape).lds_words; }
 
 int resident_capacity(int shape)
 {

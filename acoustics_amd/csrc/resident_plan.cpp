@@ -66,6 +66,56 @@ int ResPlan::tile_of(int i, int j, int k) const
 
 static int pieces(int len, int most) { return (len + most - 1) / most; }
 
+// words of a tile's six faces, each face in whole lines
+static int tile_words(int bx, int by, int bz)
+{
+    auto line = [](int n) { return (n + 15) & ~15; };
+    return 2 * (line(by * bz) + line(bx * bz) + line(bx * by));
+}
+
+// LDS words from one row of columns (along z, with its two halo columns) to
+// the next.  A wavefront's columns run over several rows; words after the halo
+// columns make the banks go on from row to row as they do within one (16
+// columns cover the 64 banks), so that its 16-byte reads do not collide.
+// Tiles that fill the LDS without them do without.
+static int row_pitch(const ResShape &sh, int by, int bz)
+{
+    const int plain = (bz + 2) * sh.column_words, even = plain + (64 - 2 * sh.column_words % 64) % 64;
+    return bz % 16 && (by + 2) * even <= sh.lds_words ? even : plain;
+}
+
+// Dispatch order of a scene's tiles: eight runs, one per XCD, each an octant
+// of the scene (halved along x, then y, then z, by number of tiles), so that
+// most neighbours share an XCD and every XCD gets its share of the damped
+// tiles; within a run the tiles with the most work first, so that the light
+// ones end up beside the heavy ones on a compute unit.
+static std::vector<int32_t> dispatch_order(const std::vector<ResTile> &tiles)
+{
+    const int n = (int)tiles.size(), per = (n + 7) / 8;
+    std::vector<int32_t> o(n);
+    for (int q = 0; q < n; ++q) o[q] = q;
+    auto centre = [&](int q, int d) {
+        const ResTile &t = tiles[q];
+        return d == 0 ? 2 * t.i0 + t.bx : d == 1 ? 2 * t.j0 + t.by : 2 * t.k0 + t.bz;
+    };
+    for (int d = 0; d < 3; ++d) {
+        const int runs = 8 >> d;   // runs of `per` tiles in each part to halve
+        for (int part = 0; part < (1 << d); ++part) {
+            const int a = std::min(n, part * runs * per), b = std::min(n, (part + 1) * runs * per);
+            std::stable_sort(o.begin() + a, o.begin() + b, [&](int x, int y) { return centre(x, d) < centre(y, d); });
+        }
+    }
+    auto weight = [&](int q) {
+        const ResTile &t = tiles[q];
+        const int axes = (t.damped & 1) + (t.damped >> 1 & 1) + (t.damped >> 2 & 1);
+        return t.bx * (axes == 0 ? 15 : axes == 1 ? 27 : 36) + (t.re > t.rb ? 200 : 0);
+    };
+    for (int part = 0; part < 8; ++part)
+        std::stable_sort(o.begin() + std::min(n, part * per), o.begin() + std::min(n, (part + 1) * per),
+                         [&](int x, int y) { return weight(x) > weight(y); });
+    return o;
+}
+
 bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
 {
     const SceneSetup &S = D.S;
@@ -93,11 +143,11 @@ bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
         for (int m = 1; m <= b.len[1]; ++m) {
             const int y = pieces(b.len[1], m);
             int z = std::min(b.len[2], RES_COLUMNS / y);
-            while (z > 1 && 2 * (y * z + b.size[0] * (y + z)) > sh.max_words) --z;
-            if (z < 1 || 2 * (y * z + b.size[0] * (y + z)) > sh.max_words) continue;
+            while (z > 1 && tile_words(b.size[0], y, z) > sh.max_words) --z;
+            if (z < 1 || tile_words(b.size[0], y, z) > sh.max_words) continue;
             const int mz = pieces(b.len[2], z);
             z = pieces(b.len[2], mz);
-            if ((y + 2) * (z + 2) > RES_LDS_COLUMNS) continue;
+            if ((y + 2) * (z + 2) * sh.column_words > sh.lds_words) continue;
             const int n = pieces(b.len[1], y) * mz;
             if (n < best || (n == best && y + z < face)) {
                 best = n;
@@ -129,11 +179,12 @@ bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
                     t.bx = std::min(b.size[0], b.lo[0] + b.len[0] - t.i0);
                     t.by = std::min(b.size[1], b.lo[1] + b.len[1] - t.j0);
                     t.bz = std::min(b.size[2], b.lo[2] + b.len[2] - t.k0);
+                    t.pitch = row_pitch(sh, t.by, t.bz);
                     t.damped = b.damped;
                     t.slab = b.slab;
-                    t.words = 2 * (t.by * t.bz + t.bx * t.bz + t.bx * t.by);
+                    t.words = tile_words(t.bx, t.by, t.bz);
                     t.word0 = (uint32_t)words;
-                    words += (uint64_t)((t.words + 7) & ~7);
+                    words += (uint64_t)((t.words + 16) & ~15);   // (tiles on lines of their own)
                     const int lo[3] = {t.i0, t.j0, t.k0}, hi[3] = {t.i0 + t.bx, t.j0 + t.by, t.k0 + t.bz};
                     for (const PSrcHost &p : S.psrc) {
                         bool hit = b.damped == 0;
@@ -149,7 +200,7 @@ bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
                 }
         P.boxes.push_back(b);
     }
-    if (words >= RES_NOWHERE) return false;
+    if (words > UINT32_MAX / 16) return false;   // byte offsets of both halves
     P.nwords = (uint32_t)words;
     // records and listener terms by tile
     const int sy = S.n[2], sx = S.n[1] * S.n[2];
@@ -180,6 +231,7 @@ bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
         P.terms.push_back({0, e.second, lt.kind, lt.kind == 0 ? (int)D.to_dev(lt.index) : lt.index, lt.beta});
         t.te = (int)P.terms.size();
     }
+    P.order = dispatch_order(P.tiles);
     return true;
 }
 
@@ -198,10 +250,11 @@ std::string resident_check(const DeviceScene &D, int shape)
         const int axes = (t.damped & 1) + (t.damped >> 1 & 1) + (t.damped >> 2 & 1);
         const int most = axes == 0 ? sh.plain : axes == 1 ? sh.one : sh.more;
         if (t.bx < 1 || t.by < 1 || t.bz < 1 || t.bx > most || t.by * t.bz > RES_COLUMNS) return "resident tile too large";
-        if ((t.by + 2) * (t.bz + 2) > RES_LDS_COLUMNS || t.words > sh.max_words) return "resident tile's halo too large";
-        if (t.words != 2 * (t.by * t.bz + t.bx * t.bz + t.bx * t.by)) return "resident tile's face words";
+        if (t.pitch < (t.bz + 2) * sh.column_words || (t.by + 2) * t.pitch > sh.lds_words || t.words > sh.max_words) return "resident tile's halo too large";
+        if (t.words != tile_words(t.bx, t.by, t.bz)) return "resident tile's face words";
         if (t.word0 < word || (uint64_t)t.word0 + (uint64_t)t.words > P.nwords) return "resident tiles share exchange words";
-        word = (uint64_t)t.word0 + (uint64_t)t.words;
+        word = (uint64_t)t.word0 + (uint64_t)t.words + 1;
+        if (word > P.nwords) return "resident tile's words";
         for (int i = t.i0; i < t.i0 + t.bx; ++i)
             for (int j = t.j0; j < t.j0 + t.by; ++j)
                 for (int k = t.k0; k < t.k0 + t.bz; ++k) {
@@ -215,6 +268,10 @@ std::string resident_check(const DeviceScene &D, int shape)
         if (t.re - t.rb > sh.max_recs || (t.re > t.rb && (t.damped || !t.skip))) return "resident records";
         for (int r = t.tb; r < t.te; ++r) ++terms[P.terms[r].slot];
     }
+    std::vector<int32_t> order(P.order);
+    std::sort(order.begin(), order.end());
+    for (size_t q = 0; q < order.size(); ++q)
+        if (order[q] != (int32_t)q || order.size() != P.tiles.size()) return "the dispatch order does not hold every tile once";
     for (uint8_t h : hit)
         if (h != 1) return "a cell lies in no resident tile";
     for (int c : recs)
@@ -313,12 +370,10 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
     for (const auto &g : groups) order.insert(order.end(), g.begin(), g.end());
     for (const ResidentScene *s : order) {
         const int m = (int)s->plan.tiles.size(), per = (m + 7) / 8;
-        // workgroup w runs on XCD w % 8: a run of consecutive tiles per XCD,
-        // so that most neighbours share one (1024 workgroups: 3.0 us per
-        // exchange against 3.9 with tiles dealt out in turn)
+        // workgroup w runs on XCD w % 8 and takes the next tile of that run
         for (int w = 0; w < 8 * per; ++w) {
             const int t = (w % 8) * per + w / 8;
-            list.push_back(t < m ? ResItem{s->dev, t, 0} : ResItem{nullptr, 0, 0});
+            list.push_back(t < m ? ResItem{s->dev, s->plan.order[t], 0} : ResItem{nullptr, 0, 0});
         }
     }
     n = (int)list.size();

@@ -35,7 +35,7 @@ __device__ __forceinline__ const AS_CONST T *cmem(const T *p) { return (const AS
 // scene with acceleration noise
 __device__ __forceinline__ double raster_accel_term(const SceneDev &S, const GhostDev &gd, long long step)
 {
-    const AS_GLOBAL double *acc = gmem(S.acc_tab) + amp_row(step) * S.n_ch + gd.obj * S.n_cpo;
+    const AS_GLOBAL double *acc = gmem(S.acc_tab) + amp_row(S, step) * S.n_ch + gd.obj * S.n_cpo;
     double v = gd.k_raster * acc[0];
     if (S.n_cpo > 1) v = fma(gd.k_vec, acc[1 + gd.vaxis], v);
     return v;
