@@ -35,7 +35,7 @@ struct Layout {
     PmlSlab *slabs;
     float *pd[3];
     float *vel[2][3];
-    float *lapv;
+    float *lapv, *inc;
     float4 *coef[3];
     int *flags[3];
     uint8_t *skip;
@@ -80,20 +80,20 @@ long long slot_cells(const SceneSetup &S) { return pad_cells((long long)S.n[0] *
 
 // Every piece of time-stepping state in one zero-initialised block: the two
 // pressure slots, the split pressures of the PML cells, both buffers of the
-// PML face velocities, and (air viscosity) the bulk cells' previous
-// Laplacian.  Each array starts on a 256-byte boundary.
+// PML face velocities, and the bulk cells' previous Laplacian (air viscosity)
+// or increment (merged staggered scheme).  Each array starts on a 256-byte boundary.
 size_t state_layout(const SceneSetup &S, long long npad, size_t off[1 + 3 + 6 + 1])
 {
     size_t o = (size_t)NUM_P_SLOTS * (size_t)npad;
     auto al = [](size_t x) { return (x + 63) / 64 * 64; };
     off[10] = o;
-    if (S.visc) o += al((size_t)npad);
+    if (S.visc || S.stag_merged) o += al((size_t)npad);
     for (int d = 0; d < 3; ++d) { off[1 + d] = o; o += al((size_t)S.n_pml); }
-    // face velocities: the PML's compact faces (collocated) or every face of the grid (staggered)
+    // face velocities: the PML's compact faces, or every face of the grid
     for (int b = 0; b < 2; ++b)
         for (int d = 0; d < 3; ++d) {
             off[4 + 3 * b + d] = o;
-            o += al(S.scheme == FDTD_SCHEME_STAGGERED ? (size_t)npad : (size_t)S.n_pml_faces[d]);
+            o += al(S.mac() ? (size_t)npad : (size_t)S.n_pml_faces[d]);
         }
     off[0] = 0;
     return o;
@@ -107,6 +107,7 @@ void carve(const SceneSetup &S, int cap, Carver &cs, Carver &c, Layout &L)
     L.state_floats = state_layout(S, slot_cells(S), off);
     L.field = cs.take<float>(L.state_floats);
     L.lapv = (L.field && S.visc) ? L.field + off[10] : nullptr;
+    L.inc = (L.field && S.stag_merged) ? L.field + off[10] : nullptr;
     for (int d = 0; d < 3; ++d) L.pd[d] = L.field ? L.field + off[1 + d] : nullptr;
     for (int b = 0; b < 2; ++b)
         for (int d = 0; d < 3; ++d) L.vel[b][d] = L.field ? L.field + off[4 + 3 * b + d] : nullptr;
@@ -329,6 +330,8 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
     D.sx = S.n[1] * sy_dev;
     D.raster = S.boundary == FDTD_BOUNDARY_RASTERIZE ? 1 : 0;
     D.scheme = S.scheme;
+    D.mac = S.mac() ? 1 : 0;
+    D.inc = L.inc;
     D.npad = npad;
     D.field = L.field;
     D.slabs = L.slabs;
@@ -480,7 +483,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                 for (int k0 = sl.lo[2]; k0 < sl.lo[2] + sl.e[2]; k0 += TK) {
                     TileDesc t{};
                     t.scene = scene_id;
-                    t.type = S.scheme == FDTD_SCHEME_STAGGERED ? TILE_MAC_PML : TILE_PML;
+                    t.type = S.mac() ? TILE_MAC_PML : TILE_PML;
                     t.i0 = i0; t.i1 = std::min(i0 + plan.pml_ti, sl.lo[0] + sl.e[0]);
                     t.j0 = j0; t.j1 = std::min(j0 + TJ, sl.lo[1] + sl.e[1]);
                     t.k0 = k0; t.k1 = std::min(k0 + TK, sl.lo[2] + sl.e[2]);
@@ -566,7 +569,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
     const int tk = std::min(plan.interior_tk_log2, std::max(0, pow2_ceil_log2(b[2] - a[2])));
     const int TK = 1 << tk, TJ = 256 >> tk;
     const int kw = b[2] - a[2];
-    const bool mac = S.scheme == FDTD_SCHEME_STAGGERED;
+    const bool mac = S.mac();
     // float4 rows start at the multiple of four at or below a[2] (the cells
     // before a[2] are read and not written); the row stride is a multiple of
     // four too, and a row's last group may be partial
@@ -763,7 +766,7 @@ static std::string check_tiles(const std::vector<TileDesc> &list, int kind, cons
         const bool ok_kind = moving ? (kind == KIND_SPECIAL || kind == KIND_ALL)
                                     : (kind == KIND_ALL || (kind == KIND_PML && pml_class) ||
                                        (kind == KIND_INTERIOR && !pml_class) || (kind == KIND_SPECIAL && t.type == TILE_SPECIAL));
-        if ((t.type == TILE_MAC || t.type == TILE_MAC_PML || t.type == TILE_MAC_VEC) != (d.scheme == FDTD_SCHEME_STAGGERED))
+        if ((t.type == TILE_MAC || t.type == TILE_MAC_PML || t.type == TILE_MAC_VEC) != (d.mac != 0))
             return "tile class does not match the scene's scheme";
         if (t.type == TILE_MAC_VEC && kind != KIND_INTERIOR && kind != KIND_ALL)
             return "staggered float4 rows outside the interior and fused launches";

@@ -97,7 +97,7 @@ struct ListenerTerm {
 // layer of cells.  A face shared by two boxes is stored in both and given the
 // same update by each.
 //
-// Merged transverse state (merge = 1, collocated scheme only): a cell of the
+// Merged transverse state (merge = 1): a cell of the
 // box that is plain along both axes other than the box axis A (no damping on
 // those axes: f1 = f3 = 1 on its faces and at the cell, no wall faces) keeps
 // only the last increment d^n = q^n - q^{n-1} of the sum q of its two
@@ -136,6 +136,15 @@ struct SceneSetup {
     double kcalp = 0, c2k2 = 0;  // c alpha dt and (c dt)^2
     int boundary = 0;
     int scheme = 0;                 // FDTD_SCHEME_*
+    // Staggered scheme in merged state (set_pml_state): cells outside the PML
+    // keep p and the last increment d = p^n - p^{n-1} less the source, instead
+    // of three face velocities.  With f1 = 1 and no damping the velocity and
+    // pressure updates reduce exactly to
+    //   d^{n+1} = d^n + (c dt / h)^2 sum_q (p_q - p),  p^{n+1} = p^n + d^{n+1} + 3 S dt
+    // (16 B per cell and step instead of 32), and the PML cells merge as the
+    // collocated scheme's do.
+    bool stag_merged = false;
+    bool mac() const { return scheme == FDTD_SCHEME_STAGGERED && !stag_merged; }   // face velocities everywhere
     // FDTD_SAMPLE_*: CENTER classifies by the cell centre, puts a
     // rasterised ghost on the face (a fully-coupled one at the solid
     // centre) with p_g = p_nbr - h grad_p . n_cell, and takes ghost values
@@ -235,8 +244,8 @@ fdtd_status build_coupled_operator(SceneSetup &S, std::string &err);
 // (f3 = f1 = 1 in the FP32 tables) and neither face is a wall.
 bool axis_plain(const SceneSetup &s, int d, int i);
 // Chooses the PML state representation: merged (the default of build_setup
-// for the collocated scheme) or the reference's per-axis split state, which
-// snapshots need.  Sets PmlSlab::merge and n_pml_merged.
+// where the scene allows it) or the reference's per-axis split state, which
+// snapshots need.  Sets PmlSlab::merge, n_pml_merged and stag_merged.
 void set_pml_state(SceneSetup &s, bool merged);
 // Engquist boundary state on the device: a face cell of layer 1 reads
 // p^{n-1} of its inner neighbour (two cells in from the exterior cell),

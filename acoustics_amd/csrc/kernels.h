@@ -103,13 +103,15 @@ struct SceneDev {
     int sx, sy;                 // strides of i and j (k fastest)
     int raster;                 // 1: rasterized ghost values, 0: fully coupled
     int scheme;                 // FDTD_SCHEME_*
+    int mac;                    // staggered scheme with a velocity on every face of the grid
+    float *inc;                 // staggered scheme, merged: the increment d per cell (null otherwise)
     long long npad;             // floats per pressure slot
     float *field;               // NUM_P_SLOTS pressure slots, full grid, k fastest
     // PML state in compact per-slab storage (PmlSlab): split pressures per
     // PML cell, face velocities per axis, double-buffered by step parity
     const PmlSlab *slabs;
     float *pd[3];
-    float *vel[2][3];           // collocated: compact PML faces; staggered: every face, full grid
+    float *vel[2][3];           // compact PML faces; mac: every face, full grid
                                 // (face d of cell c, on its low side, at c's index)
     const float4 *coef[3];      // per axis, index 0..n: {f1(face), f2(face), f3(cell), f5/h(cell)}
     const int *flags[3];        // per axis, index 0..n: 1 cell in PML, 2 face in PML, 4 sigma zero, 8 plain, 16 behind a plane constraint

@@ -181,6 +181,18 @@ __device__ __forceinline__ void emit_ghost_terms(const SceneDev &S, const TileDe
 // ---------------------------------------------------------------------------
 // interior leapfrog
 // ---------------------------------------------------------------------------
+// Sum of the pressure sources' S dt at cell (i, j, k) in step `step`.
+__device__ __forceinline__ float source_sum(const SceneDev &S, long long step, int i, int j, int k)
+{
+    float src = 0.f;
+    for (int s = 0; s < S.n_psrc; ++s) {
+        const PSrcDev ps = cmem(S.psrc)[s];
+        const AS_CONST float *g = cmem(S.gtab);
+        src = add_source(src, gmem(S.src_tab)[amp_row(S, step) * S.n_psrc + s], g[ps.goff[0] + i], g[ps.goff[1] + j], g[ps.goff[2] + k]);
+    }
+    return src;
+}
+
 __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step, bool skip_check)
 {
     const int tk = t.tk_log2;
@@ -218,6 +230,21 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
                 lapv[idx] = lc;
                 if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
             }
+        }
+        return;
+    }
+    if (S.inc) {
+        // staggered scheme, merged state (free field: no cell is skipped)
+        AS_GLOBAL float *inc = gmem(S.inc);
+        for (int i = t.i0; i < t.i1; ++i, idx += sx) {
+            const float c = pcur[idx];
+            const float dn = increment1(c, inc[idx], pcur[idx - sx], pcur[idx + sx], pcur[idx - sy], pcur[idx + sy], pcur[idx - 1],
+                                        pcur[idx + 1], lam2);
+            float pn = c + dn;
+            if (t.src) pn = fmaf(3.f, source_sum(S, step, i, j, k), pn);
+            inc[idx] = dn;
+            pnext[idx] = pn;
+            if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
         }
         return;
     }
@@ -296,6 +323,20 @@ __device__ __forceinline__ float4 leapfrog4(float4 c, float4 prev, float4 xm, fl
     return o;
 }
 
+// The merged staggered scheme's increment of four cells along k (operands as
+// leapfrog4, d the last increment).
+__device__ __forceinline__ float4 increment4(float4 c, float4 d, float4 xm, float4 xp, float4 ym, float4 yp, float zl, float zr,
+                                             float lam2)
+{
+    float4 o;
+    o.x = increment1(c.x, d.x, xm.x, xp.x, ym.x, yp.x, zl, c.y, lam2);
+    o.y = increment1(c.y, d.y, xm.y, xp.y, ym.y, yp.y, c.x, c.z, lam2);
+    o.z = increment1(c.z, d.z, xm.z, xp.z, ym.z, yp.z, c.y, c.w, lam2);
+    o.w = increment1(c.w, d.w, xm.w, xp.w, ym.w, yp.w, c.z, zr, lam2);
+    return o;
+}
+__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+
 // Whole rows, four floats per lane: wavefront w of the workgroup owns rows
 // j0 + w R .. j0 + w R + R - 1 (R = rpw rows of nk4 lanes each, R nk4 <= 64,
 // so short rows still fill the wavefront), lane l of a row the cells
@@ -303,6 +344,9 @@ __device__ __forceinline__ float4 leapfrog4(float4 c, float4 prev, float4 xm, fl
 // from the adjacent lanes; the two row ends read theirs from memory.  Plain
 // cells only (no source, no object cell); k0 and the row stride are
 // multiples of four.
+// INC: the merged staggered scheme, which keeps the increment d in place of
+// the previous level.
+template <bool INC>
 __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
 {
     // the last lane of a row may hold a partial group: its cells past k1
@@ -324,6 +368,7 @@ __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileD
     const int sx = S.sx, sy = S.sy;
     const AS_GLOBAL float *__restrict__ pcur = gmem(S.field + (size_t)slot_cur(step) * S.npad);
     AS_GLOBAL float *pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
+    AS_GLOBAL float *pold = INC ? gmem(S.inc) : pnext;
     const float lam2 = S.lam2f;
     int idx = t.i0 * sx + j * sy + k;
     if (t.i1 - t.i0 == 2 && t.te == t.tb) {
@@ -337,21 +382,37 @@ __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileD
         const float4 yp1 = *(const AS_GLOBAL float4 *)(pcur + idx + sy);
         const float4 ym2 = *(const AS_GLOBAL float4 *)(pcur + idx + sx - sy);
         const float4 yp2 = *(const AS_GLOBAL float4 *)(pcur + idx + sx + sy);
-        const float4 pv1 = *(const AS_GLOBAL float4 *)(pnext + idx);
-        const float4 pv2 = *(const AS_GLOBAL float4 *)(pnext + idx + sx);
+        const float4 pv1 = *(const AS_GLOBAL float4 *)(pold + idx);
+        const float4 pv2 = *(const AS_GLOBAL float4 *)(pold + idx + sx);
         float zl1 = __shfl_up(a1.w, 1), zr1 = __shfl_down(a1.x, 1);
         float zl2 = __shfl_up(a2.w, 1), zr2 = __shfl_down(a2.x, 1);
         if (lane == 0) { zl1 = pcur[idx - 1]; zl2 = pcur[idx + sx - 1]; }
         if (lane == nk4 - 1) { zr1 = pcur[idx + 4]; zr2 = pcur[idx + sx + 4]; }
-        const float4 o1 = leapfrog4(a1, pv1, a0, a2, ym1, yp1, zl1, zr1, lam2);
-        const float4 o2 = leapfrog4(a2, pv2, a1, a3, ym2, yp2, zl2, zr2, lam2);
+        float4 o1, o2, d1, d2;
+        if constexpr (INC) {
+            d1 = increment4(a1, pv1, a0, a2, ym1, yp1, zl1, zr1, lam2);
+            d2 = increment4(a2, pv2, a1, a3, ym2, yp2, zl2, zr2, lam2);
+            o1 = add4(a1, d1);
+            o2 = add4(a2, d2);
+        } else {
+            o1 = leapfrog4(a1, pv1, a0, a2, ym1, yp1, zl1, zr1, lam2);
+            o2 = leapfrog4(a2, pv2, a1, a3, ym2, yp2, zl2, zr2, lam2);
+        }
         if (rem == 0 && t.lead == 0) {   // whole groups only (uniform over the tile)
             if (act) {
+                if constexpr (INC) {
+                    *(AS_GLOBAL float4 *)(pold + idx) = d1;
+                    *(AS_GLOBAL float4 *)(pold + idx + sx) = d2;
+                }
                 *(AS_GLOBAL float4 *)(pnext + idx) = o1;
                 *(AS_GLOBAL float4 *)(pnext + idx + sx) = o2;
             }
         } else if (act) {
             const int n = (lane == nk4 - 1 && rem) ? rem : 4, lo = lane == 0 ? t.lead : 0;
+            if constexpr (INC) {
+                store4(pold + idx, d1, n, lo);
+                store4(pold + idx + sx, d2, n, lo);
+            }
             store4(pnext + idx, o1, n, lo);
             store4(pnext + idx + sx, o2, n, lo);
         }
@@ -363,13 +424,20 @@ __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileD
         const float4 pp = *(const AS_GLOBAL float4 *)(pcur + idx + sx);
         const float4 ym = *(const AS_GLOBAL float4 *)(pcur + idx - sy);
         const float4 yp = *(const AS_GLOBAL float4 *)(pcur + idx + sy);
-        const float4 prev = *(const AS_GLOBAL float4 *)(pnext + idx);
+        const float4 prev = *(const AS_GLOBAL float4 *)(pold + idx);
         float zl = __shfl_up(pc.w, 1), zr = __shfl_down(pc.x, 1);
         if (lane == 0) zl = pcur[idx - 1];
         if (lane == nk4 - 1) zr = pcur[idx + 4];
-        const float4 o = leapfrog4(pc, prev, pm, pp, ym, yp, zl, zr, lam2);
+        float4 o, dn;
+        if constexpr (INC) {
+            dn = increment4(pc, prev, pm, pp, ym, yp, zl, zr, lam2);
+            o = add4(pc, dn);
+        } else {
+            o = leapfrog4(pc, prev, pm, pp, ym, yp, zl, zr, lam2);
+        }
         if (act) {
             const int n = (lane == nk4 - 1 && rem) ? rem : 4, lo = lane == 0 ? t.lead : 0;
+            if constexpr (INC) store4(pold + idx, dn, n, lo);
             store4(pnext + idx, o, n, lo);
             if (t.te > t.tb) {
                 if (lo == 0) emit_cell_terms(S, t, terms, step, idx, o.x);
@@ -564,12 +632,50 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
     }
 }
 
+// A staggered scene's pulses in a PML tile (merged state), once the tile's
+// cells have been updated: S dt is added to the split pressure of every axis
+// without damping at the cell.  A pass of its own, over cells the thread has
+// just written: inside the march it took the step kernel to 82 registers
+// (5 waves a SIMD; 73 and 6 without), and it ends at once when no pulse is on.
+__device__ __forceinline__ void pml_sources(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, const TermRef *terms,
+                                            long long step)
+{
+    bool on = false;
+    for (int s = 0; s < S.n_psrc; ++s) on = on || gmem(S.src_tab)[amp_row(S, step) * S.n_psrc + s] != 0.f;
+    if (!on) return;
+    const int tk = t.tk_log2;
+    const int k = t.k0 + (threadIdx.x & ((1 << tk) - 1)), j = t.j0 + (int)(threadIdx.x >> tk);
+    if (k >= t.k1 || j >= t.j1) return;
+    AS_GLOBAL float *pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
+    const int fy = cmem(S.flags[1])[j], fz = cmem(S.flags[2])[k];
+    const bool m = sl.merge && (sl.axis == 1 || (fy & 8)) && (sl.axis == 2 || (fz & 8));
+    for (int i = t.i0; i < t.i1; ++i) {
+        const int quiet[3] = {cmem(S.flags[0])[i] & 4, fy & 4, fz & 4};
+        const int idx = i * S.sx + j * S.sy + k;
+        const int c = ((i - sl.lo[0]) * sl.e[1] + (j - sl.lo[1])) * sl.e[2] + (k - sl.lo[2]);
+        const float src = source_sum(S, step, i, j, k);
+        float pn = 0.f;
+        if (m) pn = fmaf((float)((quiet[0] ? 1 : 0) + (quiet[1] ? 1 : 0) + (quiet[2] ? 1 : 0)), src, pnext[idx]);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (m && d != sl.axis) continue;
+            AS_GLOBAL float *q = gmem(S.pd[d] + sl.cell_base) + c;
+            float n = *q;
+            if (quiet[d]) *q = n = n + src;
+            if (!m) pn = d == 0 ? n : pn + n;
+        }
+        pnext[idx] = pn;
+        if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
+    }
+}
+
 __device__ __forceinline__ void pml_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
 {
     const PmlSlab sl = cmem(S.slabs)[t.slab];
     if (sl.axis == 0) pml_tile_axis<0>(S, t, sl, terms, step);
     else if (sl.axis == 1) pml_tile_axis<1>(S, t, sl, terms, step);
     else pml_tile_axis<2>(S, t, sl, terms, step);
+    if (t.src) pml_sources(S, t, sl, terms, step);
 }
 
 // ---------------------------------------------------------------------------
@@ -1298,7 +1404,10 @@ __global__ __launch_bounds__(256) void step_kernel(const SceneDev *__restrict__ 
     if constexpr (KIND == KIND_INTERIOR) {
         // the interior launch also carries the object-adjacent cells, whose
         // FP64 gathers then hide under the interior's streaming
-        if (t.type == TILE_INTERIOR_VEC) interior_vec_tile(S, t, terms, step);
+        if (t.type == TILE_INTERIOR_VEC) {
+            if (S.inc) interior_vec_tile<true>(S, t, terms, step);
+            else interior_vec_tile<false>(S, t, terms, step);
+        }
         else if (t.type == TILE_SPECIAL) special_tile(S, t, terms, step);
         else if (t.type == TILE_MAC) mac_tile<false>(S, t, terms, step);
         else if (t.type == TILE_MAC_VEC) mac_vec_tile(S, t, terms, step);
@@ -1315,7 +1424,10 @@ __global__ __launch_bounds__(256) void step_kernel(const SceneDev *__restrict__ 
         else special_tile(S, t, terms, step);
     } else {
         if (t.type == TILE_PML) pml_tile(S, t, terms, step);
-        else if (t.type == TILE_INTERIOR_VEC) interior_vec_tile(S, t, terms, step);
+        else if (t.type == TILE_INTERIOR_VEC) {
+            if (S.inc) interior_vec_tile<true>(S, t, terms, step);
+            else interior_vec_tile<false>(S, t, terms, step);
+        }
         else if (t.type == TILE_MOVING) moving_tile(S, t, step);
         else if (t.type == TILE_SPECIAL) special_tile(S, t, terms, step);
         else if (t.type == TILE_MAC) mac_tile<false>(S, t, terms, step);

@@ -69,7 +69,8 @@ extern "C" fdtd_status fdtd_solve_noalloc(const fdtd_scene *scene, int num_steps
     std::string err;
     fdtd_status st = build_setup(*scene, D.S, err);
     if (st != FDTD_OK) { set_last_error(err); return st; }
-    set_pml_state(D.S, true);
+    // (the caller's fields of a staggered scene hold its face velocities)
+    set_pml_state(D.S, D.S.scheme == FDTD_SCHEME_COLLOCATED);
     if (D.S.moving && num_steps > D.S.mv_steps) {
         set_last_error("moving objects are planned up to stop_time (" + std::to_string(D.S.mv_steps) + " steps)");
         return FDTD_ERR_INVALID;

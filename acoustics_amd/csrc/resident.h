@@ -95,8 +95,8 @@ struct ResPlan {
 };
 
 // Why a scene cannot run resident, or null.  Which scenes can: the collocated
-// scheme with static rasterized objects, pressure sources and the merged PML
-// state.  Everything else keeps the step kernels.
+// scheme with static rasterized objects, and the staggered scheme, with
+// pressure sources and the merged state.  Everything else keeps the step kernels.
 const char *resident_refusal(const SceneSetup &S);
 // Cuts the scene for a shape; false when a tile would exceed what the kernel
 // holds per workgroup.

@@ -224,6 +224,11 @@ struct Frame {
     int ring0, cap;             // ring row of step0, rows
     uint32_t row_bytes;
     bool stuck;
+    // amplitude of the first pressure source in the step to come, fetched
+    // while the exchange of the step before runs; sources (0: none reaches the tile)
+    int src, amp_last;
+    const AS_GLOBAL float *src_tab;
+    float amp;
 
     // the scene, for code off the step loop's usual path
     __device__ __forceinline__ SceneDev scene_now() const { return *cmem(anew(scene)); }
@@ -288,6 +293,30 @@ struct Frame {
         }
         more_terms = __any(more_terms);
         stuck = false;
+        src = t.src ? S.n_psrc : 0;
+        src_tab = gmem(S.src_tab);
+        amp_last = S.amp_rows - 1;
+        amp = 0.f;
+        fetch_amp(step0);
+    }
+
+    __device__ __forceinline__ void fetch_amp(long long step)
+    {
+        if (src) amp = src_tab[(int)(step & amp_last) * src];
+    }
+    // (an amplitude of zero, once the pulse is over, adds nothing)
+    __device__ __forceinline__ bool sounding() const { return src && (amp != 0.f || src > 1); }
+    // the pressure sources' S dt at cell i of the own column in step `step`, added to v
+    __device__ __forceinline__ float add_sources(const SceneDev &Z, const ResTile &u, long long step, int i, float v) const
+    {
+        for (int p = 0; p < Z.n_psrc; ++p) {
+            const float a = p == 0 ? amp : gmem(Z.src_tab)[amp_row(Z, step) * Z.n_psrc + p];
+            if (a == 0.f) continue;
+            const PSrcDev ps = cmem(Z.psrc)[p];
+            const AS_GLOBAL float *g = gmem(Z.gtab);
+            v = add_source(v, a, g[ps.goff[0] + min(u.i0 + i, Z.n[0] - 1)], g[ps.goff[1] + u.j0 + ly], g[ps.goff[2] + u.k0 + lz]);
+        }
+        return v;
     }
 
     // Step s has been made: a cell's term takes its new pressure (in B), a
@@ -415,7 +444,9 @@ __device__ __forceinline__ void put_quad(float *B, int col, int q, const float *
 
 // Undamped cells: leapfrog, pressure sources, and the object-adjacent cells
 // of the tile in FP64 by one thread per record.
-template <int SHAPE>
+// INC: the merged staggered scheme, which keeps the increment in place of the
+// last level.
+template <int SHAPE, bool INC>
 __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, const ResTile &t)
 {
     using C = Shape<SHAPE>;
@@ -424,11 +455,10 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
     float prev[NB];
     uint32_t skip = 0;
     const float lam2 = S.lam2f;
-    const int i0 = t.i0, src = t.src ? S.n_psrc : 0;
     const bool skips = t.skip, records = t.re > t.rb;
     const int j = t.j0 + F.ly, k = t.k0 + F.lz;   // (threads without a column: the first one's)
     {
-        const AS_GLOBAL float *pp = gmem(S.field + (size_t)slot_next(F.step0) * S.npad);
+        const AS_GLOBAL float *pp = INC ? gmem(S.inc) : gmem(S.field + (size_t)slot_next(F.step0) * S.npad);
         const int idx = t.i0 * S.sx + j * S.sy + k;
 #pragma unroll
         for (int i = 0; i < NB; ++i) prev[i] = pp[idx + min(i, t.bx - 1) * S.sx];
@@ -460,20 +490,15 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
             }
         }
     }
-    // amplitudes of a step, fetched while the exchange of the one before runs
+    // accelerations of a step, fetched while the exchange of the one before runs
     double racc[NR];
-    float amp = 0.f;
-    const AS_GLOBAL float *src_tab = gmem(S.src_tab);
-    const int amp_last = S.amp_rows - 1;
-    auto amplitudes = [&](long long step) {
-        if (records) {
-            const SceneDev Z = F.scene_now();
+    auto accelerations = [&](long long step) {
+        if (!records) return;
+        const SceneDev Z = F.scene_now();
 #pragma unroll
-            for (int r = 0; r < NR; ++r) racc[r] = rat[r] >= 0 ? gmem(Z.acc_tab)[amp_row(Z, step) * Z.n_ch + robj[r]] : 0.0;
-        }
-        if (src) amp = src_tab[(int)(step & amp_last) * src];
+        for (int r = 0; r < NR; ++r) racc[r] = rat[r] >= 0 ? gmem(Z.acc_tab)[amp_row(Z, step) * Z.n_ch + robj[r]] : 0.0;
     };
-    amplitudes(F.step0);
+    accelerations(F.step0);
     for (int s = 0; s < F.steps; ++s) {
         const long long step = F.step0 + s;
         if (F.act) {
@@ -484,11 +509,17 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
                 const Quad u = quad<C::cs>(F.A, F.col, F.P, q);
                 float o[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    o[e] = leapfrog1(w.c[4 * q + e], prev[4 * q + e], 4 * q + e ? w.c[4 * q + e - 1] : w.before, w.c[4 * q + e + 1],
-                                     u.yl[e], u.yr[e], u.zl[e], u.zr[e], lam2);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) prev[4 * q + e] = w.c[4 * q + e];
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 4 * q + e;
+                    const float c = w.c[i], xm = i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
+                    if (INC) {
+                        prev[i] = increment1(c, prev[i], xm, xp, u.yl[e], u.yr[e], u.zl[e], u.zr[e], lam2);
+                        o[e] = c + prev[i];
+                    } else {
+                        o[e] = leapfrog1(c, prev[i], xm, xp, u.yl[e], u.yr[e], u.zl[e], u.zr[e], lam2);
+                        prev[i] = c;
+                    }
+                }
                 if (!skips) put_quad(F.B, F.col, q, o);
                 else {
 #pragma unroll
@@ -496,17 +527,14 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
                         if (4 * q + e < F.bx && !(skip >> (4 * q + e) & 1)) F.B[F.col + 4 * q + e] = o[e];
                 }
             }
-            // an amplitude of zero (the pulse is over) adds nothing
-            if (src && (amp != 0.f || src > 1)) {
+            if (F.sounding()) {
                 const SceneDev Z = F.scene_now();
-                for (int p = 0; p < Z.n_psrc; ++p) {
-                    const float a = p == 0 ? amp : gmem(Z.src_tab)[amp_row(Z, step) * Z.n_psrc + p];
-                    if (a == 0.f) continue;
-                    const PSrcDev ps = cmem(Z.psrc)[p];
-                    const float gy = gmem(Z.gtab)[ps.goff[1] + j], gz = gmem(Z.gtab)[ps.goff[2] + k];
-                    for (int i = 0; i < F.bx; ++i)
-                        if (!(skip >> i & 1)) F.B[F.col + i] = add_source(F.B[F.col + i], a, cmem(Z.gtab)[ps.goff[0] + i0 + i], gy, gz);
-                }
+                const ResTile u = *cmem(anew(F.tile));
+                for (int i = 0; i < F.bx; ++i)
+                    if (!(skip >> i & 1)) {
+                        float &o = F.B[F.col + i];
+                        o = INC ? fmaf(3.f, F.add_sources(Z, u, step, i, 0.f), o) : F.add_sources(Z, u, step, i, o);
+                    }
             }
         }
         if (records) {
@@ -545,12 +573,20 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
         __syncthreads();
         F.send(s);
         F.terms(s);
-        amplitudes(step + 1);
+        F.fetch_amp(step + 1);
+        accelerations(step + 1);
         F.receive(s);
         F.turn();
         __syncthreads();
     }
-    F.store_pressure(F.scene_now(), *cmem(anew(F.tile)));
+    const SceneDev Z = F.scene_now();
+    const ResTile u = *cmem(anew(F.tile));
+    F.store_pressure(Z, u);
+    if (!INC || !F.act) return;
+    const int idx = u.i0 * Z.sx + (u.j0 + anew(F.ly)) * Z.sy + u.k0 + F.lz;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+        if (i < u.bx) gmem(Z.inc)[idx + i * Z.sx] = prev[i];
 }
 
 // Face and cell coefficients of the own column along y or z.
@@ -663,9 +699,19 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, cons
                 put_quad(F.B, F.col, q, o);
             }
         }
+        if (F.act && F.sounding()) {
+            // (staggered scheme) on both undamped axes
+            const SceneDev Z = F.scene_now();
+            const ResTile u = *cmem(anew(F.tile));
+            for (int i = 0; i < F.bx; ++i) {
+                float &o = F.B[F.col + i];
+                o = fmaf(2.f, F.add_sources(Z, u, F.step0 + s, i, 0.f), o);
+            }
+        }
         __syncthreads();
         F.send(s);
         F.terms(s);
+        F.fetch_amp(F.step0 + s + 1);
         F.receive(s);
         F.turn();
         __syncthreads();
@@ -700,6 +746,7 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
     const PmlSlab sl = cmem(S.slabs)[t.slab];
     const SlabAt at(sl, t, F.ly, F.lz);
     float q0[NB], q1[NB], q2[NB], vx[NB + 1], yl[NB], yr[NB], zl[NB], zr[NB];
+    const int damped = t.damped;
     const AxisCoef cy = axis_coef(S, 1, t.j0 + F.ly), cz = axis_coef(S, 2, t.k0 + F.lz);
     {
         const int b = (int)(F.step0 & 1);
@@ -753,9 +800,24 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
                 put_quad(F.B, F.col, q, o);
             }
         }
+        if (F.act && F.sounding() && damped != 7) {
+            // (staggered scheme) on the undamped axis
+            const SceneDev Z = F.scene_now();
+            const ResTile u = *cmem(anew(F.tile));
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                if (i >= F.bx) continue;
+                const float f = F.add_sources(Z, u, F.step0 + s, i, 0.f);
+                if (damped == 6) q0[i] += f;
+                else if (damped == 5) q1[i] += f;
+                else q2[i] += f;
+                F.B[F.col + i] = q0[i] + q1[i] + q2[i];
+            }
+        }
         __syncthreads();
         F.send(s);
         F.terms(s);
+        F.fetch_amp(F.step0 + s + 1);
         F.receive(s);
         F.turn();
         __syncthreads();
@@ -843,7 +905,10 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
     __syncthreads();
     if (!gate) return;
     switch (t.damped) {
-    case 0: run_plain<SHAPE>(F, S, t); break;
+    case 0:
+        if (S.inc) run_plain<SHAPE, true>(F, S, t);
+        else run_plain<SHAPE, false>(F, S, t);
+        break;
     case 1: run_one<SHAPE, 0>(F, S, t); break;
     case 2: run_one<SHAPE, 1>(F, S, t); break;
     case 4: run_one<SHAPE, 2>(F, S, t); break;

@@ -13,7 +13,7 @@ namespace fdtd {
 
 const char *resident_refusal(const SceneSetup &S)
 {
-    if (S.scheme != FDTD_SCHEME_COLLOCATED) return "staggered scheme";
+    if (S.mac()) return "staggered scheme with face velocities";
     if (S.abc) return "Engquist boundary";
     if (S.moving) return "moving objects";
     if (S.visc) return "air viscosity";
@@ -28,7 +28,8 @@ const char *resident_refusal(const SceneSetup &S)
     // so, and every face of a damped cell but the walls is a PML face
     for (int d = 0; d < 3; ++d) {
         for (int i = 0; i < S.n[d]; ++i)
-            if ((S.cpml[d][i] != 0) == axis_plain(S, d, i)) return "PML cells without damping";
+            if ((S.cpml[d][i] != 0) == axis_plain(S, d, i) || (S.cpml[d][i] != 0) == (S.sig0[d][i] != 0))
+                return "PML cells without damping";
         for (int i = 1; i < S.n[d]; ++i)
             if ((S.fpml[d][i] != 0) != (S.cpml[d][i - 1] || S.cpml[d][i])) return "PML faces off the PML cells";
         for (int i = S.inner_lo[d]; i < S.inner_hi[d]; ++i)
@@ -187,7 +188,8 @@ bool resident_plan(const DeviceScene &D, int shape, ResPlan &P)
                     words += (uint64_t)((t.words + 16) & ~15);   // (tiles on lines of their own)
                     const int lo[3] = {t.i0, t.j0, t.k0}, hi[3] = {t.i0 + t.bx, t.j0 + t.by, t.k0 + t.bz};
                     for (const PSrcHost &p : S.psrc) {
-                        bool hit = b.damped == 0;
+                        // (collocated PML cells take no source)
+                        bool hit = b.damped == 0 || (S.stag_merged && axes < 3);
                         for (int d = 0; d < 3; ++d) hit = hit && lo[d] < p.hi[d] && hi[d] > p.lo[d];
                         t.src |= hit;
                     }
@@ -285,6 +287,9 @@ bool ResidentScene::build(const DeviceScene &D, hipStream_t st, size_t max_bytes
 {
     release();
     if (resident_refusal(D.S)) return false;
+    // (a grid that cannot fit is not cut first)
+    const ResShape most = resident_shape(RES_COARSE);
+    if (D.S.N > (int64_t)resident_capacity(RES_COARSE) * RES_COLUMNS * std::max(most.plain, most.one)) return false;
     bool ok = false;
     for (int shape = RES_FINE; shape < RES_SHAPES && !ok; ++shape)
         ok = resident_plan(D, shape, plan) && ((int)plan.tiles.size() + 7) / 8 * 8 <= resident_capacity(shape);

@@ -87,6 +87,8 @@ double algorithmic_bytes(const SceneSetup &s)
 
 double state_bytes(const SceneSetup &s)
 {
+    // merged staggered state: 16 B outside the PML, 56 split, 32 merged
+    if (s.stag_merged) return 16.0 * (double)(s.N - s.n_pml) + 56.0 * (double)s.n_pml - 24.0 * (double)s.n_pml_merged;
     return algorithmic_bytes(s) - 24.0 * (double)s.n_pml_merged;
 }
 
@@ -122,9 +124,19 @@ bool axis_plain(const SceneSetup &s, int d, int i)
 void set_pml_state(SceneSetup &s, bool merged)
 {
     s.n_pml_merged = 0;
+    s.stag_merged = merged && s.scheme == FDTD_SCHEME_STAGGERED && !s.slabs.empty();
+    for (int d = 0; d < 3 && s.stag_merged; ++d)
+        for (int i = s.inner_lo[d]; i < s.inner_hi[d]; ++i)
+            s.stag_merged = s.stag_merged && axis_plain(s, d, i) && s.sig0[d][i];
+    // the merged PML update moves a damped axis's faces only where they are
+    // PML faces; the staggered scheme moves every face, so all faces of the
+    // PML cells must be (not so when the PML ends past a cell's centre)
+    for (int d = 0; d < 3 && s.stag_merged; ++d)
+        for (int i = 1; i < s.n[d]; ++i)
+            if (s.cpml[d][i - 1] || s.cpml[d][i]) s.stag_merged = s.stag_merged && s.fpml[d][i];
     for (PmlSlab &sl : s.slabs) {
         sl.merge = 0;
-        if (!merged || s.scheme != FDTD_SCHEME_COLLOCATED) continue;
+        if (!merged || (s.scheme != FDTD_SCHEME_COLLOCATED && !s.stag_merged)) continue;
         // the march runs along x: y and z slabs merge only when x is plain
         // over their whole x range, so a column is merged or split throughout
         bool ok = true;

@@ -474,6 +474,50 @@ inline bool merged_cell(const SceneSetup &S, const PmlSlab &sl, int j, int k)
     return sl.merge && (sl.axis == 1 || axis_plain(S, 1, j)) && (sl.axis == 2 || axis_plain(S, 2, k));
 }
 
+// A staggered scene runs in merged state, which has no face velocities.  Its
+// first snapshot, saved or loaded, takes the handle to split state for good:
+// a saved one runs the steps so far again in split state (a staggered scene
+// starts at rest and is driven by its pulses alone), so that the files hold
+// every velocity and the handle goes on bit for bit as one that loads them.
+fdtd_status to_split_state(fdtd_handle *h, bool replay)
+{
+    if (!h->D.S.stag_merged) return FDTD_OK;
+    fdtd_status st = flush_series(h);
+    if (st != FDTD_OK) return st;
+    DeviceScene D;
+    D.S = h->D.S;
+    D.device = h->D.device;
+    set_pml_state(D.S, false);
+    StepProgram prog;
+    st = D.allocate_and_upload(h->stream, h->D.series_cap, LLONG_MAX);
+    if (st == FDTD_OK) {
+        std::vector<TileDesc> tiles;
+        std::vector<TermRef> terms;
+        D.append_tiles(0, tile_plan(h->tile), tiles, terms);
+        st = prog.upload({D.dev}, tiles, terms, h->stream, tile_plan(h->tile).fused);
+    }
+    if (st == FDTD_OK && replay)
+        for (long long s = 0; s < h->step && st == FDTD_OK; s += AMP_ROWS)
+            st = prog.enqueue(h->stream, s, (int)std::min<long long>(AMP_ROWS, h->step - s));
+    if (st == FDTD_OK && hipStreamSynchronize(h->stream) != hipSuccess) {
+        set_last_error("stream synchronize failed");
+        st = FDTD_ERR_DEVICE;
+    }
+    if (st != FDTD_OK) {
+        prog.release();
+        D.release();
+        return st;
+    }
+    drop_graph(h);
+    h->res_prog.release();
+    h->res.release();
+    h->prog.release();
+    h->D.release();
+    h->D = D;
+    h->prog = prog;
+    return FDTD_OK;
+}
+
 // The engine's own state file: a header, then the whole time-stepping state
 // region of the device as it lies there (pressure slots, PML state, viscous
 // Laplacian), so a handle of the same scene and state representation resumes
@@ -498,7 +542,8 @@ fdtd_status fdtd_save_snapshot(fdtd_handle *h, const char *pattern, const char *
     }
     FDTD_HIP_TRY(hipSetDevice(h->D.device));
     {
-        const fdtd_status st = settle(h);
+        fdtd_status st = settle(h);
+        if (st == FDTD_OK) st = to_split_state(h, true);
         if (st != FDTD_OK) return st;
     }
     const SceneSetup &S = h->D.S;
@@ -642,7 +687,8 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
     }
     FDTD_HIP_TRY(hipSetDevice(h->D.device));
     {
-        const fdtd_status st = settle(h);
+        fdtd_status st = settle(h);
+        if (st == FDTD_OK) st = to_split_state(h, false);
         if (st != FDTD_OK) return st;
     }
     const SceneSetup &S = h->D.S;

@@ -56,6 +56,15 @@ __device__ __forceinline__ float leapfrog1(float c, float prev, float xm, float 
     return c + fmaf(lam2, lap, c - prev);
 }
 
+// The same cell in the merged staggered scheme: its increment d^{n+1} = d^n +
+// lam2 sum_q (p_q - p^n), where the staggered update's d is f5/h times the
+// divergence of the face velocities.
+__device__ __forceinline__ float increment1(float c, float d, float xm, float xp, float ym, float yp, float zm, float zp, float lam2)
+{
+    const float lap = ((xm - c) + (xp - c)) + ((ym - c) + (yp - c)) + ((zm - c) + (zp - c));
+    return fmaf(lam2, lap, d);
+}
+
 // Face velocity update on one axis for a face whose old value is v, between
 // pressures pl (left) and pr (right); inactive faces stay at zero.  The fma
 // is explicit: a face is computed by the two cells that share it and both

@@ -327,7 +327,7 @@ const char        *fdtd_last_error(void);
 /* ------------------------------------------------------------------------- */
 typedef struct fdtd_handle fdtd_handle;
 
-/* How a PML cell of the collocated scheme keeps its state.  SPLIT is the
+/* How a PML cell keeps its state.  SPLIT is the
  * reference's state (MAC_Grid.cpp:383-508): three split pressures pDir_d and
  * the face velocities of every PML cell.  MERGED (default) gives the same
  * pressures up to FP32 rounding with fewer bytes: a cell damped along one
@@ -337,7 +337,12 @@ typedef struct fdtd_handle fdtd_handle;
  *   d^{n+1} = d^n + sum_b f5/h_b (f2_b(R) dp_R - f2_b(L) dp_L),
  *   p^{n+1} = p^n + (pDir_A^{n+1} - pDir_A^n) + d^{n+1}
  * (32 B per such cell and step instead of 56).  Snapshots need SPLIT (they
- * write every pDir_d and velocity). */
+ * write every pDir_d and velocity).  MERGED also applies to the staggered
+ * scheme: its PML cells merge the same way, and a cell outside the PML keeps
+ * the increment of its pressure instead of three face velocities (16 B instead
+ * of 32).  A staggered handle's first snapshot, saved or loaded, takes it to
+ * SPLIT for good: the steps so far are run again, so that the files hold every
+ * velocity. */
 enum {
     FDTD_PML_STATE_MERGED = 0,
     FDTD_PML_STATE_SPLIT  = 1
