@@ -163,11 +163,14 @@ TilePlan tile_plan(int id)
 // planes (plan 0), the staggered scheme 4 and 4 (plan 1: 199 us per step at
 // 256^3, against 207 us with plan 0 and 227 us as two launches).  A grid this
 // small is latency-bound and takes 2-plane PML marches (plan 10: 6.2 us per
-// step at 64^3 against 9.8; the same at 80^3, slower from 128^3 on).
+// step at 64^3 against 9.8; the same at 80^3, slower from 128^3 on).  A grid
+// well beyond the 256 MB Infinity Cache reads every halo from HBM and takes
+// plan 1's four planes and eight bands (330x290x351, 33.6 M cells: 145 us per
+// step against 159; at 256^3, 16.8 M cells, 79 against 73).
 int default_tile_plan(const SceneSetup &S)
 {
     if (S.scheme == FDTD_SCHEME_STAGGERED) return 1;
-    return S.N < 400000 ? 10 : 0;
+    return S.N < 400000 ? 10 : S.N > 25000000 ? 1 : 0;
 }
 
 size_t DeviceScene::bytes_needed(const SceneSetup &S, int series_cap)
@@ -513,8 +516,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
     // (256^3 free field 45.8 -> 41.0-41.4 us per step; the same tiles in
     // the boundary class measured 46.4)
     if (S.abc) {
-        const bool ride_rows = plan.fused && plan.interior_vec && !S.visc && S.scheme != FDTD_SCHEME_STAGGERED &&
-                               b[2] - (a[2] & ~3) <= 256;
+        const bool ride_rows = plan.fused && plan.interior_vec && !S.visc;
         const int boxes[6][6] = {
             {1, 2, 1, n[1] - 1, 1, n[2] - 1},        {n[0] - 2, n[0] - 1, 1, n[1] - 1, 1, n[2] - 1},
             {2, n[0] - 2, 1, 2, 1, n[2] - 1},        {2, n[0] - 2, n[1] - 2, n[1] - 1, 1, n[2] - 1},
@@ -590,7 +592,11 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                 mac_uniform = mac_uniform && S.f1[d][i] == S.f1[d][a[d]] && S.f2[d][i] == S.f2[d][a[d]];
                 if (i < b[d]) mac_uniform = mac_uniform && S.f5h[d][i] == S.f5h[d][a[d]];
             }
-    const bool vec = !S.visc && plan.interior_vec && kwv <= 256 && (!mac || mac_uniform);
+    const bool vec = !S.visc && plan.interior_vec && (!mac || mac_uniform);
+    // a row longer than a wavefront's 256 cells is cut into segments of equal
+    // length, a multiple of four (330x290x351: 172 -> 159 us per step against
+    // scalar tiles)
+    const int nseg = (kwv + 255) / 256, segw = ((kwv + nseg - 1) / nseg + 3) & ~3;
     auto scalar_tiles = [&](int i0, int i1, int jlo, int jhi) {
         for (int j0 = jlo; j0 < jhi; j0 += TJ)
             for (int k0 = a[2]; k0 < b[2]; k0 += TK) {
@@ -621,7 +627,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
         // 1, marches of four planes) takes G = 8: 189.7 us against 194.2 with
         // 4 and 207.4 with 2.  The Engquist free field, all rows, measured
         // 46.7 against 45.8 with groups, so it keeps single bands.
-        const int rpw = std::max(1, std::min(8, 64 / ((kwv + 3) / 4)));
+        const int rpw = std::max(1, std::min(8, 64 / ((std::min(kwv, segw) + 3) / 4)));
         const int G = S.slabs.empty() ? 1 : std::max(1, plan.band_group);
         // A z slab's row segment and the row's interior part share a 128-byte
         // line at each end of the row (16 PML cells, 64 bytes, at 256^3).  In
@@ -660,16 +666,17 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                     const int lo[3] = {i0, j0, a[2]}, hi[3] = {i1, j1, b[2]};
                     if (special_hit(lo, hi) || src_hit(lo, hi)) {
                         scalar_tiles(i0, i1, j0, j1);
-                    } else {
-                        TileDesc t{};
-                        t.scene = scene_id;
-                        t.type = mac ? TILE_MAC_VEC : TILE_INTERIOR_VEC;
-                        t.i0 = i0; t.i1 = i1; t.j0 = j0; t.j1 = j1; t.k0 = kv0; t.k1 = b[2];
-                        t.tk_log2 = 6;
-                        t.rpw = rpw;
-                        t.lead = lead;
-                        out.push_back(t);
-                    }
+                    } else
+                        for (int k0 = kv0; k0 < b[2]; k0 += segw) {
+                            TileDesc t{};
+                            t.scene = scene_id;
+                            t.type = mac ? TILE_MAC_VEC : TILE_INTERIOR_VEC;
+                            t.i0 = i0; t.i1 = i1; t.j0 = j0; t.j1 = j1; t.k0 = k0; t.k1 = std::min(k0 + segw, b[2]);
+                            t.tk_log2 = 6;
+                            t.rpw = rpw;
+                            t.lead = k0 == kv0 ? lead : 0;
+                            out.push_back(t);
+                        }
                     if (ride.empty()) continue;
                     auto it = ride.find(at(i0, j0));
                     if (it == ride.end()) continue;
