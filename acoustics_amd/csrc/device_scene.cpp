@@ -565,12 +565,13 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                 }
     }
     // object-adjacent cells
-    for (int r0 = 0; r0 < (int)S.special.size(); r0 += 256) {
+    const int per_tile = special_per_tile(S.boundary == FDTD_BOUNDARY_RASTERIZE);
+    for (int r0 = 0; r0 < (int)S.special.size(); r0 += per_tile) {
         TileDesc t{};
         t.scene = scene_id;
         t.type = TILE_SPECIAL;
         t.i0 = r0;
-        t.i1 = std::min(r0 + 256, (int)S.special.size());
+        t.i1 = std::min(r0 + per_tile, (int)S.special.size());
         out.push_back(t);
     }
     // interior: whole-row float4 tiles of four rows where the layout allows
@@ -786,7 +787,7 @@ static std::string check_tiles(const std::vector<TileDesc> &list, int kind, cons
             return "staggered float4 rows outside the interior and fused launches";
         if (!ok_kind) return "tile class does not match its launch";
         if (t.type == TILE_SPECIAL) {
-            if (t.i0 < 0 || t.i1 > d.n_special || t.i1 - t.i0 > 256) return "special tile range out of range";
+            if (t.i0 < 0 || t.i1 > d.n_special || t.i1 - t.i0 > special_per_tile(d.raster)) return "special tile range out of range";
             continue;
         }
         if (moving) {

@@ -212,6 +212,11 @@ struct TileDesc {
                                  // a multiple of four) that belong to another tile and are not written
 };
 
+// Records of a TILE_SPECIAL: one thread each; with coupled ghosts
+// COUPLED_LANES threads each, which share the ghosts' operator rows.
+enum : int { COUPLED_LANES = 8 };
+inline int special_per_tile(int raster) { return raster ? 256 : 256 / COUPLED_LANES; }
+
 struct MotionDesc {
     int scene;
 };

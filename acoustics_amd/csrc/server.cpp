@@ -369,6 +369,7 @@ fdtd_status fdtd_plan_check(const fdtd_scene *scene, int tile_config, int64_t *n
     d.n_special = (int)D.S.special.size();
     d.scheme = D.S.scheme;
     d.mac = D.S.mac() ? 1 : 0;
+    d.raster = D.S.boundary == FDTD_BOUNDARY_RASTERIZE ? 1 : 0;
     d.mv = D.S.moving ? 1 : 0;
     for (int a = 0; a < 3; ++a) { d.u_lo[a] = D.S.mv_lo[a]; d.u_n[a] = D.S.mv_hi[a] - D.S.mv_lo[a]; }
     std::vector<TileDesc> tiles;
