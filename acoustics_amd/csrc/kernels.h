@@ -57,9 +57,10 @@ __host__ __device__ inline int slot_next(long long s) { return (int)(s & 1); }
 // step, as the reference's clock runs (_simulationTime += dt).  CLK_ARRIVED
 // and CLK_GATE belong to a resident launch (resident.h): its workgroups that
 // have arrived, and whether they run (GATE_RUN) or give the block up
-// (GATE_GIVEN_UP, for good); the advance kernel shuts the gate again and leaves
-// the counter of a scene that gave up where it is.
-enum : int { CLK_STEP = 0, CLK_TARGET = 1, CLK_DONE = 2, CLK_TIME = 3, CLK_ARRIVED = 4, CLK_GATE = 5, CLK_WORDS = 8 };
+// (GATE_GIVEN_UP, for good); the advance kernel shuts the gate again.  A scene
+// that gave up has its step as its target, the true one in CLK_HELD, so that no
+// launch moves it until the host reopens it.
+enum : int { CLK_STEP = 0, CLK_TARGET = 1, CLK_DONE = 2, CLK_TIME = 3, CLK_ARRIVED = 4, CLK_GATE = 5, CLK_HELD = 6, CLK_WORDS = 8 };
 enum : unsigned long long { GATE_SHUT = 0, GATE_RUN = 1, GATE_GIVEN_UP = 2 };
 
 // the clock words of step s of a scene starting at t_start (host side)

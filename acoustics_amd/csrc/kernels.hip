@@ -1372,7 +1372,7 @@ __global__ __launch_bounds__(256) void advance_kernel(const SceneDev *__restrict
     AS_GLOBAL unsigned long long *clk = gmem(S.clock);
     const long long step = (long long)clk[CLK_STEP], target = (long long)clk[CLK_TARGET];
     if (step >= target) return;
-    const long long base = clk[CLK_GATE] == GATE_GIVEN_UP ? step : min(step + (long long)n, target);
+    const long long base = min(step + (long long)n, target);
     // rows first .. first + rows - 1, their times accumulated by one addition
     // of dt per step (the reference's clock)
     const long long first = n > 0 ? step + S.amp_rows : step;
@@ -1418,7 +1418,7 @@ __global__ __launch_bounds__(256) void advance_kernel(const SceneDev *__restrict
         clk[CLK_STEP] = (unsigned long long)base;
         clk[CLK_TIME] = (unsigned long long)__double_as_longlong(now);
         clk[CLK_ARRIVED] = 0ULL;
-        if (clk[CLK_GATE] == GATE_RUN) clk[CLK_GATE] = GATE_SHUT;
+        clk[CLK_GATE] = GATE_SHUT;
     }
 }
 

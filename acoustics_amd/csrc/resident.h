@@ -137,8 +137,8 @@ struct ResidentProgram {
     void release();
 };
 
-// Step that a scene's clock is at, and its gate shut again, for the step kernels
-// to go on from there (the stream idle).
+// Step that a scene's clock is at; one that gave up gets its target back and its
+// gate shut, for the step kernels to go on from there (the stream idle).
 fdtd_status resident_reopen(const SceneDev &dev, long long *step);
 
 // Call before a stream that had resident launches goes away, with it idle.

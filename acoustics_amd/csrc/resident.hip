@@ -894,8 +894,12 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
             if (spins >= wait_limit) {
                 u64 expect = GATE_SHUT;
                 if (__hip_atomic_compare_exchange_strong(&clk[CLK_GATE], &expect, (u64)GATE_GIVEN_UP, __ATOMIC_RELAXED,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                    // with its target at its step, nothing enqueued behind this launch moves the scene
+                    clk[CLK_HELD] = clk[CLK_TARGET];
+                    clk[CLK_TARGET] = (u64)F.step0;
                     __hip_atomic_store(trouble, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
             } else {
                 __builtin_amdgcn_s_sleep(4);
             }

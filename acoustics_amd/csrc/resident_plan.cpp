@@ -439,8 +439,11 @@ fdtd_status resident_reopen(const SceneDev &dev, long long *step)
     unsigned long long clk[CLK_WORDS];
     FDTD_HIP_TRY(hipMemcpy(clk, dev.clock, sizeof clk, hipMemcpyDeviceToHost));
     *step = (long long)clk[CLK_STEP];
+    if (clk[CLK_GATE] != GATE_GIVEN_UP) return FDTD_OK;
+    clk[CLK_TARGET] = clk[CLK_HELD];
+    clk[CLK_ARRIVED] = 0;
     clk[CLK_GATE] = GATE_SHUT;
-    FDTD_HIP_TRY(hipMemcpy(dev.clock + CLK_GATE, &clk[CLK_GATE], sizeof clk[0], hipMemcpyHostToDevice));
+    FDTD_HIP_TRY(hipMemcpy(dev.clock, clk, sizeof clk, hipMemcpyHostToDevice));
     return FDTD_OK;
 }
 

@@ -93,6 +93,20 @@ def test_given_up_blocks_are_run_by_the_step_kernels(hip_lib, monkeypatch):
             assert np.array_equal(srv.take(rid)[1], want)
 
 
+@pytest.mark.parametrize("name", ["odd", "sphere"])
+def test_short_blocks_behind_a_given_up_one(hip_lib, monkeypatch, name):
+    """Step kernels enqueued before the host knows of it leave the scene alone."""
+    sb = CASES[name]()
+    with Solver(sb, tile_config=0) as s:
+        s.step(203)
+        want = s.series()
+    monkeypatch.setenv("FDTD_RESIDENT_WAIT", "0")
+    with Solver(sb) as s:
+        for n in (70, 2, 1, 127, 3):
+            s.step(n)
+        assert np.array_equal(s.series(), want)
+
+
 def test_two_threads(hip_lib):
     """Two handles on two streams, each too large to share the device."""
     sb = CASES["largest"]()
