@@ -434,13 +434,17 @@ fdtd_status DeviceScene::read_series(long long ring_row, long long nrows, double
     if (nrows <= 0 || S.L == 0) return FDTD_OK;
     std::vector<double> rows((size_t)nrows * T);
     if (T) FDTD_HIP_TRY(hipMemcpy(rows.data(), dev.terms + (size_t)ring_row * T, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (long long r = 0; r < nrows; ++r)
-        for (int l = 0; l < S.L; ++l) {
-            double v = 0.0;
-            for (int q = S.lst_ptr[l]; q < S.lst_ptr[l + 1]; ++q) v += rows[(size_t)r * T + q];
-            out[(size_t)r * S.L + l] = v;
-        }
+    for (long long r = 0; r < nrows; ++r) sum_terms(rows.data() + (size_t)r * T, out + (size_t)r * S.L);
     return FDTD_OK;
+}
+
+void DeviceScene::sum_terms(const double *row, double *out) const
+{
+    for (int l = 0; l < S.L; ++l) {
+        double v = 0.0;
+        for (int q = S.lst_ptr[l]; q < S.lst_ptr[l + 1]; ++q) v += row[q];
+        out[l] = v;
+    }
 }
 
 void DeviceScene::release()

@@ -91,6 +91,8 @@ struct DeviceScene {
     // Listener values of ring rows [ring_row, ring_row + nrows): FP64 [nrows][L],
     // each the sum of the listener's terms in term order.
     fdtd_status read_series(long long ring_row, long long nrows, double *out) const;
+    // the same of one row's terms
+    void sum_terms(const double *row, double *out) const;
     bool needs_motion_kernel() const { return S.moving; }
 };
 

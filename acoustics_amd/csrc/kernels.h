@@ -99,6 +99,9 @@ struct MoveDev {
     double kin_dt;
 };
 
+// Terms of the longest row that is mirrored in SceneDev::tail (16 KB over PCIe).
+enum : int { TAIL_TERMS = 2048 };
+
 struct SceneDev {
     int n[3];
     int sx, sy;                 // strides of i and j (k fastest)
@@ -144,6 +147,7 @@ struct SceneDev {
     // of its terms, formed when the rows are read out
     int T, cap;                 // terms per row, rows of the ring
     double *terms;              // [cap][T]
+    double *tail;               // pinned host memory [T + 1], or null: the newest row and its step, after a block of one step
     unsigned long long *clock;  // CLK_WORDS words
     int n_obj;
     // 1: the seven-sample configuration (ghosts at 3h/4 from the fluid cell,

@@ -33,11 +33,18 @@ struct fdtd_handle {
     long long step = 0;          // steps taken
     long long flushed = 0;       // listener rows copied to host_series
     std::vector<double> host_series;
+    double *tail = nullptr;     // SceneDev::tail
     int timing = 0;             // FDTD_TIMING_*
     std::vector<hipEvent_t> ev;  // [2*i] begin, [2*i+1] end of step kernel i
     hipEvent_t call_begin = nullptr, call_end = nullptr;
     int timed_steps = 0;
 };
+
+// The mirrored row is no longer the newest (the stream idle).
+static void forget_tail(fdtd_handle *h)
+{
+    if (h->tail) h->tail[h->D.S.lst_terms.size()] = -1.0;
+}
 
 extern "C" {
 
@@ -126,6 +133,12 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
     int cap = opt.series_capacity > 0 ? opt.series_capacity : 1024;
     cap = std::max(cap, h->graph_steps + 1);
     st = h->D.allocate_and_upload(h->stream, cap, LLONG_MAX);
+    if (st == FDTD_OK && h->D.S.L > 0 && h->D.S.lst_terms.size() <= TAIL_TERMS) {
+        const size_t T = h->D.S.lst_terms.size();
+        if (hipHostMalloc(&h->tail, sizeof(double) * (T + 1)) == hipSuccess) forget_tail(h.get());
+        else h->tail = nullptr;   // (rows are then copied)
+        h->D.dev.tail = h->tail;
+    }
     if (st == FDTD_OK) {
         std::vector<TileDesc> tiles;
         std::vector<TermRef> terms;
@@ -142,6 +155,7 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
         h->res.release();
         h->prog.release();
         h->D.release();
+        if (h->tail) (void)hipHostFree(h->tail);
         if (h->own_stream) (void)hipStreamDestroy(h->stream);
         return st;
     }
@@ -168,6 +182,7 @@ fdtd_status fdtd_destroy(fdtd_handle *h)
     h->res.release();
     h->prog.release();
     h->D.release();
+    if (h->tail) (void)hipHostFree(h->tail);
     if (h->own_stream) (void)hipStreamDestroy(h->stream);
     delete h;
     return FDTD_OK;
@@ -212,6 +227,11 @@ static fdtd_status flush_series(fdtd_handle *h)
     const int cap = h->D.series_cap;
     const size_t old = h->host_series.size();
     h->host_series.resize(old + (size_t)rows * L);
+    if (rows == 1 && h->tail && h->tail[h->D.S.lst_terms.size()] == (double)(h->step - 1)) {
+        h->D.sum_terms(h->tail, h->host_series.data() + old);
+        h->flushed = h->step;
+        return FDTD_OK;
+    }
     long long r = h->flushed;
     while (r < h->step) {
         const long long ring = r % cap;
@@ -490,6 +510,7 @@ fdtd_status to_split_state(fdtd_handle *h, bool replay)
     set_pml_state(D.S, false);
     StepProgram prog;
     st = D.allocate_and_upload(h->stream, h->D.series_cap, LLONG_MAX);
+    D.dev.tail = h->tail;
     if (st == FDTD_OK) {
         std::vector<TileDesc> tiles;
         std::vector<TermRef> terms;
@@ -674,6 +695,7 @@ static fdtd_status resume_at(fdtd_handle *h, long long s)
     FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
     h->step = s;
     h->flushed = s;
+    forget_tail(h);
     h->host_series.assign((size_t)s * h->D.S.L, 0.0);
     return FDTD_OK;
 }

@@ -1,0 +1,51 @@
+"""The newest row, mirrored in host memory after a block of one step, against
+the rows read from the device: single steps, steps in blocks, rewound handles."""
+import numpy as np
+import pytest
+
+from acoustics_amd import capi, scenes
+from acoustics_amd.solver import Solver
+
+pytestmark = pytest.mark.gpu
+
+
+def scene(n_listeners, scheme=capi.FDTD_SCHEME_COLLOCATED):
+    s = scenes.base_settings((28, 33, 30), 0.005, 5)
+    s["scheme"] = scheme
+    mid = np.array(s["min_bound"]) + 0.005 * np.array([14.2, 16.4, 15.1])
+    rng = np.random.default_rng(3)
+    ears = mid + rng.uniform(-0.04, 0.04, size=(n_listeners, 3))
+    return scenes.SceneBuffers(s, pressure_sources=[scenes.gaussian_pressure_source(mid, 2e-5)], listeners=ears)
+
+
+# 256 listeners of 8 terms are the longest mirrored row
+@pytest.mark.parametrize("n_listeners", [0, 1, 33, 256, 300])
+def test_single_steps_and_blocks(hip_lib, n_listeners):
+    sb = scene(n_listeners)
+    with Solver(sb) as ref:
+        ref.step(120)
+        want = ref.series()
+    with Solver(sb) as s:
+        at = 0
+        for n in (1, 1, 7, 1, 64, 1, 1, 3, 1, 20, 1, 1, 18):
+            s.step(n)
+            at += n
+            assert np.array_equal(s.listen(), want[at - 1])
+        assert np.array_equal(s.series(), want)
+
+
+@pytest.mark.parametrize("scheme", [capi.FDTD_SCHEME_COLLOCATED, capi.FDTD_SCHEME_STAGGERED])
+def test_rewound(hip_lib, tmp_path, scheme):
+    """The mirrored row of a step is not taken for the same step made again."""
+    sb = scene(8, scheme)
+    pattern = str(tmp_path / "r_%s")
+    with Solver(sb) as s:
+        s.step(30)
+        s.save_snapshot(pattern, "x", 0)
+        s.step(4)
+        s.step(1)
+        first = s.listen()
+        s.load_snapshot(pattern, "x", 0)
+        s.step(5)
+        again = s.listen()
+        assert np.array_equal(first, again) and np.any(first)
