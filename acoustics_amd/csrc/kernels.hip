@@ -148,33 +148,33 @@ __device__ __forceinline__ double coupled_ghost(const SceneDev &S, int g, const 
 
 // ---------------------------------------------------------------------------
 // listener terms (PML_WaveSolver::FetchScalarData, MLSModeInterpolator::lookup
-// with precomputed weights): the thread that produces a term's sample writes
+// with precomputed weights): the tile that produces a term's sample writes
 // beta * sample into the scene's series ring; the terms of a listener are
 // summed when the ring is read out.  A tile lists its terms in [tb, te).
+//
+// One thread per term, once the tile's cells are written: a cell's sample is
+// read back.  (Looking for a cell's terms where it is computed walks the whole
+// list at every cell, and the tile that holds a cluster of listeners outlasted
+// the step: 96^3 with a spinning object 24.1 us per step against 21.4, and with
+// marches of four planes 36.9 against 19.0; Engquist 203x190x214 23.4, 22.0.)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void emit_cell_terms(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step,
-                                                int idx, float pn)
+__device__ __forceinline__ void emit_terms(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
 {
-    for (int q = t.tb; q < t.te; ++q) {
-        const TermRef r = cmem(terms)[q];
-        if (r.kind == 0 && r.cell == idx) gmem(S.terms)[(size_t)(step % S.cap) * S.T + r.slot] = r.beta * (double)pn;
-    }
-}
-
-__device__ __forceinline__ void emit_ghost_terms(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
-{
-    const AS_GLOBAL float *__restrict__ pcur = gmem(S.field + (size_t)slot_cur(step) * S.npad);
+    const AS_GLOBAL float *pcur = gmem(S.field + (size_t)slot_cur(step) * S.npad);
+    const AS_GLOBAL float *pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
+    AS_GLOBAL double *row = gmem(S.terms) + (size_t)(step % S.cap) * S.T;
     for (int q = t.tb + (int)threadIdx.x; q < t.te; q += (int)blockDim.x) {
-        const TermRef r = cmem(terms)[q];
-        if (r.kind == 0) continue;
+        const TermRef r = gmem(terms)[q];
         double v;
-        if (S.raster) {
+        if (r.kind == 0) {
+            v = (double)pnext[r.cell];
+        } else if (S.raster) {
             const GhostDev gd = gmem(S.ghosts)[r.cell];
             v = (double)pcur[gd.nbr] + raster_accel_term(S, gd, step);
         } else {
             v = coupled_ghost(S, r.cell, pcur, step);
         }
-        gmem(S.terms)[(size_t)(step % S.cap) * S.T + r.slot] = r.beta * v;
+        row[r.slot] = r.beta * v;
     }
 }
 
@@ -193,7 +193,7 @@ __device__ __forceinline__ float source_sum(const SceneDev &S, long long step, i
     return src;
 }
 
-__device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step, bool skip_check)
+__device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc &t, long long step, bool skip_check)
 {
     const int tk = t.tk_log2;
     const int tx = threadIdx.x & ((1 << tk) - 1), ty = threadIdx.x >> tk;
@@ -228,7 +228,6 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
             if (!skip_check || !gmem(S.skip)[idx]) {
                 pnext[idx] = pn;
                 lapv[idx] = lc;
-                if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
             }
         }
         return;
@@ -244,11 +243,10 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
             if (t.src) pn = fmaf(3.f, source_sum(S, step, i, j, k), pn);
             inc[idx] = dn;
             pnext[idx] = pn;
-            if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
         }
         return;
     }
-    if (!t.src && !skip_check && t.te == t.tb && t.i1 - t.i0 == 2) {
+    if (!t.src && !skip_check && t.i1 - t.i0 == 2) {
         // two planes with every load issued before any arithmetic
         const float a0 = pcur[idx - sx], a1 = pcur[idx], a2 = pcur[idx + sx], a3 = pcur[idx + 2 * sx];
         const float ym1 = pcur[idx - sy], yp1 = pcur[idx + sy], zm1 = pcur[idx - 1], zp1 = pcur[idx + 1];
@@ -260,7 +258,7 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
     }
     float pm = pcur[idx - sx];
     float pc = pcur[idx];
-    if (!t.src && !skip_check && t.te == t.tb) {
+    if (!t.src && !skip_check) {
         // the streaming case: 12 bytes of HBM traffic per cell
         for (int i = t.i0; i < t.i1; ++i, idx += sx) {
             const float pp = pcur[idx + sx];
@@ -289,7 +287,6 @@ __device__ __forceinline__ void interior_tile(const SceneDev &S, const TileDesc 
         if (t.src && S.n_spk) pn += speaker_at(S, i, j, k);
         if (!skip_check || !gmem(S.skip)[idx]) {
             pnext[idx] = pn;
-            if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
         }
         pm = pc;
         pc = pp;
@@ -347,7 +344,7 @@ __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(
 // INC: the merged staggered scheme, which keeps the increment d in place of
 // the previous level.
 template <bool INC>
-__device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     // the last lane of a row may hold a partial group: its cells past k1
     // (PML or row padding) are read, used as k neighbours, and not written;
@@ -371,7 +368,7 @@ __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileD
     AS_GLOBAL float *pold = INC ? gmem(S.inc) : pnext;
     const float lam2 = S.lam2f;
     int idx = t.i0 * sx + j * sy + k;
-    if (t.i1 - t.i0 == 2 && t.te == t.tb) {
+    if (t.i1 - t.i0 == 2) {
         // two planes with every load issued before any arithmetic (twice the
         // bytes in flight per wave of the marching form below)
         const float4 a0 = *(const AS_GLOBAL float4 *)(pcur + idx - sx);
@@ -439,12 +436,6 @@ __device__ __forceinline__ void interior_vec_tile(const SceneDev &S, const TileD
             const int n = (lane == nk4 - 1 && rem) ? rem : 4, lo = lane == 0 ? t.lead : 0;
             if constexpr (INC) store4(pold + idx, dn, n, lo);
             store4(pnext + idx, o, n, lo);
-            if (t.te > t.tb) {
-                if (lo == 0) emit_cell_terms(S, t, terms, step, idx, o.x);
-                if (n > 1 && lo <= 1) emit_cell_terms(S, t, terms, step, idx + 1, o.y);
-                if (n > 2 && lo <= 2) emit_cell_terms(S, t, terms, step, idx + 2, o.z);
-                if (n > 3) emit_cell_terms(S, t, terms, step, idx + 3, o.w);
-            }
         }
         pm = pc;
         pc = pp;
@@ -477,8 +468,7 @@ __device__ __forceinline__ void stb(AS_GLOBAL T *base, uint32_t off, T v)
 // the slab merges and both transverse axes are plain at it; in y and z slabs
 // x is plain over the whole slab, so merging is constant along a column.
 template <int A>
-__device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, const TermRef *terms,
-                                              long long step)
+__device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, long long step)
 {
     const int tk = t.tk_log2;
     const int tx = threadIdx.x & ((1 << tk) - 1), ty = threadIdx.x >> tk;
@@ -626,7 +616,6 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
         }
         if (solid_col || (fxC & 16)) pn = 0.f;
         stb(pnext, po, pn);
-        if (t.te > t.tb) emit_cell_terms(S, t, terms, step, (int)(po >> 2), pn);
         pm = pc;
         pc = pp;
     }
@@ -637,8 +626,7 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
 // without damping at the cell.  A pass of its own, over cells the thread has
 // just written: inside the march it took the step kernel to 82 registers
 // (5 waves a SIMD; 73 and 6 without), and it ends at once when no pulse is on.
-__device__ __forceinline__ void pml_sources(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, const TermRef *terms,
-                                            long long step)
+__device__ __forceinline__ void pml_sources(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, long long step)
 {
     bool on = false;
     for (int s = 0; s < S.n_psrc; ++s) on = on || gmem(S.src_tab)[amp_row(S, step) * S.n_psrc + s] != 0.f;
@@ -665,17 +653,16 @@ __device__ __forceinline__ void pml_sources(const SceneDev &S, const TileDesc &t
             if (!m) pn = d == 0 ? n : pn + n;
         }
         pnext[idx] = pn;
-        if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
     }
 }
 
-__device__ __forceinline__ void pml_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void pml_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     const PmlSlab sl = cmem(S.slabs)[t.slab];
-    if (sl.axis == 0) pml_tile_axis<0>(S, t, sl, terms, step);
-    else if (sl.axis == 1) pml_tile_axis<1>(S, t, sl, terms, step);
-    else pml_tile_axis<2>(S, t, sl, terms, step);
-    if (t.src) pml_sources(S, t, sl, terms, step);
+    if (sl.axis == 0) pml_tile_axis<0>(S, t, sl, step);
+    else if (sl.axis == 1) pml_tile_axis<1>(S, t, sl, step);
+    else pml_tile_axis<2>(S, t, sl, step);
+    if (t.src) pml_sources(S, t, sl, step);
 }
 
 // ---------------------------------------------------------------------------
@@ -697,7 +684,7 @@ __device__ __forceinline__ float mac_face(float4 c, float v, float pl, float pr)
 }
 
 template <bool PML>
-__device__ __forceinline__ void mac_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void mac_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     const int tk = t.tk_log2;
     const int tx = threadIdx.x & ((1 << tk) - 1), ty = threadIdx.x >> tk;
@@ -776,7 +763,6 @@ __device__ __forceinline__ void mac_tile(const SceneDev &S, const TileDesc &t, c
             pn = __fadd_rn(pc, fmaf(3.f, src, __fadd_rn(__fadd_rn(ix, iy), iz)));
         }
         pnext[idx] = pn;
-        if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, pn);
         vxL = vxR;
         pm = pc;
         pc = pp;
@@ -789,12 +775,12 @@ __device__ __forceinline__ void mac_tile(const SceneDev &S, const TileDesc &t, c
 // group (the fifth is the next lane's first, recomputed the same way), its
 // cells' low x and y faces (the high ones are recomputed by the neighbours
 // that own them) and its four pressures, marching the tile's planes with the
-// x face carried, and writes the listener terms of its cells.  Arithmetic as
+// x face carried.  Arithmetic as
 // mac_tile<false>, cell by cell.  The host
 // builds these rows only where each axis's coefficient table holds a single
 // value over the tile's faces and cells (outside the PML: f1 = 1, sigma = 0),
 // so one entry per axis is held instead of one per face.
-__device__ __forceinline__ void mac_vec_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void mac_vec_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     const int nk4 = (t.k1 - t.k0 + 3) >> 2, R = t.rpw, rem = (t.k1 - t.k0) & 3;
     const int j0w = t.j0 + (int)(threadIdx.x >> 6) * R;
@@ -862,12 +848,6 @@ __device__ __forceinline__ void mac_vec_tile(const SceneDev &S, const TileDesc &
             store4(vo1 + idx, vyL, n, lo);
             store4(vo2 + idx, make_float4(f0, f1, f2, f3), n, lo);
             store4(pnext + idx, pn, n, lo);
-            if (t.te > t.tb) {
-                if (lo == 0) emit_cell_terms(S, t, terms, step, idx, pn.x);
-                if (n > 1 && lo <= 1) emit_cell_terms(S, t, terms, step, idx + 1, pn.y);
-                if (n > 2 && lo <= 2) emit_cell_terms(S, t, terms, step, idx + 2, pn.z);
-                if (n > 3) emit_cell_terms(S, t, terms, step, idx + 3, pn.w);
-            }
         }
         vxL = vxR;
         pm = pc;
@@ -911,7 +891,7 @@ __device__ __forceinline__ double coupled_ghost_shared(const SceneDev &S, int g,
     return x;
 }
 
-__device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     const int lanes = S.raster ? 1 : COUPLED_LANES;
     const int r = t.i0 + (int)threadIdx.x / lanes, lane = (int)threadIdx.x % lanes;
@@ -969,7 +949,6 @@ __device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &
         pn += (double)speaker_at(S, i, j, k);
     }
     pnext[idx] = (float)pn;
-    if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, (float)pn);
 }
 
 // ---------------------------------------------------------------------------
@@ -987,7 +966,7 @@ __device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &
 // back in the next step from the same cell, then the current slot.  Only the
 // face cell's own thread touches its exterior cell, in either slot.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void abc_tile(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void abc_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     const int nk = t.k1 - t.k0, nj = t.j1 - t.j0;
     const int q = (int)threadIdx.x, r = q / nk;
@@ -1059,7 +1038,6 @@ __device__ __forceinline__ void abc_tile(const SceneDev &S, const TileDesc &t, c
         }
     if (t.src && S.n_spk) pn += (double)speaker_at(S, i, j, k);
     pnext[idx] = (float)pn;
-    if (t.te > t.tb) emit_cell_terms(S, t, terms, step, idx, (float)pn);
 }
 
 // ---------------------------------------------------------------------------
@@ -1448,38 +1426,41 @@ __global__ __launch_bounds__(256) void step_kernel(const SceneDev *__restrict__ 
         // the interior launch also carries the object-adjacent cells, whose
         // FP64 gathers then hide under the interior's streaming
         if (t.type == TILE_INTERIOR_VEC) {
-            if (S.inc) interior_vec_tile<true>(S, t, terms, step);
-            else interior_vec_tile<false>(S, t, terms, step);
+            if (S.inc) interior_vec_tile<true>(S, t, step);
+            else interior_vec_tile<false>(S, t, step);
         }
-        else if (t.type == TILE_SPECIAL) special_tile(S, t, terms, step);
-        else if (t.type == TILE_MAC) mac_tile<false>(S, t, terms, step);
-        else if (t.type == TILE_MAC_VEC) mac_vec_tile(S, t, terms, step);
-        else interior_tile(S, t, terms, step, t.type == TILE_INTERIOR_SKIP);
+        else if (t.type == TILE_SPECIAL) special_tile(S, t, step);
+        else if (t.type == TILE_MAC) mac_tile<false>(S, t, step);
+        else if (t.type == TILE_MAC_VEC) mac_vec_tile(S, t, step);
+        else interior_tile(S, t, step, t.type == TILE_INTERIOR_SKIP);
     } else if constexpr (KIND == KIND_PML) {
-        if (t.type == TILE_MAC_PML) mac_tile<true>(S, t, terms, step);
-        else if (t.type == TILE_ABC) abc_tile(S, t, terms, step);
-        else pml_tile(S, t, terms, step);
+        if (t.type == TILE_MAC_PML) mac_tile<true>(S, t, step);
+        else if (t.type == TILE_ABC) abc_tile(S, t, step);
+        else pml_tile(S, t, step);
     } else if constexpr (KIND == KIND_SPECIAL) {
         // with one launch per class the moving-object tiles run in this
         // launch of their own, so they do not set the register budget of the
         // streaming tiles
         if (t.type == TILE_MOVING) moving_tile(S, t, step);
-        else special_tile(S, t, terms, step);
+        else special_tile(S, t, step);
     } else {
-        if (t.type == TILE_PML) pml_tile(S, t, terms, step);
+        if (t.type == TILE_PML) pml_tile(S, t, step);
         else if (t.type == TILE_INTERIOR_VEC) {
-            if (S.inc) interior_vec_tile<true>(S, t, terms, step);
-            else interior_vec_tile<false>(S, t, terms, step);
+            if (S.inc) interior_vec_tile<true>(S, t, step);
+            else interior_vec_tile<false>(S, t, step);
         }
         else if (t.type == TILE_MOVING) moving_tile(S, t, step);
-        else if (t.type == TILE_SPECIAL) special_tile(S, t, terms, step);
-        else if (t.type == TILE_MAC) mac_tile<false>(S, t, terms, step);
-        else if (t.type == TILE_MAC_PML) mac_tile<true>(S, t, terms, step);
-        else if (t.type == TILE_MAC_VEC) mac_vec_tile(S, t, terms, step);
-        else if (t.type == TILE_ABC) abc_tile(S, t, terms, step);
-        else interior_tile(S, t, terms, step, t.type == TILE_INTERIOR_SKIP);
+        else if (t.type == TILE_SPECIAL) special_tile(S, t, step);
+        else if (t.type == TILE_MAC) mac_tile<false>(S, t, step);
+        else if (t.type == TILE_MAC_PML) mac_tile<true>(S, t, step);
+        else if (t.type == TILE_MAC_VEC) mac_vec_tile(S, t, step);
+        else if (t.type == TILE_ABC) abc_tile(S, t, step);
+        else interior_tile(S, t, step, t.type == TILE_INTERIOR_SKIP);
     }
-    if (t.te > t.tb) emit_ghost_terms(S, t, terms, step);
+    if (t.te > t.tb) {
+        __syncthreads();   // the tile's cells are written
+        emit_terms(S, t, terms, step);
+    }
 }
 
 hipError_t launch_step(int kind, const SceneDev *scenes, const TileDesc *tiles, int ntiles, int nhead, const TermRef *terms,

@@ -35,6 +35,20 @@ def test_single_steps_and_blocks(hip_lib, n_listeners):
 
 
 @pytest.mark.parametrize("scheme", [capi.FDTD_SCHEME_COLLOCATED, capi.FDTD_SCHEME_STAGGERED])
+@pytest.mark.parametrize("plan", [0, 1, 4, 10])
+def test_many_terms_in_a_tile(hip_lib, scheme, plan):
+    """2400 terms in a few tiles, some of them PML tiles, by the step kernels:
+    the resident kernel's rows."""
+    sb = scene(300, scheme)
+    with Solver(sb) as ref:
+        ref.step(90)
+        want = ref.series()
+    with Solver(sb, tile_config=plan) as s:
+        s.step(90)
+        assert np.array_equal(s.series(), want)
+
+
+@pytest.mark.parametrize("scheme", [capi.FDTD_SCHEME_COLLOCATED, capi.FDTD_SCHEME_STAGGERED])
 def test_rewound(hip_lib, tmp_path, scheme):
     """The mirrored row of a step is not taken for the same step made again."""
     sb = scene(8, scheme)
