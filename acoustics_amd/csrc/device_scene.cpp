@@ -159,18 +159,19 @@ TilePlan tile_plan(int id)
     return plans[(id >= 0 && id < kNumTilePlans) ? id : 0];
 }
 
-// One fused launch; the collocated scheme marches 2 interior and 8 PML
-// planes (plan 0), the staggered scheme 4 and 4 (plan 1: 199 us per step at
-// 256^3, against 207 us with plan 0 and 227 us as two launches).  A grid this
-// small is latency-bound and takes 2-plane PML marches (plan 10: 6.2 us per
-// step at 64^3 against 9.8; the same at 80^3, slower from 128^3 on).  A grid
-// well beyond the 256 MB Infinity Cache reads every halo from HBM and takes
-// plan 1's four planes and eight bands (330x290x351, 33.6 M cells: 145 us per
-// step against 159; at 256^3, 16.8 M cells, 79 against 73).
+// One fused launch.  Marches of four interior and four PML planes, eight bands
+// of rows together (plan 1): per step 96^3 coupled 11.2 us against 12.8 with
+// marches of 2 and 8 (plan 0), 128^3 12.3 against 15.1, 200x210x190 30.6
+// against 33.7, 256^3 70.7 against 73.4, 330x290x351 144.7 against 157, the
+// staggered 180x170x190 25.8 against 28.6 and 300x280x310 145 against 151
+// (256^3: 95.9, 94.9).  A grid this small has too few tiles for that and takes
+// marches of two (plan 10: 6.2 us at 64^3 against 7.3; at 96^3 12.0, 11.2).
+// Without a PML plan 0's two interior planes are better (101x100x98 6.8 us
+// against 8.3, 203x190x214 21.9 and 23.1, 301x300x298 63.7 and 64.6).
 int default_tile_plan(const SceneSetup &S)
 {
-    if (S.scheme == FDTD_SCHEME_STAGGERED) return 1;
-    return S.N < 400000 ? 10 : S.N > 25000000 ? 1 : 0;
+    if (S.slabs.empty()) return 0;
+    return S.N < 400000 ? 10 : 1;
 }
 
 size_t DeviceScene::bytes_needed(const SceneSetup &S, int series_cap)

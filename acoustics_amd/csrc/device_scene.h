@@ -34,8 +34,8 @@ struct TilePlan {
 constexpr int kNumTilePlans = 11;
 TilePlan tile_plan(int id);
 struct SceneSetup;
-// The single-scene default: plan 0; plan 1 for the staggered scheme; plan 10
-// for a grid of under 400,000 cells.
+// The default for a scene: plan 1; plan 10 for a grid of under 400,000 cells;
+// plan 0 without a PML.  All three are one fused launch.
 int default_tile_plan(const SceneSetup &S);
 
 // Device buffers and uploaded tables of one scene, all in one hipMalloc arena.

@@ -116,7 +116,7 @@ fdtd_status fdtd_server::rebuild()
         const int id = (int)devs.size();
         devs.push_back(r->dev->dev);
         const int tb = (int)terms.size();
-        if (!r->res.mem && r->tiles.empty()) r->dev->append_tiles(0, tile_plan(0), r->tiles, r->terms);
+        if (!r->res.mem && r->tiles.empty()) r->dev->append_tiles(0, tile_plan(default_tile_plan(r->dev->S)), r->tiles, r->terms);
         if (r->res.mem) continue;
         for (TermRef q : r->terms) { q.scene = id; terms.push_back(q); }
         for (TileDesc t : r->tiles) { t.scene = id; t.tb += tb; t.te += tb; tiles.push_back(t); }
@@ -126,7 +126,7 @@ fdtd_status fdtd_server::rebuild()
         const fdtd_status s = res_prog[shape].upload(resident_list[shape], stream);
         if (s != FDTD_OK) return s;
     }
-    return prog.upload(devs, tiles, terms, stream, tile_plan(0).fused, motion);
+    return prog.upload(devs, tiles, terms, stream, true, motion);
 }
 
 // One block of every active request: the step kernels of those that are not
@@ -238,7 +238,7 @@ void fdtd_server::run()
                 resident += (int64_t)r->res.bytes;
                 stats.peak_resident_bytes = std::max(stats.peak_resident_bytes, resident);
             } else if (s == FDTD_OK) {
-                r->dev->append_tiles(0, tile_plan(0), r->tiles, r->terms);
+                r->dev->append_tiles(0, tile_plan(default_tile_plan(r->dev->S)), r->tiles, r->terms);
             }
             std::lock_guard<std::mutex> lk(mu);
             if (s != FDTD_OK) { finish(r, s); done_cv.notify_all(); continue; }
