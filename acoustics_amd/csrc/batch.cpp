@@ -240,7 +240,7 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
             // resident ones, then every scene's clock
             const int blk = std::min(want, (int)AMP_ROWS);
             for (int k = 0; k < blk && prog_tiles > 0; ++k) {
-                const fdtd_status s = prog.enqueue_step(st, taken + k, k);
+                const fdtd_status s = prog.enqueue_step(st, taken + k, k, blk);
                 if (s != FDTD_OK) return s;
             }
             for (ResidentProgram &p : res_prog) {

@@ -71,6 +71,16 @@ static size_t moving_cells(const SceneSetup &S)
     return (size_t)(S.mv_hi[0] - S.mv_lo[0]) * (S.mv_hi[1] - S.mv_lo[1]) * (S.mv_hi[2] - S.mv_lo[2]);
 }
 
+// Steps of moving objects classified in one launch: as many as 16 MB of classes
+// and ghost terms hold, at most 16 (the launch's 10 us are then under one per step).
+static int moving_ahead(const SceneSetup &S)
+{
+    if (S.mv_ahead) return S.mv_ahead;
+    int a = 1;
+    while (a < 16 && 2 * a * 50 * moving_cells(S) <= (16u << 20)) a *= 2;
+    return a;
+}
+
 long long pad_cells(long long N) { return (N + 63) / 64 * 64; }
 
 // Cells of one pressure slot in device storage: rows along k are padded to a
@@ -137,11 +147,11 @@ void carve(const SceneSetup &S, int cap, Carver &cs, Carver &c, Layout &L)
     L.spk = c.take<double>(8 * S.spk.size());
     L.spk_samples = c.take<double>(S.spk_samples.size());
     L.spk_field = c.take<float>(S.spk.empty() ? 0 : (size_t)(S.spk_hi[0] - S.spk_lo[0]) * (S.spk_hi[1] - S.spk_lo[1]) * (S.spk_hi[2] - S.spk_lo[2]));
-    L.ucls = c.take<uint8_t>(2 * moving_cells(S));
+    L.ucls = c.take<uint8_t>(2 * moving_ahead(S) * moving_cells(S));
     L.mobj = c.take<MoveDev>(S.moving ? S.objs.size() : 0);
     L.kin = c.take<double>(S.kin.size());
     L.pose = c.take<Geom>(S.moving ? (size_t)amp_rows(S) * S.objs.size() : 0);
-    L.ughost = c.take<double>(6 * moving_cells(S));
+    L.ughost = c.take<double>(6 * moving_ahead(S) * moving_cells(S));
     L.self = c.take<SceneDev>(1);
 }
 
@@ -200,7 +210,7 @@ fdtd_status DeviceScene::reset_to_start(hipStream_t st)
     FDTD_HIP_TRY(hipMemcpyAsync(dev.clock, clk, sizeof clk, hipMemcpyHostToDevice, st));
     FDTD_HIP_TRY(fill_amplitudes(st));
     if (S.moving)
-        FDTD_HIP_TRY(hipMemcpyAsync(dev.ucls + moving_cells(S), S.mv_cls0.data(), S.mv_cls0.size(), hipMemcpyHostToDevice, st));
+        FDTD_HIP_TRY(hipMemcpyAsync(dev.ucls + (2 * moving_ahead(S) - 1) * moving_cells(S), S.mv_cls0.data(), S.mv_cls0.size(), hipMemcpyHostToDevice, st));
     FDTD_HIP_TRY(hipStreamSynchronize(st));
     return FDTD_OK;
 }
@@ -288,7 +298,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
         FDTD_HIP_TRY(up(L.mobj, mv.data(), mv.size() * sizeof(MoveDev)));
         FDTD_HIP_TRY(up(L.kin, S.kin.data(), S.kin.size() * sizeof(double)));
         // the flags of step -1 (row 1): the classification at the start pose
-        FDTD_HIP_TRY(up(L.ucls + moving_cells(S), S.mv_cls0.data(), S.mv_cls0.size()));
+        FDTD_HIP_TRY(up(L.ucls + (2 * moving_ahead(S) - 1) * moving_cells(S), S.mv_cls0.data(), S.mv_cls0.size()));
     }
     FDTD_HIP_TRY(up(L.gtab, S.gtab.data(), S.gtab.size() * 4));
     FDTD_HIP_TRY(up(L.slabs, S.slabs.data(), S.slabs.size() * sizeof(PmlSlab)));
@@ -401,6 +411,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
     D.kin = L.kin;
     D.pose = L.pose;
     D.ughost = L.ughost;
+    D.mv_ahead = moving_ahead(S);
     D.h = S.h;
     D.rho = S.rho;
     self = L.self;
@@ -1011,6 +1022,8 @@ fdtd_status StepProgram::upload(const std::vector<SceneDev> &scenes, const std::
     }
     nmotion = (int)motion.size();
     motion_cells = 0;
+    motion_ahead = INT_MAX;
+    for (const MotionDesc &m : motion) motion_ahead = std::min(motion_ahead, devs[m.scene].mv_ahead);
     for (const MotionDesc &m : motion)
         motion_cells = std::max(motion_cells, devs[m.scene].u_n[0] * devs[m.scene].u_n[1] * devs[m.scene].u_n[2]);
     nspeaker = (int)speaker.size();
@@ -1045,9 +1058,18 @@ void StepProgram::release()
     fused = false;
 }
 
-fdtd_status StepProgram::enqueue_step(hipStream_t st, long long step, int k, hipEvent_t ev_begin, hipEvent_t ev_end) const
+fdtd_status StepProgram::enqueue_step(hipStream_t st, long long step, int k, int block, hipEvent_t ev_begin, hipEvent_t ev_end) const
 {
-    if (nmotion) FDTD_HIP_TRY(launch_motion(d_scenes, d_motion, nmotion, motion_cells, k, st));
+    if (nmotion) {
+        // the last step of a block by itself is classified with its fresh cells
+        const int at = k % motion_ahead, n = std::min(motion_ahead, block - (k - at));
+        if (n > 1) {
+            if (at == 0) FDTD_HIP_TRY(launch_motion(d_scenes, d_motion, nmotion, motion_cells, k, n, st));
+            FDTD_HIP_TRY(launch_fresh(d_scenes, d_motion, nmotion, motion_cells, k, st));
+        } else {
+            FDTD_HIP_TRY(launch_motion(d_scenes, d_motion, nmotion, motion_cells, k, 0, st));
+        }
+    }
     if (nspeaker) FDTD_HIP_TRY(launch_speaker(d_scenes, d_motion + nmotion, nspeaker, speaker_cells, k, st));
     if (ev_begin) FDTD_HIP_TRY(hipEventRecord(ev_begin, st));
     auto launch = [&](int kind, hipStream_t s) {
@@ -1078,7 +1100,7 @@ fdtd_status StepProgram::enqueue(hipStream_t st, long long step, int n, const hi
         const int blk = std::min(n - done, (int)AMP_ROWS);
         for (int k = 0; k < blk; ++k) {
             const int q = done + k;
-            fdtd_status s = enqueue_step(st, step + q, k, ev ? ev[2 * q] : nullptr, ev ? ev[2 * q + 1] : nullptr);
+            fdtd_status s = enqueue_step(st, step + q, k, blk, ev ? ev[2 * q] : nullptr, ev ? ev[2 * q + 1] : nullptr);
             if (s != FDTD_OK) return s;
         }
         FDTD_HIP_TRY(launch_advance(d_scenes, nscenes, blk, st));

@@ -127,7 +127,7 @@ struct StepProgram {
     TermRef *d_terms = nullptr;
     int ntiles[NUM_KINDS] = {0, 0, 0};
     int head[NUM_KINDS] = {0, 0, 0};   // tiles dispatched first on every step (no odd-step reversal)
-    int nmotion = 0, motion_cells = 0, nspeaker = 0, speaker_cells = 0, nscenes = 0;
+    int nmotion = 0, motion_cells = 0, motion_ahead = 1, nspeaker = 0, speaker_cells = 0, nscenes = 0;
     bool fused = false;        // everything in d_tiles[KIND_INTERIOR], launched as KIND_ALL
     const unsigned long long *order_clock = nullptr;  // step word of the first scene
     // tiles of every kind in one list; split by type here (or kept in one
@@ -152,8 +152,8 @@ struct StepProgram {
     // one advance after every AMP_ROWS steps and after the last.  ev, when
     // given, holds 2n events; ev[2q], ev[2q+1] bracket step q's kernels.
     fdtd_status enqueue(hipStream_t st, long long step, int n = 1, const hipEvent_t *ev = nullptr) const;
-    // one step's launches at block offset k, without the advance
-    fdtd_status enqueue_step(hipStream_t st, long long step, int k, hipEvent_t ev_begin = nullptr,
+    // one step's launches at offset k of a block of `block` steps, without the advance
+    fdtd_status enqueue_step(hipStream_t st, long long step, int k, int block, hipEvent_t ev_begin = nullptr,
                              hipEvent_t ev_end = nullptr) const;
 };
 

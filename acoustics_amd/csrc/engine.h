@@ -128,6 +128,7 @@ struct SceneSetup {
     double h = 0, dt = 0, c = 0, rho = 0, t_start = 0, stop_time = 0;
     double lam2 = 0;             // (c dt / h)^2
     int amp_rows = 0;            // rows of the amplitude ring (0: AMP_ROWS)
+    int mv_ahead = 0;            // steps of moving objects classified in one launch (0: by the box's size)
     bool visc = false;           // air viscosity: the bulk update keeps the previous step's Laplacian
     // time-parallel chunk: every source acts only in steps s < src_steps
     // (-1: always), the first step whose start time, counted by repeated

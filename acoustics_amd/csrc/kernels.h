@@ -168,22 +168,31 @@ struct SceneDev {
     double c;                   // sound speed
     int sp_lo[3], sp_n[3];      // box of cells within 8 widths of any speaker
     float *spk_field;           // [sp_n0 sp_n1 sp_n2]: the speakers' S dt of the step being run
-    // moving objects: the box of cells reclassified every step, their bulk
-    // flags by step parity (row s & 1 holds step s's classification), the
-    // objects' motion and a ring of their poses (row amp_row(s) holds the
-    // poses at t_s; the advance kernel refills it with the amplitudes)
-    int mv;
+    // moving objects: the box of cells reclassified every step, rings of their
+    // bulk flags and ghost terms (class_row, ghost_terms), the objects' motion
+    // and a ring of their poses (row amp_row(s) holds the poses at t_s; the
+    // advance kernel refills it with the amplitudes).  mv_ahead: steps that are
+    // classified in one launch, a power of two
+    int mv, mv_ahead;
     int u_lo[3], u_n[3];
-    uint8_t *ucls;              // [2][u_n0 u_n1 u_n2], z fastest: 1 bulk, 0 solid
+    uint8_t *ucls;              // [2 mv_ahead][u_n0 u_n1 u_n2], z fastest: 1 bulk, 0 solid
     const MoveDev *mobj;        // [n_obj]
     const double *kin;          // keyframes, 8 doubles each
     Geom *pose;                 // [amp_rows][n_obj]
-    double *ughost;             // [6][u cells]: ghost term of each solid neighbour of a fluid cell (-x, +x, ..., +z)
+    double *ughost;             // [mv_ahead][6][u cells]: ghost term of each solid neighbour of a fluid cell (-x, +x, ..., +z)
     double h, rho, bmin[3];
 };
 
 // ring row of step s's amplitudes, times and poses
 __host__ __device__ inline int amp_row(const SceneDev &S, long long s) { return (int)(s & (long long)(S.amp_rows - 1)); }
+
+// row of a moving scene's classes in step s
+__host__ __device__ inline int class_row(const SceneDev &S, long long s) { return (int)(s & (long long)(2 * S.mv_ahead - 1)); }
+// and its ghost terms
+__host__ __device__ inline double *ghost_terms(const SceneDev &S, long long s)
+{
+    return S.ughost + (size_t)(s & (long long)(S.mv_ahead - 1)) * 6 * ((size_t)S.u_n[0] * S.u_n[1] * S.u_n[2]);
+}
 
 // A listener term handled by the tile that produces its sample: kind 0 is
 // the new pressure of flat cell `cell`; kind 1 the value of ghost entry
@@ -245,8 +254,11 @@ hipError_t launch_advance(const SceneDev *scenes, int nscenes, int n, hipStream_
 // per-step reclassification of each scene's box, zeroed new solid cells,
 // filled fresh cells and the ghost terms of the box's fluid cells; six
 // threads per cell along x (max_cells: the largest box of the list), one
-// scene per y.
-hipError_t launch_motion(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, hipStream_t s);
+// scene per y.  nsteps > 0: the classes and ghost terms of that many steps from
+// clock + k on (at most the scenes' mv_ahead), and launch_fresh before each.
+hipError_t launch_motion(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, int nsteps, hipStream_t s);
+// The zeroed and fresh cells of step clock + k, whose classes are there.
+hipError_t launch_fresh(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, hipStream_t s);
 // Speaker sources, before the step kernels of step clock + k: the speakers'
 // S dt over each listed scene's speaker box.
 hipError_t launch_speaker(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, hipStream_t s);

@@ -76,6 +76,7 @@ extern "C" fdtd_status fdtd_solve_noalloc(const fdtd_scene *scene, int num_steps
         return FDTD_ERR_INVALID;
     }
     D.S.amp_rows = AMP_ROWS_BOUNDED;   // the scratch is bounded
+    D.S.mv_ahead = 1;
     const int cap = AMP_ROWS_BOUNDED;   // one step block of listener rows, read out after each block
     size_t state_b = 0, table_b = 0;
     DeviceScene::region_bytes(D.S, cap, &state_b, &table_b);

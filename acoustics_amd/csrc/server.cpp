@@ -139,7 +139,7 @@ fdtd_status fdtd_server::run_block()
     for (int done = 0; done < block;) {
         const int blk = std::min(block - done, (int)AMP_ROWS);
         for (int k = 0; k < blk && kernels; ++k) {
-            const fdtd_status s = prog.enqueue_step(stream, done + k, k);
+            const fdtd_status s = prog.enqueue_step(stream, done + k, k, blk);
             if (s != FDTD_OK) return s;
         }
         for (ResidentProgram &p : res_prog) {
@@ -338,6 +338,7 @@ int64_t fdtd_scene_device_bytes(const fdtd_scene *scene)
     SceneSetup S;
     std::string err;
     if (build_setup(*scene, S, err) != FDTD_OK) { set_last_error(err); return -1; }
+    S.mv_ahead = 1;
     return (int64_t)DeviceScene::bytes_needed(S, 1);
 }
 
@@ -517,6 +518,7 @@ fdtd_status fdtd_server_submit(fdtd_server *s, const fdtd_scene *scene, int num_
         return FDTD_ERR_INVALID;
     }
     r->steps = num_steps;
+    r->setup.mv_ahead = 1;   // its memory counts against the budget
     r->bytes = DeviceScene::bytes_needed(r->setup, num_steps);
     r->submitted = Clock::now();
     std::lock_guard<std::mutex> lk(s->mu);
