@@ -160,9 +160,9 @@ void carve(const SceneSetup &S, int cap, Carver &cs, Carver &c, Layout &L)
 TilePlan tile_plan(int id)
 {
     // {interior k threads (log2), interior planes, PML planes, whole-row float4 interior, one launch,
-    //  PML k threads (log2)[, bands of float4 rows taken together]}
+    //  PML k threads (log2)[, bands of float4 rows taken together[, interior planes without a PML]]}
     static const TilePlan plans[kNumTilePlans] = {
-        {6, 2, 8, true, true, 6, 4}, {6, 4, 4, true, true, 6, 8}, {6, 8, 8, true, true, 6},   {6, 4, 8, true, false, 6},
+        {6, 4, 4, true, true, 6, 8, 2}, {6, 4, 4, true, true, 6, 8}, {6, 8, 8, true, true, 6},   {6, 4, 8, true, false, 6},
         {6, 8, 8, false, false, 6}, {6, 4, 8, true, true, 5},   {6, 4, 16, true, true, 6},  {6, 4, 8, true, true, 6},
         {6, 4, 4, false, false, 6}, {6, 4, 8, true, true, 4},   {6, 2, 2, true, true, 6},
     };
@@ -170,18 +170,18 @@ TilePlan tile_plan(int id)
 }
 
 // One fused launch.  Marches of four interior and four PML planes, eight bands
-// of rows together (plan 1): per step 96^3 coupled 11.2 us against 12.8 with
-// marches of 2 and 8 (plan 0), 128^3 12.3 against 15.1, 200x210x190 30.6
-// against 33.7, 256^3 70.7 against 73.4, 330x290x351 144.7 against 157, the
+// of rows together (plans 0 and 1): per step 96^3 coupled 11.2 us against 12.8
+// with marches of 2 and 8 in four bands, 128^3 12.3 against 15.1, 200x210x190
+// 30.6 against 33.7, 256^3 70.7 against 73.4, 330x290x351 144.7 against 157, the
 // staggered 180x170x190 25.8 against 28.6 and 300x280x310 145 against 151
 // (256^3: 95.9, 94.9).  A grid this small has too few tiles for that and takes
 // marches of two (plan 10: 6.2 us at 64^3 against 7.3; at 96^3 12.0, 11.2).
-// Without a PML plan 0's two interior planes are better (101x100x98 6.8 us
-// against 8.3, 203x190x214 21.9 and 23.1, 301x300x298 63.7 and 64.6).
+// Without a PML two interior planes are better (101x100x98 6.8 us against 8.3,
+// 203x190x214 21.9 and 23.1, 301x300x298 63.7 and 64.6).
 int default_tile_plan(const SceneSetup &S)
 {
-    if (S.slabs.empty()) return 0;
-    return S.N < 400000 ? 10 : 1;
+    if (S.scheme == FDTD_SCHEME_STAGGERED) return 1;
+    return S.N < 400000 ? 10 : 0;
 }
 
 size_t DeviceScene::bytes_needed(const SceneSetup &S, int series_cap)
@@ -609,6 +609,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                 mac_uniform = mac_uniform && S.f1[d][i] == S.f1[d][a[d]] && S.f2[d][i] == S.f2[d][a[d]];
                 if (i < b[d]) mac_uniform = mac_uniform && S.f5h[d][i] == S.f5h[d][a[d]];
             }
+    const int ti = S.slabs.empty() && plan.open_ti ? plan.open_ti : plan.interior_ti;
     const bool vec = !S.visc && plan.interior_vec && (!mac || mac_uniform);
     // a row longer than a wavefront's 256 cells is cut into segments of equal
     // length, a multiple of four (330x290x351: 172 -> 159 us per step against
@@ -630,7 +631,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
             }
     };
     if (!vec) {
-        for (int i0 = a[0]; i0 < b[0]; i0 += plan.interior_ti) scalar_tiles(i0, std::min(i0 + plan.interior_ti, b[0]), a[1], b[1]);
+        for (int i0 = a[0]; i0 < b[0]; i0 += ti) scalar_tiles(i0, std::min(i0 + ti, b[0]), a[1], b[1]);
     } else {
         // short rows share a wavefront: rpw rows of kwv/4 lanes each.  The
         // tiles of a band of rows follow each other along x, so a tile's x
@@ -665,7 +666,7 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                 const TileDesc &z = out[q];
                 const int li = z.i1 - 1, lj = z.j1 - 1;
                 if (li < a[0] || li >= b[0] || lj < a[1] || lj >= b[1]) continue;
-                const int i0t = a[0] + (li - a[0]) / plan.interior_ti * plan.interior_ti;
+                const int i0t = a[0] + (li - a[0]) / ti * ti;
                 const int j0t = a[1] + (lj - a[1]) / (4 * rpw) * (4 * rpw);
                 ride[at(i0t, j0t)].push_back(z);
                 moved[q] = 1;
@@ -676,8 +677,8 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
             out.resize(w);
         }
         for (int jg = a[1]; jg < b[1]; jg += G * 4 * rpw) {
-            for (int i0 = a[0]; i0 < b[0]; i0 += plan.interior_ti) {
-                const int i1 = std::min(i0 + plan.interior_ti, b[0]);
+            for (int i0 = a[0]; i0 < b[0]; i0 += ti) {
+                const int i1 = std::min(i0 + ti, b[0]);
                 for (int j0 = jg; j0 < std::min(b[1], jg + G * 4 * rpw); j0 += 4 * rpw) {
                     const int j1 = std::min(j0 + 4 * rpw, b[1]);
                     const int lo[3] = {i0, j0, a[2]}, hi[3] = {i1, j1, b[2]};

@@ -30,12 +30,13 @@ struct TilePlan {
     bool fused = false;        // one launch for all tile classes
     int pml_tk_log2 = 6;       // PML slab columns: up to 1 << pml_tk_log2 along k, 256 >> it along j
     int band_group = 1;        // float4 row tiles: this many bands of rows advance along x together
+    int open_ti = 0;           // interior planes of a grid without a PML (0: interior_ti)
 };
 constexpr int kNumTilePlans = 11;
 TilePlan tile_plan(int id);
 struct SceneSetup;
-// The default for a scene: plan 1; plan 10 for a grid of under 400,000 cells;
-// plan 0 without a PML.  All three are one fused launch.
+// The default for a scene: plan 0; plan 1 for the staggered scheme; plan 10 for
+// a grid of under 400,000 cells.  All three are one fused launch.
 int default_tile_plan(const SceneSetup &S);
 
 // Device buffers and uploaded tables of one scene, all in one hipMalloc arena.

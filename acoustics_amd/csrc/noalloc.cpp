@@ -90,7 +90,7 @@ extern "C" fdtd_status fdtd_solve_noalloc(const fdtd_scene *scene, int num_steps
     if (((uintptr_t)fields & 255u) != 0) { set_last_error("fields must be 256-byte aligned"); return FDTD_ERR_INVALID; }
     if (D.S.L > 0 && num_steps > 0 && !series) { set_last_error("null series buffer"); return FDTD_ERR_INVALID; }
     const int plan = D.S.scheme == FDTD_SCHEME_STAGGERED ? 3 : 0;   // fdtd_create's default plans
-    const TilePlan tp = tile_plan(plan);
+    TilePlan tp = tile_plan(plan);
     D.sy_dev = row_stride(D.S);   // (the tile builder indexes device rows)
     std::vector<TileDesc> tiles;
     std::vector<TermRef> terms;
@@ -99,7 +99,15 @@ extern "C" fdtd_status fdtd_solve_noalloc(const fdtd_scene *scene, int num_steps
     if (D.needs_motion_kernel()) motion.push_back({0});
     const size_t npre = motion.size() + (D.S.spk.empty() ? 0 : 1);
     const size_t table_region = (table_b + 255) & ~(size_t)255;
-    const size_t prog_b = StepProgram::bytes_needed(1, tiles, tp.fused, terms.size(), npre);
+    size_t prog_b = StepProgram::bytes_needed(1, tiles, tp.fused, terms.size(), npre);
+    if (table_region + prog_b > kScratchBytes) {
+        // longer marches are fewer tiles
+        tp = tile_plan(6);
+        tiles.clear();
+        terms.clear();
+        D.append_tiles(0, tp, tiles, terms);
+        prog_b = StepProgram::bytes_needed(1, tiles, tp.fused, terms.size(), npre);
+    }
     if (table_region + prog_b > kScratchBytes) {
         set_last_error("the scene's tables and step program need " + std::to_string(table_region + prog_b) +
                        " bytes of scratch; fdtd_solve_noalloc holds at most " + std::to_string(kScratchBytes));
