@@ -184,6 +184,17 @@ int default_tile_plan(const SceneSetup &S)
     return S.N < 400000 ? 10 : 0;
 }
 
+size_t DeviceScene::base_layout(size_t off[11]) const
+{
+    SceneSetup old;
+    old.visc = S.visc;
+    old.scheme = S.scheme;
+    old.stag_merged = S.stag_merged;
+    old.n_pml = S.n_pml;
+    for (int d = 0; d < 3; ++d) old.n_pml_faces[d] = S.base_faces[d];
+    return state_layout(old, npad, off);
+}
+
 size_t DeviceScene::bytes_needed(const SceneSetup &S, int series_cap)
 {
     Carver c;

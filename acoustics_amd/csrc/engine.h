@@ -117,7 +117,7 @@ struct ListenerTerm {
 struct PmlSlab {
     int32_t lo[3], e[3];
     int32_t axis;                // the box's damped axis (x slabs 0, y slabs 1, z slabs 2)
-    int32_t merge;               // 1: merged transverse state for eligible cells
+    int32_t merge;               // 1: merged transverse state in every cell; 0: split state in every cell
     int64_t cell_base;
     int64_t v_base[3];
 };
@@ -176,8 +176,18 @@ struct SceneSetup {
     // never updated (MAC_Grid.cpp:521-919)
     bool abc = false;
     int64_t n_pml = 0;
-    std::vector<PmlSlab> slabs;        // the PML as up to six disjoint boxes
-    int64_t n_pml_faces[3] = {0, 0, 0};  // compact face-velocity entries per axis
+    // the PML as up to six disjoint slabs, and as the boxes its state is stored
+    // in (set_pml_state): a slab that merges is cut where merged cells meet split
+    // ones, so that a box holds one kind.  The split cells along the grid's
+    // edges then lie close together: in a slab that spans the grid they are the
+    // ends of its rows, 64 of every 1024 bytes of nine arrays, whose half-used
+    // lines took 24 of 68 us per step at 256^3 for 4% of the cells, most of it
+    // because the state no longer fitted the 256 MB Infinity Cache (now 57 us;
+    // 256x256x250 75 -> 55, 330x290x351 144 -> 138).  With compact
+    // face-velocity entries per axis.
+    std::vector<PmlSlab> base_slabs, slabs;
+    int64_t base_faces[3] = {0, 0, 0}, n_pml_faces[3] = {0, 0, 0};
+    bool pml_merged = false;           // every slab merges
     int64_t n_pml_merged = 0;           // PML cells holding merged transverse state
     // sources
     std::vector<PSrcHost> psrc;
@@ -246,7 +256,7 @@ fdtd_status build_coupled_operator(SceneSetup &S, std::string &err);
 bool axis_plain(const SceneSetup &s, int d, int i);
 // Chooses the PML state representation: merged (the default of build_setup
 // where the scene allows it) or the reference's per-axis split state, which
-// snapshots need.  Sets PmlSlab::merge, n_pml_merged and stag_merged.
+// snapshots need.  Sets slabs, n_pml_faces, n_pml_merged, pml_merged and stag_merged.
 void set_pml_state(SceneSetup &s, bool merged);
 // Engquist boundary state on the device: a face cell of layer 1 reads
 // p^{n-1} of its inner neighbour (two cells in from the exterior cell),

@@ -463,12 +463,10 @@ __device__ __forceinline__ void stb(AS_GLOBAL T *base, uint32_t off, T v)
     *(AS_GLOBAL T *)((AS_GLOBAL char *)base + off) = v;
 }
 
-// A = the slab's damped axis.  Threads run along z (lanes) and y (rows) and
-// march along x, carrying the x face between planes.  A cell is merged when
-// the slab merges and both transverse axes are plain at it; in y and z slabs
-// x is plain over the whole slab, so merging is constant along a column.
-template <int A>
-__device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, long long step)
+// Cells damped along two or three axes, or every PML cell without the merged
+// state: a split pressure per axis and the faces of all three.  Threads run along
+// z (lanes) and y (rows) and march along x, carrying the x face between planes.
+__device__ __forceinline__ void pml_split_tile(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, long long step)
 {
     const int tk = t.tk_log2;
     const int tx = threadIdx.x & ((1 << tk) - 1), ty = threadIdx.x >> tk;
@@ -477,7 +475,7 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
     const int nx = S.n[0], ny = S.n[1], nz = S.n[2];
     const AS_GLOBAL float *__restrict__ pcur = gmem(S.field + (size_t)slot_cur(step) * S.npad);
     AS_GLOBAL float *__restrict__ pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
-    // compact storage of this slab: cells (and x faces) have plane stride
+    // compact storage of this box: cells (and x faces) have plane stride
     // e1*e2; y faces (e1+1)*e2; z faces e1*(e2+1)
     const int e0 = sl.e[0], e1 = sl.e[1], e2 = sl.e[2];
     const int li0 = t.i0 - sl.lo[0], lj = j - sl.lo[1], lk = k - sl.lo[2];
@@ -514,22 +512,8 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
     const bool yr_on = has_yR && ((fyR & 2) || ck), yr_ci = has_yR;
     const bool zl_on = k >= 1 && ((fzL & 2) || cj), zl_ci = k >= 1;
     const bool zr_on = has_zR && ((fzR & 2) || cj), zr_ci = has_zR;
-    // the high y / z face of this column is stored here when it is the slab's last layer
+    // the high y / z face of this column is stored here when it is the box's last layer
     const bool own_yR = lj == e1 - 1, own_zR = lk == e2 - 1;
-
-    // merged or split; a split axis keeps its pDir and faces.  The low face of
-    // a merged cell is still updated when the cell below it in the slab is
-    // split on that axis (that cell reads it as its high face).
-    const bool mg = sl.merge != 0;
-    const bool py = A == 1 || (fyL & 8), pz = A == 2 || (fzL & 8);
-    const bool m = mg && py && pz;
-    const bool sx = A == 0 || !m, sy = A == 1 || !m, sz = A == 2 || !m;
-    const int fyM = lj >= 1 ? fy[j - 1] : 0, fzM = lk >= 1 ? fz[k - 1] : 0;
-    const bool need_yL = sy || (lj >= 1 && !(mg && (A == 1 || (fyM & 8)) && pz));
-    const bool need_zL = sz || (lk >= 1 && !(mg && py && (A == 2 || (fzM & 8))));
-    // merged state: the increment d in the lower transverse axis's array; q
-    // itself is p - pDir_A
-    AS_GLOBAL float *__restrict__ darr = A == 0 ? pd1 : pd0;
 
     // byte offsets
     const uint32_t sx4 = 4u * (uint32_t)S.sx, sy4 = 4u * (uint32_t)S.sy;
@@ -546,78 +530,151 @@ __device__ __forceinline__ void pml_tile_axis(const SceneDev &S, const TileDesc 
     float pc = ldb(pcur, po);
     // the x face on the low side of the current cell (updated value), carried
     // from one plane to the next: cell i's high face is cell i+1's low face
-    float vxL = 0.f;
-    if (sx) vxL = face_update(t.i0 >= 1 && ((fx[t.i0] & 2) || ox), cx[t.i0], ldb(vi0, co), pm, pc);
+    float vxL = face_update(t.i0 >= 1 && ((fx[t.i0] & 2) || ox), cx[t.i0], ldb(vi0, co), pm, pc);
     const int ilast = sl.lo[0] + e0 - 1;
     for (int i = t.i0; i < t.i1; ++i, po += sx4, co += cs4, yo += ys4, zo += zs4) {
         const bool last = i + 1 >= nx;
         const float pp = ldb(pcur, po + (last ? 0u : sx4));
         const float ym = ldb(pcur, po - ym4), yp = ldb(pcur, po + yp4);
         const float zm = ldb(pcur, po - zm4), zp = ldb(pcur, po + zp4);
-        float vxr_old = 0.f, vyl_old = 0.f, vyr_old = 0.f, vzl_old = 0.f, vzr_old = 0.f;
-        float q0 = 0.f, q1 = 0.f, q2 = 0.f, qd = 0.f;
-        if (sx) { vxr_old = ldb(vi0, co + cs4); q0 = ldb(pd0, co); }
-        if (need_yL) vyl_old = ldb(vi1, yo);
-        if (sy) { vyr_old = ldb(vi1, yo + e24); q1 = ldb(pd1, co); }
-        if (need_zL) vzl_old = ldb(vi2, zo);
-        if (sz) { vzr_old = ldb(vi2, zo + 4u); q2 = ldb(pd2, co); }
-        if (m) qd = ldb(darr, co);
+        const float vxr_old = ldb(vi0, co + cs4), vyl_old = ldb(vi1, yo), vyr_old = ldb(vi1, yo + e24);
+        const float vzl_old = ldb(vi2, zo), vzr_old = ldb(vi2, zo + 4u);
+        const float q0 = ldb(pd0, co), q1 = ldb(pd1, co), q2 = ldb(pd2, co);
         const int fxC = fx[i], fxR = last ? 0 : fx[i + 1];
         const float4 cxC = cx[i], cxR = cx[min(i + 1, nx)];
         const bool ci = fxC & 1;
-        float n0 = 0.f, n1 = 0.f, n2 = 0.f;
         // x: high face (new), low face carried
-        if (sx) {
-            const float vxR = last ? 0.f : face_update((fxR & 2) || ox, cxR, vxr_old, pc, pp);
-            stb(vo0, co, vxL);
-            if (i == ilast) stb(vo0, co + cs4, vxR);
-            n0 = split_update(cxC, q0, vxR - vxL);
-            stb(pd0, co, n0);
-            vxL = vxR;
-        }
-        // y
-        float vyL = 0.f;
-        if (need_yL) {
-            vyL = face_update(yl_on || (ci && yl_ci), cyL, vyl_old, ym, pc);
-            stb(vo1, yo, vyL);
-        }
-        if (sy) {
-            const float vyR = face_update(yr_on || (ci && yr_ci), cyR, vyr_old, pc, yp);
-            if (own_yR) stb(vo1, yo + e24, vyR);
-            n1 = split_update(cyL, q1, vyR - vyL);
-            stb(pd1, co, n1);
-        }
-        // z
-        float vzL = 0.f;
-        if (need_zL) {
-            vzL = face_update(zl_on || (ci && zl_ci), czL, vzl_old, zm, pc);
-            stb(vo2, zo, vzL);
-        }
-        if (sz) {
-            const float vzR = face_update(zr_on || (ci && zr_ci), czR, vzr_old, pc, zp);
-            if (own_zR) stb(vo2, zo + 4u, vzR);
-            n2 = split_update(czL, q2, vzR - vzL);
-            stb(pd2, co, n2);
-        }
-        float pn;
-        if (m) {
-            float lap = 0.f;
-            if constexpr (A != 0) lap = transverse_add(lap, cxC.w, cxC.y, cxR.y, pm, pc, pp);
-            if constexpr (A != 1) lap = transverse_add(lap, cyL.w, cyL.y, cyR.y, ym, pc, yp);
-            if constexpr (A != 2) lap = transverse_add(lap, czL.w, czL.y, czR.y, zm, pc, zp);
-            // p^{n+1} = p^n + (pDir_A^{n+1} - pDir_A^n) + d^{n+1}: only
-            // increments are rounded before the last addition
-            const float dn = qd + lap;
-            const float dA = (A == 0 ? n0 : A == 1 ? n1 : n2) - (A == 0 ? q0 : A == 1 ? q1 : q2);
-            stb(darr, co, dn);
-            pn = pc + (dA + dn);
-        } else {
-            pn = n0 + n1 + n2;
-        }
+        const float vxR = last ? 0.f : face_update((fxR & 2) || ox, cxR, vxr_old, pc, pp);
+        const float vyL = face_update(yl_on || (ci && yl_ci), cyL, vyl_old, ym, pc);
+        const float vyR = face_update(yr_on || (ci && yr_ci), cyR, vyr_old, pc, yp);
+        const float vzL = face_update(zl_on || (ci && zl_ci), czL, vzl_old, zm, pc);
+        const float vzR = face_update(zr_on || (ci && zr_ci), czR, vzr_old, pc, zp);
+        stb(vo0, co, vxL);
+        if (i == ilast) stb(vo0, co + cs4, vxR);
+        stb(vo1, yo, vyL);
+        if (own_yR) stb(vo1, yo + e24, vyR);
+        stb(vo2, zo, vzL);
+        if (own_zR) stb(vo2, zo + 4u, vzR);
+        const float n0 = split_update(cxC, q0, vxR - vxL);
+        const float n1 = split_update(cyL, q1, vyR - vyL);
+        const float n2 = split_update(czL, q2, vzR - vzL);
+        stb(pd0, co, n0);
+        stb(pd1, co, n1);
+        stb(pd2, co, n2);
+        float pn = n0 + n1 + n2;
         if (solid_col || (fxC & 16)) pn = 0.f;
         stb(pnext, po, pn);
+        vxL = vxR;
         pm = pc;
         pc = pp;
+    }
+}
+
+// Cells damped along A only, in the merged state (PmlSlab::merge): the split
+// pressure and the faces along A, and the increment d of the transverse sum,
+// whose lower axis's array holds it.  Each cell has its own few values and no
+// lane branches, so two planes have every load issued before any arithmetic.
+// Bound: the memory side (32 bytes a cell and step; the instructions take a
+// quarter of the time).  Beside pml_split_tile in one body with a branch per
+// axis: 92 VALU and 70 SALU instructions a cell against 68 and 40, no faster by
+// itself, but it is what lets a box hold one kind of cell.
+template <int A>
+__device__ __forceinline__ void pml_merged_axis(const SceneDev &S, const TileDesc &t, const PmlSlab &sl, long long step)
+{
+    const int tk = t.tk_log2;
+    const int k = t.k0 + (int)(threadIdx.x & ((1 << tk) - 1)), j = t.j0 + (int)(threadIdx.x >> tk);
+    if (k >= t.k1 || j >= t.j1) return;
+    const int nx = S.n[0], ny = S.n[1], nz = S.n[2];
+    const AS_GLOBAL float *__restrict__ pcur = gmem(S.field + (size_t)slot_cur(step) * S.npad);
+    AS_GLOBAL float *__restrict__ pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
+    const int e1 = sl.e[1], e2 = sl.e[2];
+    const int li0 = t.i0 - sl.lo[0], lj = j - sl.lo[1], lk = k - sl.lo[2];
+    const int vb = (int)(step & 1);
+    AS_GLOBAL float *__restrict__ pq = gmem(S.pd[A] + sl.cell_base);
+    AS_GLOBAL float *__restrict__ pi = gmem(S.pd[A == 0 ? 1 : 0] + sl.cell_base);   // the increment d
+    const AS_GLOBAL float *__restrict__ vi = gmem(S.vel[vb][A] + sl.v_base[A]);
+    AS_GLOBAL float *__restrict__ vo = gmem(S.vel[vb ^ 1][A] + sl.v_base[A]);
+    const AS_CONST float4 *__restrict__ cx = cmem(S.coef[0]);
+    const AS_CONST int *__restrict__ fx = cmem(S.flags[0]);
+    const AS_CONST float4 *cy = cmem(S.coef[1]), *cz = cmem(S.coef[2]);
+    const float4 cyL = cy[j], czL = cz[k], cyR = cy[min(j + 1, ny)], czR = cz[min(k + 1, nz)];
+    // the faces along A, for A != 0: updated, and the high one stored here
+    const int ja = A == 1 ? j : k, na = A == 1 ? ny : nz;
+    const AS_CONST int *fa = cmem(S.flags[A]);
+    const int fyz = cmem(S.flags[1])[j] | cmem(S.flags[2])[k], other = A == 0 ? fyz : A == 1 ? cmem(S.flags[2])[k] : cmem(S.flags[1])[j];
+    const bool has_l = A != 0 && ja >= 1, has_r = A != 0 && ja + 1 < na, solid = fyz & 16;
+    const bool l_on = has_l && ((fa[ja] & 2) || (other & 1)), r_on = has_r && ((fa[min(ja + 1, na - 1)] & 2) || (other & 1));
+    const bool own = A == 1 ? lj == e1 - 1 : A == 2 ? lk == e2 - 1 : false;
+    const uint32_t sx4 = 4u * (uint32_t)S.sx, sy4 = 4u * (uint32_t)S.sy, cs4 = 4u * (uint32_t)(e1 * e2);
+    const uint32_t ym4 = j > 0 ? sy4 : 0u, yp4 = j < ny - 1 ? sy4 : 0u;
+    const uint32_t zm4 = k > 0 ? 4u : 0u, zp4 = k < nz - 1 ? 4u : 0u;
+    uint32_t po = 4u * (uint32_t)(t.i0 * S.sx + j * S.sy + k);
+    uint32_t co = 4u * (uint32_t)((li0 * e1 + lj) * e2 + lk);
+    // faces along A: plane stride, this column's low face, from it to the high one
+    const uint32_t vs4 = A == 0 ? cs4 : A == 1 ? 4u * (uint32_t)((e1 + 1) * e2) : 4u * (uint32_t)(e1 * (e2 + 1));
+    uint32_t fo = A == 0 ? co : A == 1 ? 4u * (uint32_t)((li0 * (e1 + 1) + lj) * e2 + lk) : 4u * (uint32_t)((li0 * e1 + lj) * (e2 + 1) + lk);
+    const uint32_t hi4 = A == 0 ? cs4 : A == 1 ? 4u * (uint32_t)e2 : 4u;
+
+    float pm = ldb(pcur, po - (t.i0 > 0 ? sx4 : 0u));
+    float pc = ldb(pcur, po);
+    float vL = 0.f;   // A == 0: the updated low face of the next plane
+    if (A == 0) vL = face_update(t.i0 >= 1 && ((fx[t.i0] & 2) || (other & 1)), cx[t.i0], ldb(vi, fo), pm, pc);
+    const int ilast = sl.lo[0] + sl.e[0] - 1;
+    for (int i = t.i0; i < t.i1; i += 2, po += 2u * sx4, co += 2u * cs4, fo += 2u * vs4) {
+        const int planes = min(2, t.i1 - i);
+        float pp[2], ym[2], yp[2], zm[2], zp[2], q[2], d[2], vl[2], vr[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            // (a plane past the tile loads the last one's values)
+            const uint32_t at = u < planes ? (uint32_t)u : 0u;
+            const uint32_t p = po + at * sx4, c = co + at * cs4, v = fo + at * vs4;
+            pp[u] = ldb(pcur, p + (i + (int)at + 1 < nx ? sx4 : 0u));
+            ym[u] = ldb(pcur, p - ym4);
+            yp[u] = ldb(pcur, p + yp4);
+            zm[u] = ldb(pcur, p - zm4);
+            zp[u] = ldb(pcur, p + zp4);
+            q[u] = ldb(pq, c);
+            d[u] = ldb(pi, c);
+            if (A != 0) vl[u] = ldb(vi, v);
+            vr[u] = ldb(vi, v + hi4);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (u >= planes) break;
+            const bool last = i + u + 1 >= nx;
+            const float4 cxC = cx[i + u], cxR = cx[min(i + u + 1, nx)];
+            float4 cA;
+            float dv;
+            if (A == 0) {
+                const float vR = last ? 0.f : face_update((fx[min(i + u + 1, nx - 1)] & 2) || (other & 1), cxR, vr[u], pc, pp[u]);
+                stb(vo, fo + (uint32_t)u * vs4, vL);
+                if (i + u == ilast) stb(vo, fo + (uint32_t)u * vs4 + hi4, vR);
+                dv = vR - vL;
+                vL = vR;
+                cA = cxC;
+            } else {
+                const float l = face_update(l_on || (has_l && (fx[i + u] & 1)), A == 1 ? cyL : czL, vl[u], A == 1 ? ym[u] : zm[u], pc);
+                const float r = face_update(r_on || (has_r && (fx[i + u] & 1)), A == 1 ? cyR : czR, vr[u], pc, A == 1 ? yp[u] : zp[u]);
+                stb(vo, fo + (uint32_t)u * vs4, l);
+                if (own) stb(vo, fo + (uint32_t)u * vs4 + hi4, r);
+                dv = r - l;
+                cA = A == 1 ? cyL : czL;
+            }
+            const float n = split_update(cA, q[u], dv);
+            float lap = 0.f;
+            if (A != 0) lap = transverse_add(lap, cxC.w, cxC.y, cxR.y, pm, pc, pp[u]);
+            if (A != 1) lap = transverse_add(lap, cyL.w, cyL.y, cyR.y, ym[u], pc, yp[u]);
+            if (A != 2) lap = transverse_add(lap, czL.w, czL.y, czR.y, zm[u], pc, zp[u]);
+            const float dn = d[u] + lap;
+            stb(pq, co + (uint32_t)u * cs4, n);
+            stb(pi, co + (uint32_t)u * cs4, dn);
+            // p^{n+1} = p^n + (pDir_A^{n+1} - pDir_A^n) + d^{n+1}: only
+            // increments are rounded before the last addition
+            const float pn = pc + ((n - q[u]) + dn);
+            stb(pnext, po + (uint32_t)u * sx4, solid || (fx[i + u] & 16) ? 0.f : pn);
+            pm = pc;
+            pc = pp[u];
+        }
     }
 }
 
@@ -636,7 +693,7 @@ __device__ __forceinline__ void pml_sources(const SceneDev &S, const TileDesc &t
     if (k >= t.k1 || j >= t.j1) return;
     AS_GLOBAL float *pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
     const int fy = cmem(S.flags[1])[j], fz = cmem(S.flags[2])[k];
-    const bool m = sl.merge && (sl.axis == 1 || (fy & 8)) && (sl.axis == 2 || (fz & 8));
+    const bool m = sl.merge;
     for (int i = t.i0; i < t.i1; ++i) {
         const int quiet[3] = {cmem(S.flags[0])[i] & 4, fy & 4, fz & 4};
         const int idx = i * S.sx + j * S.sy + k;
@@ -659,9 +716,10 @@ __device__ __forceinline__ void pml_sources(const SceneDev &S, const TileDesc &t
 __device__ __forceinline__ void pml_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
     const PmlSlab sl = cmem(S.slabs)[t.slab];
-    if (sl.axis == 0) pml_tile_axis<0>(S, t, sl, step);
-    else if (sl.axis == 1) pml_tile_axis<1>(S, t, sl, step);
-    else pml_tile_axis<2>(S, t, sl, step);
+    if (!sl.merge) pml_split_tile(S, t, sl, step);
+    else if (sl.axis == 0) pml_merged_axis<0>(S, t, sl, step);
+    else if (sl.axis == 1) pml_merged_axis<1>(S, t, sl, step);
+    else pml_merged_axis<2>(S, t, sl, step);
     if (t.src) pml_sources(S, t, sl, step);
 }
 

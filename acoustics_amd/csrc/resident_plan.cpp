@@ -22,8 +22,7 @@ const char *resident_refusal(const SceneSetup &S)
     if (S.boundary != FDTD_BOUNDARY_RASTERIZE) return "coupled ghost cells";
     if (S.n_cpo != 1) return "acceleration noise";
     if (S.slabs.empty()) return "no PML";
-    for (const PmlSlab &sl : S.slabs)
-        if (!sl.merge) return "split PML state";
+    if (!S.pml_merged) return "split PML state";
     // a cell is damped along an axis exactly where that axis's segment says
     // so, and every face of a damped cell but the walls is a PML face
     for (int d = 0; d < 3; ++d) {

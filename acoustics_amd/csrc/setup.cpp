@@ -124,7 +124,7 @@ bool axis_plain(const SceneSetup &s, int d, int i)
 void set_pml_state(SceneSetup &s, bool merged)
 {
     s.n_pml_merged = 0;
-    s.stag_merged = merged && s.scheme == FDTD_SCHEME_STAGGERED && !s.slabs.empty();
+    s.stag_merged = merged && s.scheme == FDTD_SCHEME_STAGGERED && !s.base_slabs.empty();
     for (int d = 0; d < 3 && s.stag_merged; ++d)
         for (int i = s.inner_lo[d]; i < s.inner_hi[d]; ++i)
             s.stag_merged = s.stag_merged && axis_plain(s, d, i) && s.sig0[d][i];
@@ -134,21 +134,42 @@ void set_pml_state(SceneSetup &s, bool merged)
     for (int d = 0; d < 3 && s.stag_merged; ++d)
         for (int i = 1; i < s.n[d]; ++i)
             if (s.cpml[d][i - 1] || s.cpml[d][i]) s.stag_merged = s.stag_merged && s.fpml[d][i];
-    for (PmlSlab &sl : s.slabs) {
-        sl.merge = 0;
-        if (!merged || (s.scheme != FDTD_SCHEME_COLLOCATED && !s.stag_merged)) continue;
+    s.slabs.clear();
+    s.pml_merged = !s.base_slabs.empty();
+    int64_t cells = 0, faces[3] = {0, 0, 0};
+    for (const PmlSlab &base : s.base_slabs) {
+        bool ok = merged && (s.scheme == FDTD_SCHEME_COLLOCATED || s.stag_merged);
         // the march runs along x: y and z slabs merge only when x is plain
         // over their whole x range, so a column is merged or split throughout
-        bool ok = true;
-        if (sl.axis != 0)
-            for (int i = sl.lo[0]; i < sl.lo[0] + sl.e[0] && ok; ++i) ok = axis_plain(s, 0, i);
-        if (!ok) continue;
-        sl.merge = 1;
-        int64_t ny = 0, nz = 0;
-        for (int j = sl.lo[1]; j < sl.lo[1] + sl.e[1]; ++j) ny += (sl.axis == 1 || axis_plain(s, 1, j));
-        for (int k = sl.lo[2]; k < sl.lo[2] + sl.e[2]; ++k) nz += (sl.axis == 2 || axis_plain(s, 2, k));
-        s.n_pml_merged += (int64_t)sl.e[0] * ny * nz;
+        if (base.axis != 0)
+            for (int i = base.lo[0]; i < base.lo[0] + base.e[0] && ok; ++i) ok = axis_plain(s, 0, i);
+        s.pml_merged = s.pml_merged && ok;
+        auto cuts = [&](int d) {
+            std::vector<int> at{base.lo[d]};
+            for (int i = base.lo[d] + 1; i < base.lo[d] + base.e[d] && ok && d != base.axis; ++i)
+                if (axis_plain(s, d, i) != axis_plain(s, d, i - 1)) at.push_back(i);
+            at.push_back(base.lo[d] + base.e[d]);
+            return at;
+        };
+        const std::vector<int> cj = cuts(1), ck = cuts(2);
+        for (size_t a = 0; a + 1 < cj.size(); ++a)
+            for (size_t b = 0; b + 1 < ck.size(); ++b) {
+                PmlSlab sl = base;
+                sl.lo[1] = cj[a]; sl.e[1] = cj[a + 1] - cj[a];
+                sl.lo[2] = ck[b]; sl.e[2] = ck[b + 1] - ck[b];
+                sl.merge = ok && (sl.axis == 1 || axis_plain(s, 1, cj[a])) && (sl.axis == 2 || axis_plain(s, 2, ck[b]));
+                sl.cell_base = cells;
+                const int64_t n = (int64_t)sl.e[0] * sl.e[1] * sl.e[2];
+                cells += n;
+                for (int d = 0; d < 3; ++d) {
+                    sl.v_base[d] = faces[d];
+                    faces[d] += (int64_t)(sl.e[0] + (d == 0)) * (sl.e[1] + (d == 1)) * (sl.e[2] + (d == 2));
+                }
+                if (sl.merge) s.n_pml_merged += n;
+                s.slabs.push_back(sl);
+            }
     }
+    for (int d = 0; d < 3; ++d) s.n_pml_faces[d] = faces[d];
 }
 
 namespace {
@@ -538,6 +559,7 @@ fdtd_status build_setup(const fdtd_scene &sc, SceneSetup &S, std::string &err)
     }
     S.n_pml = S.abc ? 0 : S.N - (int64_t)(S.inner_hi[0] - S.inner_lo[0]) * (S.inner_hi[1] - S.inner_lo[1]) * (S.inner_hi[2] - S.inner_lo[2]);
     S.slabs.clear();
+    S.base_slabs.clear();
     for (int d = 0; d < 3; ++d) S.n_pml_faces[d] = 0;
     S.n_pml_merged = 0;
     if (!S.abc) {
@@ -548,7 +570,6 @@ fdtd_status build_setup(const fdtd_scene &sc, SceneSetup &S, std::string &err)
             {a[0], b[0], 0, a[1], 0, n[2]}, {a[0], b[0], b[1], n[1], 0, n[2]},
             {a[0], b[0], a[1], b[1], 0, a[2]}, {a[0], b[0], a[1], b[1], b[2], n[2]},
         };
-        S.slabs.clear();
         int64_t cells = 0, faces[3] = {0, 0, 0};
         for (const auto &bx : boxes) {
             PmlSlab sl{};
@@ -561,10 +582,10 @@ fdtd_status build_setup(const fdtd_scene &sc, SceneSetup &S, std::string &err)
                 sl.v_base[d] = faces[d];
                 faces[d] += (int64_t)(sl.e[0] + (d == 0)) * (sl.e[1] + (d == 1)) * (sl.e[2] + (d == 2));
             }
-            S.slabs.push_back(sl);
+            S.base_slabs.push_back(sl);
         }
         if (cells != S.n_pml) { err = "internal: PML slab decomposition does not cover the PML"; return FDTD_ERR_INVALID; }
-        for (int d = 0; d < 3; ++d) S.n_pml_faces[d] = faces[d];
+        for (int d = 0; d < 3; ++d) S.base_faces[d] = faces[d];
         set_pml_state(S, true);
     }
 

@@ -487,13 +487,6 @@ void for_pml_faces(const SceneSetup &S, int d, F fn)
     }
 }
 
-// A cell of a merging slab is merged when both axes other than the slab axis
-// are plain there (the kernel's rule; x is plain over y and z slabs that merge).
-inline bool merged_cell(const SceneSetup &S, const PmlSlab &sl, int j, int k)
-{
-    return sl.merge && (sl.axis == 1 || axis_plain(S, 1, j)) && (sl.axis == 2 || axis_plain(S, 2, k));
-}
-
 // A staggered scene runs in merged state, which has no face velocities.  Its
 // first snapshot, saved or loaded, takes the handle to split state for good:
 // a saved one runs the steps so far again in split state (a staggered scene
@@ -549,6 +542,40 @@ struct EngineStateHeader {
     int64_t step, n_cells, state_floats, npad;
 };
 constexpr char kStateMagic[8] = {'F', 'D', 'T', 'D', 'S', 'T', 'A', 'T'};
+
+// State files of version 1 hold a merged PML by its six slabs; version 2, and
+// the engine, by the boxes they are cut into.
+std::vector<float> by_boxes(const DeviceScene &D, const std::vector<float> &old)
+{
+    const SceneSetup &S = D.S;
+    size_t off[11];
+    D.base_layout(off);
+    std::vector<float> raw(D.state_floats, 0.f);
+    // everything but the PML's arrays keeps its place
+    std::copy(old.begin(), old.begin() + (ptrdiff_t)std::min(off[1], raw.size()), raw.begin());
+    for (const PmlSlab &sl : S.slabs)
+        for (const PmlSlab &b : S.base_slabs) {
+            bool in = true;
+            for (int d = 0; d < 3; ++d) in = in && sl.lo[d] >= b.lo[d] && sl.lo[d] + sl.e[d] <= b.lo[d] + b.e[d];
+            if (!in) continue;
+            // cells (a = 0), and the faces of axis a - 1
+            for (int a = 0; a < 4; ++a) {
+                const int E[3] = {sl.e[0] + (a == 1), sl.e[1] + (a == 2), sl.e[2] + (a == 3)};
+                const int F[3] = {b.e[0] + (a == 1), b.e[1] + (a == 2), b.e[2] + (a == 3)};
+                const int64_t to0 = a ? sl.v_base[a - 1] : sl.cell_base, from0 = a ? b.v_base[a - 1] : b.cell_base;
+                for (int q = 0; q < (a ? 2 : 3); ++q) {
+                    const float *src = old.data() + off[a ? 4 + 3 * q + a - 1 : 1 + q] + from0;
+                    float *dst = raw.data() + ((a ? D.dev.vel[q][a - 1] : D.dev.pd[q]) - D.dev.field) + to0;
+                    for (int i = 0; i < E[0]; ++i)
+                        for (int j = 0; j < E[1]; ++j)
+                            for (int k = 0; k < E[2]; ++k)
+                                dst[((int64_t)i * E[1] + j) * E[2] + k] =
+                                    src[((int64_t)(i + sl.lo[0] - b.lo[0]) * F[1] + j + sl.lo[1] - b.lo[1]) * F[2] + k + sl.lo[2] - b.lo[2]];
+                }
+            }
+        }
+    return raw;
+}
 
 }  // namespace
 
@@ -610,7 +637,7 @@ fdtd_status fdtd_save_snapshot(fdtd_handle *h, const char *pattern, const char *
                     const long long c = sl.cell_base + ((long long)li * sl.e[1] + lj) * sl.e[2] + lk;
                     const int j = sl.lo[1] + lj, k = sl.lo[2] + lk;
                     const long long g = ((long long)(sl.lo[0] + li) * S.n[1] + j) * S.n[2] + k;
-                    if (!merged_cell(S, sl, j, k)) {
+                    if (!sl.merge) {
                         for (int d = 0; d < 3; ++d) full[d][g] = comp[d][c];
                     } else {
                         const int A = sl.axis, lower = A == 0 ? 1 : 0;
@@ -639,24 +666,12 @@ fdtd_status fdtd_save_snapshot(fdtd_handle *h, const char *pattern, const char *
             // a transverse face between two merged cells is not kept by the
             // merged state (the files hold zero there); every other face is
             for (const PmlSlab &sl : S.slabs) {
+                if (sl.merge && d != sl.axis) continue;
                 const int E[3] = {sl.e[0] + (d == 0), sl.e[1] + (d == 1), sl.e[2] + (d == 2)};
                 for (int li = 0; li < E[0]; ++li)
                     for (int lj = 0; lj < E[1]; ++lj)
                         for (int lk = 0; lk < E[2]; ++lk) {
                             const int i = sl.lo[0] + li, j = sl.lo[1] + lj, k = sl.lo[2] + lk;
-                            if (d != sl.axis && sl.merge) {
-                                // the cells on either side of the face inside this box
-                                const int lo_l = (d == 1 ? lj : lk) - 1, hi_l = (d == 1 ? lj : lk);
-                                const int ext = d == 1 ? sl.e[1] : sl.e[2];
-                                bool kept = false;
-                                for (int side = 0; side < 2; ++side) {
-                                    const int l = side ? hi_l : lo_l;
-                                    if (l < 0 || l >= ext) continue;
-                                    const int jj = d == 1 ? sl.lo[1] + l : j, kk = d == 2 ? sl.lo[2] + l : k;
-                                    kept = kept || !merged_cell(S, sl, jj, kk);
-                                }
-                                if (!kept) continue;
-                            }
                             const long long c = sl.v_base[d] + ((long long)li * E[1] + lj) * E[2] + lk;
                             fv[face_index(S.n, d, i, j, k)] = vc[c];
                         }
@@ -668,7 +683,7 @@ fdtd_status fdtd_save_snapshot(fdtd_handle *h, const char *pattern, const char *
     {
         EngineStateHeader hd{};
         std::memcpy(hd.magic, kStateMagic, 8);
-        hd.version = 1;
+        hd.version = merged ? 2 : 1;
         hd.pml_state = merged ? FDTD_PML_STATE_MERGED : FDTD_PML_STATE_SPLIT;
         hd.scheme = S.scheme;
         hd.step = s;
@@ -721,14 +736,17 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
     {
         std::ifstream is(snap_name(pattern, simulator_id, numbering, "engine_state.bin"), std::ios::binary);
         EngineStateHeader hd{};
+        size_t off[11];
         if (is && is.read(reinterpret_cast<char *>(&hd), sizeof hd) && std::memcmp(hd.magic, kStateMagic, 8) == 0 &&
-            hd.version == 1 && hd.n_cells == N && hd.scheme == S.scheme && hd.state_floats == (int64_t)h->D.state_floats &&
+            (hd.version == 1 || hd.version == 2) && hd.n_cells == N && hd.scheme == S.scheme &&
+            hd.state_floats == (int64_t)(merged && hd.version == 1 ? h->D.base_layout(off) : h->D.state_floats) &&
             hd.npad == h->D.npad && hd.pml_state == (merged ? FDTD_PML_STATE_MERGED : FDTD_PML_STATE_SPLIT) && hd.step >= 0) {
-            std::vector<float> raw(h->D.state_floats);
+            std::vector<float> raw(hd.state_floats);
             if (!is.read(reinterpret_cast<char *>(raw.data()), (std::streamsize)(raw.size() * 4))) {
                 set_last_error("engine state file: short file");
                 return FDTD_ERR_INVALID;
             }
+            if (merged && hd.version == 1) raw = by_boxes(h->D, raw);
             FDTD_HIP_TRY(hipMemcpy(h->D.dev.field, raw.data(), raw.size() * 4, hipMemcpyHostToDevice));
             return resume_at(h, hd.step);
         }
@@ -797,7 +815,7 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
                     const long long c = sl.cell_base + ((long long)li * sl.e[1] + lj) * sl.e[2] + lk;
                     const int i = sl.lo[0] + li, j = sl.lo[1] + lj, k = sl.lo[2] + lk;
                     const long long g = ((long long)i * S.n[1] + j) * S.n[2] + k;
-                    if (!merged_cell(S, sl, j, k)) {
+                    if (!sl.merge) {
                         for (int d = 0; d < 3; ++d) comp[d][c] = (float)pml[d][g];
                         continue;
                     }
