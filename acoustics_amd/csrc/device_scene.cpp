@@ -1084,12 +1084,13 @@ fdtd_status StepProgram::enqueue_step(hipStream_t st, long long step, int k, int
     }
     if (nspeaker) FDTD_HIP_TRY(launch_speaker(d_scenes, d_motion + nmotion, nspeaker, speaker_cells, k, st));
     if (ev_begin) FDTD_HIP_TRY(hipEventRecord(ev_begin, st));
+    const int at = block == 1 ? k | STEP_ALONE : k;
     auto launch = [&](int kind, hipStream_t s) {
         // fused: every class in the interior list, except the moving-object tiles
         if (fused && kind == KIND_INTERIOR)
-            return launch_step(KIND_ALL, d_scenes, d_tiles[kind], ntiles[kind], head[kind], d_terms, order_clock, k, s);
+            return launch_step(KIND_ALL, d_scenes, d_tiles[kind], ntiles[kind], head[kind], d_terms, order_clock, at, s);
         if (fused && kind == KIND_PML) return hipSuccess;
-        return launch_step(kind, d_scenes, d_tiles[kind], ntiles[kind], head[kind], d_terms, order_clock, k, s);
+        return launch_step(kind, d_scenes, d_tiles[kind], ntiles[kind], head[kind], d_terms, order_clock, at, s);
     };
     // (running the PML slabs on a second stream beside the interior was
     // measured slower than one stream and is not offered)

@@ -147,7 +147,7 @@ struct SceneDev {
     // of its terms, formed when the rows are read out
     int T, cap;                 // terms per row, rows of the ring
     double *terms;              // [cap][T]
-    double *tail;               // pinned host memory [T + 1], or null: the newest row and its step, after a block of one step
+    double *tail;               // pinned host memory [T + 1], or null: the newest row and its step, after a step run by itself (STEP_ALONE)
     unsigned long long *clock;  // CLK_WORDS words
     int n_obj;
     // 1: the seven-sample configuration (ghosts at 3h/4 from the fluid cell,
@@ -244,6 +244,9 @@ enum : int { KIND_INTERIOR = 0, KIND_PML = 1, KIND_SPECIAL = 2, NUM_KINDS = 3, K
 // last and the Infinity Cache still holds.  k: the step's offset in its block.
 // nhead: the first nhead tiles (a multiple of eight) keep their place on odd
 // steps too.
+// STEP_ALONE in k: a step enqueued by itself, whose listener row goes to
+// SceneDev::tail as well.
+enum : int { STEP_ALONE = 1 << 30 };
 hipError_t launch_step(int kind, const SceneDev *scenes, const TileDesc *tiles, int ntiles, int nhead, const TermRef *terms,
                        const unsigned long long *order_clock, int k, hipStream_t s);
 // Moves every scene of the launch n steps on (clamped to its target) and

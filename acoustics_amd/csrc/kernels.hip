@@ -158,7 +158,7 @@ __device__ __forceinline__ double coupled_ghost(const SceneDev &S, int g, const 
 // the step: 96^3 with a spinning object 24.1 us per step against 21.4, and with
 // marches of four planes 36.9 against 19.0; Engquist 203x190x214 23.4, 22.0.)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void emit_terms(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step)
+__device__ __forceinline__ void emit_terms(const SceneDev &S, const TileDesc &t, const TermRef *terms, long long step, bool mirror)
 {
     const AS_GLOBAL float *pcur = gmem(S.field + (size_t)slot_cur(step) * S.npad);
     const AS_GLOBAL float *pnext = gmem(S.field + (size_t)slot_next(step) * S.npad);
@@ -174,7 +174,9 @@ __device__ __forceinline__ void emit_terms(const SceneDev &S, const TileDesc &t,
         } else {
             v = coupled_ghost(S, r.cell, pcur, step);
         }
-        row[r.slot] = r.beta * v;
+        v *= r.beta;
+        row[r.slot] = v;
+        if (mirror) gmem(S.tail)[r.slot] = v;
     }
 }
 
@@ -1438,14 +1440,6 @@ __global__ __launch_bounds__(256) void advance_kernel(const SceneDev *__restrict
     const long long step = (long long)clk[CLK_STEP], target = (long long)clk[CLK_TARGET];
     if (step >= target) return;
     const long long base = min(step + (long long)n, target);
-    // A caller that listens after every step waits for this launch anyway: the
-    // row goes to host memory here, and no copy has to be launched and waited
-    // for after it (64^3, step and listen: 36 -> 21 us).
-    if (n == 1 && S.tail) {
-        const AS_GLOBAL double *row = gmem(S.terms) + (size_t)(step % S.cap) * S.T;
-        for (int q = threadIdx.x; q < S.T; q += blockDim.x) gmem(S.tail)[q] = row[q];
-        if (threadIdx.x == 0) gmem(S.tail)[S.T] = (double)step;
-    }
     // rows first .. first + rows - 1, their times accumulated by one addition
     // of dt per step (the reference's clock)
     const long long first = n > 0 ? step + S.amp_rows : step;
@@ -1504,11 +1498,19 @@ __global__ __launch_bounds__(256) void step_kernel(const SceneDev *__restrict__ 
                                                    int ntiles, int nhead, const TermRef *__restrict__ terms,
                                                    const unsigned long long *__restrict__ order_clock, int k)
 {
-    const TileDesc t = gmem(tiles)[tile_of(blockIdx.x, ntiles, nhead, order_clock, k)];
+    // A caller that listens after every step waits for this launch anyway: the
+    // row goes to host memory as well, and no copy has to be launched and waited
+    // for (64^3, step and listen: 36 -> 22 us, and 17.5 without an advance launch).
+    const bool alone = k & STEP_ALONE;
+    k &= ~STEP_ALONE;
+    const int w = tile_of(blockIdx.x, ntiles, nhead, order_clock, k);
+    const TileDesc t = gmem(tiles)[w];
     if (t.type == TILE_EMPTY) return;
     const SceneDev &S = scenes[t.scene];
     const long long step = (long long)S.clock[CLK_STEP] + k;
     if (step >= (long long)S.clock[CLK_TARGET]) return;
+    const bool mirror = alone && S.tail;
+    if (KIND != KIND_PML && KIND != KIND_SPECIAL && mirror && w == 0 && threadIdx.x == 0) gmem(S.tail)[S.T] = (double)step;
     if constexpr (KIND == KIND_INTERIOR) {
         // the interior launch also carries the object-adjacent cells, whose
         // FP64 gathers then hide under the interior's streaming
@@ -1546,7 +1548,7 @@ __global__ __launch_bounds__(256) void step_kernel(const SceneDev *__restrict__ 
     }
     if (t.te > t.tb) {
         __syncthreads();   // the tile's cells are written
-        emit_terms(S, t, terms, step);
+        emit_terms(S, t, terms, step, mirror);
     }
 }
 

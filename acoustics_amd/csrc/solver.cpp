@@ -31,6 +31,7 @@ struct fdtd_handle {
     int graph_steps = 0;
     hipGraphExec_t graph_exec = nullptr;
     long long step = 0;          // steps taken
+    int lead = 0;                // steps run one by one since the device clock was advanced
     long long flushed = 0;       // listener rows copied to host_series
     std::vector<double> host_series;
     double *tail = nullptr;     // SceneDev::tail
@@ -198,6 +199,7 @@ static fdtd_status settle(fdtd_handle *h)
     if (*h->res_prog.trouble > 1) { set_last_error("a resident launch lost its neighbours"); return FDTD_ERR_DEVICE; }
     *h->res_prog.trouble = 0;
     h->res_prog.n = 0;
+    h->lead = 0;   // (what was enqueued behind it has not run)
     long long at = 0;
     {
         const fdtd_status st = resident_reopen(h->D.dev, &at);
@@ -269,6 +271,14 @@ static bool capturing(hipStream_t st)
     return hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
 }
 
+// Brings the device clock up to the steps run one by one.
+static fdtd_status catch_up(fdtd_handle *h)
+{
+    if (h->lead) FDTD_HIP_TRY(launch_advance(h->prog.d_scenes, 1, h->lead, h->stream));
+    h->lead = 0;
+    return FDTD_OK;
+}
+
 fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
 {
     if (!h || nsteps < 0) return FDTD_ERR_INVALID;
@@ -309,7 +319,21 @@ fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
             fdtd_status st = flush_series(h);
             if (st != FDTD_OK) return st;
         }
-        if (use_graph) {
+        // Single steps run at growing offsets from the device clock, which moves
+        // on, with the amplitudes' ring, before anything else and once the ring
+        // is used up: a step that is waited for is one launch (64^3, step and
+        // listen: 17.5 us against 21.4).  On the handle's own stream only: a
+        // caller's may be captured, and a replay finds the clock elsewhere.
+        const bool single = block == 1 && h->own_stream && !use_graph && !per_step;
+        if (!single || h->lead == AMP_ROWS - 1) {
+            const fdtd_status st = catch_up(h);
+            if (st != FDTD_OK) return st;
+        }
+        if (single) {
+            const fdtd_status st = h->prog.enqueue_step(h->stream, h->step, h->lead, 1);
+            if (st != FDTD_OK) return st;
+            ++h->lead;
+        } else if (use_graph) {
             if (!h->graph_exec) {
                 fdtd_status st = build_graph(h);
                 if (st != FDTD_OK) return st;
@@ -529,6 +553,7 @@ fdtd_status to_split_state(fdtd_handle *h, bool replay)
     h->D.release();
     h->D = D;
     h->prog = prog;
+    h->lead = 0;
     return FDTD_OK;
 }
 
@@ -709,6 +734,7 @@ static fdtd_status resume_at(fdtd_handle *h, long long s)
     FDTD_HIP_TRY(h->D.fill_amplitudes(h->stream));
     FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
     h->step = s;
+    h->lead = 0;
     h->flushed = s;
     forget_tail(h);
     h->host_series.assign((size_t)s * h->D.S.L, 0.0);

@@ -34,6 +34,25 @@ def test_single_steps_and_blocks(hip_lib, n_listeners):
         assert np.array_equal(s.series(), want)
 
 
+@pytest.mark.parametrize("kw", [dict(), dict(tile_config=3), dict(steps_per_graph=8)])
+def test_more_single_steps_than_the_amplitude_ring_holds(hip_lib, kw):
+    """The device clock follows after 255 of them, and before anything else."""
+    sb = scenes.config2(seed=5, n=40, n_listeners=6, radius=0.03, shell=0.05)[0]
+    with Solver(sb) as ref:
+        ref.step(700)
+        want, field = ref.series(), ref.pressure()
+    with Solver(sb, **kw) as s:
+        for n in [1] * 300 + [5, 1, 1, 16, 1, 40] + [1] * 257 + [2, 1]:
+            s.step(n)
+        s.set_timing(True)
+        s.step(3)
+        s.set_timing(False)
+        left = 700 - s.info()["step_index"]
+        for _ in range(left):
+            s.step(1)
+        assert np.array_equal(s.series(), want) and np.array_equal(s.pressure(), field)
+
+
 @pytest.mark.parametrize("scheme", [capi.FDTD_SCHEME_COLLOCATED, capi.FDTD_SCHEME_STAGGERED])
 @pytest.mark.parametrize("plan", [0, 1, 4, 10])
 def test_many_terms_in_a_tile(hip_lib, scheme, plan):
