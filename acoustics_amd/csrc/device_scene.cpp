@@ -538,23 +538,24 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
     // whole, the y faces inside x, the z faces inside x and y), cut into
     // tiles of at most 256 cells.  A z-face cell is one float of a row's
     // first or last line: when the float4 rows run in the fused launch, the
-    // z faces are cut into tiles of 64 planes by 4 rows that follow the row
-    // tile holding their last column, while those lines are in the L2
-    // (256^3 free field 45.8 -> 41.0-41.4 us per step; the same tiles in
-    // the boundary class measured 46.4)
+    // z faces are cut into tiles of 8 planes by 4 rows with both ends of each
+    // row (the end of one and the start of the next share a line), which
+    // follow the row tile holding their last column, while those lines are in
+    // the L2 (203x190x214: 20.3 us per step, 21.2 with 32 planes, 22.0 with
+    // tiles of 64 planes and one end; 256^3 32.9, 34.0 and 34.0)
     if (S.abc) {
-        const bool ride_rows = plan.fused && plan.interior_vec && !S.visc;
+        const bool ride_rows = plan.fused && plan.interior_vec && !S.visc && n[2] > 4;
         const int boxes[6][6] = {
             {1, 2, 1, n[1] - 1, 1, n[2] - 1},        {n[0] - 2, n[0] - 1, 1, n[1] - 1, 1, n[2] - 1},
             {2, n[0] - 2, 1, 2, 1, n[2] - 1},        {2, n[0] - 2, n[1] - 2, n[1] - 1, 1, n[2] - 1},
             {2, n[0] - 2, 2, n[1] - 2, 1, 2},        {2, n[0] - 2, 2, n[1] - 2, n[2] - 2, n[2] - 1},
         };
-        for (int f = 0; f < 6; ++f) {
+        for (int f = 0; f < (ride_rows ? 5 : 6); ++f) {
             const int *bx = boxes[f];
-            const bool zface = ride_rows && f >= 4;
+            const bool ends = ride_rows && f == 4;
             const int ek = bx[5] - bx[4], ej = bx[3] - bx[2], ei = bx[1] - bx[0];
-            const int tk = std::min(ek, 256), tj = zface ? std::min(ej, 4) : std::min(ej, std::max(1, 256 / tk));
-            const int ti = zface ? std::min(ei, 64) : std::min(ei, std::max(1, 256 / (tk * tj)));
+            const int tk = std::min(ek, 256), tj = ends ? std::min(ej, 4) : std::min(ej, std::max(1, 256 / tk));
+            const int ti = ends ? std::min(ei, 8) : std::min(ei, std::max(1, 256 / (tk * tj)));
             for (int i0 = bx[0]; i0 < bx[1]; i0 += ti)
                 for (int j0 = bx[2]; j0 < bx[3]; j0 += tj)
                     for (int k0 = bx[4]; k0 < bx[5]; k0 += tk) {
@@ -563,10 +564,11 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
                         t.type = TILE_ABC;
                         t.i0 = i0; t.i1 = std::min(i0 + ti, bx[1]);
                         t.j0 = j0; t.j1 = std::min(j0 + tj, bx[3]);
-                        t.k0 = k0; t.k1 = std::min(k0 + tk, bx[5]);
+                        t.k0 = k0; t.k1 = ends ? n[2] - 1 : std::min(k0 + tk, bx[5]);
+                        t.rpw = ends ? n[2] - 3 : 0;
                         const int lo[3] = {t.i0, t.j0, t.k0}, hi[3] = {t.i1, t.j1, t.k1};
                         t.src = src_hit(lo, hi);
-                        if (zface) row_end.push_back(out.size());
+                        if (ends) row_end.push_back(out.size());
                         out.push_back(t);
                     }
         }
@@ -757,7 +759,7 @@ void DeviceScene::assign_terms(int scene_id, size_t base, std::vector<TileDesc> 
         for (int q : column[(size_t)i * S.n[1] + j]) {
             const TileDesc &t = out[q];
             const int kfirst = t.k0 + ((t.type == TILE_INTERIOR_VEC || t.type == TILE_MAC_VEC) ? t.lead : 0);   // cells the tile writes
-            if (k >= kfirst && k < t.k1 && (best < 0 || q < best)) best = q;
+            if (k >= kfirst && k < t.k1 && (k - kfirst) % tile_kstep(t) == 0 && (best < 0 || q < best)) best = q;
         }
         return best;
     };
@@ -836,8 +838,10 @@ static std::string check_tiles(const std::vector<TileDesc> &list, int kind, cons
                 if (lo[a] < 1 || hi[a] > d.n[a] - 1 || lo[a] >= hi[a]) return "boundary tile outside layers 1 .. n-2";
                 plane = plane || (hi[a] - lo[a] == 1 && (lo[a] == 1 || lo[a] == d.n[a] - 2));
             }
+            const int ks = tile_kstep(t), nk = (t.k1 - t.k0 + ks - 1) / ks;
+            if (ks > 1) plane = nk == 2 && t.k0 == 1 && t.k0 + ks == d.n[2] - 2;   // both ends of rows
             if (!plane) return "boundary tile off the layer-1 shell";
-            if ((int64_t)(t.i1 - t.i0) * (t.j1 - t.j0) * (t.k1 - t.k0) > 256) return "boundary tile too large";
+            if ((int64_t)(t.i1 - t.i0) * (t.j1 - t.j0) * nk > 256) return "boundary tile too large";
             continue;
         }
         // a float4 row tile reads from k0 and writes from k0 + lead

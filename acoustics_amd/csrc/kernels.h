@@ -221,7 +221,8 @@ struct TileDesc {
     int src;                     // tile intersects a pressure-source box
     int slab;                    // TILE_PML: index into SceneDev::slabs
     int tb, te;                  // listener terms [tb, te) of the program's TermRef table
-    int rpw;                     // TILE_INTERIOR_VEC: rows per wavefront (the tile holds 4 * rpw rows)
+    int rpw;                     // TILE_INTERIOR_VEC: rows per wavefront (the tile holds 4 * rpw rows);
+                                 // TILE_ABC: distance along k from one cell to the next (0: 1)
     int lead;                    // TILE_INTERIOR_VEC: cells at the start of each row's first group (from k0,
                                  // a multiple of four) that belong to another tile and are not written
 };
@@ -230,6 +231,9 @@ struct TileDesc {
 // COUPLED_LANES threads each, which share the ghosts' operator rows.
 enum : int { COUPLED_LANES = 8 };
 inline int special_per_tile(int raster) { return raster ? 256 : 256 / COUPLED_LANES; }
+
+// Distance along k between a tile's cells.
+__host__ __device__ inline int tile_kstep(const TileDesc &t) { return t.type == TILE_ABC && t.rpw ? t.rpw : 1; }
 
 struct MotionDesc {
     int scene;

@@ -1028,9 +1028,9 @@ __device__ __forceinline__ void special_tile(const SceneDev &S, const TileDesc &
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void abc_tile(const SceneDev &S, const TileDesc &t, long long step)
 {
-    const int nk = t.k1 - t.k0, nj = t.j1 - t.j0;
+    const int ks = tile_kstep(t), nk = (t.k1 - t.k0 + ks - 1) / ks, nj = t.j1 - t.j0;
     const int q = (int)threadIdx.x, r = q / nk;
-    const int k = t.k0 + (q - r * nk), j = t.j0 + r % nj, i = t.i0 + r / nj;
+    const int k = t.k0 + (q - r * nk) * ks, j = t.j0 + r % nj, i = t.i0 + r / nj;
     if (i >= t.i1) return;
     const int ijk[3] = {i, j, k};
     const int st[3] = {S.sx, S.sy, 1};

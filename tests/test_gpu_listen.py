@@ -82,3 +82,24 @@ def test_rewound(hip_lib, tmp_path, scheme):
         s.step(5)
         again = s.listen()
         assert np.array_equal(first, again) and np.any(first)
+
+
+@pytest.mark.parametrize("div", [(20, 21, 22), (37, 9, 13), (11, 40, 8)])
+def test_listeners_at_both_ends_of_engquist_rows(hip_lib, div):
+    """Tiles with both ends of rows against the boundary class's own tiles (plan 4)."""
+    s = scenes.base_settings(div, 0.005, 0)
+    lo = np.array(s["min_bound"])
+    rng = np.random.default_rng(4)
+    ears = lo + 0.005 * np.concatenate([rng.uniform([2.6] * 3, np.array(div) - 2.6, size=(20, 3)) for _ in range(2)])
+    ears[:20, 2] = lo[2] + 0.005 * 1.7
+    ears[20:, 2] = lo[2] + 0.005 * (div[2] - 1.7)
+    sb = scenes.SceneBuffers(s, pressure_sources=[scenes.gaussian_pressure_source(lo + 0.005 * (np.array(div) * 0.5), 2e-5)],
+                             listeners=ears)
+    out = []
+    for plan in (4, 0, 10):
+        with Solver(sb, tile_config=plan) as v:
+            v.step(120)
+            out.append((v.series(), v.pressure()))
+    assert np.any(out[0][0])
+    for series, p in out[1:]:
+        assert np.array_equal(series, out[0][0]) and np.array_equal(p, out[0][1])
