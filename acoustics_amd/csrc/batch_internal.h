@@ -49,7 +49,12 @@ struct BatchRunner {
     void free_buffers();                              // with the stream idle
     fdtd_status autotune(hipStream_t st);
     fdtd_status advance(hipStream_t st, int nsteps);
-    bool any_resident() const { return res_prog[RES_FINE].n > 0 || res_prog[RES_COARSE].n > 0; }
+    bool any_resident() const
+    {
+        for (const ResidentProgram &p : res_prog)
+            if (p.n > 0) return true;
+        return false;
+    }
     bool all_resident() const;
     fdtd_status list_resident(hipStream_t st);        // (re)builds the resident launches
     // Waits for the stream and completes blocks that a resident launch gave up.

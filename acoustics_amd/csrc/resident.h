@@ -29,13 +29,17 @@ struct ResBox {
     int32_t first;              // its first tile
     int32_t damped;             // bit d: axis d is damped
     int32_t slab;               // PML slab that stores its state (-1: no damped axis)
-    int32_t pad;
+    int32_t swap;               // its tiles' columns run along y
 };
 
+// A tile in its own frame: columns along its first axis, x, or y with swap (the
+// second axis is then x).  A class damped along x is thin there: along y it gives
+// longer columns and fewer tiles.
 struct ResTile {
     int32_t i0, j0, k0, bx, by, bz;
+    int32_t swap;
     int32_t pitch;              // LDS words from one row of columns (along z) to the next
-    int32_t damped, slab;
+    int32_t damped, slab;       // (axes of the grid)
     uint32_t word0;             // its first word in the exchange buffer and in the route table
     int32_t words;              // faces' cells: x low, x high, y low, y high, z low, z high (one more word follows)
     int32_t tb, te;             // listener terms
@@ -70,13 +74,14 @@ struct ResItem {
 };
 
 // Tile shapes: cells per column by number of damped axes, and the LDS words
-// of a column (its cells, the x-high halo after them, the x-low halo last).
+// of a column (its cells, the high halo after them, the low halo last).
 struct ResShape {
     int plain, one, more;
-    int column_words, lds_words;  // of one of the two buffers
+    int column_words, lds_words;  // of one buffer
+    int buffers;                // of pressures
     int max_words, max_recs;    // face words and records a tile may hold
 };
-enum : int { RES_FINE = 0, RES_COARSE = 1, RES_SHAPES = 2 };
+enum : int { RES_FINE = 0, RES_COARSE = 1, RES_LARGE = 2, RES_SHAPES = 3 };
 ResShape resident_shape(int shape);
 
 struct SceneSetup;

@@ -37,11 +37,22 @@ struct Shape;
 template <>
 struct Shape<RES_FINE> {
     static constexpr int plain = 8, one = 8, more = 8, cs = 12, words = 4, recs = 2, waves = 3, lds = 4608;
+    static constexpr bool in_place = false;
 };
 // larger grids: as many cells per workgroup as registers and LDS hold
 template <>
 struct Shape<RES_COARSE> {
     static constexpr int plain = 16, one = 12, more = 8, cs = 20, words = 6, recs = 3, waves = 3, lds = 6500;
+    static constexpr bool in_place = false;
+};
+// grids beyond that: two workgroups a compute unit with 256 registers a lane,
+// and pressures in one LDS buffer, so new ones wait in registers for a barrier.
+// Slower where RES_COARSE fits (128^3 8.4 us per step against 5.3: two waves a
+// SIMD hide less), faster than the step kernels beyond (144x146x144 7.9 us against 14.6).
+template <>
+struct Shape<RES_LARGE> {
+    static constexpr int plain = 32, one = 24, more = 16, cs = 36, words = 10, recs = 3, waves = 2, lds = 15000;
+    static constexpr bool in_place = true;
 };
 
 typedef unsigned long long u64;
@@ -67,13 +78,24 @@ __device__ __forceinline__ int anew(int v)
 // the cell itself and of its neighbour across the face, global cell across it)
 struct FaceCell {
     int own, halo;      // LDS words
-    int i, j, k;        // the neighbour's cell
+    int i, j, k;        // the neighbour's cell (tile's frame)
     bool real;          // (the last words of a face stand for no cell)
 };
 
 // Words of a face, rounded up to whole 128-byte lines: a line then has one
 // sender per neighbour.
 __device__ __forceinline__ int face_words(int n) { return (n + 15) & ~15; }
+
+// a[d] of a struct in device memory (a copy of it that is indexed by a variable
+// would go to scratch memory)
+template <class T>
+__device__ __forceinline__ T pick(const T (&a)[3], int d) { return cmem(&a[0])[d]; }
+
+// a tile's axes in the grid: its columns', and the one across
+__device__ __forceinline__ int column_axis(const ResTile &t) { return t.swap ? 1 : 0; }
+__device__ __forceinline__ int across_axis(const ResTile &t) { return t.swap ? 0 : 1; }
+__device__ __forceinline__ int column_stride(const SceneDev &S, const ResTile &t) { return t.swap ? S.sy : S.sx; }
+__device__ __forceinline__ int across_stride(const SceneDev &S, const ResTile &t) { return t.swap ? S.sx : S.sy; }
 
 template <int CS>
 __device__ __forceinline__ FaceCell face_cell(const ResTile &t, int w)
@@ -138,8 +160,11 @@ __global__ __launch_bounds__(RES_THREADS) void route_kernel(const ResScene *__re
             continue;
         }
         r.lds = (uint32_t)f.own | ((uint32_t)f.halo << 16);
-        if (f.i >= 0 && f.j >= 0 && f.k >= 0 && f.i < S.n[0] && f.j < S.n[1] && f.k < S.n[2]) {
-            const int x[3] = {f.i, f.j, f.k};
+        const int x[3] = {t.swap ? f.j : f.i, t.swap ? f.i : f.j, f.k};
+        if (x[0] >= 0 && x[1] >= 0 && x[2] >= 0 && x[0] < S.n[0] && x[1] < S.n[1] && x[2] < S.n[2]) {
+            // the face's axis, and whether it is the tile's low one
+            const int a = f.i < t.i0 || f.i >= t.i0 + t.bx ? column_axis(t) : f.j < t.j0 || f.j >= t.j0 + t.by ? across_axis(t) : 2;
+            const bool low = f.i < t.i0 || f.j < t.j0 || f.k < t.k0;
             for (int b = 0; b < R.nboxes; ++b) {
                 const ResBox B = cmem(R.boxes)[b];
                 int at[3];
@@ -152,15 +177,12 @@ __global__ __launch_bounds__(RES_THREADS) void route_kernel(const ResScene *__re
                 const int q = B.first + ((at[0] / B.size[0]) * B.count[1] + at[1] / B.size[1]) * B.count[2] + at[2] / B.size[2];
                 const ResTile o = gmem(R.tiles)[q];
                 const int nyz = face_words(o.by * o.bz), nxz = face_words(o.bx * o.bz), nxy = face_words(o.bx * o.by);
-                const int li = x[0] - o.i0, lj = x[1] - o.j0, lk = x[2] - o.k0;
+                const int li = (o.swap ? x[1] : x[0]) - o.i0, lj = (o.swap ? x[0] : x[1]) - o.j0, lk = x[2] - o.k0;
                 // the own cell is across the neighbour's opposite face
                 int word;
-                if (f.i < t.i0) word = nyz + lj * o.bz + lk;
-                else if (f.i >= t.i0 + t.bx) word = lj * o.bz + lk;
-                else if (f.j < t.j0) word = 2 * nyz + nxz + li * o.bz + lk;
-                else if (f.j >= t.j0 + t.by) word = 2 * nyz + li * o.bz + lk;
-                else if (f.k < t.k0) word = 2 * (nyz + nxz) + nxy + li * o.by + lj;
-                else word = 2 * (nyz + nxz) + li * o.by + lj;
+                if (a == column_axis(o)) word = (low ? nyz : 0) + lj * o.bz + lk;
+                else if (a == across_axis(o)) word = 2 * nyz + (low ? nxz : 0) + li * o.bz + lk;
+                else word = 2 * (nyz + nxz) + (low ? nxy : 0) + li * o.by + lj;
                 r.to = o.word0 + (uint32_t)word;
                 break;
             }
@@ -169,11 +191,11 @@ __global__ __launch_bounds__(RES_THREADS) void route_kernel(const ResScene *__re
     }
 }
 
-// the x table entry of face / cell i: a wall face gets zero factors
-__device__ __forceinline__ float4 x_entry(const SceneDev &S, int i)
+// the table entry of face / cell i along axis d: a wall face gets zero factors
+__device__ __forceinline__ float4 table_entry(const SceneDev *S, int d, int i)
 {
-    float4 c = gmem(S.coef[0])[min(i, S.n[0])];
-    if (i <= 0 || i >= S.n[0]) { c.x = 0.f; c.y = 0.f; }
+    float4 c = gmem(pick(S->coef, d))[min(i, pick(S->n, d))];
+    if (i <= 0 || i >= pick(S->n, d)) { c.x = 0.f; c.y = 0.f; }
     return c;
 }
 
@@ -200,7 +222,7 @@ struct Frame {
     const ResScene *res;
     const ResTile *tile;
     float *A, *B;               // this step's pressures and the next's, in LDS
-    float4 *X;                  // x table of the tile's cells and faces, in LDS
+    float4 *X;                  // table of the tile's cells and faces along its columns, in LDS
     long long step0;
     int steps;
     uint32_t tag;
@@ -236,13 +258,14 @@ struct Frame {
     __device__ __forceinline__ static int place(const SceneDev &S, const ResTile &t, int cell)
     {
         const int i = cell / S.sx, r = cell - i * S.sx, j = r / S.sy, k = r - j * S.sy;
-        return (j - t.j0 + 1) * t.pitch + (k - t.k0 + 1) * C::cs + (i - t.i0);
+        const int u = t.swap ? j : i, v = t.swap ? i : j;
+        return (v - t.j0 + 1) * t.pitch + (k - t.k0 + 1) * C::cs + (u - t.i0);
     }
 
     // p^{step} of the tile and its halo, both buffers cleared before
     __device__ __forceinline__ void load(const SceneDev &S, const ResScene &R, const ResTile &t)
     {
-        const int tid = (int)threadIdx.x, n = 2 * C::lds;
+        const int tid = (int)threadIdx.x, n = (C::in_place ? 1 : 2) * C::lds;
         for (int q = tid; q < n; q += RES_THREADS) A[q] = 0.f;
         bx = t.bx;
         P = t.pitch;
@@ -250,14 +273,14 @@ struct Frame {
         ly = act ? tid / t.bz : 0;
         lz = act ? tid - ly * t.bz : 0;
         col = (ly + 1) * P + (lz + 1) * C::cs;
-        if (tid <= C::plain) X[tid] = x_entry(S, t.i0 + tid);
+        if (tid <= C::plain) X[tid] = table_entry(scene, column_axis(t), t.i0 + tid);
         __syncthreads();
         const AS_GLOBAL float *pc = gmem(S.field + (size_t)slot_cur(step0) * S.npad);
         if (act) {
-            const int idx = t.i0 * S.sx + (t.j0 + ly) * S.sy + t.k0 + lz;
+            const int su = column_stride(S, t), idx = t.i0 * su + (t.j0 + ly) * across_stride(S, t) + t.k0 + lz;
 #pragma unroll
             for (int i = 0; i < C::plain; ++i)
-                if (i < t.bx) A[col + i] = pc[idx + i * S.sx];
+                if (i < t.bx) A[col + i] = pc[idx + i * su];
         }
         words = R.words;
         half = R.nwords * 8u;
@@ -271,8 +294,9 @@ struct Frame {
             lds[m] = r.lds * 4u;
             if (w < t.words) {
                 const FaceCell f = face_cell<C::cs>(t, w);
-                if (f.real && f.i >= 0 && f.j >= 0 && f.k >= 0 && f.i < S.n[0] && f.j < S.n[1] && f.k < S.n[2])
-                    A[f.halo] = pc[f.i * S.sx + f.j * S.sy + f.k];
+                const int i = t.swap ? f.j : f.i, j = t.swap ? f.i : f.j;
+                if (f.real && i >= 0 && j >= 0 && f.k >= 0 && i < S.n[0] && j < S.n[1] && f.k < S.n[2])
+                    A[f.halo] = pc[i * S.sx + j * S.sy + f.k];
             }
         }
         // one term per thread of the usual kind (a cell's new pressure) is
@@ -314,25 +338,29 @@ struct Frame {
             if (a == 0.f) continue;
             const PSrcDev ps = cmem(Z.psrc)[p];
             const AS_GLOBAL float *g = gmem(Z.gtab);
-            v = add_source(v, a, g[ps.goff[0] + min(u.i0 + i, Z.n[0] - 1)], g[ps.goff[1] + u.j0 + ly], g[ps.goff[2] + u.k0 + lz]);
+            const int x = u.swap ? u.j0 + ly : min(u.i0 + i, Z.n[0] - 1), y = u.swap ? min(u.i0 + i, Z.n[1] - 1) : u.j0 + ly;
+            v = add_source(v, a, g[ps.goff[0] + x], g[ps.goff[1] + y], g[ps.goff[2] + u.k0 + lz]);
         }
         return v;
     }
 
     // Step s has been made: a cell's term takes its new pressure (in B), a
-    // ghost's its value in that step (from A).
+    // ghost's its value in that step (from A; in place, before the cells are
+    // written, with GHOSTS).
+    template <bool GHOSTS = false>
     __device__ __forceinline__ void terms(int s) const
     {
         if (!terms_here) return;
         const int row = ring0 + s < cap ? ring0 + s : ring0 + s - cap;
-        if (has_term) *(AS_GLOBAL double *)((AS_GLOBAL char *)term_to + (size_t)row * row_bytes) = term_beta * (double)B[term_at];
+        if (has_term && !GHOSTS) *(AS_GLOBAL double *)((AS_GLOBAL char *)term_to + (size_t)row * row_bytes) = term_beta * (double)B[term_at];
         if (!more_terms) return;
         const SceneDev S = scene_now();
         const ResScene R = *cmem(anew(res));
         const ResTile t = *cmem(anew(tile));
         for (int q = t.tb + (int)threadIdx.x; q < t.te; q += RES_THREADS) {
             const TermRef r = gmem(R.terms)[q];
-            if (r.kind == 0 && q < t.tb + RES_THREADS) continue;
+            if (r.kind == 0 && (GHOSTS || q < t.tb + RES_THREADS)) continue;
+            if (C::in_place && r.kind != 0 && !GHOSTS) continue;
             double v;
             if (r.kind == 0) v = (double)B[place(S, t, r.cell)];
             else {
@@ -386,18 +414,29 @@ struct Frame {
         B = q;
     }
 
+    // (in place, the last step) the level before the newest, which the step overwrites
+    __device__ __forceinline__ void store_old() const
+    {
+        if (!act) return;
+        const SceneDev S = scene_now();
+        const ResTile t = *cmem(anew(tile));
+        AS_GLOBAL float *pp = gmem(S.field + (size_t)slot_next(step0 + steps) * S.npad);
+        const int su = column_stride(S, t), idx = t.i0 * su + (t.j0 + anew(ly)) * across_stride(S, t) + t.k0 + lz;
+        for (int i = 0; i < t.bx; ++i) pp[idx + i * su] = A[col + i];
+    }
+
     // the last two levels of the own cells, into the slots of step step0 + steps
     __device__ __forceinline__ void store_pressure(const SceneDev &S, const ResTile &t) const
     {
         if (!act) return;
         const long long s = step0 + steps;
         AS_GLOBAL float *pc = gmem(S.field + (size_t)slot_cur(s) * S.npad), *pp = gmem(S.field + (size_t)slot_next(s) * S.npad);
-        const int idx = t.i0 * S.sx + (t.j0 + anew(ly)) * S.sy + t.k0 + lz;
+        const int su = column_stride(S, t), idx = t.i0 * su + (t.j0 + anew(ly)) * across_stride(S, t) + t.k0 + lz;
 #pragma unroll
         for (int i = 0; i < C::plain; ++i)
             if (i < t.bx) {
-                pc[idx + i * S.sx] = A[col + i];
-                pp[idx + i * S.sx] = B[col + i];
+                pc[idx + i * su] = A[col + i];
+                if (!C::in_place) pp[idx + i * su] = B[col + i];
             }
     }
 };
@@ -407,7 +446,7 @@ struct Frame {
 template <int CS, int NB>
 struct Column {
     float c[NB + 1], before;    // cells 0 .. NB (cell bx is the x-high halo); the x-low halo
-    __device__ __forceinline__ Column(const float *A, int col)
+    __device__ __forceinline__ void load(const float *A, int col)
     {
 #pragma unroll
         for (int q = 0; q < NB / 4; ++q) {
@@ -440,6 +479,26 @@ __device__ __forceinline__ Quad quad(const float *A, int col, int P, int q)
 __device__ __forceinline__ void put_quad(float *B, int col, int q, const float *o)
 {
     *(float4 *)(B + col + 4 * q) = make_float4(o[0], o[1], o[2], o[3]);
+}
+
+// In place: every thread has read what it needs of this step's pressures, and
+// may write the next ones.
+template <int SHAPE>
+__device__ __forceinline__ void before_writes(Frame<SHAPE> &F, int s)
+{
+    if constexpr (Shape<SHAPE>::in_place) {
+        F.template terms<true>(s);
+        if (s == F.steps - 1) F.store_old();
+        __syncthreads();
+    }
+}
+// Writes a column of new pressures; (in place) cells past the tile's last as put_quad.
+template <int NB>
+__device__ __forceinline__ void put_column(float *B, int col, int bx, const float *o)
+{
+#pragma unroll
+    for (int q = 0; q < NB / 4; ++q)
+        if (4 * q < bx) put_quad(B, col, q, o + 4 * q);
 }
 
 // Undamped cells: leapfrog, pressure sources, and the object-adjacent cells
@@ -501,8 +560,12 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
     accelerations(F.step0);
     for (int s = 0; s < F.steps; ++s) {
         const long long step = F.step0 + s;
+        // new pressures: four at a time, or (in place) in the column, from which
+        // each cell has been read by the time it is replaced
+        Column<C::cs, NB> w;
         if (F.act) {
-            const Column<C::cs, NB> w(F.A, F.col);
+            w.load(F.A, F.col);
+            float left = w.before;
 #pragma unroll
             for (int q = 0; q < NB / 4; ++q) {
                 if (4 * q >= F.bx) continue;
@@ -511,7 +574,7 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = 4 * q + e;
-                    const float c = w.c[i], xm = i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
+                    const float c = w.c[i], xm = C::in_place ? left : i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
                     if (INC) {
                         prev[i] = increment1(c, prev[i], xm, xp, u.yl[e], u.yr[e], u.zl[e], u.zr[e], lam2);
                         o[e] = c + prev[i];
@@ -519,24 +582,19 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
                         o[e] = leapfrog1(c, prev[i], xm, xp, u.yl[e], u.yr[e], u.zl[e], u.zr[e], lam2);
                         prev[i] = c;
                     }
+                    if (C::in_place) { left = c; w.c[i] = o[e]; }
                 }
-                if (!skips) put_quad(F.B, F.col, q, o);
-                else {
+                if constexpr (!C::in_place) {
+                    if (!skips) put_quad(F.B, F.col, q, o);
+                    else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (4 * q + e < F.bx && !(skip >> (4 * q + e) & 1)) F.B[F.col + 4 * q + e] = o[e];
-                }
-            }
-            if (F.sounding()) {
-                const SceneDev Z = F.scene_now();
-                const ResTile u = *cmem(anew(F.tile));
-                for (int i = 0; i < F.bx; ++i)
-                    if (!(skip >> i & 1)) {
-                        float &o = F.B[F.col + i];
-                        o = INC ? fmaf(3.f, F.add_sources(Z, u, step, i, 0.f), o) : F.add_sources(Z, u, step, i, o);
+                        for (int e = 0; e < 4; ++e)
+                            if (4 * q + e < F.bx && !(skip >> (4 * q + e) & 1)) F.B[F.col + 4 * q + e] = o[e];
                     }
+                }
             }
         }
+        float rnow[NR];
         if (records) {
             const SceneDev Z = F.scene_now();
             const ResTile u = *cmem(anew(F.tile));
@@ -567,8 +625,33 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
                     }
                 }
                 rprev[r] = cf;
-                F.B[rat[r]] = (float)pn;
+                rnow[r] = (float)pn;
             }
+        }
+        before_writes(F, s);
+        if (F.act) {
+            if constexpr (C::in_place) {
+                if (!skips) put_column<NB>(F.B, F.col, F.bx, w.c);
+                else {
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+                        if (i < F.bx && !(skip >> i & 1)) F.B[F.col + i] = w.c[i];
+                }
+            }
+            if (F.sounding()) {
+                const SceneDev Z = F.scene_now();
+                const ResTile u = *cmem(anew(F.tile));
+                for (int i = 0; i < F.bx; ++i)
+                    if (!(skip >> i & 1)) {
+                        float &o = F.B[F.col + i];
+                        o = INC ? fmaf(3.f, F.add_sources(Z, u, step, i, 0.f), o) : F.add_sources(Z, u, step, i, o);
+                    }
+            }
+        }
+        if (records) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+                if (rat[r] >= 0) F.B[rat[r]] = rnow[r];
         }
         __syncthreads();
         F.send(s);
@@ -593,14 +676,14 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
 struct AxisCoef {
     float l1, l2, r1, r2, c3, c5;   // faces low and high {f1, f2}, cell {f3, f5/h}; a wall face stays at zero
 };
-__device__ __forceinline__ AxisCoef axis_coef(const SceneDev &S, int d, int i)
+__device__ __forceinline__ AxisCoef axis_coef(const SceneDev *S, int d, int i)
 {
-    const float4 lo = gmem(S.coef[d])[i], hi = gmem(S.coef[d])[i + 1];
+    const float4 lo = gmem(pick(S->coef, d))[i], hi = gmem(pick(S->coef, d))[i + 1];
     AxisCoef a;
     a.l1 = i > 0 ? lo.x : 0.f;
     a.l2 = i > 0 ? lo.y : 0.f;
-    a.r1 = i + 1 < S.n[d] ? hi.x : 0.f;
-    a.r2 = i + 1 < S.n[d] ? hi.y : 0.f;
+    a.r1 = i + 1 < pick(S->n, d) ? hi.x : 0.f;
+    a.r2 = i + 1 < pick(S->n, d) ? hi.y : 0.f;
     a.c3 = lo.z;
     a.c5 = lo.w;
     return a;
@@ -613,19 +696,33 @@ __device__ __forceinline__ float split_step(float f3, float f5, float q, float d
 {
     return fmaf(f5, dv, f3 * q);
 }
-// compact offsets of the own column's cells and faces in its slab
+// compact offsets of the own column's cells and faces in its slab: the cell's,
+// and the low faces' along the tile's axes, of column cell i
 struct SlabAt {
-    const PmlSlab &sl;
-    int e1, e2, li, lj, lk;
+    int c, cu, u, uu, v, vu, vh, w, wu;
     __device__ SlabAt(const PmlSlab &s, const ResTile &t, int ly, int lz)
-        : sl(s), e1(s.e[1]), e2(s.e[2]), li(t.i0 - s.lo[0]), lj(t.j0 + ly - s.lo[1]), lk(t.k0 + lz - s.lo[2]) {}
-    __device__ __forceinline__ int cell(int i) const { return ((li + i) * e1 + lj) * e2 + lk; }   // and the x face
-    __device__ __forceinline__ int fy(int i, int h) const { return ((li + i) * (e1 + 1) + lj + h) * e2 + lk; }
-    __device__ __forceinline__ int fz(int i, int h) const { return ((li + i) * e1 + lj) * (e2 + 1) + lk + h; }
+    {
+        const int e1 = s.e[1], e2 = s.e[2];
+        const int x = (t.swap ? t.j0 + ly : t.i0) - s.lo[0], y = (t.swap ? t.i0 : t.j0 + ly) - s.lo[1], z = t.k0 + lz - s.lo[2];
+        c = (x * e1 + y) * e2 + z;                   // and the x face
+        const int yf = (x * (e1 + 1) + y) * e2 + z;  // the y face
+        w = (x * e1 + y) * (e2 + 1) + z;
+        cu = t.swap ? e2 : e1 * e2;
+        u = t.swap ? yf : c;
+        uu = cu;
+        v = t.swap ? c : yf;
+        vu = t.swap ? e2 : (e1 + 1) * e2;
+        vh = t.swap ? e1 * e2 : e2;
+        wu = t.swap ? e2 + 1 : e1 * (e2 + 1);
+    }
+    __device__ __forceinline__ int cell(int i) const { return c + i * cu; }
+    __device__ __forceinline__ int fu(int i) const { return u + i * uu; }
+    __device__ __forceinline__ int fv(int i, int h) const { return v + i * vu + h * vh; }
+    __device__ __forceinline__ int fw(int i, int h) const { return w + i * wu + h; }
 };
 
-// Cells damped along axis D only (the merged PML state): pDir along D, both
-// faces along D, and the increment of the transverse sum.
+// Cells damped along axis D of the tile only (the merged PML state): pDir along
+// it, both faces along it, and the increment of the transverse sum.
 template <int SHAPE, int D>
 __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, const ResTile &t)
 {
@@ -633,32 +730,35 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, cons
     constexpr int NB = C::one;
     const PmlSlab sl = cmem(S.slabs)[t.slab];
     const SlabAt at(sl, t, F.ly, F.lz);
-    AS_GLOBAL float *pq = gmem(S.pd[D] + sl.cell_base), *pi = gmem(S.pd[D == 0 ? 1 : 0] + sl.cell_base);
+    const int gu = column_axis(t), gv = across_axis(t), g = D == 0 ? gu : D == 1 ? gv : 2;   // axes of the grid; g the damped one
+    AS_GLOBAL float *pq = gmem(pick(F.scene->pd, g) + sl.cell_base), *pi = gmem(pick(F.scene->pd, g == 0 ? 1 : 0) + sl.cell_base);
     float q0[NB], dd[NB], vl[D == 0 ? NB + 1 : NB], vr[D == 0 ? 1 : NB];
-    const AxisCoef cy = axis_coef(S, 1, t.j0 + F.ly), cz = axis_coef(S, 2, t.k0 + F.lz);
+    const AxisCoef cy = axis_coef(F.scene, gv, t.j0 + F.ly), cz = axis_coef(F.scene, 2, t.k0 + F.lz);
     {
-        const AS_GLOBAL float *v = gmem((F.step0 & 1 ? S.vel[1][D] : S.vel[0][D]) + sl.v_base[D]);
+        const AS_GLOBAL float *v = gmem((F.step0 & 1 ? pick(F.scene->vel[1], g) : pick(F.scene->vel[0], g)) + pick(S.slabs[t.slab].v_base, g));
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             const int e = min(i, t.bx - 1);
             q0[i] = pq[at.cell(e)];
             dd[i] = pi[at.cell(e)];
-            if (D == 0) vl[i] = v[at.cell(e)];
-            if (D == 1) { vl[i] = v[at.fy(e, 0)]; vr[i] = v[at.fy(e, 1)]; }
-            if (D == 2) { vl[i] = v[at.fz(e, 0)]; vr[i] = v[at.fz(e, 1)]; }
+            if (D == 0) vl[i] = v[at.fu(e)];
+            if (D == 1) { vl[i] = v[at.fv(e, 0)]; vr[i] = v[at.fv(e, 1)]; }
+            if (D == 2) { vl[i] = v[at.fw(e, 0)]; vr[i] = v[at.fw(e, 1)]; }
         }
         if (D == 0) {
             // the high face of the last cell (compile-time places only)
-            const float last = v[at.cell(t.bx)];
+            const float last = v[at.fu(t.bx)];
 #pragma unroll
             for (int i = 1; i <= NB; ++i)
                 if (i == t.bx) vl[i] = last;
         }
     }
-    const float4 xp0 = cmem(S.coef[0])[t.i0];   // D != 0: x is plain over the tile, one entry for all
+    const float4 xp0 = cmem(pick(F.scene->coef, gu))[t.i0];   // D != 0: plain along the columns, one entry for all
     for (int s = 0; s < F.steps; ++s) {
+        Column<C::cs, NB> w;
         if (F.act) {
-            const Column<C::cs, NB> w(F.A, F.col);
+            w.load(F.A, F.col);
+            float left = w.before;
             float before = 0.f;                 // D == 0: the updated low face of the next cell
 #pragma unroll
             for (int q = 0; q < NB / 4; ++q) {
@@ -668,7 +768,7 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, cons
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = 4 * q + e;
-                    const float c = w.c[i], xm = i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
+                    const float c = w.c[i], xm = C::in_place ? left : i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
                     float n, lap = 0.f;
                     const float qo = q0[i];
                     if (D == 0) {
@@ -695,9 +795,14 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, cons
                     dd[i] = dn;
                     q0[i] = n;
                     o[e] = c + (dA + dn);
+                    if (C::in_place) { left = c; w.c[i] = o[e]; }
                 }
-                put_quad(F.B, F.col, q, o);
+                if constexpr (!C::in_place) put_quad(F.B, F.col, q, o);
             }
+        }
+        before_writes(F, s);
+        if constexpr (C::in_place) {
+            if (F.act) put_column<NB>(F.B, F.col, F.bx, w.c);
         }
         if (F.act && F.sounding()) {
             // (staggered scheme) on both undamped axes
@@ -722,17 +827,18 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, cons
     if (!F.act) return;
     const PmlSlab zl_ = cmem(Z.slabs)[u.slab];
     const SlabAt to(zl_, u, anew(F.ly), anew(F.lz));
-    AS_GLOBAL float *zq = gmem(Z.pd[D] + zl_.cell_base), *zi = gmem(Z.pd[D == 0 ? 1 : 0] + zl_.cell_base);
-    AS_GLOBAL float *v = gmem(((F.step0 + F.steps) & 1 ? Z.vel[1][D] : Z.vel[0][D]) + zl_.v_base[D]);
+    const int h = D == 0 ? column_axis(u) : D == 1 ? across_axis(u) : 2;
+    AS_GLOBAL float *zq = gmem(pick(F.scene->pd, h) + zl_.cell_base), *zi = gmem(pick(F.scene->pd, h == 0 ? 1 : 0) + zl_.cell_base);
+    AS_GLOBAL float *v = gmem(((F.step0 + F.steps) & 1 ? pick(F.scene->vel[1], h) : pick(F.scene->vel[0], h)) + pick(Z.slabs[u.slab].v_base, h));
 #pragma unroll
     for (int i = 0; i <= NB; ++i) {
         if (i < NB && i < u.bx) {
             zq[to.cell(i)] = q0[i];
             zi[to.cell(i)] = dd[i];
-            if (D == 1) { v[to.fy(i, 0)] = vl[i]; if (F.ly == u.by - 1) v[to.fy(i, 1)] = vr[i]; }
-            if (D == 2) { v[to.fz(i, 0)] = vl[i]; if (F.lz == u.bz - 1) v[to.fz(i, 1)] = vr[i]; }
+            if (D == 1) { v[to.fv(i, 0)] = vl[i]; if (F.ly == u.by - 1) v[to.fv(i, 1)] = vr[i]; }
+            if (D == 2) { v[to.fw(i, 0)] = vl[i]; if (F.lz == u.bz - 1) v[to.fw(i, 1)] = vr[i]; }
         }
-        if (D == 0 && i <= u.bx) v[to.cell(i)] = vl[i];
+        if (D == 0 && i <= u.bx) v[to.fu(i)] = vl[i];
     }
 }
 
@@ -746,32 +852,36 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
     const PmlSlab sl = cmem(S.slabs)[t.slab];
     const SlabAt at(sl, t, F.ly, F.lz);
     float q0[NB], q1[NB], q2[NB], vx[NB + 1], yl[NB], yr[NB], zl[NB], zr[NB];
-    const int damped = t.damped;
-    const AxisCoef cy = axis_coef(S, 1, t.j0 + F.ly), cz = axis_coef(S, 2, t.k0 + F.lz);
+    // (in the tile's frame)
+    const int damped = t.swap ? (t.damped & 4) | (t.damped & 1) << 1 | (t.damped >> 1 & 1) : t.damped;
+    const int gu = column_axis(t), gv = across_axis(t);
+    const AxisCoef cy = axis_coef(F.scene, gv, t.j0 + F.ly), cz = axis_coef(F.scene, 2, t.k0 + F.lz);
     {
         const int b = (int)(F.step0 & 1);
-        const AS_GLOBAL float *v0 = gmem((b ? S.vel[1][0] : S.vel[0][0]) + sl.v_base[0]), *v1 = gmem((b ? S.vel[1][1] : S.vel[0][1]) + sl.v_base[1]);
+        const AS_GLOBAL float *v0 = gmem((b ? pick(F.scene->vel[1], gu) : pick(F.scene->vel[0], gu)) + pick(S.slabs[t.slab].v_base, gu)), *v1 = gmem((b ? pick(F.scene->vel[1], gv) : pick(F.scene->vel[0], gv)) + pick(S.slabs[t.slab].v_base, gv));
         const AS_GLOBAL float *v2 = gmem((b ? S.vel[1][2] : S.vel[0][2]) + sl.v_base[2]);
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             const int e = min(i, t.bx - 1), c = at.cell(e);
-            vx[i] = v0[c];
-            q0[i] = gmem(S.pd[0] + sl.cell_base)[c];
-            q1[i] = gmem(S.pd[1] + sl.cell_base)[c];
+            vx[i] = v0[at.fu(e)];
+            q0[i] = gmem(pick(F.scene->pd, gu) + sl.cell_base)[c];
+            q1[i] = gmem(pick(F.scene->pd, gv) + sl.cell_base)[c];
             q2[i] = gmem(S.pd[2] + sl.cell_base)[c];
-            yl[i] = v1[at.fy(e, 0)];
-            yr[i] = v1[at.fy(e, 1)];
-            zl[i] = v2[at.fz(e, 0)];
-            zr[i] = v2[at.fz(e, 1)];
+            yl[i] = v1[at.fv(e, 0)];
+            yr[i] = v1[at.fv(e, 1)];
+            zl[i] = v2[at.fw(e, 0)];
+            zr[i] = v2[at.fw(e, 1)];
         }
-        const float last = v0[at.cell(t.bx)];
+        const float last = v0[at.fu(t.bx)];
 #pragma unroll
         for (int i = 1; i <= NB; ++i)
             if (i == t.bx) vx[i] = last;
     }
     for (int s = 0; s < F.steps; ++s) {
+        Column<C::cs, NB> w;
         if (F.act) {
-            const Column<C::cs, NB> w(F.A, F.col);
+            w.load(F.A, F.col);
+            float left = w.before;
             float before = 0.f;
 #pragma unroll
             for (int q = 0; q < NB / 4; ++q) {
@@ -781,7 +891,7 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = 4 * q + e;
-                    const float c = w.c[i], xm = i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
+                    const float c = w.c[i], xm = C::in_place ? left : i ? w.c[i - 1] : w.before, xp = w.c[i + 1];
                     const float4 xl = F.X[i], xr = F.X[i + 1];
                     if (i == 0) before = face_step(xl.x, xl.y, vx[0], xm, c);
                     const float after = face_step(xr.x, xr.y, vx[i + 1], c, xp);
@@ -796,9 +906,14 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
                     zr[i] = face_step(cz.r1, cz.r2, zr[i], c, u.zr[e]);
                     q2[i] = split_step(cz.c3, cz.c5, q2[i], zr[i] - zl[i]);
                     o[e] = q0[i] + q1[i] + q2[i];
+                    if (C::in_place) { left = c; w.c[i] = o[e]; }
                 }
-                put_quad(F.B, F.col, q, o);
+                if constexpr (!C::in_place) put_quad(F.B, F.col, q, o);
             }
+        }
+        before_writes(F, s);
+        if constexpr (C::in_place) {
+            if (F.act) put_column<NB>(F.B, F.col, F.bx, w.c);
         }
         if (F.act && F.sounding() && damped != 7) {
             // (staggered scheme) on the undamped axis
@@ -829,20 +944,21 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
     const PmlSlab zl_ = cmem(Z.slabs)[u.slab];
     const SlabAt to(zl_, u, anew(F.ly), anew(F.lz));
     const int b = (int)((F.step0 + F.steps) & 1);
-    AS_GLOBAL float *v0 = gmem((b ? Z.vel[1][0] : Z.vel[0][0]) + zl_.v_base[0]), *v1 = gmem((b ? Z.vel[1][1] : Z.vel[0][1]) + zl_.v_base[1]);
+    const int hu = column_axis(u), hv = across_axis(u);
+    AS_GLOBAL float *v0 = gmem((b ? pick(F.scene->vel[1], hu) : pick(F.scene->vel[0], hu)) + pick(Z.slabs[u.slab].v_base, hu)), *v1 = gmem((b ? pick(F.scene->vel[1], hv) : pick(F.scene->vel[0], hv)) + pick(Z.slabs[u.slab].v_base, hv));
     AS_GLOBAL float *v2 = gmem((b ? Z.vel[1][2] : Z.vel[0][2]) + zl_.v_base[2]);
 #pragma unroll
     for (int i = 0; i <= NB; ++i) {
-        if (i <= u.bx) v0[to.cell(i)] = vx[i];
+        if (i <= u.bx) v0[to.fu(i)] = vx[i];
         if (i < NB && i < u.bx) {
             const int c = to.cell(i);
-            gmem(Z.pd[0] + zl_.cell_base)[c] = q0[i];
-            gmem(Z.pd[1] + zl_.cell_base)[c] = q1[i];
+            gmem(pick(F.scene->pd, hu) + zl_.cell_base)[c] = q0[i];
+            gmem(pick(F.scene->pd, hv) + zl_.cell_base)[c] = q1[i];
             gmem(Z.pd[2] + zl_.cell_base)[c] = q2[i];
-            v1[to.fy(i, 0)] = yl[i];
-            if (F.ly == u.by - 1) v1[to.fy(i, 1)] = yr[i];
-            v2[to.fz(i, 0)] = zl[i];
-            if (F.lz == u.bz - 1) v2[to.fz(i, 1)] = zr[i];
+            v1[to.fv(i, 0)] = yl[i];
+            if (F.ly == u.by - 1) v1[to.fv(i, 1)] = yr[i];
+            v2[to.fw(i, 0)] = zl[i];
+            if (F.lz == u.bz - 1) v2[to.fw(i, 1)] = zr[i];
         }
     }
 }
@@ -879,7 +995,7 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
     F.trouble = trouble;
     F.X = xtab;
     F.A = lds;
-    F.B = lds + Shape<SHAPE>::lds;
+    F.B = Shape<SHAPE>::in_place ? lds : lds + Shape<SHAPE>::lds;
     if (threadIdx.x == 0) {
         u64 expect = GATE_SHUT;
         const u64 n = __hip_atomic_fetch_add(&clk[CLK_ARRIVED], 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1ULL;
@@ -908,7 +1024,8 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
     }
     __syncthreads();
     if (!gate) return;
-    switch (t.damped) {
+    // damped axes in the tile's frame
+    switch (t.swap ? (t.damped & 4) | (t.damped & 1) << 1 | (t.damped >> 1 & 1) : t.damped) {
     case 0:
         if (S.inc) run_plain<SHAPE, true>(F, S, t);
         else run_plain<SHAPE, false>(F, S, t);
@@ -922,16 +1039,30 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
 
 }  // namespace
 
-ResShape resident_shape(int shape)
+// f(Shape<shape>, the shape's kernel)
+template <class F>
+static auto with_shape(int shape, F f)
 {
-    auto of = [](auto c) {
-        using C = decltype(c);
-        return ResShape{C::plain, C::one, C::more, C::cs, C::lds, C::words * RES_THREADS, C::recs * RES_THREADS};
-    };
-    return shape == RES_FINE ? of(Shape<RES_FINE>{}) : of(Shape<RES_COARSE>{});
+    switch (shape) {
+    case RES_FINE: return f(Shape<RES_FINE>{}, resident_kernel<RES_FINE>);
+    case RES_COARSE: return f(Shape<RES_COARSE>{}, resident_kernel<RES_COARSE>);
+    default: return f(Shape<RES_LARGE>{}, resident_kernel<RES_LARGE>);
+    }
 }
 
-static size_t lds_bytes(int shape) { return sizeof(float) * 2 * (size_t)resident_shape(shape).lds_words; }
+ResShape resident_shape(int shape)
+{
+    return with_shape(shape, [](auto c, auto) {
+        using C = decltype(c);
+        return ResShape{C::plain, C::one, C::more, C::cs, C::lds, C::in_place ? 1 : 2, C::words * RES_THREADS, C::recs * RES_THREADS};
+    });
+}
+
+static size_t lds_bytes(int shape)
+{
+    const ResShape sh = resident_shape(shape);
+    return sizeof(float) * (size_t)sh.buffers * (size_t)sh.lds_words;
+}
 
 int resident_capacity(int shape)
 {
@@ -939,9 +1070,7 @@ int resident_capacity(int shape)
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return 0;
     const size_t bytes = lds_bytes(shape);
-    const hipError_t e = shape == RES_FINE
-                             ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, resident_kernel<RES_FINE>, RES_THREADS, bytes)
-                             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, resident_kernel<RES_COARSE>, RES_THREADS, bytes);
+    const hipError_t e = with_shape(shape, [&](auto, auto k) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, RES_THREADS, bytes); });
     if (e != hipSuccess) return 0;
     return per * cus;
 }
@@ -949,10 +1078,10 @@ int resident_capacity(int shape)
 hipError_t launch_resident_routes(const ResScene *scene, int ntiles, int shape, hipStream_t s)
 {
     if (ntiles <= 0) return hipSuccess;
-    if (shape == RES_FINE)
-        hipLaunchKernelGGL(route_kernel<Shape<RES_FINE>::cs>, dim3(ntiles), dim3(RES_THREADS), 0, s, scene);
-    else
-        hipLaunchKernelGGL(route_kernel<Shape<RES_COARSE>::cs>, dim3(ntiles), dim3(RES_THREADS), 0, s, scene);
+    with_shape(shape, [&](auto c, auto) {
+        hipLaunchKernelGGL(route_kernel<decltype(c)::cs>, dim3(ntiles), dim3(RES_THREADS), 0, s, scene);
+        return 0;
+    });
     return hipGetLastError();
 }
 
@@ -961,10 +1090,10 @@ hipError_t launch_resident(int shape, const ResItem *items, int n, int nsteps, u
 {
     if (n <= 0) return hipSuccess;
     const size_t bytes = lds_bytes(shape);
-    if (shape == RES_FINE)
-        hipLaunchKernelGGL(resident_kernel<RES_FINE>, dim3(n), dim3(RES_THREADS), bytes, s, items, nsteps, tag, wait_limit, trouble);
-    else
-        hipLaunchKernelGGL(resident_kernel<RES_COARSE>, dim3(n), dim3(RES_THREADS), bytes, s, items, nsteps, tag, wait_limit, trouble);
+    with_shape(shape, [&](auto, auto k) {
+        hipLaunchKernelGGL(k, dim3(n), dim3(RES_THREADS), bytes, s, items, nsteps, tag, wait_limit, trouble);
+        return 0;
+    });
     return hipGetLastError();
 }
 

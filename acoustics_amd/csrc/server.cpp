@@ -133,7 +133,9 @@ fdtd_status fdtd_server::rebuild()
 // resident, the resident launches, and the clocks, AMP_ROWS steps at a time.
 fdtd_status fdtd_server::run_block()
 {
-    if (res_prog[RES_FINE].n == 0 && res_prog[RES_COARSE].n == 0) return prog.enqueue(stream, 0, block);
+    bool any = false;
+    for (const ResidentProgram &p : res_prog) any = any || p.n > 0;
+    if (!any) return prog.enqueue(stream, 0, block);
     bool kernels = false;
     for (int k = 0; k < NUM_KINDS; ++k) kernels = kernels || prog.ntiles[k] > 0;
     for (int done = 0; done < block;) {

@@ -126,3 +126,34 @@ def test_two_threads(hip_lib):
     for t in th:
         t.join()
     assert all(np.array_equal(g, want) for g in got)
+
+
+def _large(kind, div):
+    rng = np.random.default_rng(8)
+    if kind == "staggered":
+        s = scenes.base_settings(div, 0.005, 8)
+        s["scheme"] = capi.FDTD_SCHEME_STAGGERED
+        mid = np.array(s["min_bound"]) + 0.005 * np.array(div) * [0.5, 0.08, 0.5]   # the pulse reaches into the PML
+        ears = mid + rng.uniform(0.0, 0.06, size=(12, 3))
+        return scenes.SceneBuffers(s, pressure_sources=[scenes.gaussian_pressure_source(mid, 2e-5)], listeners=ears)
+    return scenes._small_object_scene(rng, div, 0.005, 8, 2, 24)
+
+
+@pytest.mark.parametrize("kind", ["objects", "staggered"])
+@pytest.mark.parametrize("div", [(139, 89, 190), (144, 146, 144), (97, 210, 133)])
+def test_grids_for_the_largest_tiles(hip_lib, kind, div):
+    """Too many tiles of the other shapes: columns of up to 32 cells, along x and y, in one LDS buffer."""
+    sb = _large(kind, div)
+    print(f"case: large {kind} {div}", flush=True)
+    with Solver(sb, tile_config=0) as s:
+        s.step(150)
+        want, field = s.series(), s.pressure()
+        s.step(61)
+        more = s.pressure()
+    with Solver(sb) as s:
+        for n in (1, 70, 79):
+            s.step(n)
+        assert np.array_equal(s.series(), want) and np.array_equal(s.pressure(), field)
+        s.step(60)
+        s.step(1)      # a step kernel goes on from the block's two levels
+        assert np.array_equal(s.pressure(), more)
