@@ -321,6 +321,11 @@ struct Frame {
         src_tab = gmem(S.src_tab);
         amp_last = S.amp_rows - 1;
         amp = 0.f;
+        if (src) {
+            const PSrcDev ps = cmem(S.psrc)[0];
+            const int gu = t.swap ? ps.goff[1] : ps.goff[0], n = t.swap ? S.n[1] : S.n[0];
+            if (tid < C::plain) along()[tid] = gmem(S.gtab)[gu + min(t.i0 + tid, n - 1)];
+        }
         fetch_amp(step0);
     }
 
@@ -330,11 +335,27 @@ struct Frame {
     }
     // (an amplitude of zero, once the pulse is over, adds nothing)
     __device__ __forceinline__ bool sounding() const { return src && (amp != 0.f || src > 1); }
-    // the pressure sources' S dt at cell i of the own column in step `step`, added to v
-    __device__ __forceinline__ float add_sources(const SceneDev &Z, const ResTile &u, long long step, int i, float v) const
+    // the first source's factor along the columns (after the table in LDS) ...
+    __device__ __forceinline__ float *along() const { return (float *)(X + C::plain + 1); }
+    // ... and across them and along z, for a step's add_sources
+    struct Across { float v, z; };
+    __device__ __forceinline__ Across across(const SceneDev &Z, const ResTile &u) const
     {
-        for (int p = 0; p < Z.n_psrc; ++p) {
-            const float a = p == 0 ? amp : gmem(Z.src_tab)[amp_row(Z, step) * Z.n_psrc + p];
+        const PSrcDev ps = cmem(Z.psrc)[0];
+        const AS_GLOBAL float *g = gmem(Z.gtab);
+        return {g[(u.swap ? ps.goff[0] : ps.goff[1]) + u.j0 + ly], g[ps.goff[2] + u.k0 + lz]};
+    }
+    // the pressure sources' S dt at cell i of the own column in step `step`, added to v.
+    // The first one's factors are at hand: a staggered pulse never ends, and
+    // loaded cell by cell they held up its tiles in every step (150x97x133:
+    // 10.7 us per step, now 7.0; kept in registers for all steps they cost the
+    // other tiles 3%)
+    __device__ __forceinline__ float add_sources(const SceneDev &Z, const ResTile &u, Across w, long long step, int i, float v) const
+    {
+        // (only the in-place shape's tiles swap)
+        if (amp != 0.f) v = C::in_place && u.swap ? add_source(v, amp, w.v, along()[i], w.z) : add_source(v, amp, along()[i], w.v, w.z);
+        for (int p = 1; p < Z.n_psrc; ++p) {
+            const float a = gmem(Z.src_tab)[amp_row(Z, step) * Z.n_psrc + p];
             if (a == 0.f) continue;
             const PSrcDev ps = cmem(Z.psrc)[p];
             const AS_GLOBAL float *g = gmem(Z.gtab);
@@ -641,10 +662,11 @@ __device__ __forceinline__ void run_plain(Frame<SHAPE> &F, const SceneDev &S, co
             if (F.sounding()) {
                 const SceneDev Z = F.scene_now();
                 const ResTile u = *cmem(anew(F.tile));
+                const auto w = F.across(Z, u);
                 for (int i = 0; i < F.bx; ++i)
                     if (!(skip >> i & 1)) {
                         float &o = F.B[F.col + i];
-                        o = INC ? fmaf(3.f, F.add_sources(Z, u, step, i, 0.f), o) : F.add_sources(Z, u, step, i, o);
+                        o = INC ? fmaf(3.f, F.add_sources(Z, u, w, step, i, 0.f), o) : F.add_sources(Z, u, w, step, i, o);
                     }
             }
         }
@@ -808,9 +830,10 @@ __device__ __forceinline__ void run_one(Frame<SHAPE> &F, const SceneDev &S, cons
             // (staggered scheme) on both undamped axes
             const SceneDev Z = F.scene_now();
             const ResTile u = *cmem(anew(F.tile));
+            const auto w = F.across(Z, u);
             for (int i = 0; i < F.bx; ++i) {
                 float &o = F.B[F.col + i];
-                o = fmaf(2.f, F.add_sources(Z, u, F.step0 + s, i, 0.f), o);
+                o = fmaf(2.f, F.add_sources(Z, u, w, F.step0 + s, i, 0.f), o);
             }
         }
         __syncthreads();
@@ -919,10 +942,11 @@ __device__ __forceinline__ void run_more(Frame<SHAPE> &F, const SceneDev &S, con
             // (staggered scheme) on the undamped axis
             const SceneDev Z = F.scene_now();
             const ResTile u = *cmem(anew(F.tile));
+            const auto w = F.across(Z, u);
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 if (i >= F.bx) continue;
-                const float f = F.add_sources(Z, u, F.step0 + s, i, 0.f);
+                const float f = F.add_sources(Z, u, w, F.step0 + s, i, 0.f);
                 if (damped == 6) q0[i] += f;
                 else if (damped == 5) q1[i] += f;
                 else q2[i] += f;
@@ -975,7 +999,7 @@ __global__ __launch_bounds__(RES_THREADS, Shape<SHAPE>::waves) void resident_ker
 {
     extern __shared__ __align__(16) float lds[];
     __shared__ int gate;
-    __shared__ float4 xtab[Shape<SHAPE>::plain + 1];
+    __shared__ float4 xtab[Shape<SHAPE>::plain + 1 + Shape<SHAPE>::plain / 4];
     const ResItem it = items[blockIdx.x];
     if (!it.scene) return;
     // uniform data by way of the constant address space: scalar loads, scalar registers
