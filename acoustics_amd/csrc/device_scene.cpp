@@ -648,16 +648,14 @@ void DeviceScene::append_tiles(int scene_id, const TilePlan &plan, std::vector<T
     } else {
         // short rows share a wavefront: rpw rows of kwv/4 lanes each.  The
         // tiles of a band of rows follow each other along x, so a tile's x
-        // halo (two planes of its rows, twice its y halo) was just read by the
-        // tile before it and is still in the L2 (at 256^3: 73.4 us per step
-        // against 75.6 with the y-neighbours adjacent; the Engquist free field
-        // 46.0 against 51.9).  With PML slabs, G = band_group bands advance
-        // along x together (G tiles per x step), so the rows between them are
-        // read once for both neighbours' y halos: 72.4 us against 73.2 at
-        // 256^3 with G = 4 (2 and 8: 73.1, 72.9); the staggered scheme (plan
-        // 1, marches of four planes) takes G = 8: 189.7 us against 194.2 with
-        // 4 and 207.4 with 2.  The Engquist free field, all rows, measured
-        // 46.7 against 45.8 with groups, so it keeps single bands.
+        // halo was just read by the tile before it and is still in the L2 (at
+        // 256^3, marches of two: 73.4 us per step against 75.6 with the
+        // y-neighbours adjacent; the Engquist free field 46.0 against 51.9).
+        // With PML slabs, G = band_group bands advance along x together (G tiles
+        // per x step), so the rows between them are read once for both
+        // neighbours' y halos: 300x290x280, marches of four, 103.2 us with
+        // G = 8, 103.8 with 4 and 107.9 with one.  The Engquist free field, all
+        // rows, measured 46.7 against 45.8 with groups, so it keeps single bands.
         const int rpw = std::max(1, std::min(8, 64 / ((std::min(kwv, segw) + 3) / 4)));
         const int G = S.slabs.empty() ? 1 : std::max(1, plan.band_group);
         // A z slab's row segment and the row's interior part share a 128-byte

@@ -6,8 +6,8 @@
 // workgroups in flight, 1.9 us with 512, 3.0 us with 1024 (a bare exchange of
 // 1024 words each); nothing else is read from or written to memory.  Measured
 // per step: 64^3 with a 10-cell PML (206 workgroups) 2.1 us, of which the
-// arithmetic alone 0.9 and the exchange alone 1.5 (the step kernels: 6.6);
-// 128^3 with a 12-cell PML (733) 5.4 us, 2.9 and 5.0 (17.9).
+// arithmetic alone 0.9 and the exchange alone 1.5 (the step kernels: 6.0);
+// 128^3 with a 12-cell PML (733) 5.2 us, 2.9 and 5.0 (12.3).
 //
 // * Each face pressure travels in one 8-byte word with the step's tag above
 //   it, so the data is its own flag: no store is waited for before a flag is

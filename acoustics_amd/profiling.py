@@ -31,7 +31,7 @@ STEP_KERNELS = ("step_kernel<0>", "step_kernel<1>", "step_kernel<2>", "step_kern
 KERNEL_ROLE = {"step_kernel<0>": "interior + object-adjacent cells", "step_kernel<1>": "PML slabs",
                "step_kernel<2>": "object-adjacent cells",
                "step_kernel<3>": "one step, all tile classes (PML, interior, object-adjacent) + listener terms",
-               "advance_kernel": "block advance (step counter, amplitude ring for the next 64 steps)"}
+               "advance_kernel": "block advance (step counter, amplitude ring for the next 256 steps)"}
 
 
 def copy(mib, iters):
@@ -55,7 +55,7 @@ def step(n, steps, tile, scheme="collocated", boundary="rasterize"):
         bc = FDTD_BOUNDARY_FULLY_COUPLED if boundary == "coupled" else FDTD_BOUNDARY_RASTERIZE
         sb, _ = scenes.config3(seed=3, n=n, h=0.64 / n, boundary=bc)
     with Solver(sb, tile_config=tile) as s:
-        # eager (one dispatch per kernel per step, one advance per 64 steps),
+        # eager (one dispatch per kernel per step, one advance per 256 steps),
         # no timing events between the kernels
         s.step(steps)
         s.synchronize()
