@@ -483,7 +483,8 @@ fdtd_status fdtd_batch_read_listener_series(fdtd_batch *b, int scene, double *ou
     b->R.reap();
     const DeviceScene &D = *b->R.scenes[scene];
     const long long rows = std::min<long long>(b->R.taken, b->R.targets[scene]);
-    return D.read_series(0, rows, out);
+    b->R.stage.open();
+    return D.read_series(0, rows, out, &b->R.stage, b->stream);
 }
 
 fdtd_status fdtd_time_chunk(const fdtd_settings *in, int64_t num_steps, int chunk, fdtd_settings *out,

@@ -34,6 +34,7 @@ struct BatchRunner {
     // launches by tile shape
     std::vector<std::unique_ptr<ResidentScene>> res;
     ResidentProgram res_prog[RES_SHAPES];
+    SeriesStage stage;
     bool res_listed = false;
     int plan = 0;
     int graph_steps = 32;
@@ -68,6 +69,7 @@ struct BatchRunner {
             if (r) r->release();
         res.clear();
         for (ResidentProgram &p : res_prog) p.release();
+        stage.close();
     }
     ~BatchRunner();
 };

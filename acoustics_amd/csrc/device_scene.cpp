@@ -48,6 +48,7 @@ struct Layout {
     int32_t *op_ptr, *op_idx, *oc_ptr, *oc_ch;
     double *op_w, *oc_w;
     double *terms;
+    int32_t *lst_ptr;
     unsigned long long *clock;
     double *t_tab;
     double *acc_tab;
@@ -140,6 +141,7 @@ void carve(const SceneSetup &S, int cap, Carver &cs, Carver &c, Layout &L)
     L.oc_ch = c.take<int32_t>(S.oc_ch.size());
     L.oc_w = c.take<double>(S.oc_w.size());
     L.terms = c.take<double>((size_t)cap * std::max<size_t>(1, S.lst_terms.size()));
+    L.lst_ptr = c.take<int32_t>((size_t)S.L + 1);
     L.clock = c.take<unsigned long long>(CLK_WORDS);
     L.t_tab = c.take<double>(amp_rows(S));
     L.acc_tab = c.take<double>((size_t)amp_rows(S) * S.objs.size() * S.n_cpo);
@@ -312,6 +314,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
         FDTD_HIP_TRY(up(L.ucls + (2 * moving_ahead(S) - 1) * moving_cells(S), S.mv_cls0.data(), S.mv_cls0.size()));
     }
     FDTD_HIP_TRY(up(L.gtab, S.gtab.data(), S.gtab.size() * 4));
+    FDTD_HIP_TRY(up(L.lst_ptr, S.lst_ptr.data(), S.lst_ptr.size() * sizeof(int32_t)));
     FDTD_HIP_TRY(up(L.slabs, S.slabs.data(), S.slabs.size() * sizeof(PmlSlab)));
     std::vector<PSrcDev> ps;
     for (const PSrcHost &h : S.psrc) {
@@ -396,6 +399,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
     D.T = (int)S.lst_terms.size();
     D.cap = cap;
     D.terms = L.terms;
+    D.lst_ptr = L.lst_ptr;
     D.clock = L.clock;
     D.n_obj = (int)S.objs.size();
     D.seven = S.sampling == FDTD_SAMPLE_SEVEN ? 1 : 0;
@@ -451,10 +455,20 @@ hipError_t DeviceScene::upload_grid(float *dst, const float *dense) const
                        (size_t)S.n[0] * S.n[1], hipMemcpyHostToDevice);
 }
 
-fdtd_status DeviceScene::read_series(long long ring_row, long long nrows, double *out) const
+fdtd_status DeviceScene::read_series(long long ring_row, long long nrows, double *out, const SeriesStage *stage, hipStream_t st) const
 {
     const size_t T = S.lst_terms.size();
     if (nrows <= 0 || S.L == 0) return FDTD_OK;
+    if (stage && stage->host && T > 0 && (size_t)S.L <= SeriesStage::DOUBLES) {
+        const long long most = (long long)(SeriesStage::DOUBLES / (size_t)S.L);
+        for (long long r = 0; r < nrows; r += most) {
+            const long long n = std::min(most, nrows - r);
+            FDTD_HIP_TRY(launch_sum_terms(dev.terms + (size_t)(ring_row + r) * T, (int)T, dev.lst_ptr, S.L, n, stage->host, st));
+            FDTD_HIP_TRY(hipStreamSynchronize(st));
+            std::memcpy(out + (size_t)r * S.L, stage->host, sizeof(double) * (size_t)n * S.L);
+        }
+        return FDTD_OK;
+    }
     std::vector<double> rows((size_t)nrows * T);
     if (T) FDTD_HIP_TRY(hipMemcpy(rows.data(), dev.terms + (size_t)ring_row * T, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
     for (long long r = 0; r < nrows; ++r) sum_terms(rows.data() + (size_t)r * T, out + (size_t)r * S.L);

@@ -40,6 +40,14 @@ struct SceneSetup;
 int default_tile_plan(const SceneSetup &S);
 
 // Device buffers and uploaded tables of one scene, all in one hipMalloc arena.
+// Pinned host memory that listener rows come over in.
+struct SeriesStage {
+    enum : size_t { DOUBLES = 32768 };
+    double *host = nullptr;
+    void open() { if (!host && hipHostMalloc(&host, sizeof(double) * DOUBLES) != hipSuccess) { (void)hipGetLastError(); host = nullptr; } }
+    void close() { if (host) (void)hipHostFree(host); host = nullptr; }
+};
+
 struct DeviceScene {
     SceneSetup S;
     int device = 0;
@@ -92,8 +100,10 @@ struct DeviceScene {
     void append_tiles(int scene_id, const TilePlan &plan, std::vector<TileDesc> &out, std::vector<TermRef> &terms) const;
     void assign_terms(int scene_id, size_t base, std::vector<TileDesc> &out, std::vector<TermRef> &terms) const;
     // Listener values of ring rows [ring_row, ring_row + nrows): FP64 [nrows][L],
-    // each the sum of the listener's terms in term order.
-    fdtd_status read_series(long long ring_row, long long nrows, double *out) const;
+    // each the sum of the listener's terms in term order; summed on st (idle) by
+    // way of `stage`, or, without one, on the host.
+    fdtd_status read_series(long long ring_row, long long nrows, double *out, const SeriesStage *stage = nullptr,
+                            hipStream_t st = nullptr) const;
     // the same of one row's terms
     void sum_terms(const double *row, double *out) const;
     bool needs_motion_kernel() const { return S.moving; }

@@ -147,6 +147,7 @@ struct SceneDev {
     // of its terms, formed when the rows are read out
     int T, cap;                 // terms per row, rows of the ring
     double *terms;              // [cap][T]
+    const int32_t *lst_ptr;     // [L + 1]: listener l's terms are [lst_ptr[l], lst_ptr[l + 1])
     double *tail;               // pinned host memory [T + 1], or null: the newest row and its step, after a step run by itself (STEP_ALONE)
     unsigned long long *clock;  // CLK_WORDS words
     int n_obj;
@@ -266,6 +267,9 @@ hipError_t launch_advance(const SceneDev *scenes, int nscenes, int n, hipStream_
 hipError_t launch_motion(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, int nsteps, hipStream_t s);
 // The zeroed and fresh cells of step clock + k, whose classes are there.
 hipError_t launch_fresh(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, hipStream_t s);
+// Sums of each listener's terms, in their order, for `rows` ring rows starting at
+// `terms`: out[row][listener], which may be pinned host memory.
+hipError_t launch_sum_terms(const double *terms, int T, const int32_t *lst_ptr, int L, long long rows, double *out, hipStream_t s);
 // Speaker sources, before the step kernels of step clock + k: the speakers'
 // S dt over each listed scene's speaker box.
 hipError_t launch_speaker(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, hipStream_t s);

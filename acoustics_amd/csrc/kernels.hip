@@ -1594,6 +1594,30 @@ hipError_t launch_speaker(const SceneDev *scenes, const MotionDesc *list, int n,
     return hipGetLastError();
 }
 
+// A listener's value is the sum of its terms, about eight: formed here, an eighth
+// of the ring crosses to the host, and it crosses while the sums are formed.
+// (1000 rows of 64 listeners: 0.40 ms copied and summed on the host, 0.05 here.)
+__global__ __launch_bounds__(256) void sum_terms_kernel(const double *__restrict__ terms, int T, const int32_t *__restrict__ lst_ptr,
+                                                        int L, long long n, double *__restrict__ out)
+{
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    const long long row = q / L;
+    const int l = (int)(q - row * L), end = gmem(lst_ptr)[l + 1];
+    const AS_GLOBAL double *t = gmem(terms) + (size_t)row * T;
+    double v = 0.0;
+    for (int e = gmem(lst_ptr)[l]; e < end; ++e) v += t[e];
+    gmem(out)[q] = v;
+}
+
+hipError_t launch_sum_terms(const double *terms, int T, const int32_t *lst_ptr, int L, long long rows, double *out, hipStream_t s)
+{
+    const long long n = rows * L;
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(sum_terms_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, terms, T, lst_ptr, L, n, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_motion(const SceneDev *scenes, const MotionDesc *list, int n, int max_cells, int k, int nsteps, hipStream_t s)
 {
     if (n <= 0 || max_cells <= 0) return hipSuccess;

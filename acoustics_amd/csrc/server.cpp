@@ -80,6 +80,7 @@ struct fdtd_server {
     // rebuild needs no graph capture)
     StepProgram prog;
     ResidentProgram res_prog[RES_SHAPES];
+    SeriesStage stage;
     bool dirty = true;
     int block = 64;
 
@@ -184,6 +185,7 @@ fdtd_status fdtd_server::settle()
 void fdtd_server::run()
 {
     (void)hipSetDevice(device);
+    stage.open();
     for (;;) {
         std::vector<Request *> admit;
         {
@@ -274,7 +276,7 @@ void fdtd_server::run()
                         const int L = r->dev->S.L;
                         if (!check || !L) continue;
                         row.resize(L);
-                        fdtd_status s = r->dev->read_series(r->launched - 1, 1, row.data());
+                        fdtd_status s = r->dev->read_series(r->launched - 1, 1, row.data(), &stage, stream);
                         for (double v : row)
                             if (!std::isfinite(v)) { s = FDTD_ERR_NONFINITE; break; }
                         if (s != FDTD_OK) {
@@ -288,7 +290,7 @@ void fdtd_server::run()
                     const int L = r->dev->S.L;
                     r->result.resize((size_t)r->steps * L);
                     fdtd_status s = FDTD_OK;
-                    if (r->steps && L) s = r->dev->read_series(0, r->steps, r->result.data());
+                    if (r->steps && L) s = r->dev->read_series(0, r->steps, r->result.data(), &stage, stream);
                     for (double v : r->result)
                         if (!std::isfinite(v)) { s = FDTD_ERR_NONFINITE; break; }
                     finish(r, s);
@@ -317,6 +319,7 @@ void fdtd_server::run()
     (void)hipStreamSynchronize(stream);
     resident_forget_stream(stream);
     for (ResidentProgram &p : res_prog) p.release();
+    stage.close();
     std::lock_guard<std::mutex> lk(mu);
     for (Request *r : active) finish(r, FDTD_ERR_CANCELLED);
     active.clear();

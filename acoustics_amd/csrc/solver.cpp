@@ -35,6 +35,7 @@ struct fdtd_handle {
     long long flushed = 0;       // listener rows copied to host_series
     std::vector<double> host_series;
     double *tail = nullptr;     // SceneDev::tail
+    SeriesStage stage;
     int timing = 0;             // FDTD_TIMING_*
     std::vector<hipEvent_t> ev;  // [2*i] begin, [2*i+1] end of step kernel i
     hipEvent_t call_begin = nullptr, call_end = nullptr;
@@ -134,6 +135,7 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
     int cap = opt.series_capacity > 0 ? opt.series_capacity : 1024;
     cap = std::max(cap, h->graph_steps + 1);
     st = h->D.allocate_and_upload(h->stream, cap, LLONG_MAX);
+    if (st == FDTD_OK && h->D.S.L > 0) h->stage.open();
     if (st == FDTD_OK && h->D.S.L > 0 && h->D.S.lst_terms.size() <= TAIL_TERMS) {
         const size_t T = h->D.S.lst_terms.size();
         if (hipHostMalloc(&h->tail, sizeof(double) * (T + 1)) == hipSuccess) forget_tail(h.get());
@@ -157,6 +159,7 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
         h->prog.release();
         h->D.release();
         if (h->tail) (void)hipHostFree(h->tail);
+        h->stage.close();
         if (h->own_stream) (void)hipStreamDestroy(h->stream);
         return st;
     }
@@ -184,6 +187,7 @@ fdtd_status fdtd_destroy(fdtd_handle *h)
     h->prog.release();
     h->D.release();
     if (h->tail) (void)hipHostFree(h->tail);
+    h->stage.close();
     if (h->own_stream) (void)hipStreamDestroy(h->stream);
     delete h;
     return FDTD_OK;
@@ -238,7 +242,7 @@ static fdtd_status flush_series(fdtd_handle *h)
     while (r < h->step) {
         const long long ring = r % cap;
         const long long n = std::min<long long>(h->step - r, cap - ring);
-        fdtd_status st = h->D.read_series(ring, n, h->host_series.data() + old + (size_t)(r - h->flushed) * L);
+        fdtd_status st = h->D.read_series(ring, n, h->host_series.data() + old + (size_t)(r - h->flushed) * L, &h->stage, h->stream);
         if (st != FDTD_OK) return st;
         r += n;
     }

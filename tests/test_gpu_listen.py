@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from acoustics_amd import capi, scenes
-from acoustics_amd.solver import Solver
+from acoustics_amd.solver import Batch, Solver
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +32,22 @@ def test_single_steps_and_blocks(hip_lib, n_listeners):
             at += n
             assert np.array_equal(s.listen(), want[at - 1])
         assert np.array_equal(s.series(), want)
+
+
+@pytest.mark.parametrize("n_listeners", [1, 77, 256])
+def test_rows_read_in_pieces(hip_lib, n_listeners):
+    """More rows than come over at once, summed on the device, against rows summed one by one on the host."""
+    sb = scene(n_listeners)
+    with Solver(sb) as s:
+        s.step(500)
+        got = s.series()
+    with Solver(sb, series_capacity=64) as s:
+        for k in range(500):
+            s.step(1)
+            assert np.array_equal(s.listen(), got[k])
+    with Batch([sb, sb], [500, 333]) as b:
+        b.run()
+        assert np.array_equal(b.series(0), got) and np.array_equal(b.series(1), got[:333])
 
 
 @pytest.mark.parametrize("kw", [dict(), dict(tile_config=3), dict(steps_per_graph=8)])
