@@ -122,6 +122,14 @@ struct PmlSlab {
     int64_t v_base[3];
 };
 
+// Cells up to which the staggered scheme keeps increments in place of its face
+// velocities.  Such grids are held on the chip, where the state's size decides
+// (150x97x133 32 us per step with velocities, 7.0).  By step kernels the smaller
+// state is faster too (256^3 169 -> 90 us), but a large grid's short pulse
+// leaves it: what its listeners then hear, 1e-4 of the pulse, is the rounding
+// of either form (1e-3 of itself from 64 bits), and the scheme's own form stays.
+constexpr int64_t STAG_MERGED_CELLS = 3000000;
+
 struct SceneSetup {
     int n[3] = {0, 0, 0};
     int64_t N = 0;

@@ -124,7 +124,7 @@ bool axis_plain(const SceneSetup &s, int d, int i)
 void set_pml_state(SceneSetup &s, bool merged)
 {
     s.n_pml_merged = 0;
-    s.stag_merged = merged && s.scheme == FDTD_SCHEME_STAGGERED && !s.base_slabs.empty();
+    s.stag_merged = merged && s.scheme == FDTD_SCHEME_STAGGERED && !s.base_slabs.empty() && s.N <= STAG_MERGED_CELLS;
     for (int d = 0; d < 3 && s.stag_merged; ++d)
         for (int i = s.inner_lo[d]; i < s.inner_hi[d]; ++i)
             s.stag_merged = s.stag_merged && axis_plain(s, d, i) && s.sig0[d][i];

@@ -338,11 +338,11 @@ typedef struct fdtd_handle fdtd_handle;
  *   p^{n+1} = p^n + (pDir_A^{n+1} - pDir_A^n) + d^{n+1}
  * (32 B per such cell and step instead of 56).  Snapshots need SPLIT (they
  * write every pDir_d and velocity).  MERGED also applies to the staggered
- * scheme: its PML cells merge the same way, and a cell outside the PML keeps
- * the increment of its pressure instead of three face velocities (16 B instead
- * of 32).  A staggered handle's first snapshot, saved or loaded, takes it to
- * SPLIT for good: the steps so far are run again, so that the files hold every
- * velocity. */
+ * scheme on grids of up to 3 million cells: its PML cells merge the same way,
+ * and a cell outside the PML keeps the increment of its pressure instead of
+ * three face velocities (16 B instead of 32).  Such a handle's first snapshot,
+ * saved or loaded, takes it to SPLIT for good: the steps so far are run again,
+ * so that the files hold every velocity.  Larger staggered grids are SPLIT. */
 enum {
     FDTD_PML_STATE_MERGED = 0,
     FDTD_PML_STATE_SPLIT  = 1
