@@ -359,7 +359,7 @@ fdtd_status DeviceScene::place(hipStream_t st, int cap, long long target_steps, 
     D.sx = S.n[1] * sy_dev;
     D.raster = S.boundary == FDTD_BOUNDARY_RASTERIZE ? 1 : 0;
     D.scheme = S.scheme;
-    D.mac = S.mac() ? 1 : 0;
+    D.mac = S.mac() ? (S.N > MAC_STREAM_CELLS ? 2 : 1) : 0;
     D.inc = L.inc;
     D.npad = npad;
     D.field = L.field;

@@ -130,6 +130,14 @@ struct PmlSlab {
 // of either form (1e-3 of itself from 64 bits), and the scheme's own form stays.
 constexpr int64_t STAG_MERGED_CELLS = 3000000;
 
+// Cells from which such a grid's rows are written past the caches: its two
+// buffers of velocities and two slots of pressure, 32 B per cell, then no longer
+// fit the Infinity Cache (256 MiB), and lines left there push out what the
+// step still reads.  us per step, cached and streamed: 160^3 38.6 and 56.9, 200^3
+// 91.4 and 97.0, 210^3 112.1 and 108.6, 220^3 130.8 and 121.3, 256^3 168 and 154,
+// 300x280x310 312.8 and 280.8.
+constexpr int64_t MAC_STREAM_CELLS = 9000000;
+
 struct SceneSetup {
     int n[3] = {0, 0, 0};
     int64_t N = 0;

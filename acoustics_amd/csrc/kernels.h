@@ -107,7 +107,7 @@ struct SceneDev {
     int sx, sy;                 // strides of i and j (k fastest)
     int raster;                 // 1: rasterized ghost values, 0: fully coupled
     int scheme;                 // FDTD_SCHEME_*
-    int mac;                    // staggered scheme with a velocity on every face of the grid
+    int mac;                    // staggered scheme with a velocity on every face of the grid (2: over MAC_STREAM_CELLS)
     float *inc;                 // staggered scheme, merged: the increment d per cell (null otherwise)
     long long npad;             // floats per pressure slot
     float *field;               // NUM_P_SLOTS pressure slots, full grid, k fastest

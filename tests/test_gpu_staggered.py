@@ -67,3 +67,21 @@ def test_staggered_float4_rows_carry_listeners(hip_lib):
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
     assert rel_l2(outs[0], ref) <= TOL
+
+
+def test_rows_past_the_caches(hip_lib):
+    """A grid of just over nine million cells, whose float4 rows are stored past
+    the caches: ragged rows, the same bits as the scalar tiles, fused or not."""
+    sb, _ = scenes.staggered_free_field(seed=10, div=(206, 211, 209), pml=6, n_listeners=8)
+    print(f"case: staggered rows past the caches divisions={sb.divisions}", flush=True)
+    base = None
+    for plan in (8, -1, 1, 3):
+        with Solver(sb, tile_config=plan) as s:
+            s.step(60)
+            out = (s.series(), s.pressure())
+        if base is None:
+            base = out
+            assert np.abs(out[1]).max() > 0
+        else:
+            assert np.array_equal(out[0], base[0]), plan
+            assert np.array_equal(out[1], base[1]), plan
