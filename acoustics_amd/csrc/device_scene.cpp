@@ -175,8 +175,9 @@ TilePlan tile_plan(int id)
 // of rows together (plans 0 and 1): per step 96^3 coupled 11.2 us against 12.8
 // with marches of 2 and 8 in four bands, 128^3 12.3 against 15.1, 200x210x190
 // 30.6 against 33.7, 256^3 70.7 against 73.4, 330x290x351 144.7 against 157; the
-// staggered scheme with its velocities 45.6, 167.9 and 312.7 at 180x170x190, 256^3
-// and 300x280x310 against 50.4, 172.7 and 323.3 with PML marches of 8.  A grid this
+// staggered scheme with its velocities (rows stored through the caches) 45.6, 167.9
+// and 312.7 at 180x170x190, 256^3 and 300x280x310 against 50.4, 172.7 and 323.3 with
+// PML marches of 8.  A grid this
 // small has too few tiles for that and takes marches of two (plan 10: 6.2 us at
 // 64^3 against 7.3; at 96^3 12.0, 11.2).
 // Without a PML two interior planes are better (101x100x98 6.8 us against 8.3,
