@@ -94,6 +94,25 @@ fdtd_status BatchRunner::list_resident(hipStream_t st)
     return FDTD_OK;
 }
 
+// Scenes that finish later return at once on their device clocks.
+fdtd_status BatchRunner::list_whole(hipStream_t st)
+{
+    std::vector<SceneDev> devs;
+    std::vector<TileDesc> tiles;
+    std::vector<TermRef> terms;
+    std::vector<MotionDesc> motion;
+    for (size_t i = 0; i < scenes.size(); ++i) {
+        if (!scenes[i] || done[i]) continue;
+        const int id = (int)devs.size();
+        devs.push_back(scenes[i]->dev);
+        scenes[i]->append_tiles(id, tile_plan(default_tile_plan(scenes[i]->S)), tiles, terms);
+        if (scenes[i]->needs_motion_kernel()) motion.push_back({id});
+    }
+    const fdtd_status s = whole.upload(devs, tiles, terms, st, true, motion);
+    whole_listed = s == FDTD_OK;
+    return s;
+}
+
 fdtd_status BatchRunner::settle(hipStream_t st)
 {
     FDTD_HIP_TRY(hipStreamSynchronize(st));
@@ -235,7 +254,17 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
             if (s != FDTD_OK) return s;
         }
         const int want = (int)std::min<long long>(left, remaining);
-        if (any_resident()) {
+        if (any_resident() && capturing(st)) {
+            if (!whole_listed) {
+                const fdtd_status s = list_whole(st);
+                if (s != FDTD_OK) return s;
+            }
+            const fdtd_status s = whole.enqueue(st, taken, want);
+            if (s != FDTD_OK) return s;
+            taken += want;
+            left -= want;
+            ++blocks;
+        } else if (any_resident()) {
             // the step kernels of the other scenes, then the block of the
             // resident ones, then every scene's clock
             const int blk = std::min(want, (int)AMP_ROWS);
@@ -420,8 +449,10 @@ static fdtd_status batch_fill(fdtd_batch *b, const fdtd_scene *scenes, const int
         R.done.push_back(num_steps[i] == 0);
     }
     if (opt.tile_config >= 0 && opt.tile_config < kNumTilePlans) { R.plan = opt.tile_config; return R.rebuild(b->stream); }
-    if (R.all_resident()) return R.rebuild(b->stream);   // no step kernel to tune
-    return R.autotune(b->stream);
+    // (no step kernel to tune where all are resident)
+    const fdtd_status st = R.all_resident() ? R.rebuild(b->stream) : R.autotune(b->stream);
+    // a caller's stream may be captured later, when nothing can be allocated
+    return st == FDTD_OK && opt.stream && R.any_resident() ? R.list_whole(b->stream) : st;
 }
 
 extern "C" {

@@ -36,6 +36,11 @@ struct BatchRunner {
     ResidentProgram res_prog[RES_SHAPES];
     SeriesStage stage;
     bool res_listed = false;
+    // every scene's step kernels, for steps enqueued while the stream is
+    // captured: a resident launch's tags are its own, and a replay would take
+    // the words of the replay before for its neighbours'
+    StepProgram whole;
+    bool whole_listed = false;
     int plan = 0;
     int graph_steps = 32;
     hipGraphExec_t exec = nullptr;
@@ -58,6 +63,7 @@ struct BatchRunner {
     }
     bool all_resident() const;
     fdtd_status list_resident(hipStream_t st);        // (re)builds the resident launches
+    fdtd_status list_whole(hipStream_t st);
     // Waits for the stream and completes blocks that a resident launch gave up.
     fdtd_status settle(hipStream_t st);
     void release_scenes()
@@ -69,6 +75,7 @@ struct BatchRunner {
             if (r) r->release();
         res.clear();
         for (ResidentProgram &p : res_prog) p.release();
+        whole.release();
         stage.close();
     }
     ~BatchRunner();

@@ -39,6 +39,13 @@ struct SceneSetup;
 // a grid of under 400,000 cells.  All three are one fused launch.
 int default_tile_plan(const SceneSetup &S);
 
+// Whether what is enqueued on a stream is being recorded in a graph.
+inline bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
+}
+
 // Device buffers and uploaded tables of one scene, all in one hipMalloc arena.
 // Pinned host memory that listener rows come over in.
 struct SeriesStage {

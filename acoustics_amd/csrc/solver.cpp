@@ -269,12 +269,6 @@ static fdtd_status build_graph(fdtd_handle *h)
 // stores the whole state.
 constexpr int kResidentSteps = 4;
 
-static bool capturing(hipStream_t st)
-{
-    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone;
-}
-
 // Brings the device clock up to the steps run one by one.
 static fdtd_status catch_up(fdtd_handle *h)
 {

@@ -1,0 +1,31 @@
+"""What the host enqueues, followed without a GPU: tests/host/host_runtime.cpp
+stands in for the HIP runtime under the built library, and checks each launch
+against the clocks, memory, streams and devices it is made for."""
+import os
+import subprocess
+
+import pytest
+
+from acoustics_amd import capi
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SCENARIOS = [
+    "batch_capture",   # a batch's blocks on a captured stream
+]
+
+
+@pytest.fixture(scope="session")
+def host_runtime(tmp_path_factory):
+    capi.load_library()
+    exe = str(tmp_path_factory.mktemp("host") / "host_runtime")
+    lib = os.path.join(ROOT, "acoustics_amd", "lib")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"),
+                    "-rdynamic", "-o", exe, os.path.join(ROOT, "tests", "host", "host_runtime.cpp"), "-L" + lib,
+                    "-lfdtd_acoustics", "-Wl,-rpath," + lib], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("name", SCENARIOS)
+def test_host_path(host_runtime, name):
+    r = subprocess.run([host_runtime, name], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
