@@ -188,6 +188,12 @@ int default_tile_plan(const SceneSetup &S)
     return S.N < 400000 ? 10 : 0;
 }
 
+size_t DeviceScene::floats_of(const SceneSetup &S)
+{
+    size_t off[11];
+    return state_layout(S, slot_cells(S), off);
+}
+
 size_t DeviceScene::base_layout(size_t off[11]) const
 {
     SceneSetup old;

@@ -82,6 +82,8 @@ struct DeviceScene {
     fdtd_status place(hipStream_t stream, int series_cap, long long target, char *state_base, char *table_base);
     void release();
     float *slot(int s) const { return dev.field + (size_t)s * (size_t)npad; }
+    // floats of a scene's state
+    static size_t floats_of(const SceneSetup &S);
     // offsets (pd at 1, vel at 4 + 3 buffer) and floats of the state were it stored by base_slabs
     size_t base_layout(size_t off[11]) const;
     // device index of a dense host cell index (k fastest, rows of n2)

@@ -747,12 +747,15 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
         return FDTD_ERR_UNSUPPORTED;
     }
     FDTD_HIP_TRY(hipSetDevice(h->D.device));
-    {
-        fdtd_status st = settle(h);
-        if (st == FDTD_OK) st = to_split_state(h, false);
-        if (st != FDTD_OK) return st;
+    fdtd_status st = settle(h);
+    if (st != FDTD_OK) return st;
+    // every file is read before the handle is touched: a load that fails leaves it as it is
+    SceneSetup split;
+    if (h->D.S.stag_merged) {
+        split = h->D.S;
+        set_pml_state(split, false);
     }
-    const SceneSetup &S = h->D.S;
+    const SceneSetup &S = h->D.S.stag_merged ? split : h->D.S;
     const long long N = S.N;
     const bool mac = S.scheme == FDTD_SCHEME_STAGGERED;
     const bool merged = S.n_pml_merged > 0;
@@ -763,7 +766,7 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
         size_t off[11];
         if (is && is.read(reinterpret_cast<char *>(&hd), sizeof hd) && std::memcmp(hd.magic, kStateMagic, 8) == 0 &&
             (hd.version == 1 || hd.version == 2) && hd.n_cells == N && hd.scheme == S.scheme &&
-            hd.state_floats == (int64_t)(merged && hd.version == 1 ? h->D.base_layout(off) : h->D.state_floats) &&
+            hd.state_floats == (int64_t)(merged && hd.version == 1 ? h->D.base_layout(off) : DeviceScene::floats_of(S)) &&
             hd.npad == h->D.npad && hd.pml_state == (merged ? FDTD_PML_STATE_MERGED : FDTD_PML_STATE_SPLIT) && hd.step >= 0) {
             std::vector<float> raw(hd.state_floats);
             if (!is.read(reinterpret_cast<char *>(raw.data()), (std::streamsize)(raw.size() * 4))) {
@@ -771,6 +774,7 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
                 return FDTD_ERR_INVALID;
             }
             if (merged && hd.version == 1) raw = by_boxes(h->D, raw);
+            if ((st = to_split_state(h, false)) != FDTD_OK) return st;
             FDTD_HIP_TRY(hipMemcpy(h->D.dev.field, raw.data(), raw.size() * 4, hipMemcpyHostToDevice));
             return resume_at(h, hd.step);
         }
@@ -796,7 +800,6 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
         }
     }
     std::vector<double> cur, prev;
-    fdtd_status st;
     if (mac) {
         if ((st = read_matrix(snap_name(pattern, simulator_id, numbering, "p_pml_full.dat"), N, 1, cur)) != FDTD_OK) return st;
         prev.assign(N, 0.0);
@@ -809,14 +812,6 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
     // the Engquist boundary keeps p^{n-1} of each face cell's inner neighbour
     // at the face cell's exterior cell of the current slot
     abc_pack_state(S, prev.data(), cur.data());
-    // the whole state starts from zero: faces and cells the snapshot does not hold stay at rest
-    FDTD_HIP_TRY(h->D.zero_state(h->stream));
-    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
-    std::vector<float> f(N);
-    for (long long c = 0; c < N; ++c) f[c] = (float)cur[c];
-    FDTD_HIP_TRY(h->D.upload_grid(h->D.slot(slot_cur(s)), f.data()));
-    for (long long c = 0; c < N; ++c) f[c] = (float)prev[c];
-    FDTD_HIP_TRY(h->D.upload_grid(h->D.slot(slot_next(s)), f.data()));
     std::vector<double> pml[3], vel[3];
     for (int d = 0; d < 3; ++d)
         if ((st = read_matrix(snap_name(pattern, simulator_id, numbering, "p_pml_" + std::to_string(d) + ".dat"), N, 1, pml[d])) != FDTD_OK)
@@ -856,6 +851,16 @@ fdtd_status fdtd_load_snapshot(fdtd_handle *h, const char *pattern, const char *
                     }
                     comp[lower][c] = (float)dd;
                 }
+    // (the scene is in the state that S describes from here on)
+    if ((st = to_split_state(h, false)) != FDTD_OK) return st;
+    // the whole state starts from zero: faces and cells the snapshot does not hold stay at rest
+    FDTD_HIP_TRY(h->D.zero_state(h->stream));
+    FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    std::vector<float> f(N);
+    for (long long c = 0; c < N; ++c) f[c] = (float)cur[c];
+    FDTD_HIP_TRY(h->D.upload_grid(h->D.slot(slot_cur(s)), f.data()));
+    for (long long c = 0; c < N; ++c) f[c] = (float)prev[c];
+    FDTD_HIP_TRY(h->D.upload_grid(h->D.slot(slot_next(s)), f.data()));
     for (int d = 0; d < 3; ++d)
         if (S.n_pml) FDTD_HIP_TRY(hipMemcpy(h->D.dev.pd[d], comp[d].data(), S.n_pml * 4, hipMemcpyHostToDevice));
     const int vb = (int)(s & 1);

@@ -420,9 +420,29 @@ void batch_capture()
     fdtd_batch_destroy(h);
 }
 
+// A load that finds no files leaves a staggered handle where it is.
+void failed_load()
+{
+    Scene a(48, 40, 44, 6, FDTD_SCHEME_STAGGERED);
+    fdtd_handle *h = nullptr;
+    CHECK(fdtd_create(&a.sc, nullptr, &h) == FDTD_OK);
+    CHECK(fdtd_step(h, 100) == FDTD_OK);
+    CHECK(count("resident") == 1);
+    const size_t held = g_mem.size();
+    CHECK(fdtd_load_snapshot(h, "/nonexistent/%s", "0", 1) == FDTD_ERR_INVALID);
+    CHECK(g_mem.size() == held);
+    CHECK(fdtd_step(h, 40) == FDTD_OK);
+    CHECK(count("resident") == 2);
+    CHECK(clocks() == std::vector<long long>{140});
+    double p[2];
+    CHECK(fdtd_listen(h, p) == FDTD_OK);
+    fdtd_destroy(h);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
+    {"failed_load", failed_load},
 };
 
 }  // namespace

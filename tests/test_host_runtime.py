@@ -11,6 +11,7 @@ from acoustics_amd import capi
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SCENARIOS = [
     "batch_capture",   # a batch's blocks on a captured stream
+    "failed_load",     # a snapshot that is not there
 ]
 
 
