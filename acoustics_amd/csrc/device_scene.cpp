@@ -467,6 +467,10 @@ fdtd_status DeviceScene::read_series(long long ring_row, long long nrows, double
 {
     const size_t T = S.lst_terms.size();
     if (nrows <= 0 || S.L == 0) return FDTD_OK;
+    if (ring_row < 0 || ring_row + nrows > series_cap) {
+        set_last_error("listener rows outside the series ring");
+        return FDTD_ERR_INVALID;
+    }
     if (stage && stage->host && T > 0 && (size_t)S.L <= SeriesStage::DOUBLES) {
         const long long most = (long long)(SeriesStage::DOUBLES / (size_t)S.L);
         for (long long r = 0; r < nrows; r += most) {

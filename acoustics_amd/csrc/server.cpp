@@ -274,7 +274,8 @@ void fdtd_server::run()
                     r->launched += block;
                     if (r->launched < r->steps) {
                         const int L = r->dev->S.L;
-                        if (!check || !L) continue;
+                        // (none yet after a first block that was given up)
+                        if (!check || !L || r->launched <= 0) continue;
                         row.resize(L);
                         fdtd_status s = r->dev->read_series(r->launched - 1, 1, row.data(), &stage, stream);
                         for (double v : row)

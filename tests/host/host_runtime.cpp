@@ -245,7 +245,11 @@ hipError_t hipFree(void *p)
 {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
     if (!p) return hipSuccess;
-    if (!g_mem.erase((char *)p)) bad("hipFree of memory that is not there");
+    auto it = g_mem.find((char *)p);
+    if (it == g_mem.end()) { bad("hipFree of memory that is not there"); return hipErrorInvalidValue; }
+    for (auto s = g_scenes.begin(); s != g_scenes.end();)
+        s = (char *)s->first >= it->first && (char *)s->first < it->first + it->second.n ? g_scenes.erase(s) : std::next(s);
+    g_mem.erase(it);
     std::free(p);
     return hipSuccess;
 }
@@ -439,10 +443,38 @@ void failed_load()
     fdtd_destroy(h);
 }
 
+// A request whose first block is given up and falls on a finiteness check has no row to check yet.
+void server_check()
+{
+    Scene a(40, 40, 40, 6), b(44, 40, 40, 6);
+    fdtd_server_options o;
+    fdtd_server_options_default(&o);
+    o.steps_per_block = 8;
+    fdtd_server *s = nullptr;
+    CHECK(fdtd_server_create(&o, &s) == FDTD_OK);
+    g_gives_up = [](const SceneDev &S) { return S.clock[CLK_TARGET] == 83 && S.clock[CLK_STEP] == 0; };
+    int64_t id[2];
+    const int steps[2] = {15 * 8, 83};   // the second one's first block is the sixteenth
+    const Scene *sc[2] = {&a, &b};
+    for (int q = 0; q < 2; ++q) {
+        CHECK(fdtd_server_submit(s, &sc[q]->sc, steps[q], &id[q]) == FDTD_OK);
+        CHECK(fdtd_server_wait(s, id[q], 60000) == FDTD_OK);
+        std::vector<double> out(2 * (size_t)steps[q]);
+        double ms;
+        CHECK(fdtd_server_take_result(s, id[q], out.data(), &ms) == FDTD_OK);
+    }
+    fdtd_server_stats st;
+    CHECK(fdtd_server_get_stats(s, &st) == FDTD_OK && st.completed == 2 && st.blocks_run >= 26);
+    CHECK(count("resident") == 16);
+    CHECK(count("step") >= 83);
+    fdtd_server_destroy(s);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
     {"failed_load", failed_load},
+    {"server_check", server_check},
 };
 
 }  // namespace

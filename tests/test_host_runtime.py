@@ -12,6 +12,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SCENARIOS = [
     "batch_capture",   # a batch's blocks on a captured stream
     "failed_load",     # a snapshot that is not there
+    "server_check",    # a request given up before its first row, on a finiteness check
 ]
 
 
