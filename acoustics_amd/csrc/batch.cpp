@@ -39,11 +39,11 @@ fdtd_status BatchRunner::rebuild(hipStream_t st)
     }
     prog_tiles = tiles.size();
     dead_tiles = 0;
-    if (devs.empty()) { prog.release(); return FDTD_OK; }
     if (!res_listed) {
         const fdtd_status s = list_resident(st);
         if (s != FDTD_OK) return s;
     }
+    if (devs.empty()) { prog.release(); return FDTD_OK; }
     const bool fused = tile_plan(plan).fused;
     size_t npre = motion.size();
     for (const SceneDev &d : devs) npre += d.n_spk ? 1 : 0;
@@ -80,13 +80,16 @@ bool BatchRunner::all_resident() const
 }
 
 // A finished scene's workgroups return at once on its device clock, so the
-// launches keep their lists until a scene leaves the resident set.
+// launches keep their lists until a scene leaves the resident set or is stopped
+// by the host, whose device clock would let it run: nothing moves its clock on or
+// shuts its gate any more, and a launch that finds the gate open does not wait
+// for its neighbours to be there.
 fdtd_status BatchRunner::list_resident(hipStream_t st)
 {
     for (int shape = 0; shape < RES_SHAPES; ++shape) {
         std::vector<const ResidentScene *> list;
         for (size_t i = 0; i < scenes.size(); ++i)
-            if (scenes[i] && res[i] && res[i]->plan.shape == shape) list.push_back(res[i].get());
+            if (scenes[i] && !done[i] && res[i] && res[i]->plan.shape == shape) list.push_back(res[i].get());
         const fdtd_status s = res_prog[shape].upload(list, st);
         if (s != FDTD_OK) return s;
     }
@@ -128,7 +131,7 @@ fdtd_status BatchRunner::settle(hipStream_t st)
         long long at = 0;
         fdtd_status s = resident_reopen(D.dev, &at);
         if (s != FDTD_OK) return s;
-        const long long due = std::min<long long>(taken, D.target);
+        const long long due = std::min<long long>(taken, targets[i]);
         if (at >= due) continue;
         // the steps it lacks, and from now on all of its steps, by the step kernels
         std::vector<TileDesc> tiles;
@@ -249,6 +252,7 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
             remaining = std::max(remaining, targets[i] - taken);
         }
         if (remaining == 0) break;
+        if (cut) res_listed = whole_listed = false;
         if (cut || (dead_tiles > 0 && (double)dead_tiles >= kRebuildDeadShare * (double)prog_tiles)) {
             fdtd_status s = rebuild(st);
             if (s != FDTD_OK) return s;

@@ -470,11 +470,42 @@ void server_check()
     fdtd_server_destroy(s);
 }
 
+// A time chunk that is stopped early leaves the resident launches: its clock no
+// longer moves, so no launch may find its gate as the one before left it.
+void cut_chunk()
+{
+    Scene a(40, 40, 40, 6);
+    fdtd_settings &s = a.sc.settings;
+    s.time_parallel = 1;
+    s.num_time_chunks = 4;
+    const int64_t steps = 16000;            // chunks of 16000, 12000, 8000 and 4000 steps, sources in the first 4000
+    s.overlap_time = 12000.5 * s.time_step;
+    // the second one is quiet from step 4100 on, and stops 0.05 s (6000 steps) later
+    g_signal = [](const SceneDev &S, long long step) { return S.cap == 12000 && step > 4100 ? 0.0 : 1.0; };
+    std::vector<double> out((size_t)steps * 2);
+    int64_t run[4];
+    CHECK(fdtd_run_time_parallel(&a.sc, steps, nullptr, out.data(), run) == FDTD_OK);
+    CHECK(run[0] == 16000 && run[1] > 10050 && run[1] < 10150 && run[2] == 8000 && run[3] == 4000);
+    // one launch per block of 32 steps; the stopped chunk, and the finished ones,
+    // are in none after the block it was stopped in
+    std::map<const void *, int> launches;
+    for (const Call &c : g_log)
+        if (c.what == "resident scene") ++launches[c.scene];
+    CHECK(launches.size() == 4);
+    int all = 0;
+    for (const auto &e : launches) {
+        all += e.second == 500;
+        CHECK(e.second == 500 || e.second <= (run[1] + 31) / 32);
+    }
+    CHECK(all == 1);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
     {"failed_load", failed_load},
     {"server_check", server_check},
+    {"cut_chunk", cut_chunk},
 };
 
 }  // namespace

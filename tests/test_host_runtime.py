@@ -13,6 +13,7 @@ SCENARIOS = [
     "batch_capture",   # a batch's blocks on a captured stream
     "failed_load",     # a snapshot that is not there
     "server_check",    # a request given up before its first row, on a finiteness check
+    "cut_chunk",       # a time chunk stopped early
 ]
 
 
