@@ -21,6 +21,7 @@ namespace fdtd {
 fdtd_status BatchRunner::rebuild(hipStream_t st)
 {
     drop_graph();
+    listed = false;
     std::vector<SceneDev> devs;
     std::vector<TileDesc> tiles;
     std::vector<TermRef> terms;
@@ -43,7 +44,7 @@ fdtd_status BatchRunner::rebuild(hipStream_t st)
         const fdtd_status s = list_resident(st);
         if (s != FDTD_OK) return s;
     }
-    if (devs.empty()) { prog.release(); return FDTD_OK; }
+    if (devs.empty()) { prog.release(); listed = true; return FDTD_OK; }
     const bool fused = tile_plan(plan).fused;
     size_t npre = motion.size();
     for (const SceneDev &d : devs) npre += d.n_spk ? 1 : 0;
@@ -69,6 +70,7 @@ fdtd_status BatchRunner::rebuild(hipStream_t st)
     const fdtd_status s = prog.upload(devs, tiles, terms, st, fused, motion, pbuf[b], pbytes, pstage[b]);
     if (s != FDTD_OK) return s;
     FDTD_HIP_TRY(hipEventRecord(pdone[b], st));
+    listed = true;
     return FDTD_OK;
 }
 
@@ -125,6 +127,7 @@ fdtd_status BatchRunner::settle(hipStream_t st)
         gave_up = gave_up || p.gave_up();
     }
     if (!gave_up) return FDTD_OK;
+    res_listed = listed = false;   // (also where this ends early)
     for (size_t i = 0; i < scenes.size(); ++i) {
         if (!scenes[i] || !res[i]) continue;
         DeviceScene &D = *scenes[i];
@@ -148,7 +151,6 @@ fdtd_status BatchRunner::settle(hipStream_t st)
     }
     for (ResidentProgram &p : res_prog)
         if (p.trouble) *p.trouble = 0;
-    res_listed = false;
     return rebuild(st);
 }
 
@@ -253,7 +255,7 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
         }
         if (remaining == 0) break;
         if (cut) res_listed = whole_listed = false;
-        if (cut || (dead_tiles > 0 && (double)dead_tiles >= kRebuildDeadShare * (double)prog_tiles)) {
+        if (!listed || cut || (dead_tiles > 0 && (double)dead_tiles >= kRebuildDeadShare * (double)prog_tiles)) {
             fdtd_status s = rebuild(st);
             if (s != FDTD_OK) return s;
         }

@@ -41,6 +41,7 @@ struct BatchRunner {
     // the words of the replay before for its neighbours'
     StepProgram whole;
     bool whole_listed = false;
+    bool listed = false;                              // prog and the resident launches hold the scenes as they are
     int plan = 0;
     int graph_steps = 32;
     hipGraphExec_t exec = nullptr;

@@ -12,10 +12,12 @@
 
 namespace fdtd {
 
+// (the error is taken with it: left behind, it would be the next launch's)
 #define FDTD_HIP_TRY(expr)                                                     \
     do {                                                                       \
         hipError_t e_ = (expr);                                                \
         if (e_ != hipSuccess) {                                                \
+            (void)hipGetLastError();                                           \
             set_last_error(std::string(#expr) + ": " + hipGetErrorString(e_)); \
             return e_ == hipErrorOutOfMemory ? FDTD_ERR_OOM : FDTD_ERR_DEVICE; \
         }                                                                      \

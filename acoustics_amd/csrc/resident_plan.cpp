@@ -398,7 +398,6 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
             list.push_back(t < m ? ResItem{s->dev, s->plan.order[t], 0} : ResItem{nullptr, 0, 0});
         }
     }
-    n = (int)list.size();
     if (!trouble) {
         FDTD_HIP_TRY(hipHostMalloc(&trouble, sizeof(int)));
         *trouble = 0;
@@ -412,6 +411,7 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
     FDTD_HIP_TRY(hipMalloc(&items, sizeof(ResItem) * list.size()));
     FDTD_HIP_TRY(hipMemcpyAsync(items, list.data(), sizeof(ResItem) * list.size(), hipMemcpyHostToDevice, st));
     FDTD_HIP_TRY(hipStreamSynchronize(st));
+    n = (int)list.size();   // (nothing is launched before the list is there)
     return FDTD_OK;
 }
 

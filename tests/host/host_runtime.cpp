@@ -7,6 +7,7 @@
 // usage: host_runtime SCENARIO   (prints what went wrong; exit status 0 if nothing)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -500,12 +501,42 @@ void cut_chunk()
     CHECK(all == 1);
 }
 
+// Device memory that runs out while a batch lists its scenes anew: the call
+// fails, nothing is launched over lists that are not there, and the batch goes
+// on once there is memory.
+void no_memory_for_lists()
+{
+    Scene a(40, 40, 40, 6), b(44, 40, 40, 6), c(112, 120, 128, 8);   // the third one of another tile shape
+    for (int k = 0; k < 8; ++k) {
+        const fdtd_scene sc[3] = {a.sc, b.sc, c.sc};
+        const int steps[3] = {300, 301, 302};
+        fdtd_batch *h = nullptr;
+        CHECK(fdtd_batch_create(sc, steps, 3, nullptr, &h) == FDTD_OK);
+        g_gives_up = [](const SceneDev &S) { return S.clock[CLK_TARGET] == 301 || S.clock[CLK_TARGET] == 302; };
+        CHECK(fdtd_batch_step(h, 64) == FDTD_OK);
+        double row[302 * 2];
+        g_fail_malloc = k;
+        const fdtd_status st = fdtd_batch_read_listener_series(h, 0, row);
+        CHECK(st == FDTD_OK || st == FDTD_ERR_OOM);
+        if (st == FDTD_OK) CHECK(fdtd_batch_step(h, 64) == FDTD_OK);
+        else (void)fdtd_batch_step(h, 64);
+        g_fail_malloc = -1;
+        g_gives_up = [](const SceneDev &) { return false; };
+        CHECK(fdtd_batch_run(h) == FDTD_OK);
+        std::vector<long long> want{300, 301, 302}, got = clocks();
+        std::sort(got.begin(), got.end());
+        CHECK(got == want);
+        fdtd_batch_destroy(h);
+    }
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
     {"failed_load", failed_load},
     {"server_check", server_check},
     {"cut_chunk", cut_chunk},
+    {"no_memory_for_lists", no_memory_for_lists},
 };
 
 }  // namespace

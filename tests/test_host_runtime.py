@@ -14,6 +14,7 @@ SCENARIOS = [
     "failed_load",     # a snapshot that is not there
     "server_check",    # a request given up before its first row, on a finiteness check
     "cut_chunk",       # a time chunk stopped early
+    "no_memory_for_lists",   # no device memory while scenes are listed anew
 ]
 
 
