@@ -139,7 +139,7 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
     if (st == FDTD_OK && h->D.S.L > 0 && h->D.S.lst_terms.size() <= TAIL_TERMS) {
         const size_t T = h->D.S.lst_terms.size();
         if (hipHostMalloc(&h->tail, sizeof(double) * (T + 1)) == hipSuccess) forget_tail(h.get());
-        else h->tail = nullptr;   // (rows are then copied)
+        else { (void)hipGetLastError(); h->tail = nullptr; }   // (rows are then copied)
         h->D.dev.tail = h->tail;
     }
     if (st == FDTD_OK) {
@@ -151,8 +151,12 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
         st = h->prog.upload({h->D.dev}, tiles, terms, h->stream, tile_plan(h->tile).fused, motion);
     }
     // a tile plan or graph blocks that the caller asked for are what runs
-    if (st == FDTD_OK && opt.tile_config < 0 && h->graph_steps == 0 && h->res.build(h->D, h->stream))
-        st = h->res_prog.upload({&h->res}, h->stream);
+    if (st == FDTD_OK && opt.tile_config < 0 && h->graph_steps == 0 && h->res.build(h->D, h->stream) &&
+        h->res_prog.upload({&h->res}, h->stream) != FDTD_OK) {
+        // (no memory for its list: the step kernels run it all)
+        h->res_prog.release();
+        h->res.release();
+    }
     if (st != FDTD_OK) {
         h->res_prog.release();
         h->res.release();

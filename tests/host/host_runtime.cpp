@@ -530,6 +530,24 @@ void no_memory_for_lists()
     }
 }
 
+// Without pinned memory for the newest row and the read-out, rows are copied.
+void no_pinned_memory()
+{
+    for (int resident = 0; resident < 2; ++resident) {
+        Scene a(40, 40, 40, 6);
+        if (!resident) a.sc.settings.air_viscosity_alpha = 2e-6;
+        fdtd_handle *h = nullptr;
+        g_fail_pinned = true;
+        CHECK(fdtd_create(&a.sc, nullptr, &h) == FDTD_OK);
+        g_fail_pinned = false;
+        if (!h) continue;
+        CHECK(fdtd_step(h, 30) == FDTD_OK);
+        double p[2];
+        CHECK(fdtd_listen(h, p) == FDTD_OK);
+        fdtd_destroy(h);
+    }
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -537,6 +555,7 @@ const Scenario kScenarios[] = {
     {"server_check", server_check},
     {"cut_chunk", cut_chunk},
     {"no_memory_for_lists", no_memory_for_lists},
+    {"no_pinned_memory", no_pinned_memory},
 };
 
 }  // namespace

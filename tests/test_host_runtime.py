@@ -15,6 +15,7 @@ SCENARIOS = [
     "server_check",    # a request given up before its first row, on a finiteness check
     "cut_chunk",       # a time chunk stopped early
     "no_memory_for_lists",   # no device memory while scenes are listed anew
+    "no_pinned_memory",      # nor pinned memory for listener rows
 ]
 
 
