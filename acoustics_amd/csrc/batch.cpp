@@ -515,6 +515,7 @@ fdtd_status fdtd_batch_steps_done(fdtd_batch *b, int scene, int64_t *steps)
 fdtd_status fdtd_batch_read_listener_series(fdtd_batch *b, int scene, double *out)
 {
     if (!b || scene < 0 || scene >= (int)b->R.scenes.size()) return FDTD_ERR_INVALID;
+    const OnDevice on(b->device);
     const fdtd_status s = b->R.settle(b->stream);
     if (s != FDTD_OK) return s;
     b->R.reap();

@@ -23,6 +23,20 @@ namespace fdtd {
         }                                                                      \
     } while (0)
 
+// Selects a device for a call that only reads, which may launch and allocate, and
+// leaves the caller's selected afterwards.
+struct OnDevice {
+    int was = -1;
+    explicit OnDevice(int dev)
+    {
+        if (hipGetDevice(&was) == hipSuccess && was == dev) was = -1;
+        else (void)hipSetDevice(dev);
+    }
+    ~OnDevice() { if (was >= 0) (void)hipSetDevice(was); }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+};
+
 // Tile shapes of one plan (chosen by the autotuner).
 struct TilePlan {
     int interior_tk_log2 = 6;  // 64 threads along k, 4 rows along j

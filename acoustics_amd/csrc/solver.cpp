@@ -360,6 +360,7 @@ fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
 fdtd_status fdtd_synchronize(fdtd_handle *h)
 {
     if (!h) return FDTD_ERR_INVALID;
+    const OnDevice on(h->D.device);
     return settle(h);
 }
 
@@ -397,6 +398,7 @@ fdtd_status fdtd_listen(fdtd_handle *h, double *out)
 {
     if (!h || (!out && h->D.S.L)) return FDTD_ERR_INVALID;
     if (h->step == 0) { std::fill(out, out + h->D.S.L, 0.0); return FDTD_OK; }
+    const OnDevice on(h->D.device);
     fdtd_status st = flush_series(h);
     if (st != FDTD_OK) return st;
     const int L = h->D.S.L;
@@ -409,6 +411,7 @@ fdtd_status fdtd_listen(fdtd_handle *h, double *out)
 fdtd_status fdtd_read_listener_series(fdtd_handle *h, int64_t first, int64_t n, double *out)
 {
     if (!h || first < 0 || n < 0 || first + n > h->step) { set_last_error("rows out of range"); return FDTD_ERR_INVALID; }
+    const OnDevice on(h->D.device);
     fdtd_status st = flush_series(h);
     if (st != FDTD_OK) return st;
     const int L = h->D.S.L;
@@ -419,6 +422,7 @@ fdtd_status fdtd_read_listener_series(fdtd_handle *h, int64_t first, int64_t n, 
 fdtd_status fdtd_read_pressure(fdtd_handle *h, double *out)
 {
     if (!h || !out) return FDTD_ERR_INVALID;
+    const OnDevice on(h->D.device);
     const fdtd_status st = settle(h);
     if (st != FDTD_OK) return st;
     const int slot = slot_cur(h->step);  // p^{step}: the newest field

@@ -548,6 +548,42 @@ void no_pinned_memory()
     }
 }
 
+// What reads a handle or batch of device 1 while device 0 is selected launches
+// and allocates on device 1, and leaves device 0 selected.
+void other_device()
+{
+    Scene a(40, 40, 40, 6), b(44, 40, 40, 6);
+    g_gives_up = [](const SceneDev &S) { return S.clock[CLK_TARGET] == 301; };
+    for (int gives_up = 0; gives_up < 2; ++gives_up) {
+        if (gives_up) g_gives_up = [](const SceneDev &) { return true; };
+        fdtd_options o;
+        fdtd_options_default(&o);
+        o.device = 1;
+        std::vector<double> out(64000);
+        for (int call = 0; call < 4; ++call) {
+            fdtd_handle *h = nullptr;
+            CHECK(fdtd_create(&a.sc, &o, &h) == FDTD_OK);
+            CHECK(fdtd_step(h, 64) == FDTD_OK);
+            t_dev = 0;
+            CHECK((call == 0 ? fdtd_listen(h, out.data()) : call == 1 ? fdtd_read_listener_series(h, 0, 64, out.data()) :
+                   call == 2 ? fdtd_read_pressure(h, out.data()) : fdtd_synchronize(h)) == FDTD_OK);
+            CHECK(t_dev == 0);
+            CHECK(fdtd_destroy(h) == FDTD_OK);
+        }
+        const fdtd_scene sc[2] = {a.sc, b.sc};
+        const int steps[2] = {300, 301};
+        fdtd_batch *h = nullptr;
+        t_dev = 1;
+        CHECK(fdtd_batch_create(sc, steps, 2, nullptr, &h) == FDTD_OK);
+        CHECK(fdtd_batch_step(h, 64) == FDTD_OK);
+        t_dev = 0;
+        CHECK(fdtd_batch_read_listener_series(h, 0, out.data()) == FDTD_OK);
+        CHECK(t_dev == 0);
+        for (const auto &e : g_mem) CHECK(e.second.dev == 1);
+        CHECK(fdtd_batch_destroy(h) == FDTD_OK);
+    }
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -556,6 +592,7 @@ const Scenario kScenarios[] = {
     {"cut_chunk", cut_chunk},
     {"no_memory_for_lists", no_memory_for_lists},
     {"no_pinned_memory", no_pinned_memory},
+    {"other_device", other_device},
 };
 
 }  // namespace

@@ -16,6 +16,7 @@ SCENARIOS = [
     "cut_chunk",       # a time chunk stopped early
     "no_memory_for_lists",   # no device memory while scenes are listed anew
     "no_pinned_memory",      # nor pinned memory for listener rows
+    "other_device",          # reads while another device is selected
 ]
 
 
