@@ -434,6 +434,7 @@ static fdtd_status batch_fill(fdtd_batch *b, const fdtd_scene *scenes, const int
     else { FDTD_HIP_TRY(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)); b->own_stream = true; }
     BatchRunner &R = b->R;
     R.graph_steps = std::max(0, opt.steps_per_graph);
+    for (ResidentProgram &p : R.res_prog) p.callers_stream = !b->own_stream;
     for (int i = 0; i < n; ++i) {
         if (num_steps[i] < 0) { set_last_error("negative step count"); return FDTD_ERR_INVALID; }
         auto ds = std::make_unique<DeviceScene>();

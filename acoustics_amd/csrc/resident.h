@@ -133,6 +133,7 @@ struct ResidentProgram {
     uint32_t tag = 1;
     int *trouble = nullptr;     // pinned host memory: see launch_resident
     int wait_limit = 0;
+    bool callers_stream = false;   // the stream may be captured between launches
     // Scenes of one shape.  They are listed so that their workgroups fill the
     // device side by side; a scene's start at a multiple of eight and follow
     // each other within an XCD.
@@ -157,7 +158,8 @@ hipError_t launch_resident_routes(const ResScene *scene, int ntiles, int shape, 
 // buffers.  wait_limit bounds the wait for the scene's other workgroups to be
 // dispatched; past it the scene gives the block up untouched, and every
 // later one, and `trouble` (host memory) becomes 1.  A later wait that does not end sets it to 2.
+// done: an event that the launch's end completes.
 hipError_t launch_resident(int shape, const ResItem *items, int n, int nsteps, uint32_t tag, int wait_limit,
-                           int *trouble, hipStream_t s);
+                           int *trouble, hipStream_t s, hipEvent_t done);
 
 }  // namespace fdtd

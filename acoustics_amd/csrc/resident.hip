@@ -24,6 +24,8 @@
 //   columns are 16-byte reads.
 #include <climits>
 
+#include <hip/hip_ext.h>
+
 #include "resident.h"
 #include "stencil.h"
 
@@ -1110,12 +1112,12 @@ hipError_t launch_resident_routes(const ResScene *scene, int ntiles, int shape, 
 }
 
 hipError_t launch_resident(int shape, const ResItem *items, int n, int nsteps, uint32_t tag, int wait_limit,
-                           int *trouble, hipStream_t s)
+                           int *trouble, hipStream_t s, hipEvent_t done)
 {
     if (n <= 0) return hipSuccess;
     const size_t bytes = lds_bytes(shape);
     with_shape(shape, [&](auto, auto k) {
-        hipLaunchKernelGGL(k, dim3(n), dim3(RES_THREADS), bytes, s, items, nsteps, tag, wait_limit, trouble);
+        hipExtLaunchKernelGGL(k, dim3(n), dim3(RES_THREADS), bytes, s, nullptr, done, 0, items, nsteps, tag, wait_limit, trouble);
         return 0;
     });
     return hipGetLastError();

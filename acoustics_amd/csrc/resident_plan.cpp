@@ -417,38 +417,29 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
 
 // Two resident launches on different streams could each hold a part of the
 // device and wait for the rest of it until both give up.  So launches of one
-// process follow each other on a device: a launch on another stream than the
-// one before waits for that stream's work so far.
+// process follow each other on a device: each leaves an event, and one on another
+// stream waits for that.  The event is the launch's own completion (64^3, blocks
+// of 4 steps: 27 us a block; recorded behind it 30, without one 26).  A caller's
+// stream may be under capture by then, where the runtime refuses to wait for its
+// earlier events, and touching one spoils the capture: a stream that nobody else
+// knows waits for a launch on such a stream at once, and leaves the event.
 namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_order;
-hipStream_t g_last[kMaxDevices] = {};
-bool g_used[kMaxDevices] = {};
+struct Last {
+    hipEvent_t done = nullptr;      // left on `stream`, or, if that is a caller's, on relay
+    hipEvent_t handed = nullptr;    // from a caller's stream to relay
+    hipStream_t relay = nullptr;
+    hipStream_t stream = nullptr;
+    bool used = false;
+} g_last[kMaxDevices];
 }  // namespace
-
-static fdtd_status follow_last(hipStream_t st)
-{
-    int dev = 0;
-    FDTD_HIP_TRY(hipGetDevice(&dev));
-    if (dev < 0 || dev >= kMaxDevices) return FDTD_ERR_DEVICE;
-    if (g_used[dev] && g_last[dev] != st) {
-        hipEvent_t e;
-        FDTD_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        hipError_t r = hipEventRecord(e, g_last[dev]);
-        if (r == hipSuccess) r = hipStreamWaitEvent(st, e, 0);
-        (void)hipEventDestroy(e);
-        FDTD_HIP_TRY(r);
-    }
-    g_used[dev] = true;
-    g_last[dev] = st;
-    return FDTD_OK;
-}
 
 void resident_forget_stream(hipStream_t st)
 {
     std::lock_guard<std::mutex> lk(g_order);
-    for (int d = 0; d < kMaxDevices; ++d)
-        if (g_used[d] && g_last[d] == st) g_used[d] = false;
+    for (Last &l : g_last)
+        if (l.used && l.stream == st) l.used = false;
 }
 
 fdtd_status resident_reopen(const SceneDev &dev, long long *step)
@@ -466,11 +457,26 @@ fdtd_status resident_reopen(const SceneDev &dev, long long *step)
 
 fdtd_status ResidentProgram::enqueue(hipStream_t st, int nsteps)
 {
+    if (n <= 0) return FDTD_OK;
     std::lock_guard<std::mutex> lk(g_order);
-    const fdtd_status s = follow_last(st);
-    if (s != FDTD_OK) return s;
-    FDTD_HIP_TRY(launch_resident(shape, items, n, nsteps, tag, wait_limit, trouble, st));
+    int dev = 0;
+    FDTD_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices) return FDTD_ERR_DEVICE;
+    Last &last = g_last[dev];
+    if (!last.done) {
+        FDTD_HIP_TRY(hipEventCreateWithFlags(&last.handed, hipEventDisableTiming));
+        FDTD_HIP_TRY(hipStreamCreateWithFlags(&last.relay, hipStreamNonBlocking));
+        FDTD_HIP_TRY(hipEventCreateWithFlags(&last.done, hipEventDisableTiming));
+    }
+    if (last.used && last.stream != st) FDTD_HIP_TRY(hipStreamWaitEvent(st, last.done, 0));
+    FDTD_HIP_TRY(launch_resident(shape, items, n, nsteps, tag, wait_limit, trouble, st, callers_stream ? last.handed : last.done));
     tag += (uint32_t)nsteps + 1;
+    if (callers_stream) {
+        FDTD_HIP_TRY(hipStreamWaitEvent(last.relay, last.handed, 0));
+        FDTD_HIP_TRY(hipEventRecord(last.done, last.relay));
+    }
+    last.stream = st;
+    last.used = true;
     return FDTD_OK;
 }
 

@@ -150,6 +150,7 @@ fdtd_status fdtd_create(const fdtd_scene *scene, const fdtd_options *opt_in, fdt
         if (h->D.needs_motion_kernel()) motion.push_back({0});
         st = h->prog.upload({h->D.dev}, tiles, terms, h->stream, tile_plan(h->tile).fused, motion);
     }
+    h->res_prog.callers_stream = !h->own_stream;
     // a tile plan or graph blocks that the caller asked for are what runs
     if (st == FDTD_OK && opt.tile_config < 0 && h->graph_steps == 0 && h->res.build(h->D, h->stream) &&
         h->res_prog.upload({&h->res}, h->stream) != FDTD_OK) {

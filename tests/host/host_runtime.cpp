@@ -221,6 +221,13 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **a, size_t, hipStr
     return hipSuccess;
 }
 
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s);
+hipError_t hipExtLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t m, hipStream_t st, hipEvent_t, hipEvent_t stop, int)
+{
+    const hipError_t r = hipLaunchKernel(f, g, b, a, m, st);
+    return r != hipSuccess || !stop ? r : hipEventRecord(stop, st);
+}
+
 hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
 hipError_t hipGetDevice(int *d) { *d = t_dev; return hipSuccess; }
 hipError_t hipSetDevice(int d) { t_dev = d; return hipSuccess; }
@@ -335,6 +342,8 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
 {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
+    const Stream *on = ((Event *)e)->on;
+    if (on && on->capturing && !stream_of(s)->capturing) bad("a wait for an event of a stream under capture");
     g_log.push_back({"wait", stream_of(s), stream_of(s)->capturing, ((Event *)e)->on});
     return hipSuccess;
 }
@@ -584,6 +593,35 @@ void other_device()
     }
 }
 
+// Two handles whose blocks follow each other: the second one's waits for the
+// first one's, and nothing is enqueued for it on the first one's stream, which
+// its owner may be capturing.
+void captured_neighbour()
+{
+    Scene a(128, 128, 128, 12);
+    fdtd_options o;
+    fdtd_options_default(&o);
+    hipStream_t st = new_stream();
+    o.stream = st;
+    fdtd_handle *h[2] = {nullptr, nullptr};
+    CHECK(fdtd_create(&a.sc, &o, &h[0]) == FDTD_OK);
+    CHECK(fdtd_create(&a.sc, nullptr, &h[1]) == FDTD_OK);
+    CHECK(fdtd_step(h[0], 64) == FDTD_OK);
+    forget();
+    (void)hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed);
+    CHECK(fdtd_step(h[1], 64) == FDTD_OK);
+    hipGraph_t g = nullptr;
+    (void)hipStreamEndCapture(st, &g);
+    bool waited = false;
+    for (const Call &c : g_log) {
+        if (c.stream == stream_of(st)) bad("%s on the other handle's stream", c.what.c_str());
+        waited = waited || c.what == "wait";
+    }
+    CHECK(waited && count("resident") == 1);
+    CHECK((clocks() == std::vector<long long>{64, 64}));
+    for (fdtd_handle *x : h) CHECK(fdtd_destroy(x) == FDTD_OK);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -593,6 +631,7 @@ const Scenario kScenarios[] = {
     {"no_memory_for_lists", no_memory_for_lists},
     {"no_pinned_memory", no_pinned_memory},
     {"other_device", other_device},
+    {"captured_neighbour", captured_neighbour},
 };
 
 }  // namespace

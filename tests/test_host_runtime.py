@@ -17,6 +17,7 @@ SCENARIOS = [
     "no_memory_for_lists",   # no device memory while scenes are listed anew
     "no_pinned_memory",      # nor pinned memory for listener rows
     "other_device",          # reads while another device is selected
+    "captured_neighbour",    # blocks of two handles, one stream under capture
 ]
 
 
