@@ -120,7 +120,9 @@ fdtd_status BatchRunner::list_whole(hipStream_t st)
 
 fdtd_status BatchRunner::settle(hipStream_t st)
 {
+    const uint64_t seq = resident_seq();
     FDTD_HIP_TRY(hipStreamSynchronize(st));
+    resident_idle(st, seq);
     bool gave_up = false;
     for (const ResidentProgram &p : res_prog) {
         if (p.trouble && *p.trouble > 1) { set_last_error("a resident launch lost its neighbours"); return FDTD_ERR_DEVICE; }

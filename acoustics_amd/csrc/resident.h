@@ -130,6 +130,7 @@ struct ResidentScene {
 struct ResidentProgram {
     ResItem *items = nullptr;   // device
     int n = 0, shape = RES_FINE;
+    int room = 0;               // workgroups of the shape that the device holds
     uint32_t tag = 1;
     int *trouble = nullptr;     // pinned host memory: see launch_resident
     int wait_limit = 0;
@@ -146,6 +147,11 @@ struct ResidentProgram {
 // Step that a scene's clock is at; one that gave up gets its target back and its
 // gate shut, for the step kernels to go on from there (the stream idle).
 fdtd_status resident_reopen(const SceneDev &dev, long long *step);
+
+// After a wait for a stream: what had been launched on it when resident_seq was
+// called, before the wait, runs no more.
+uint64_t resident_seq();
+void resident_idle(hipStream_t st, uint64_t seq);
 
 // Call before a stream that had resident launches goes away, with it idle.
 void resident_forget_stream(hipStream_t st);

@@ -373,7 +373,7 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
     // Workgroups are dispatched in list order, and a scene starts when all of
     // its own are on the device: scenes that fill the device together stand
     // next to each other (largest first, each into the first group with room).
-    const int room = resident_capacity(shape);
+    room = resident_capacity(shape);
     std::vector<const ResidentScene *> order(scenes);
     std::stable_sort(order.begin(), order.end(), [](const ResidentScene *a, const ResidentScene *b) {
         return a->plan.tiles.size() > b->plan.tiles.size();
@@ -416,30 +416,60 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
 }
 
 // Two resident launches on different streams could each hold a part of the
-// device and wait for the rest of it until both give up.  So launches of one
-// process follow each other on a device: each leaves an event, and one on another
-// stream waits for that.  The event is the launch's own completion (64^3, blocks
-// of 4 steps: 27 us a block; recorded behind it 30, without one 26).  A caller's
-// stream may be under capture by then, where the runtime refuses to wait for its
-// earlier events, and touching one spoils the capture: a stream that nobody else
-// knows waits for a launch on such a stream at once, and leaves the event.
+// device and wait for the rest of it until both give up.  So those of one process
+// that do not fit a device together follow each other there: each leaves an event,
+// and a launch that does not fit beside all that other streams may still have
+// running waits for them.  (Two tile shapes do not share a device by a count of
+// workgroups, so they follow each other too.)  The event is the launch's own
+// completion (64^3, blocks of 4 steps: 27 us a block; recorded behind it 30,
+// without one 26).  A caller's stream may be under capture by then, where the
+// runtime refuses to wait for its earlier events, and touching one spoils the
+// capture: a stream that nobody else knows waits for a launch on such a stream at
+// once, and leaves the event.
 namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_order;
-struct Last {
-    hipEvent_t done = nullptr;      // left on `stream`, or, if that is a caller's, on relay
-    hipEvent_t handed = nullptr;    // from a caller's stream to relay
-    hipStream_t relay = nullptr;
+uint64_t g_seq = 0;
+// what a stream may still have running
+struct Flight {
     hipStream_t stream = nullptr;
-    bool used = false;
-} g_last[kMaxDevices];
+    hipEvent_t done = nullptr;      // of its last launch; left on `stream`, or, if that is a caller's, on the relay
+    hipEvent_t handed = nullptr;    // from a caller's stream to the relay
+    int n = 0, shape = -1;          // workgroups of its largest launch (0: idle); -1: of several shapes
+    bool covered = false;           // another stream's launch waits for it: whoever waits for that waits for this
+    uint64_t seq = 0;
+};
+struct Order {
+    hipStream_t relay = nullptr;
+    std::vector<Flight> flights;
+} g_order_of[kMaxDevices];
 }  // namespace
+
+uint64_t resident_seq()
+{
+    std::lock_guard<std::mutex> lk(g_order);
+    return g_seq;
+}
+
+void resident_idle(hipStream_t st, uint64_t seq)
+{
+    std::lock_guard<std::mutex> lk(g_order);
+    for (Order &o : g_order_of)
+        for (Flight &f : o.flights)
+            if (f.stream == st && f.seq <= seq) f.n = 0;
+}
 
 void resident_forget_stream(hipStream_t st)
 {
     std::lock_guard<std::mutex> lk(g_order);
-    for (Last &l : g_last)
-        if (l.used && l.stream == st) l.used = false;
+    for (Order &o : g_order_of)
+        for (size_t q = 0; q < o.flights.size();) {
+            Flight &f = o.flights[q];
+            if (f.stream != st) { ++q; continue; }
+            if (f.done) (void)hipEventDestroy(f.done);
+            if (f.handed) (void)hipEventDestroy(f.handed);
+            o.flights.erase(o.flights.begin() + (ptrdiff_t)q);
+        }
 }
 
 fdtd_status resident_reopen(const SceneDev &dev, long long *step)
@@ -462,21 +492,41 @@ fdtd_status ResidentProgram::enqueue(hipStream_t st, int nsteps)
     int dev = 0;
     FDTD_HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= kMaxDevices) return FDTD_ERR_DEVICE;
-    Last &last = g_last[dev];
-    if (!last.done) {
-        FDTD_HIP_TRY(hipEventCreateWithFlags(&last.handed, hipEventDisableTiming));
-        FDTD_HIP_TRY(hipStreamCreateWithFlags(&last.relay, hipStreamNonBlocking));
-        FDTD_HIP_TRY(hipEventCreateWithFlags(&last.done, hipEventDisableTiming));
+    Order &order = g_order_of[dev];
+    size_t own = 0;
+    while (own < order.flights.size() && order.flights[own].stream != st) ++own;
+    if (own == order.flights.size()) {
+        Flight f;
+        f.stream = st;
+        FDTD_HIP_TRY(hipEventCreateWithFlags(&f.done, hipEventDisableTiming));
+        FDTD_HIP_TRY(hipEventCreateWithFlags(&f.handed, hipEventDisableTiming));
+        if (!order.relay) FDTD_HIP_TRY(hipStreamCreateWithFlags(&order.relay, hipStreamNonBlocking));
+        order.flights.push_back(f);
     }
-    if (last.used && last.stream != st) FDTD_HIP_TRY(hipStreamWaitEvent(st, last.done, 0));
-    FDTD_HIP_TRY(launch_resident(shape, items, n, nsteps, tag, wait_limit, trouble, st, callers_stream ? last.handed : last.done));
+    int together = n;
+    bool fits = true;
+    for (const Flight &f : order.flights)
+        if (f.stream != st && f.n) {
+            together += f.n;
+            fits = fits && f.shape == shape;
+        }
+    if (!fits || together > room)
+        for (Flight &f : order.flights)
+            if (f.stream != st && f.n && !f.covered) {
+                FDTD_HIP_TRY(hipStreamWaitEvent(st, f.done, 0));
+                f.covered = true;
+            }
+    Flight &f = order.flights[own];
+    FDTD_HIP_TRY(launch_resident(shape, items, n, nsteps, tag, wait_limit, trouble, st, callers_stream ? f.handed : f.done));
     tag += (uint32_t)nsteps + 1;
+    f.shape = f.n && f.shape != shape ? -1 : shape;
+    f.n = std::max(f.n, n);
+    f.covered = false;
+    f.seq = ++g_seq;
     if (callers_stream) {
-        FDTD_HIP_TRY(hipStreamWaitEvent(last.relay, last.handed, 0));
-        FDTD_HIP_TRY(hipEventRecord(last.done, last.relay));
+        FDTD_HIP_TRY(hipStreamWaitEvent(order.relay, f.handed, 0));
+        FDTD_HIP_TRY(hipEventRecord(f.done, order.relay));
     }
-    last.stream = st;
-    last.used = true;
     return FDTD_OK;
 }
 

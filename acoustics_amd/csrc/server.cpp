@@ -159,6 +159,7 @@ fdtd_status fdtd_server::run_block()
 // are where their clocks say and go on with the step kernels.
 fdtd_status fdtd_server::settle()
 {
+    resident_idle(stream, resident_seq());   // (nobody else launches on it)
     bool gave_up = false;
     for (const ResidentProgram &p : res_prog) {
         if (p.trouble && *p.trouble > 1) return FDTD_ERR_DEVICE;

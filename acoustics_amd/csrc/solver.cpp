@@ -203,7 +203,9 @@ fdtd_status fdtd_destroy(fdtd_handle *h)
 // run them, and the scene from then on.
 static fdtd_status settle(fdtd_handle *h)
 {
+    const uint64_t seq = resident_seq();
     FDTD_HIP_TRY(hipStreamSynchronize(h->stream));
+    resident_idle(h->stream, seq);
     if (!h->res_prog.trouble || *h->res_prog.trouble == 0) return FDTD_OK;
     if (*h->res_prog.trouble > 1) { set_last_error("a resident launch lost its neighbours"); return FDTD_ERR_DEVICE; }
     *h->res_prog.trouble = 0;

@@ -622,6 +622,28 @@ void captured_neighbour()
     for (fdtd_handle *x : h) CHECK(fdtd_destroy(x) == FDTD_OK);
 }
 
+// Blocks that fit the device together wait for nothing on other streams; one that does
+// not fit beside them waits for them, and for none that have been waited for by the host.
+void side_by_side()
+{
+    Scene a(64, 64, 64, 10), b(128, 128, 128, 12);
+    fdtd_handle *h[5];
+    for (int i = 0; i < 5; ++i) CHECK(fdtd_create(i < 4 ? &a.sc : &b.sc, nullptr, &h[i]) == FDTD_OK);
+    auto waits = [&](int i) {
+        forget();
+        CHECK(fdtd_step(h[i], 64) == FDTD_OK && count("resident") == 1);
+        return count("wait");
+    };
+    for (int i = 0; i < 3; ++i) CHECK(waits(i) == 0);
+    CHECK(waits(0) == 0 && waits(2) == 0);
+    CHECK(waits(3) == 3);                       // 4 x 208 workgroups of 768
+    CHECK(waits(4) == 1);                       // of the other shape: behind the one that waited for all
+    CHECK(waits(1) == 1);
+    for (fdtd_handle *x : h) CHECK(fdtd_synchronize(x) == FDTD_OK);
+    CHECK(waits(3) == 0 && waits(0) == 0 && waits(4) == 2);
+    for (fdtd_handle *x : h) CHECK(fdtd_destroy(x) == FDTD_OK);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -632,6 +654,7 @@ const Scenario kScenarios[] = {
     {"no_pinned_memory", no_pinned_memory},
     {"other_device", other_device},
     {"captured_neighbour", captured_neighbour},
+    {"side_by_side", side_by_side},
 };
 
 }  // namespace

@@ -18,6 +18,7 @@ SCENARIOS = [
     "no_pinned_memory",      # nor pinned memory for listener rows
     "other_device",          # reads while another device is selected
     "captured_neighbour",    # blocks of two handles, one stream under capture
+    "side_by_side",          # blocks of several handles
 ]
 
 
