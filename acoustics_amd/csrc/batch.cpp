@@ -262,7 +262,10 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
             if (s != FDTD_OK) return s;
         }
         const int want = (int)std::min<long long>(left, remaining);
-        if (any_resident() && capturing(st)) {
+        int least = 0;
+        for (const ResidentProgram &p : res_prog) least = std::max(least, p.least());
+        // (a longer call's last steps are not worth listing the step kernels for)
+        if (any_resident() && (nsteps < least || capturing(st))) {
             if (!whole_listed) {
                 const fdtd_status s = list_whole(st);
                 if (s != FDTD_OK) return s;
@@ -275,7 +278,7 @@ fdtd_status BatchRunner::advance(hipStream_t st, int nsteps)
         } else if (any_resident()) {
             // the step kernels of the other scenes, then the block of the
             // resident ones, then every scene's clock
-            const int blk = std::min(want, (int)AMP_ROWS);
+            const int blk = want <= AMP_ROWS ? want : want < AMP_ROWS + least ? want / 2 : (int)AMP_ROWS;
             for (int k = 0; k < blk && prog_tiles > 0; ++k) {
                 const fdtd_status s = prog.enqueue_step(st, taken + k, k, blk);
                 if (s != FDTD_OK) return s;

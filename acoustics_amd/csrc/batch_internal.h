@@ -36,9 +36,9 @@ struct BatchRunner {
     ResidentProgram res_prog[RES_SHAPES];
     SeriesStage stage;
     bool res_listed = false;
-    // every scene's step kernels, for steps enqueued while the stream is
-    // captured: a resident launch's tags are its own, and a replay would take
-    // the words of the replay before for its neighbours'
+    // every scene's step kernels, for calls of a few steps, and for steps enqueued
+    // while the stream is captured: a resident launch's tags are its own, and a
+    // replay would take the words of the replay before for its neighbours'
     StepProgram whole;
     bool whole_listed = false;
     bool listed = false;                              // prog and the resident launches hold the scenes as they are

@@ -126,6 +126,13 @@ struct ResidentScene {
     void release();
 };
 
+// Steps from which a launch beats the step kernels: it loads and stores the whole
+// state, once for each time its workgroups fill the device (`rounds`).  us per
+// block, launched resident and by step kernels: 64^3 18 + 2 a step and 6.5 a step;
+// 128^3 40 + 4 and 13; 144x144x144 45 + 8 and 14, and four of them in a batch 250 +
+// 38 and 47; eight of 64^3 45 + 6 and 20.
+inline int resident_least(int shape, int rounds) { return shape == RES_LARGE ? 8 * rounds : 4; }
+
 // The launches of a set of resident scenes.
 struct ResidentProgram {
     ResItem *items = nullptr;   // device
@@ -141,6 +148,7 @@ struct ResidentProgram {
     fdtd_status upload(const std::vector<const ResidentScene *> &scenes, hipStream_t st);
     fdtd_status enqueue(hipStream_t st, int nsteps);
     bool gave_up() const { return trouble && *trouble != 0; }
+    int least() const { return n > 0 ? resident_least(shape, (n + room - 1) / room) : 0; }
     void release();
 };
 

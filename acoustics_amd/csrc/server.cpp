@@ -236,8 +236,12 @@ void fdtd_server::run()
             r->dev = std::make_unique<DeviceScene>();
             r->dev->S = std::move(r->setup);
             fdtd_status s = r->dev->allocate_and_upload(upload, std::max(1, r->steps), r->steps);
-            // resident where it fits the device and the budget
-            if (s == FDTD_OK && r->res.build(*r->dev, upload, (size_t)std::max<int64_t>(0, opt.hbm_budget_bytes - resident))) {
+            // resident where it fits the device and the budget, and the blocks are long enough
+            // for it among a few others
+            if (s == FDTD_OK && r->res.build(*r->dev, upload, (size_t)std::max<int64_t>(0, opt.hbm_budget_bytes - resident)) &&
+                block < resident_least(r->res.plan.shape, 4))
+                r->res.release();
+            if (s == FDTD_OK && r->res.mem) {
                 std::lock_guard<std::mutex> lk(mu);
                 r->bytes += r->res.bytes;
                 resident += (int64_t)r->res.bytes;

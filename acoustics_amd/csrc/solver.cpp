@@ -272,10 +272,6 @@ static fdtd_status build_graph(fdtd_handle *h)
     return FDTD_OK;
 }
 
-// Fewer steps than this run as step kernels: a resident launch loads and
-// stores the whole state.
-constexpr int kResidentSteps = 4;
-
 // Brings the device clock up to the steps run one by one.
 static fdtd_status catch_up(fdtd_handle *h)
 {
@@ -344,7 +340,7 @@ fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
                 if (st != FDTD_OK) return st;
             }
             FDTD_HIP_TRY(hipGraphLaunch(h->graph_exec, h->stream));
-        } else if (h->res_prog.n > 0 && !per_step && block >= kResidentSteps && !capturing(h->stream)) {
+        } else if (h->res_prog.n > 0 && !per_step && block >= h->res_prog.least() && !capturing(h->stream)) {
             fdtd_status st = h->res_prog.enqueue(h->stream, block);
             if (st != FDTD_OK) return st;
             FDTD_HIP_TRY(launch_advance(h->D.self, 1, block, h->stream));

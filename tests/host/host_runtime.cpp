@@ -644,6 +644,52 @@ void side_by_side()
     for (fdtd_handle *x : h) CHECK(fdtd_destroy(x) == FDTD_OK);
 }
 
+// Blocks too short to pay for a resident launch's load and store of the state are step kernels.
+void short_blocks()
+{
+    Scene a(40, 40, 40, 6), b(44, 40, 40, 6), c(144, 146, 144, 8);   // the third one in the largest tiles
+    auto resident = [&](auto step) {
+        forget();
+        CHECK(step() == FDTD_OK);
+        return count("resident") > 0;
+    };
+    {
+        const fdtd_scene sc[2] = {a.sc, b.sc};
+        const int steps[2] = {600, 601};
+        fdtd_batch *h = nullptr;
+        CHECK(fdtd_batch_create(sc, steps, 2, nullptr, &h) == FDTD_OK);
+        CHECK(!resident([&] { return fdtd_batch_step(h, 1); }) && count("step") >= 1);
+        CHECK(!resident([&] { return fdtd_batch_step(h, 3); }) && count("step") >= 3);
+        CHECK(resident([&] { return fdtd_batch_step(h, 4); }));
+        CHECK(!resident([&] { return fdtd_batch_step(h, 2); }));
+        CHECK((clocks() == std::vector<long long>{10, 10}));
+        // a long call's remainder joins its last blocks
+        CHECK(resident([&] { return fdtd_batch_step(h, 258); }) && count("step") == 0 && count("resident") == 2);
+        CHECK(resident([&] { return fdtd_batch_run(h); }) && count("step") == 0);
+        CHECK(fdtd_batch_destroy(h) == FDTD_OK);
+    }
+    {
+        fdtd_handle *h = nullptr;
+        CHECK(fdtd_create(&c.sc, nullptr, &h) == FDTD_OK);
+        CHECK(!resident([&] { return fdtd_step(h, 7); }));
+        CHECK(resident([&] { return fdtd_step(h, 8); }));
+        CHECK(fdtd_destroy(h) == FDTD_OK);
+    }
+    for (int block : {2, 16}) {
+        fdtd_server_options o;
+        fdtd_server_options_default(&o);
+        o.steps_per_block = block;
+        fdtd_server *s = nullptr;
+        int64_t id;
+        CHECK(fdtd_server_create(&o, &s) == FDTD_OK);
+        CHECK(resident([&] {
+            const fdtd_status st = fdtd_server_submit(s, block == 2 ? &a.sc : &c.sc, 40, &id);
+            return st == FDTD_OK ? fdtd_server_wait(s, id, 60000) : st;
+        }) == false);
+        CHECK(fdtd_server_destroy(s) == FDTD_OK);
+    }
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -655,6 +701,7 @@ const Scenario kScenarios[] = {
     {"other_device", other_device},
     {"captured_neighbour", captured_neighbour},
     {"side_by_side", side_by_side},
+    {"short_blocks", short_blocks},
 };
 
 }  // namespace

@@ -19,6 +19,7 @@ SCENARIOS = [
     "other_device",          # reads while another device is selected
     "captured_neighbour",    # blocks of two handles, one stream under capture
     "side_by_side",          # blocks of several handles
+    "short_blocks",          # blocks of a few steps
 ]
 
 
