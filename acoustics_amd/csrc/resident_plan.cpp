@@ -403,10 +403,13 @@ fdtd_status ResidentProgram::upload(const std::vector<const ResidentScene *> &sc
         *trouble = 0;
     }
     if (!wait_limit) {
-        // about a second; another launch that holds the device for longer
-        // sends this one's scenes to the step kernels
+        // 7 ms, three times the longest block (256 steps of 9 us); whatever holds
+        // the device for longer, another process's launch for one, sends this
+        // one's scenes to the step kernels. With 230 ms, three processes that
+        // solve 1000 steps at 128^3 each took 230 to 480 ms for them instead of the
+        // step kernels' 16 to 44.
         const char *w = std::getenv("FDTD_RESIDENT_WAIT");
-        wait_limit = w ? std::atoi(w) : 1 << 20;
+        wait_limit = w ? std::atoi(w) : 1 << 15;
     }
     FDTD_HIP_TRY(hipMalloc(&items, sizeof(ResItem) * list.size()));
     FDTD_HIP_TRY(hipMemcpyAsync(items, list.data(), sizeof(ResItem) * list.size(), hipMemcpyHostToDevice, st));

@@ -18,6 +18,11 @@ namespace fdtd {
 const std::string &get_last_error();
 }
 
+// Steps that a handle runs by step kernels after its block was given up, before
+// it tries again: the 7 ms that a try may wait are a tenth of them. Twice as many
+// after each further one.
+constexpr long long kResidentPause = 8192;
+
 struct fdtd_handle {
     DeviceScene D;
     StepProgram prog;
@@ -25,6 +30,8 @@ struct fdtd_handle {
     // step kernels run single steps, and the whole scene elsewhere)
     ResidentScene res;
     ResidentProgram res_prog;
+    long long res_from = 0;      // step from which blocks run resident (again)
+    long long res_pause = kResidentPause;
     hipStream_t stream = nullptr;
     bool own_stream = false;
     int tile = 0;
@@ -200,7 +207,7 @@ fdtd_status fdtd_destroy(fdtd_handle *h)
 
 // Waits for the stream and completes steps that a resident launch gave up
 // (its workgroups could not all be on the device at once): the step kernels
-// run them, and the scene from then on.
+// run them, and the scene for a while from then on.
 static fdtd_status settle(fdtd_handle *h)
 {
     const uint64_t seq = resident_seq();
@@ -209,7 +216,8 @@ static fdtd_status settle(fdtd_handle *h)
     if (!h->res_prog.trouble || *h->res_prog.trouble == 0) return FDTD_OK;
     if (*h->res_prog.trouble > 1) { set_last_error("a resident launch lost its neighbours"); return FDTD_ERR_DEVICE; }
     *h->res_prog.trouble = 0;
-    h->res_prog.n = 0;
+    h->res_from = h->step + h->res_pause;
+    h->res_pause *= 2;
     h->lead = 0;   // (what was enqueued behind it has not run)
     long long at = 0;
     {
@@ -340,7 +348,7 @@ fdtd_status fdtd_step(fdtd_handle *h, int nsteps)
                 if (st != FDTD_OK) return st;
             }
             FDTD_HIP_TRY(hipGraphLaunch(h->graph_exec, h->stream));
-        } else if (h->res_prog.n > 0 && !per_step && block >= h->res_prog.least() && !capturing(h->stream)) {
+        } else if (h->res_prog.n > 0 && h->step >= h->res_from && !per_step && block >= h->res_prog.least() && !capturing(h->stream)) {
             fdtd_status st = h->res_prog.enqueue(h->stream, block);
             if (st != FDTD_OK) return st;
             FDTD_HIP_TRY(launch_advance(h->D.self, 1, block, h->stream));

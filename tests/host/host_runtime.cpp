@@ -75,6 +75,7 @@ struct Block { size_t n; int dev; };
 std::map<char *, Block> g_mem;
 long g_fail_malloc = -1;        // device allocations left before one fails (-1: none does)
 bool g_fail_pinned = false;
+int g_patience = 0;             // the last resident launch's wait limit
 
 // what the resident kernel does
 std::function<bool(const SceneDev &)> g_gives_up = [](const SceneDev &) { return false; };
@@ -210,6 +211,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **a, size_t, hipStr
         const int n = (int)g.x, steps = arg<int>(a, 1);
         int *trouble = arg<int *>(a, 4);
         for (const ResScene *r : scenes_of(items, n)) g_log.push_back({"resident scene", s, s->capturing, r->S->clock});
+        g_patience = arg<int>(a, 3);
         if (s->capturing) bad("a resident launch is recorded in a graph");
         run = [=] { run_resident(items, n, steps, trouble); };
     } else if (is("sum_terms_kernel")) {
@@ -690,6 +692,40 @@ void short_blocks()
     }
 }
 
+// A handle whose block was given up, because something else held the device, runs
+// step kernels for a while and then tries again, after longer and longer whiles.
+void tries_again()
+{
+    Scene a(40, 40, 40, 6);
+    fdtd_handle *h = nullptr;
+    CHECK(fdtd_create(&a.sc, nullptr, &h) == FDTD_OK);
+    std::vector<double> out(2);
+    g_gives_up = [](const SceneDev &) { return true; };
+    long long last = 0, pause = 0;
+    int tries = 0;
+    for (long long s = 0; s < 200000; s += 250) {
+        forget();
+        CHECK(fdtd_step(h, 250) == FDTD_OK && fdtd_listen(h, out.data()) == FDTD_OK);
+        CHECK(clocks() == std::vector<long long>{s + 250});
+        if (!count("resident")) continue;
+        if (tries) {
+            CHECK(s - last >= 8000 && s - last >= 2 * pause - 500);
+            pause = s - last;
+        }
+        last = s;
+        ++tries;
+    }
+    CHECK(tries >= 3 && tries <= 6);
+    g_gives_up = [](const SceneDev &) { return false; };
+    CHECK(fdtd_step(h, 400000) == FDTD_OK);
+    forget();
+    CHECK(fdtd_step(h, 250) == FDTD_OK);
+    CHECK(count("resident") == 1 && count("step") == 0);
+    // not more than some hundredths of a second (a spin takes 0.2 us)
+    CHECK(g_patience > 0 && g_patience <= 1 << 16);
+    CHECK(fdtd_destroy(h) == FDTD_OK);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -702,6 +738,7 @@ const Scenario kScenarios[] = {
     {"captured_neighbour", captured_neighbour},
     {"side_by_side", side_by_side},
     {"short_blocks", short_blocks},
+    {"tries_again", tries_again},
 };
 
 }  // namespace

@@ -20,6 +20,7 @@ SCENARIOS = [
     "captured_neighbour",    # blocks of two handles, one stream under capture
     "side_by_side",          # blocks of several handles
     "short_blocks",          # blocks of a few steps
+    "tries_again",           # a handle that gave a block up
 ]
 
 
