@@ -340,7 +340,7 @@ typedef struct fdtd_handle fdtd_handle;
  * write every pDir_d and velocity).  MERGED also applies to the staggered
  * scheme on grids of up to 3 million cells: its PML cells merge the same way,
  * and a cell outside the PML keeps the increment of its pressure instead of
- * three face velocities (16 B instead of 32).  Such a handle's first snapshot,
+ * three face velocities (16 B instead of 32); no less accurate on average.  Such a handle's first snapshot,
  * saved or loaded, takes it to SPLIT for good: the steps so far are run again,
  * so that the files hold every velocity.  Larger staggered grids are SPLIT. */
 enum {
