@@ -454,7 +454,7 @@ fdtd_status fdtd_get_info(fdtd_handle *h, fdtd_info *o)
     for (long long q = 0; q < h->step; ++q) t += S.dt;
     o->time = t;
     o->bytes_per_step = algorithmic_bytes(S);
-    o->device_bytes = (int64_t)h->D.arena_bytes;
+    o->device_bytes = (int64_t)(h->D.arena_bytes + h->res.bytes);
     o->n_pml_merged_cells = S.n_pml_merged;
     o->state_bytes_per_step = state_bytes(S);
     return FDTD_OK;

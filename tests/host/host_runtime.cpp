@@ -726,6 +726,20 @@ void tries_again()
     CHECK(fdtd_destroy(h) == FDTD_OK);
 }
 
+// The device memory that a handle reports holds its resident tables too.
+void device_bytes()
+{
+    Scene a(64, 64, 64, 10);
+    fdtd_handle *h = nullptr;
+    CHECK(fdtd_create(&a.sc, nullptr, &h) == FDTD_OK);
+    fdtd_info o;
+    CHECK(fdtd_get_info(h, &o) == FDTD_OK);
+    size_t held = 0;
+    for (const auto &e : g_mem) held += e.second.n;
+    CHECK((size_t)o.device_bytes <= held && o.device_bytes >= 0.95 * (double)held);   // (the launch lists are not counted)
+    CHECK(fdtd_destroy(h) == FDTD_OK);
+}
+
 struct Scenario { const char *name; void (*run)(); };
 const Scenario kScenarios[] = {
     {"batch_capture", batch_capture},
@@ -739,6 +753,7 @@ const Scenario kScenarios[] = {
     {"side_by_side", side_by_side},
     {"short_blocks", short_blocks},
     {"tries_again", tries_again},
+    {"device_bytes", device_bytes},
 };
 
 }  // namespace

@@ -21,6 +21,7 @@ SCENARIOS = [
     "side_by_side",          # blocks of several handles
     "short_blocks",          # blocks of a few steps
     "tries_again",           # a handle that gave a block up
+    "device_bytes",          # what fdtd_get_info says of it
 ]
 
 
